@@ -9,9 +9,9 @@
 #include <string.h>
 
 #include <mutex>
+#include <vector>
 
-#include "hot_device.h"
-#include "hot_host.h"
+#include "phase.h"
 
 namespace hot {
 
@@ -59,8 +59,8 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 static BwdLayout bwd_layout(int64_t L, int64_t O, int64_t I, const hot_config* c) {
   BwdLayout b;
   const int64_t lp = (L / c->hla_n) * c->hla_r;
-  b.ld_g = round_up(O, GEMM_KTILE) * c->gx_bits / 8;
-  b.ld_w = round_up(O, GEMM_KTILE) * c->w_bits / 8;
+  b.ld_g = round_up(O * c->gx_bits / 8, 128);      // whole 128-byte lines (what is past O is zero)
+  b.ld_w = round_up(O * c->w_bits / 8, 128);
   b.ld_gp = round_up(lp, GEMM_KTILE);
   size_t o = 0;
   b.off_hq = o;   o += STAT_SLOT_BYTES;
@@ -72,7 +72,7 @@ static BwdLayout bwd_layout(int64_t L, int64_t O, int64_t I, const hot_config* c
   b.off_qg = o;   o += align256((size_t)L * b.ld_g);
   b.off_qw = o;   o += align256((size_t)I * b.ld_w);
   b.off_qgp = o;  o += align256((size_t)O * b.ld_gp);
-  const GemmSplit px = gemm_split_plan(L, I, O, c->gx_bits), pw = gemm_split_plan(O, I, lp, 8);
+  const GemmSplit px = gemm_split_plan(L, I, b.ld_g * 8 / c->gx_bits, c->gx_bits), pw = gemm_split_plan(O, I, lp, 8);
   b.split_bytes = px.ws_bytes > pw.ws_bytes ? px.ws_bytes : pw.ws_bytes;
   b.off_split = o; o += align256(b.split_bytes);
   {  // the workspace query knows no input type: room for the larger partition of the two element sizes
@@ -85,20 +85,10 @@ static BwdLayout bwd_layout(int64_t L, int64_t O, int64_t I, const hot_config* c
   return b;
 }
 
-__global__ void clear3_kernel(uint32_t* p0, int n0, uint32_t* p1, int n1, uint32_t* p2, int n2) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n0) { p0[i] = 0u; return; }
-  i -= n0;
-  if (i < n1) { p1[i] = 0u; return; }
-  i -= n1;
-  if (i < n2) p2[i] = 0u;
-}
-
-// One stream or two.  Forking and joining the side stream costs the host three event record / wait
-// pairs, about 60 us on top of the 23 us the ten launches take (measured); that is hidden only when
-// the kernels of the call run longer than it.  Calls with little arithmetic (both products together
-// below 30 GOP: ViT-B proj at 12608 tokens, 23 GOP, runs 75 us on one stream against 85 us with the
-// side stream; qkv, 70 GOP, 123 against 108) keep everything on the caller's stream.
+// One stream or two.  The transform + quantise work is two launches either way; the second stream carries the g_x
+// product beside the g_W product.  Forking and joining it costs the host two event record / wait pairs, 21 us
+// (measured), which only long calls hide: calls with little arithmetic (both products together below 30 GOP, e.g.
+// ViT-B proj at 12608 tokens) keep everything on the caller's stream.
 static int backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* c) {
   if (c->streams == 1 || c->streams == 2) return c->streams;
   const double lp = (double)((L / c->hla_n) * c->hla_r);
@@ -111,6 +101,9 @@ static const int32_t* identity_rows() {
   static const Rows rows;   // initialised once, thread-safe
   return rows.v;
 }
+
+// Whether W's job shares the launches of a phase (Hadamard blocks of up to 16; with stochastic rounding of 16).
+static bool w_joins_phase(const hot_config* c) { return c->w_round == HOT_ROUND_STOCH ? c->n_o == CW_ROWS : c->n_o <= CW_ROWS; }
 
 }  // namespace hot
 
@@ -228,13 +221,14 @@ enum {
   K_GEMM_GW = 7,
   K_COUNT = 8
 };
+// Slots of the stage timing (hot_linear_backward with times4)
+enum { STAGE_STATS = 0, STAGE_QUANT = 1, STAGE_GEMM = 2, STAGE_COUNT = 3 };
 
-// The two W kernels are small (a few MB) and cannot fill the chip; they run on a side stream beside
-// the g_y kernels.  One side stream and three events per device, created on first use (default
+// The side stream of the g_x product.  One per device with its two events, created on first use (default
 // priority) and kept for the life of the process; a mutex keeps the fork / join of one call together.
 struct SideLane {
   hipStream_t stream = nullptr;
-  hipEvent_t fork = nullptr, fork2 = nullptr, join = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
   bool tried = false, ok = false;
 };
 static std::mutex g_side_mutex;
@@ -248,17 +242,23 @@ static SideLane* side_lane_locked() {
     s.tried = true;
     s.ok = hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess &&
            hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) == hipSuccess &&
-           hipEventCreateWithFlags(&s.fork2, hipEventDisableTiming) == hipSuccess &&
            hipEventCreateWithFlags(&s.join, hipEventDisableTiming) == hipSuccess;
     if (!s.ok) (void)hipGetLastError();
   }
   return s.ok ? &s : nullptr;
 }
 
+// Events recorded along a timed call: event i + 1 follows the i-th group of launches, slot_of[i] names the group.
+struct Marks {
+  hipEvent_t* ev;
+  int* slot_of;
+  bool split;        // one group per kernel (every job launched on its own) instead of one per stage
+  int seq = 0;
+};
+
 static int run_backward(const void* gy, const void* w, int dtype, const void* xq, const float* sx, int64_t L,
                         int64_t O, int64_t I, const hot_config* cfg, void* gx, void* gw, int out_dtype,
-                        void* workspace, size_t workspace_bytes, hipEvent_t* ev /* K_COUNT + 1 or null */,
-                        int* slot_of /* K_COUNT: kernel group measured by event pair i, i + 1 */, hipStream_t st,
+                        void* workspace, size_t workspace_bytes, Marks* marks, hipStream_t st,
                         void* gb = nullptr /* [O] of out_dtype: column sums of g_y, or null */) {
   const char* who = "hot_linear_backward";
   if (int e = check_cfg(cfg, who)) return e;
@@ -284,166 +284,203 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   float* sw = (float*)(ws + b.off_sw);
   float* sgp = (float*)(ws + b.off_sgp);
   const int64_t lp = (L / cfg->hla_n) * cfg->hla_r;
-  // timing: event i + 1 is recorded after the i-th kernel group of the launch order; slot_of[i] names it
-  int seq = 0;
+  if (marks) (void)hipEventRecord(marks->ev[0], st);
   auto mark = [&](int slot) {
-    if (!ev) return;
-    slot_of[seq] = slot;
-    (void)hipEventRecord(ev[++seq], st);
+    if (!marks) return;
+    marks->slot_of[marks->seq] = slot;
+    (void)hipEventRecord(marks->ev[++marks->seq], st);
   };
-  // event to record between the two kernels of a token-wise call (statistics pass, quantise pass)
-  auto mid = [&](int slot) -> hipEvent_t {
-    if (!ev) return nullptr;
-    slot_of[seq] = slot;
-    return ev[++seq];
-  };
-  if (ev) (void)hipEventRecord(ev[0], st);
-  // one launch zeroes every statistic of the call (absmax slots, per-channel maxima)
-  {
-    const int n0 = (int)(STAT_SLOT_BYTES / 4), n1 = (int)(colwise_stats_bytes_impl(I) / 4), n2 = (int)(colwise_stats_bytes_impl(O) / 4);
-    const int total = n0 + n1 + n2;
-    hipLaunchKernelGGL(clear3_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                       (uint32_t*)(ws + b.off_hq), n0, (uint32_t*)(ws + b.off_colw), n1, (uint32_t*)(ws + b.off_colg), n2);
+  const bool split = marks && marks->split;
+  int rc;
+  // The jobs.  g_y: HLA along tokens + quantise, transposed (g_W operand); Hadamard along O + quantise (g_x operand).
+  // W: Hadamard along O + quantise, stored [I, O].  Blocks of up to 128 tokens and Hadamard blocks of up to 16 share
+  // the launches of the two phases (phase.h); larger ones have kernels of their own.
+  const bool big = cfg->hla_n > COL_MAX_N, w_short = w_joins_phase(cfg);
+  ColJob gj, wj;
+  rc = col_job_impl(wj, w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed, HOT_STREAM_W,
+                    cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw, colwise_workspace_bytes_impl(I), who,
+                    1, 0, false, w_short);
+  if (rc) return rc;
+  // With one step per tensor both quantisers of g_y need the absmax of their transform first: the statistics pass of
+  // the token-wise job delivers both from a single read of g_y.
+  const bool row_tensor = cfg->gx_scale == HOT_SCALE_TENSOR;
+  const bool hq_job = cfg->n_o <= CW_ROWS && (row_tensor ? (!big || (cfg->n_o == 16 && O % 16 == 0)) : O <= HQ_ROW_MAX_K);
+  const bool row_fused = hq_job && row_tensor;
+  float* const slots = (float*)(ws + b.off_hq);
+  if (!big) {
+    rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
+                      HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg, colwise_workspace_bytes_impl(O), who,
+                      1, 0, false, false);
+    if (rc) return rc;
+    if (row_fused) col_job_row_stat(gj, cfg->n_o);
+    if (gb) gj.a.colsum = (float*)(ws + b.off_colsum);
   }
-  mark(K_CLEAR);
-  // W: Hadamard along O + quantise, stored [I, O]
-  auto quantise_w = [&](hipStream_t s2) {
-    return colwise_quant_impl(w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed,
-                              HOT_STREAM_W, cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw,
-                              ws + b.off_colw, colwise_workspace_bytes_impl(I), s2, who, nullptr, /*stats_cleared=*/true,
-                              mid(K_W_STATS));
+  HqArgs hj;
+  if (hq_job) {
+    const float* stat = !row_tensor ? nullptr : big ? slots : gj.a.row_absmax;
+    rc = hq_job_impl(hj, gy, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg, b.ld_g, sg,
+                     stat, big ? STAT_SLOTS : row_tensor ? gj.a.npart : 0, big ? STAT_SLOT_STRIDE : 1, 1);
+    if (rc) return rc;
+  }
+  ColsumArgs sj;
+  if (gb) {
+    sj.partial = (const float*)(ws + b.off_colsum); sj.C = O; sj.out = gb; sj.out_dtype = out_dtype;
+    sj.strips = (int32_t)colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, dtype == HOT_F32 ? 4 : 2);
+  }
+
+  // statistics
+  if (!big) col_job_clear(gj, st);
+  if (split) mark(K_CLEAR);
+  const bool w_joins = w_short && !split;
+  if (!big) {
+    rc = phase_launch(0, dtype, &gj, w_joins ? &wj : nullptr, nullptr, nullptr, st);
+    if (rc) return rc;
+    if (split) mark(K_GY_STATS);
+  } else if (w_joins) {
+    rc = phase_launch(0, dtype, nullptr, &wj, nullptr, nullptr, st);
+    if (rc) return rc;
+  }
+  auto w_alone = [&](int pass) { return w_short ? phase_launch(pass, dtype, nullptr, &wj, nullptr, nullptr, st) : phase_launch(pass, dtype, &wj, nullptr, nullptr, nullptr, st); };
+  if (!w_joins && (rc = w_alone(0))) return rc;
+  if (split) mark(K_W_STATS);
+  if (marks && !split) mark(STAGE_STATS);
+
+  // transform + quantise
+  if (big) {
+    rc = colwise_quant_impl(gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed, HOT_STREAM_GW,
+                            cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg,
+                            hla_workspace_bytes_impl(L, O, cfg->hla_n, cfg->hla_r), st, who, row_fused ? slots : nullptr,
+                            gb ? (float*)(ws + b.off_colsum) : nullptr);
+    if (rc) return rc;
+  }
+  if (split) {
+    if (!big && (rc = phase_launch(1, dtype, &gj, nullptr, nullptr, gb ? &sj : nullptr, st))) return rc;
+    if (big && gb && (rc = colsum_finish_impl(sj, st))) return rc;
+    mark(K_GY_HLA);
+    if (hq_job && (rc = phase_launch(1, dtype, nullptr, nullptr, &hj, nullptr, st))) return rc;
+  } else {
+    rc = phase_launch(1, dtype, big ? nullptr : &gj, w_joins ? &wj : nullptr, hq_job ? &hj : nullptr, gb ? &sj : nullptr, st);
+    if (rc) return rc;
+  }
+  if (!hq_job) {
+    rc = hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg,
+                         b.ld_g, sg, slots, STAT_SLOT_BYTES, st, false);
+    if (rc) return rc;
+  }
+  if (split) mark(K_GY_HQ);
+  if (!w_joins && (rc = w_alone(1))) return rc;
+  if (split) mark(K_W_QUANT);
+  if (marks && !split) mark(STAGE_QUANT);
+
+  // the products: g_x = (qG . qW^T) sG sW / n_o and g_W = (qGp . xq^T) sGp sx / hla_n
+  const GemmProduct px = {ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, b.ld_g * 8 / cfg->gx_bits, sg,
+                          cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, I};
+  const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
+                          1.0f / (float)cfg->hla_n, gw, I};
+  if (!split && cfg->streams != 2 && gemm_pair_possible(pw, px)) {
+    rc = gemm_pair_impl(pw, px, out_dtype, st);
+    if (!rc && marks) mark(STAGE_GEMM);
+    return rc;
+  }
+  auto run_gemm = [&](const GemmProduct& p, hipStream_t s2) {
+    // (no split on the side stream: the split workspace belongs to the g_W product)
+    return gemm_i8_impl(p.A, p.lda, p.B, p.ldb, p.bits, p.M, p.N, p.K, p.scale_a, p.a_per_row, p.scale_b, p.post_scale, p.out, out_dtype,
+                        p.ldo, nullptr, s2, s2 == st && b.split_bytes ? ws + b.off_split : nullptr, s2 == st ? b.split_bytes : 0);
   };
-  // Without per-kernel timing, independent kernels overlap on the side stream: first the W kernels
-  // beside the g_y statistics.
+  // Beside the g_W product when that has fewer tiles than the chip has CUs and cannot fill it alone (two large
+  // products only get in each other's way).
   std::unique_lock<std::mutex> side_guard(g_side_mutex, std::defer_lock);
   SideLane* side = nullptr;
-  if (!ev && backward_streams(L, O, I, cfg) == 2) {
+  if (!marks && backward_streams(L, O, I, cfg) == 2 && ((O + 127) / 128) * ((I + 127) / 128) < 256) {
     side_guard.lock();
     side = side_lane_locked();
     if (!side) side_guard.unlock();
   }
-  // Once the side stream has been forked, every way out of this function joins it again: the
-  // caller's stream waits for what the side stream was given, also when a later stage refuses, so
-  // that no kernel of the call still runs (on the workspace) behind work the caller queues next,
-  // and a capture of the caller's stream is never left with an unjoined branch.
+  // Once the side stream has been forked, every way out of this function joins it again: the caller's stream waits
+  // for what the side stream was given, also when a launch refuses, so that no kernel of the call still runs (on the
+  // workspace) behind work the caller queues next, and a capture of the caller's stream is never left with an unjoined branch.
   struct SideJoin {
     SideLane* side = nullptr;
     hipStream_t st = nullptr;
-    bool forked = false, joined = false;
     ~SideJoin() {
-      if (!forked || joined) return;
+      if (!side) return;
       if (hipEventRecord(side->join, side->stream) == hipSuccess) (void)hipStreamWaitEvent(st, side->join, 0);
     }
   } side_join;
-  int rc = HOT_OK;
   if (side) {
     rc = check_hip(hipEventRecord(side->fork, st), "hipEventRecord");
     if (!rc) rc = check_hip(hipStreamWaitEvent(side->stream, side->fork, 0), "hipStreamWaitEvent");
     if (rc) return rc;
-    side_join.side = side; side_join.st = st; side_join.forked = true;
-    rc = quantise_w(side->stream);
+    side_join.side = side; side_join.st = st;
+    rc = run_gemm(px, side->stream);
     if (rc) return rc;
   }
-  // g_y: HLA along tokens + quantise, transposed (g_W operand); Hadamard along O + quantise (g_x
-  // operand).  With one step per tensor both quantisers need the absmax of their transform first:
-  // the statistics pass of the token-wise kernel delivers both from a single read of g_y.
-  const bool fuse = cfg->gx_scale == HOT_SCALE_TENSOR && cfg->n_o == 16 && O % 16 == 0 && cfg->gw_scale != HOT_SCALE_SAWB;
-  // Side stream, beside the g_W GEMM on the main stream: always the row-wise quantise pass of g_y (a
-  // streaming kernel next to a matrix kernel); the g_x GEMM too when the g_W GEMM has fewer tiles
-  // than the chip has CUs and cannot fill it alone (two large GEMMs only get in each other's way).
-  const bool hq_aside = side != nullptr;
-  const bool gx_aside = side != nullptr && ((O + 127) / 128) * ((I + 127) / 128) < 256;
-  rc = colwise_quant_impl(gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round,
-                          cfg->seed, HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp,
-                          ws + b.off_colg, hla_workspace_bytes_impl(L, O, cfg->hla_n, cfg->hla_r), st, who,
-                          fuse ? (float*)(ws + b.off_hq) : nullptr, /*stats_cleared=*/true,
-                          hq_aside ? side->fork2 : mid(K_GY_STATS), gb ? (float*)(ws + b.off_colsum) : nullptr);
+  rc = run_gemm(pw, st);
   if (rc) return rc;
-  // bias gradient: the partial column sums of the statistics pass, added up by a small kernel that
-  // rides on the side stream behind the row-wise quantise pass, beside the large kernels of the main
-  // stream (here, in order, when there is no side stream)
-  auto finish_bias = [&](hipStream_t s2) {
-    if (!gb) return (int)HOT_OK;
-    const int64_t strips = colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, dtype == HOT_F32 ? 4 : 2);
-    return colsum_finish_impl((const float*)(ws + b.off_colsum), strips, O, gb, out_dtype, s2);
-  };
-  if (!side && (rc = finish_bias(st))) return rc;
-  mark(K_GY_HLA);
-  // g_x operand of g_y on the side stream: a streaming kernel beside the g_W GEMM
-  auto quantise_gy_rows = [&](hipStream_t s2) {
-    return hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX,
-                           cfg->gx_scale, ws + b.off_qg, b.ld_g, sg, ws + b.off_hq, STAT_SLOT_BYTES, s2, fuse);
-  };
-  auto gemm_gx = [&](hipStream_t s2) {
-    // g_x = (qG . qW^T) sG sW / n_o   (never split here: the split workspace belongs to the g_W GEMM)
-    return gemm_i8_impl(ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, O, sg,
-                        cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, out_dtype, I, nullptr, s2,
-                        s2 == st && b.split_bytes ? ws + b.off_split : nullptr, s2 == st ? b.split_bytes : 0);
-  };
-  if (hq_aside) {
-    // The statistics pass on the main stream feeds the row-wise quantiser only when it delivers the
-    // fused absmax; with per-token steps (or an absmax pass of its own) the row-wise kernel starts
-    // at once, beside the statistics pass.  The partial column sums always come from that pass.
-    if (fuse) rc = check_hip(hipStreamWaitEvent(side->stream, side->fork2, 0), "hipStreamWaitEvent");
-    if (!rc) rc = quantise_gy_rows(side->stream);
-    if (!rc && gb && !fuse) rc = check_hip(hipStreamWaitEvent(side->stream, side->fork2, 0), "hipStreamWaitEvent");
-    if (!rc) rc = finish_bias(side->stream);
-    if (!rc && gx_aside) rc = gemm_gx(side->stream);
-    if (rc) return rc;
+  if (split) mark(K_GEMM_GW);
+  if (!side && (rc = run_gemm(px, st))) return rc;
+  if (split) mark(K_GEMM_GX);
+  if (marks && !split) mark(STAGE_GEMM);
+  return HOT_OK;
+}
+
+// Timing events, kept for the next timed call: a set is taken for the length of a call and put back after it.
+struct EventSet { int dev; hipEvent_t ev[K_COUNT + 1]; };
+static std::mutex g_event_mutex;
+static std::vector<EventSet> g_event_sets;
+constexpr size_t EVENT_SETS_KEPT = 16;
+
+static int take_events(EventSet* out) {
+  int dev = 0;
+  if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
+  {
+    std::lock_guard<std::mutex> lock(g_event_mutex);
+    for (size_t i = 0; i < g_event_sets.size(); ++i)
+      if (g_event_sets[i].dev == dev) {
+        *out = g_event_sets[i];
+        g_event_sets[i] = g_event_sets.back();
+        g_event_sets.pop_back();
+        return HOT_OK;
+      }
   }
-  if (side) {
-    rc = check_hip(hipEventRecord(side->join, side->stream), "hipEventRecord");
-    if (rc) return rc;
-  }
-  // g_W = (qGp . xq^T) sGp sx / hla_n, right after the kernel that wrote its large operand
-  rc = gemm_i8_impl(ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
-                    1.0f / (float)cfg->hla_n, gw, out_dtype, I, nullptr, st,
-                    b.split_bytes ? ws + b.off_split : nullptr, b.split_bytes);
-  if (rc) return rc;
-  mark(K_GEMM_GW);
-  if (!hq_aside) {
-    rc = quantise_gy_rows(st);
-    if (rc) return rc;
-    mark(K_GY_HQ);
-  }
-  if (side) {
-    rc = check_hip(hipStreamWaitEvent(st, side->join, 0), "hipStreamWaitEvent");
-    if (rc) return rc;
-    side_join.joined = true;
-  } else {
-    rc = quantise_w(st);
-    if (rc) return rc;
-    mark(K_W_QUANT);
-  }
-  if (!gx_aside) {
-    rc = gemm_gx(st);
-    if (rc) return rc;
-    mark(K_GEMM_GX);
+  out->dev = dev;
+  for (int i = 0; i <= K_COUNT; ++i) {
+    if (int rc = check_hip(hipEventCreate(&out->ev[i]), "hipEventCreate")) {
+      while (i-- > 0) (void)hipEventDestroy(out->ev[i]);
+      return rc;
+    }
   }
   return HOT_OK;
 }
 
-// Runs the backward with an event after every kernel group and returns the K_COUNT durations (s).
+static void put_events(const EventSet& s) {
+  {
+    std::lock_guard<std::mutex> lock(g_event_mutex);
+    if (g_event_sets.size() < EVENT_SETS_KEPT) { g_event_sets.push_back(s); return; }
+  }
+  for (int i = 0; i <= K_COUNT; ++i) (void)hipEventDestroy(s.ev[i]);
+}
+
+// Runs the backward with an event after every group of launches (split: every kernel, else every stage) and returns
+// the durations of the `slots` groups in seconds.
 static int run_backward_timed(const void* gy, const void* w, int dtype, const void* xq, const float* sx, int64_t L,
                               int64_t O, int64_t I, const hot_config* cfg, void* gx, void* gw, int out_dtype,
-                              void* workspace, size_t workspace_bytes, float* secs, hipStream_t st) {
-  hipEvent_t ev[K_COUNT + 1];
+                              void* workspace, size_t workspace_bytes, bool split, float* secs, int slots, hipStream_t st) {
+  EventSet set;
   int slot_of[K_COUNT];
-  for (int i = 0; i <= K_COUNT; ++i) ev[i] = nullptr;
-  for (int i = 0; i < K_COUNT; ++i) { slot_of[i] = -1; secs[i] = 0.f; }
-  int rc = HOT_OK;
-  for (int i = 0; i <= K_COUNT && !rc; ++i) rc = check_hip(hipEventCreate(&ev[i]), "hipEventCreate");
-  if (!rc) rc = run_backward(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, ev, slot_of, st);
-  if (!rc) rc = check_hip(hipEventSynchronize(ev[K_COUNT]), "hipEventSynchronize");
+  for (int i = 0; i < slots; ++i) secs[i] = 0.f;
+  if (int rc = take_events(&set)) return rc;
+  Marks marks{set.ev, slot_of, split};
+  int rc = run_backward(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, &marks, st);
+  if (!rc) rc = check_hip(hipEventSynchronize(set.ev[marks.seq]), "hipEventSynchronize");
   if (!rc) {
-    for (int i = 0; i < K_COUNT; ++i) {
+    for (int i = 0; i < marks.seq; ++i) {
       float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
-      if (slot_of[i] >= 0) secs[slot_of[i]] = ms * 1e-3f;
+      (void)hipEventElapsedTime(&ms, set.ev[i], set.ev[i + 1]);
+      secs[slot_of[i]] += ms * 1e-3f;
     }
   }
-  for (int i = 0; i <= K_COUNT; ++i)
-    if (ev[i]) (void)hipEventDestroy(ev[i]);
+  put_events(set);
   return rc;
 }
 
@@ -452,17 +489,14 @@ int hot_linear_backward(const void* gy, const void* w, int dtype, const void* xq
                         void* workspace, size_t workspace_bytes, float* times4, void* hip_stream) {
   if (!times4)
     return run_backward(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, nullptr,
-                        nullptr, (hipStream_t)hip_stream);
-  float k[K_COUNT];
+                        (hipStream_t)hip_stream);
+  // the reference op returns {fwht, quant, gemm, dequant} (HLQ_backward_kernel.cu:729-733): here the launches that
+  // only measure, those that transform and quantise (with blocks above 128 tokens these hold g_y's statistics too), both
+  // products, and 0 for the dequantisation, which is the products' epilogue
   const int rc = run_backward_timed(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes,
-                                    k, (hipStream_t)hip_stream);
-  if (rc) return rc;
-  // the reference op returns {fwht, quant, gemm, dequant} (HLQ_backward_kernel.cu:729-733)
-  times4[0] = k[K_CLEAR] + k[K_GY_STATS] + k[K_W_STATS];          // transform passes that only measure
-  times4[1] = k[K_GY_HLA] + k[K_GY_HQ] + k[K_W_QUANT];            // transform + quantise passes
-  times4[2] = k[K_GEMM_GX] + k[K_GEMM_GW];                        // both GEMMs
-  times4[3] = 0.f;                                                // dequantisation: fused into the GEMMs' epilogues
-  return HOT_OK;
+                                    false, times4, STAGE_COUNT, (hipStream_t)hip_stream);
+  times4[3] = 0.f;
+  return rc;
 }
 
 int hot_linear_backward_bias(const void* gy, const void* w, int dtype, const void* xq, const float* sx, int64_t L,
@@ -470,7 +504,7 @@ int hot_linear_backward_bias(const void* gy, const void* w, int dtype, const voi
                              void* workspace, size_t workspace_bytes, void* hip_stream) {
   if (!gb) return fail(HOT_ERR_INVALID, "hot_linear_backward_bias: null pointer");
   return run_backward(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, nullptr,
-                      nullptr, (hipStream_t)hip_stream, gb);
+                      (hipStream_t)hip_stream, gb);
 }
 
 // ---- g_x through a low-rank projection along the tokens ---------------------------------------------
@@ -555,7 +589,7 @@ int hot_gx_lowrank(const void* gy, const void* w, int dtype, int64_t L, int64_t 
   } else {
     rc = colwise_quant_impl(gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, bits, cfg->gx_round, cfg->seed,
                             HOT_STREAM_GX, HOT_SCALE_TENSOR, ws + b.off_qg, b.ld_g, bits == 4, sg, ws + b.off_colg,
-                            b.colg_bytes, st, who, nullptr, false, nullptr, nullptr, 1, 0, true);
+                            b.colg_bytes, st, who, nullptr, nullptr, 1, 0, true);
   }
   if (rc) return rc;
   zero_pad_impl(ws + b.off_qg, b.lp, O * bits / 8, b.ld_g, st);
@@ -778,7 +812,7 @@ int hot_abc_forward_batched(const void* x, int dtype, int64_t B, int64_t T, int6
   const int64_t kg = kpad_group(T, cfg);
   return colwise_quant_impl(x, dtype, B * T, I, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->act_bits, cfg->act_round, cfg->seed,
                             HOT_STREAM_ACT, cfg->act_scale, xq_out, B * kg, 0, sx_out, workspace, workspace_bytes,
-                            (hipStream_t)hip_stream, who, nullptr, false, nullptr, nullptr, (int)B, kg);
+                            (hipStream_t)hip_stream, who, nullptr, nullptr, (int)B, kg);
 }
 
 int hot_backward_batched_ranges(int64_t B, int64_t T, int64_t O, int64_t I, const hot_config* cfg) {
@@ -812,23 +846,37 @@ int hot_linear_backward_batched(const void* gy, const void* w, int dtype, const 
   float* sg = (float*)(ws + b.off_sg);
   float* sw = (float*)(ws + b.off_sw);
   float* sgp = (float*)(ws + b.off_sgp);
-  // W: Hadamard along O + quantise, stored [I, O]
-  int rc = colwise_quant_impl(w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed,
-                              HOT_STREAM_W, cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw,
-                              colwise_workspace_bytes_impl(I), st, who);
+  // W: Hadamard along O + quantise, stored [I, O].  g_y: HLA inside every sample, one step per sample (or per sample
+  // and channel), transposed -> g_W operand; Hadamard along O, one step per sample (or per token) -> g_x operand, whose
+  // product reads a step per row.  Two phases of independent jobs (phase.h).
+  const bool w_short = w_joins_phase(cfg), row_tensor = cfg->gx_scale == HOT_SCALE_TENSOR;
+  const bool hq_job = cfg->n_o <= CW_ROWS && (row_tensor || O <= HQ_ROW_MAX_K);
+  ColJob gj, wj;
+  int rc = col_job_impl(wj, w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed, HOT_STREAM_W,
+                        cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw, colwise_workspace_bytes_impl(I), who,
+                        1, 0, false, w_short);
+  if (!rc) rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
+                             HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg,
+                             colwise_group_workspace_bytes_impl(O, (int)B), who, (int)B, b.kg, false, false);
   if (rc) return rc;
-  // g_y: Hadamard along O, one step per sample (or per token) -> g_x operand; the GEMM reads a step per row
-  rc = hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale,
-                       ws + b.off_qg, b.ld_g, sg, ws + b.off_hq, b.off_sg - b.off_hq, st, false,
-                       cfg->gx_scale == HOT_SCALE_TENSOR ? T : 0, nullptr);
+  HqArgs hj;
+  if (hq_job) {
+    if (row_tensor) col_job_row_stat(gj, cfg->n_o);
+    rc = hq_job_impl(hj, gy, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg, b.ld_g, sg,
+                     gj.a.row_absmax, B > 1 ? 1 : gj.a.npart, B > 1 ? GS : 1, B);
+    if (rc) return rc;
+  }
+  col_job_clear(gj, st);
+  rc = phase_launch(0, dtype, &gj, w_short ? &wj : nullptr, nullptr, nullptr, st);
+  if (!rc && !w_short) rc = phase_launch(0, dtype, &wj, nullptr, nullptr, nullptr, st);
+  if (!rc) rc = phase_launch(1, dtype, &gj, w_short ? &wj : nullptr, hq_job ? &hj : nullptr, nullptr, st);
+  if (!rc && !w_short) rc = phase_launch(1, dtype, &wj, nullptr, nullptr, nullptr, st);
+  if (!rc && !hq_job)
+    rc = hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale,
+                         ws + b.off_qg, b.ld_g, sg, ws + b.off_hq, b.off_sg - b.off_hq, st, false, row_tensor ? T : 0, nullptr);
   if (rc) return rc;
-  rc = gemm_i8_impl(ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, O, sg, 1, sw, 1.0f / (float)cfg->n_o, gx,
-                    out_dtype, I, nullptr, st);
-  if (rc) return rc;
-  // g_y: HLA inside every sample, one step per sample (or per sample and channel), transposed -> g_W operand
-  rc = colwise_quant_impl(gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
-                          HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg,
-                          colwise_group_workspace_bytes_impl(O, (int)B), st, who, nullptr, false, nullptr, nullptr, (int)B, b.kg);
+  rc = gemm_i8_impl(ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, O, sg, cfg->gx_scale == HOT_SCALE_ROW || B > 1 || !hq_job, sw,
+                    1.0f / (float)cfg->n_o, gx, out_dtype, I, nullptr, st);   // (one sample: one step for the whole operand)
   if (rc) return rc;
   // g_W = sum over samples of (qGp_b . xq_b^T) sGp_b sx_b / hla_n
   return gemm_i8_grouped_impl(ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, O, I, (int)B, b.kg, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
@@ -839,8 +887,8 @@ int hot_linear_backward_kernels(const void* gy, const void* w, int dtype, const 
                                 int64_t O, int64_t I, const hot_config* cfg, void* gx, void* gw, int out_dtype,
                                 void* workspace, size_t workspace_bytes, float* times8, void* hip_stream) {
   if (!times8) return fail(HOT_ERR_INVALID, "hot_linear_backward_kernels: null times8");
-  return run_backward_timed(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, times8,
-                            (hipStream_t)hip_stream);
+  return run_backward_timed(gy, w, dtype, xq, sx, L, O, I, cfg, gx, gw, out_dtype, workspace, workspace_bytes, true, times8,
+                            K_COUNT, (hipStream_t)hip_stream);
 }
 
 }  // extern "C"

@@ -19,6 +19,8 @@
 // Tiling: 256 threads = 2x2 waves; each wave owns (32 WM) x (32 WN) outputs as
 // WM x WN MFMA tiles; K advances 128 codes per stage with the next stage's
 // global loads in flight during the MFMAs (double-buffered LDS).
+#include <string.h>
+
 #include <mutex>
 #include <type_traits>
 #include <utility>
@@ -320,6 +322,7 @@ __device__ __forceinline__ void gemm_epilogue_staged(const v16i (&acc)[WM][WN], 
   constexpr int PITCH = ROWB + 16;
   constexpr int CPR = ROWB / 16;                        // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;                         // rows one wave-wide store covers
+  static_assert(64 % CPR == 0 && 32 % RPI == 0, "a store covers whole rows of the fragment, and no row past it");
   typedef typename Quad<OutT>::type quad_t;
   OutT* out = reinterpret_cast<OutT*>(g.out);
   const int m = lane & 31, half = lane >> 5;
@@ -656,9 +659,15 @@ gemm_i8_pipe_kernel(const GemmArgs g) {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
+// LDS of the kernel: S stages, and a spare KiB when the chunks of a stage do not come out even
+template <int WM, int WN, int GM, int GN, int S, int RB>
+constexpr int slot_ring_bytes() {
+  const int rows = 32 * (WM * GM + WN * GN), chunks = rows * RB / 1024;
+  return S * rows * RB + (chunks % 4 ? 1024 : 0);
+}
+
 template <int WM, int WN, int GM, int GN, int BITS, int S, int RB, typename OutT>
-__global__ void __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(1, (WM * WN <= 8 ? 2 : 1))))
-gemm_i8_slot_kernel(const GemmArgs g) {
+__device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uint8_t* ring) {
   static_assert(GM * GN == 4, "four waves");
   static_assert(RB == 64 || RB == 128, "stage rows of 64 or 128 bytes");
   constexpr int BM = 32 * WM * GM, BN = 32 * WN * GN;
@@ -668,7 +677,7 @@ gemm_i8_slot_kernel(const GemmArgs g) {
   constexpr int ROWS = BM + BN, CHUNKS = ROWS / RPC, LPW = (CHUNKS + 3) / 4;
   constexpr bool SPARE = LPW * 4 != CHUNKS;
   constexpr int STAGE_BYTES = ROWS * RB;
-  constexpr int RING_BYTES = S * STAGE_BYTES + (SPARE ? 1024 : 0);
+  constexpr int RING_BYTES = slot_ring_bytes<WM, WN, GM, GN, S, RB>();
   static_assert(S >= 2 && RING_BYTES <= 160 * 1024, "two or more LDS stages within 160 KiB");
   constexpr int NF = WM * WN;                       // accumulator fragments per wave
   constexpr int NM = NF * (BITS == 4 ? 2 : 1);      // MFMAs (slots) per round
@@ -677,13 +686,12 @@ gemm_i8_slot_kernel(const GemmArgs g) {
   constexpr int DPS = (LPW + NM - 1) / NM;          // DMA instructions per slot of the refilling round
   constexpr int RPSL = (NR + NM - 1) / NM;          // fragment reads per slot (1 unless NR > NM)
   static_assert(NR <= H || BITS != 4, "the reads of a round fit the first half of the round before");
-  __shared__ __attribute__((aligned(1024))) uint8_t ring[RING_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / GN, wn = wave % GN;
   int tm, tn;
-  tile_of(g, (int)blockIdx.x, tm, tn);
+  tile_of(g, block, tm, tn);
   const int64_t row0 = (int64_t)tm * BM, col0 = (int64_t)tn * BN;
   constexpr bool EARLY_SCALES = NF <= 4 && BITS != 16;
   float sa_row[WM];
@@ -883,6 +891,13 @@ gemm_i8_slot_kernel(const GemmArgs g) {
     return;
   }
   gemm_epilogue<WM, WN, BITS, OutT>(acc, g, row0 + wm * WM * 32, col0 + wn * WN * 32, lane, sa_row, sb);
+}
+
+template <int WM, int WN, int GM, int GN, int BITS, int S, int RB, typename OutT>
+__global__ void __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(1, (WM * WN <= 8 ? 2 : 1))))
+gemm_i8_slot_kernel(const GemmArgs g) {
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[slot_ring_bytes<WM, WN, GM, GN, S, RB>()];
+  gemm_slot_body<WM, WN, GM, GN, BITS, S, RB, OutT>(g, (int)blockIdx.x, ring);
 }
 
 // ---------------------------------------------------------------------------
@@ -1350,21 +1365,37 @@ static int dispatch_out(int out_dtype, int variant, GemmArgs& g, hipStream_t st)
   }
 }
 
+// Checks a product and fills the arguments that every kernel takes.
+static int gemm_fill(GemmArgs& g, const GemmProduct& p, int out_dtype, int32_t* acc_out) {
+  if (!p.A || !p.B || !p.scale_a || !p.scale_b || !p.out) return fail(HOT_ERR_INVALID, "hot_gemm_i8: null pointer");
+  if (p.M < 0 || p.N < 0 || p.K <= 0) return fail(HOT_ERR_INVALID, "hot_gemm_i8: bad shape %lld x %lld x %lld", (long long)p.M, (long long)p.N, (long long)p.K);
+  if (p.bits != 4 && p.bits != 8) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: bits=%d (4 or 8)", p.bits);
+  const int64_t kpad = round_up(p.K, GEMM_KTILE);
+  const int64_t need = kpad * p.bits / 8;
+  if (p.lda < need || p.ldb < need || (p.lda & 15) || (p.ldb & 15))
+    return fail(HOT_ERR_INVALID, "hot_gemm_i8: row pitches (%lld, %lld) must be multiples of 16 and >= %lld bytes", (long long)p.lda, (long long)p.ldb, (long long)need);
+  if (((uintptr_t)p.A & 15) || ((uintptr_t)p.B & 15)) return fail(HOT_ERR_INVALID, "hot_gemm_i8: operands must be 16-byte aligned");
+  if (p.ldo < p.N) return fail(HOT_ERR_INVALID, "hot_gemm_i8: ldo=%lld < N", (long long)p.ldo);
+  if (p.bits == 4 && p.K > (int64_t)(0x7FFFFFFF / (112 * 112))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for the scaled INT4 accumulator");
+  if (p.bits == 8 && p.K > (int64_t)(0x7FFFFFFF / (127 * 127))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for int32 accumulation");
+  memset(&g, 0, sizeof(g));
+  g.A = (const uint8_t*)p.A; g.B = (const uint8_t*)p.B; g.lda = p.lda; g.ldb = p.ldb; g.M = p.M; g.N = p.N;
+  g.ktiles = (int)(kpad / G_BK);
+  g.scale_a = p.scale_a; g.scale_b = p.scale_b; g.post_scale = p.post_scale; g.a_per_row = p.a_per_row;
+  g.out = p.out; g.ldo = p.ldo; g.acc_out = acc_out;
+  g.vec_out = ((p.ldo & 3) == 0 && ((uintptr_t)p.out & 15) == 0) ? 1 : 0;
+  g.vec16 = (((uintptr_t)p.out & 15) == 0 && ((p.ldo * (out_dtype == HOT_F32 ? 4 : 2)) & 15) == 0) ? 1 : 0;
+  g.splits = 1; g.gsplits = 1;
+  return HOT_OK;
+}
+
 int gemm_i8_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int bits, int64_t M, int64_t N,
                  int64_t K, const float* scale_a, int a_per_row, const float* scale_b, float post_scale,
                  void* out, int out_dtype, int64_t ldo, int32_t* acc_out, hipStream_t st, void* split_ws,
                  size_t split_ws_bytes, int variant) {
-  if (!A || !B || !scale_a || !scale_b || !out) return fail(HOT_ERR_INVALID, "hot_gemm_i8: null pointer");
-  if (M < 0 || N < 0 || K <= 0) return fail(HOT_ERR_INVALID, "hot_gemm_i8: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
-  if (bits != 4 && bits != 8) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: bits=%d (4 or 8)", bits);
-  const int64_t kpad = round_up(K, GEMM_KTILE);
-  const int64_t need = kpad * bits / 8;
-  if (lda < need || ldb < need || (lda & 15) || (ldb & 15))
-    return fail(HOT_ERR_INVALID, "hot_gemm_i8: row pitches (%lld, %lld) must be multiples of 16 and >= %lld bytes", (long long)lda, (long long)ldb, (long long)need);
-  if (((uintptr_t)A & 15) || ((uintptr_t)B & 15)) return fail(HOT_ERR_INVALID, "hot_gemm_i8: operands must be 16-byte aligned");
-  if (ldo < N) return fail(HOT_ERR_INVALID, "hot_gemm_i8: ldo=%lld < N", (long long)ldo);
-  if (bits == 4 && K > (int64_t)(0x7FFFFFFF / (112 * 112))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for the scaled INT4 accumulator");
-  if (bits == 8 && K > (int64_t)(0x7FFFFFFF / (127 * 127))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for int32 accumulation");
+  GemmArgs g;
+  const GemmProduct p = {A, lda, B, ldb, bits, M, N, K, scale_a, a_per_row, scale_b, post_scale, out, ldo};
+  if (int rc = gemm_fill(g, p, out_dtype, acc_out)) return rc;
   if (variant < HOT_GEMM_AUTO || variant >= HOT_GEMM_VARIANTS) return fail(HOT_ERR_INVALID, "hot_gemm_i8: unknown kernel variant %d", variant);
   if (M == 0 || N == 0) return HOT_OK;
   const size_t ws_have = split_ws ? split_ws_bytes : 0;
@@ -1372,15 +1403,6 @@ int gemm_i8_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int bit
   const bool small_ptrs = M * lda < (1ll << 32) && N * ldb < (1ll << 32);
   if (variant != HOT_GEMM_REG_128 && !small_ptrs)
     return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: operands of 4 GiB or more take the register-staged kernel only");
-  GemmArgs g;
-  g.A = (const uint8_t*)A; g.B = (const uint8_t*)B; g.lda = lda; g.ldb = ldb; g.M = M; g.N = N;
-  g.ktiles = (int)(kpad / G_BK);
-  g.scale_a = scale_a; g.scale_b = scale_b; g.post_scale = post_scale; g.a_per_row = a_per_row;
-  g.out = out; g.ldo = ldo; g.acc_out = acc_out; g.bias = nullptr;
-  g.vec_out = ((ldo & 3) == 0 && ((uintptr_t)out & 15) == 0) ? 1 : 0;
-  g.vec16 = (((uintptr_t)out & 15) == 0 && ((ldo * (out_dtype == HOT_F32 ? 4 : 2)) & 15) == 0) ? 1 : 0;
-  g.splits = 1; g.partials = nullptr;
-  g.groups = 0; g.group_stages = 0; g.gsplits = 1; g.gper = 0; g.gscale_a = nullptr; g.gscale_b = nullptr; g.gpart = nullptr; g.ldp = 0;
   if (variant == HOT_GEMM_DMA_128_SPLITK) {
     const GemmSplit plan = gemm_split_plan(M, N, K, bits);
     if (plan.splits < 2) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: the split-K kernel needs a product of fewer than 256 tiles of 128 x 128 and a long K");
@@ -1390,6 +1412,86 @@ int gemm_i8_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int bit
     g.partials = (v4i*)split_ws;
   }
   return bits == 4 ? dispatch_out<4>(out_dtype, variant, g, st) : dispatch_out<8>(out_dtype, variant, g, st);
+}
+
+// ---- two products in one launch -----------------------------------------------------------------------
+//
+// The two products of a backward pass do not depend on each other.  Launched one after the other each leaves CUs
+// idle in its last round, and a lone workgroup per CU leaves the matrix cores idle while it fills its ring and while it
+// stores; here both share a grid and two workgroups share a CU (at most 80 KiB of LDS and 256 registers each), so that
+// one's loads and stores lie under the other's MFMAs.  The g_W tiles come first: they run longest, and g_x tiles fill
+// in behind them.  Two tilings, g_x / g_W:
+//   128 x 128 (2 stages) / 64 x 128 (3 stages): while the g_W product makes fewer than 256 tiles of 192 x 128, i.e.
+//     one long tile per CU would be its latency.  Measured against one after the other by gemm_plan_impl (us,
+//     bf16 results): 12608 x 768 x 3072 INT4 + 3072 x 768 x 7092: 50.2 / 57.5; 768 wide (proj): 21.4 / 31.0; 25216 x 768
+//     x 3072 + 3072 x 768 x 7092: 69.1 / 86.1; 3003 x 520 x 1000 + 1000 x 520 x 3003: 11.8 / 19.3; 128 tokens: 5.3 / 10.0
+//   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008 INT4 + 11008 x 4096 x 4096: 409 / 456;
+//     8192 x 11008 x 4096 + 4096 x 11008 x 2080: 348 / 424; 8192 x 4096 x 4096 + 4096^3: 174 / 187
+// (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174).
+struct PairArgs {
+  GemmArgs w, x;
+  uint32_t w_blocks;      // a multiple of 8: blockIdx % 8 stays the XCD of the second product's tiles
+};
+
+template <int XBITS, bool LARGE, typename OutT>
+__global__ void __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+gemm_pair_kernel(const PairArgs p) {
+  constexpr int XM = LARGE ? 3 : 2, WM = LARGE ? 3 : 2, WN = LARGE ? 2 : 1, WGM = LARGE ? 2 : 1, WGN = LARGE ? 2 : 4, WS = LARGE ? 2 : 3;
+  constexpr int LX = slot_ring_bytes<XM, 2, 2, 2, 2, 128>(), LW = slot_ring_bytes<WM, WN, WGM, WGN, WS, 128>();
+  static_assert(LX <= 80 * 1024 && LW <= 80 * 1024, "two workgroups per CU");
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[LX > LW ? LX : LW];
+  // (the arguments are read inside the branch that uses them: both products' would overflow the scalar registers)
+  typedef const __attribute__((address_space(4))) PairArgs* segment_t;
+  segment_t k = (segment_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  const PairArgs& q = *(const PairArgs*)k;
+  if (blockIdx.x < p.w_blocks) {
+    if ((int)blockIdx.x < q.w.tiles_m * q.w.tiles_n) gemm_slot_body<WM, WN, WGM, WGN, 8, WS, 128, OutT>(q.w, (int)blockIdx.x, ring);
+  } else {
+    gemm_slot_body<XM, 2, 2, 2, XBITS, 2, 128, OutT>(q.x, (int)(blockIdx.x - p.w_blocks), ring);
+  }
+}
+
+static void pair_tiles(GemmArgs& g, int bm, int bn) {
+  g.tiles_m = (int)((g.M + bm - 1) / bm);
+  g.tiles_n = (int)((g.N + bn - 1) / bn);
+  g.group_m = pick_group_m(g.tiles_m, g.tiles_n, 2);
+}
+
+template <int XBITS, bool LARGE, typename OutT>
+static int launch_pair(PairArgs& p, hipStream_t st) {
+  pair_tiles(p.w, LARGE ? 192 : 64, 128);
+  pair_tiles(p.x, LARGE ? 192 : 128, 128);
+  p.w_blocks = (uint32_t)round_up((int64_t)p.w.tiles_m * p.w.tiles_n, 8);
+  const int64_t total = (int64_t)p.w_blocks + (int64_t)p.x.tiles_m * p.x.tiles_n;
+  if (total > (1 << 30)) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: too many tiles");
+  hipLaunchKernelGGL((gemm_pair_kernel<XBITS, LARGE, OutT>), dim3((unsigned)total), dim3(G_THREADS), 0, st, p);
+  return check_launch("gemm_pair_kernel");
+}
+
+bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
+  auto fits = [](const GemmProduct& p) {
+    return p.M > 0 && p.N > 0 && p.K > 0 && (round_up(p.K, GEMM_KTILE) * p.bits / 8) % 128 == 0 && p.M * p.lda < (1ll << 32) && p.N * p.ldb < (1ll << 32);
+  };
+  return w.bits == 8 && fits(w) && fits(x);
+}
+
+int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
+  PairArgs p;
+  if (int rc = gemm_fill(p.w, w, out_dtype, nullptr)) return rc;
+  if (int rc = gemm_fill(p.x, x, out_dtype, nullptr)) return rc;
+  if (!gemm_pair_possible(w, x)) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: the paired kernel takes rows of whole 128-byte lines");
+  const bool large = ((w.M + 191) / 192) * ((w.N + 127) / 128) >= 256;
+#define HOT_PAIR_CASE(OUT)                                                                                          \
+  return x.bits == 4 ? (large ? launch_pair<4, true, OUT>(p, st) : launch_pair<4, false, OUT>(p, st))               \
+                     : (large ? launch_pair<8, true, OUT>(p, st) : launch_pair<8, false, OUT>(p, st))
+  switch (out_dtype) {
+    case HOT_F32: HOT_PAIR_CASE(float);
+    case HOT_BF16: HOT_PAIR_CASE(bf16_t);
+    case HOT_F16: HOT_PAIR_CASE(f16_t);
+    default: return fail(HOT_ERR_INVALID, "hot_gemm_i8: bad out dtype %d", out_dtype);
+  }
+#undef HOT_PAIR_CASE
 }
 
 // out[M, N] = A[M, K] . B[N, K]^T (+ bias[N]) on bf16 operands, fp32 accumulation

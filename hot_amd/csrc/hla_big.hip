@@ -392,9 +392,10 @@ int dispatch_runs(int m, const BigArgs& a, void* out, int64_t ld_out, hipStream_
   }
 }
 
-__global__ void big_clear_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n) {
+__global__ void big_clear_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n, float* row_absmax) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < (int64_t)(STAT_BYTES / 4)) stat[i] = 0.f;
+  if (row_absmax && i < (int64_t)(STAT_SLOT_BYTES / 4)) row_absmax[i] = 0.f;
   if (i < C) colmax[i] = 0.f;
   if (i < n) tab[i] = -1;
 }
@@ -448,7 +449,7 @@ __global__ void __launch_bounds__(256) big_table_kernel(int32_t* tab, const TabR
 // rows in its own LDS bitmap; thread i of the grid clears word i of the statistics and of the
 // per-channel maxima, writes -1 for natural row i when it is dropped, and the entry of the i-th row of
 // the caller's list.  Dropped and kept rows are disjoint, so the two writes never meet.
-__global__ void __launch_bounds__(256) big_prepare_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n, const TabRows p) {
+__global__ void __launch_bounds__(256) big_prepare_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n, float* row_absmax, const TabRows p) {
   __shared__ uint32_t s_map[8192 / 32];
   __shared__ uint32_t s_below[8192 / 32];
   const int tid = threadIdx.x;
@@ -467,6 +468,7 @@ __global__ void __launch_bounds__(256) big_prepare_kernel(float* stat, float* co
   __syncthreads();
   const int64_t i = (int64_t)blockIdx.x * 256 + tid;
   if (i < (int64_t)(STAT_BYTES / 4)) stat[i] = 0.f;
+  if (row_absmax && i < (int64_t)(STAT_SLOT_BYTES / 4)) row_absmax[i] = 0.f;
   if (i < C) colmax[i] = 0.f;
   if (i < n && !((s_map[i >> 5] >> (i & 31)) & 1u)) tab[i] = -1;
   if (i < p.count) {
@@ -701,7 +703,7 @@ size_t hla_big_workspace_bytes_impl(int64_t R, int64_t C, int n, int r) {
 int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const int32_t* rows, int r, int bits,
                  int rounding, uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_out,
                  float* scales_out, void* workspace, size_t workspace_bytes, hipStream_t st, const char* who,
-                 hipEvent_t after_stats, float* row16_absmax_out, bool rowmajor, int store4) {
+                 float* row16_absmax_out, bool rowmajor, int store4) {
   const int m = n / 64;
   if (n < 256 || n > 8192 || (n & (n - 1))) return fail(HOT_ERR_UNSUPPORTED, "%s: block size %d (a power of two, 256 .. 8192)", who, n);
   const int64_t NB = R / n, kout = NB * r;
@@ -750,11 +752,11 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
       tab_row_put(tr.packed, k, rows[k]);
     }
     hipLaunchKernelGGL(big_prepare_kernel, dim3((unsigned)((nclr + 255) / 256)), dim3(256), 0, st, a.stat, a.colmax, C,
-                       (int32_t*)(ws + b.off_tab), n, tr);
+                       (int32_t*)(ws + b.off_tab), n, row16_absmax_out, tr);
     if (int rc = check_launch("big_prepare_kernel")) return rc;
   } else {
     hipLaunchKernelGGL(big_clear_kernel, dim3((unsigned)((nclr + 255) / 256)), dim3(256), 0, st, a.stat, a.colmax, C,
-                       (int32_t*)(ws + b.off_tab), n);
+                       (int32_t*)(ws + b.off_tab), n, row16_absmax_out);
     if (int rc = build_row_table((int32_t*)(ws + b.off_tab), n, rows, r, nullptr, st, who)) return rc;
   }
   const dim3 g1((unsigned)gx, (unsigned)(R / 64));
@@ -788,7 +790,6 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
   // (with absmax steps the run-major quantise pass reads the statistic itself and publishes the steps)
   if (!(run_major && scale_mode != HOT_SCALE_SAWB))
     hipLaunchKernelGGL(big_finalize_kernel, dim3(1), dim3(256), 0, st, a, (int64_t)gx * NB * a.nk, kout);
-  if (after_stats) (void)hipEventRecord(after_stats, st);
   if (rowmajor) {
     // untransposed [NB r, C]: the quantise pass writes the destination itself (INT8), or its [Kout, C]
     // scratch, which a second kernel packs two channels to a byte

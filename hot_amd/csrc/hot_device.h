@@ -211,6 +211,45 @@ __device__ __forceinline__ float stat_slots_max(const float* slots, int lane) {
   return wave_max(lane < 16 ? slots[lane * 32] : 0.f);
 }
 
+// Maximum of the n values p[0], p[stride], ... (n >= 1, all >= 0) as far as this one of 256 threads reads them: sixteen loads are in
+// flight at a time, one after the other they would cost a memory latency each.
+__device__ __forceinline__ float part_max(const float* p, int n, int stride, int tid) {
+  float m = 0.f;
+  for (int base = tid; base < n; base += 256 * 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int i = base + 256 * u;
+      v[u] = p[(i < n ? i : n - 1) * stride];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) m = fmaxf(m, v[u]);
+  }
+  return m;
+}
+
+// rint(x / d) with rcp = 1 / d (correctly rounded) for |x / d| <= 128, in three instructions, almost always: adding
+// 1.5 * 2^23 in the fused multiply-add rounds x * rcp to an integer, whose two's complement stands in the low bits of
+// the sum.  x * rcp is within 2^-17 of x / d and the fp32 quotient within 2^-18, so both round to the same
+// integer unless x * rcp lies within 2^-16 of a half-integer: `dev` collects the largest distance from the chosen
+// integer, and where rint_unsure(dev) says so the caller takes rint_div_exact for the values it covers.
+constexpr float RINT_MAGIC = 12582912.0f;
+__device__ __forceinline__ uint32_t rint_div_bits(float x, float rcp, float& dev) {
+  const float t = __builtin_fmaf(x, rcp, RINT_MAGIC);
+  dev = fmaxf(dev, fabsf(__builtin_fmaf(x, rcp, -(t - RINT_MAGIC))));
+  return as_u(t);
+}
+__device__ __forceinline__ bool rint_unsure(float dev) { return dev > 0.5f - 1.52587890625e-05f; }
+// The same with the IEEE quotient, without a division: two residual corrections of x * rcp.  The first leaves a
+// quotient within an ulp, from which the second gives the correctly rounded one (Markstein: its residual is exact and
+// rcp is the rounded reciprocal).
+__device__ __forceinline__ uint32_t rint_div_exact(float x, float d, float rcp) {
+  float q = x * rcp;
+  q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
+  q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
+  return as_u(rintf(q) + RINT_MAGIC);
+}
+
 // rint(x / d) with rcp = 1 / d precomputed: the product x * rcp is within 1.5 * 2^-23 |x/d| of
 // the correctly rounded quotient, so it rounds to the same integer unless it lies within 2^-14 of
 // a half-integer (|x/d| <= 128); only then is the IEEE division carried out.

@@ -38,6 +38,13 @@ int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int 
 // own; scales_out then holds M entries (the step of each row's sample, the form the GEMM epilogue
 // reads), group_steps (may be null) the M / group_rows steps, and the workspace 128 bytes per sample.
 
+// The row-wise quantiser (blocks of up to 16; per-row steps: K <= HQ_ROW_MAX_K) as a job of a quantise phase (phase.h).
+// stat: nstat absmax values stat_stride floats apart; with groups > 1 one per sample, stat_stride apart, and scales_out [M].
+struct HqArgs;
+int hq_job_impl(HqArgs& a, const void* in, int64_t M, int64_t K, int n, int bits, int rounding, uint64_t seed, uint32_t rng_stream,
+                int scale_mode, void* codes_out, int64_t ld_codes, float* scales_out, const float* stat, int nstat, int stat_stride,
+                int64_t groups);
+
 // Logarithmic quantiser of the row-wise transformed tensor (luq_quantizer_BWD): codes 0 / +-2^j split as
 // 16 a + b into two planes of kp bytes per row ([M, 2 kp]), one step; the workspace holds STAT_SLOT_BYTES.
 int hq_luq_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int bits, uint64_t seed, void* codes_out,
@@ -60,8 +67,8 @@ int colwise_quant_impl(const void* in, int dtype, int64_t R, int64_t C, int n, c
                        int bits, int rounding, uint64_t seed, uint32_t rng_stream, int scale_mode,
                        void* codes_out, int64_t ld_out, int store4, float* scales_out, void* workspace,
                        size_t workspace_bytes, hipStream_t st, const char* who, float* row16_absmax_out = nullptr,
-                       bool stats_cleared = false, hipEvent_t after_stats = nullptr, float* colsum_partial = nullptr,
-                       int groups = 1, int64_t kpad_group = 0, bool rowmajor = false);
+                       float* colsum_partial = nullptr, int groups = 1, int64_t kpad_group = 0, bool rowmajor = false);
+// row16_absmax_out, colsum_partial: blocks above 128 tokens only (shorter ones: ColJob, phase.h).
 // rowmajor: codes stored untransposed, [NB r, C] with ld_out bytes per coefficient row (bytes past the C
 // channels of a row are left alone: zero_pad_impl clears them), one step for the tensor.
 void zero_pad_impl(void* codes, int64_t rows, int64_t row_bytes, int64_t ld, hipStream_t st);
@@ -77,26 +84,24 @@ size_t hla_expand_big_workspace_bytes_impl(int64_t nb, int64_t C, int n);
 // (scales_out: [groups], or [groups][C] with per-channel steps); the codes of sample g take the bytes
 // [g * kpad_group, (g + 1) * kpad_group) of every output row, zero-filled behind the sample's codes.
 size_t colwise_group_workspace_bytes_impl(int64_t C, int groups);
-// Column sums of the input of a colwise_quant_impl call (the bias gradient when the input is g_y):
-// with colsum_partial the call also writes colsum_strips_impl(...) rows of C partial sums (fp32; elem_bytes
-// = size of an input element, on which the partition of the passes depends; one
-// row per run of token blocks of its statistics pass, which holds the sum of every block as
-// coefficient 0); colsum_finish_impl adds the rows in a fixed order and rounds once to the output type.
+// Column sums of the input of a token-wise call (the bias gradient when the input is g_y): the call also writes
+// colsum_strips_impl(...) rows of C partial sums (fp32; elem_bytes = size of an input element, on which the
+// partition of the passes depends), one row per run of token blocks of its statistics pass, which holds the sum of
+// every block as coefficient 0; colsum_finish_impl adds the rows in a fixed order and rounds once to the output type.
 int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes);
-int colsum_finish_impl(const float* partial, int64_t strips, int64_t C, void* out, int out_dtype, hipStream_t st);
+struct ColsumArgs;
+int colsum_finish_impl(const ColsumArgs& a, hipStream_t st);
 size_t colwise_workspace_bytes_impl(int64_t C);
-size_t colwise_stats_bytes_impl(int64_t C);  // leading part of the workspace that must be zero before the statistics pass
 
 // Blocks of 256 .. 8192 tokens (two-level transform through an fp32 workspace); same contract as
 // colwise_quant_impl without the packed-INT4 store.
 int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const int32_t* rows, int r, int bits,
                  int rounding, uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_out,
                  float* scales_out, void* workspace, size_t workspace_bytes, hipStream_t st, const char* who,
-                 hipEvent_t after_stats = nullptr, float* row16_absmax_out = nullptr, bool rowmajor = false,
-                 int store4 = 0);
+                 float* row16_absmax_out = nullptr, bool rowmajor = false, int store4 = 0);
 // rowmajor: the codes are stored untransposed, [NB r, C] with ld_out bytes per coefficient row (store4:
 // two channels to a byte).
-// row16_absmax_out (STAT_SLOTS partial maxima, zero before the call; C a multiple of 16, absmax steps):
+// row16_absmax_out (STAT_SLOTS partial maxima, cleared by the call's first launch; C a multiple of 16, absmax steps):
 // stage 1 also delivers the absmax of the row-wise 16-point Hadamard of the input.
 size_t hla_big_workspace_bytes_impl(int64_t R, int64_t C, int n, int r);
 // Workspace of a token-wise transform of [R, C] with blocks of n tokens and r kept rows, either path.
@@ -106,6 +111,18 @@ int gemm_i8_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int bit
                  int64_t K, const float* scale_a, int a_per_row, const float* scale_b, float post_scale,
                  void* out, int out_dtype, int64_t ldo, int32_t* acc_out, hipStream_t st, void* split_ws = nullptr,
                  size_t split_ws_bytes = 0, int variant = HOT_GEMM_AUTO);
+// One product, and two of them in one launch (results of one type): w INT8, rows of both in whole 128-byte lines.
+struct GemmProduct {
+  const void* A; int64_t lda;
+  const void* B; int64_t ldb;
+  int bits;
+  int64_t M, N, K;
+  const float* scale_a; int a_per_row;
+  const float* scale_b; float post_scale;
+  void* out; int64_t ldo;
+};
+bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x);
+int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st);
 int gemm_bf16_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N, int64_t K,
                    const void* bias, void* out, int out_dtype, int64_t ldo, hipStream_t st, int variant);
 // The hot_gemm_variant that gemm_i8_impl picks for a product when `ws_bytes` of workspace come with it.

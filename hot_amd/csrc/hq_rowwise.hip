@@ -17,92 +17,12 @@
 // HBM traffic per element: sizeof(in) read once + bits/8 written; per-row
 // scales add 4 bytes per row.  Per-tensor scales need the global absmax first,
 // which costs a second read of the input.
-#include "hot_device.h"
 #include "hot_host.h"
+#include "hq_device.h"
 
 namespace hot {
 
 static_assert(STAT_SLOT_BYTES == HOT_HQ_WORKSPACE_BYTES, "the public workspace size of hot_hq_rowwise is the slot array");
-
-constexpr int EPL = 8;  // elements per lane-chunk
-
-template <typename T>
-__device__ __forceinline__ void load_chunk(const T* p, float* x) {
-  constexpr int EPV = vec_traits<T>::EPV;
-  const uint4* v = reinterpret_cast<const uint4*>(p);
-#pragma unroll
-  for (int i = 0; i < EPL / EPV; ++i) {
-    const uint4 raw = v[i];
-    unpack_vec<T>(raw, x + i * EPV);
-  }
-}
-
-// FWHT of the N-element blocks formed by N/EPL adjacent lanes.  N = 8 stands for every block that
-// fits one lane's chunk: its actual size `nrt` (1, 2, 4 or 8) arrives at run time.
-template <int N>
-__device__ __forceinline__ void fwht_lanes(float* x, int lane, int nrt) {
-#pragma unroll
-  for (int h = 1; h < EPL; h <<= 1) {
-    if (N > EPL || h < nrt) {   // no early exit: the stage loop must unroll for x to stay in registers
-#pragma unroll
-      for (int j = 0; j < EPL; ++j) {
-        if ((j & h) == 0) {
-          const float a = x[j], b = x[j + h];
-          x[j] = a + b;
-          x[j + h] = a - b;
-        }
-      }
-    }
-  }
-  // lower lane: own + partner ; upper lane: partner - own  ==  partner + (-own)
-  if constexpr (N >= 16) {
-    const uint32_t sg = (lane & 1) ? 0x80000000u : 0u;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) x[j] = as_f(as_u(x[j]) ^ sg) + lane_xor<1>(x[j]);
-  }
-  if constexpr (N >= 32) {
-    const uint32_t sg = (lane & 2) ? 0x80000000u : 0u;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) x[j] = as_f(as_u(x[j]) ^ sg) + lane_xor<2>(x[j]);
-  }
-  if constexpr (N >= 64) {
-    const uint32_t sg = (lane & 4) ? 0x80000000u : 0u;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) x[j] = as_f(as_u(x[j]) ^ sg) + lane_xor<4>(x[j]);
-  }
-}
-
-template <int BITS, int ROUND>
-__device__ __forceinline__ void quant_store_chunk(const float* x, float d, float rcp, uint64_t e0, uint64_t seed,
-                                                  uint32_t stream, int8_t* out_row_chunk) {
-  constexpr int QMAX = (1 << (BITS - 1)) - 1;
-  int q[EPL];
-  if constexpr (ROUND == 0) {
-    // |x / d| <= qmax (1 + 2^-22) because d comes from the absmax: no clamp needed
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) q[j] = (int)rint_div_fast(x[j], d, rcp);
-  } else {
-    uint32_t r[EPL];
-    sr_bits8(e0 >> 3, seed, stream, r);          // e0 is a multiple of EPL = 8
-    const float rcpk = rcp * 65536.0f;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) q[j] = q_stoch_fix(x[j], rcpk, r[j], QMAX);
-  }
-  if constexpr (BITS == 4) {
-    uint32_t w = 0;
-#pragma unroll
-    for (int j = 0; j < EPL; ++j) w |= (uint32_t)(q[j] & 0xF) << (4 * j);
-    *reinterpret_cast<uint32_t*>(out_row_chunk) = w;
-  } else {
-    uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      w0 |= (uint32_t)(q[j] & 0xFF) << (8 * j);
-      w1 |= (uint32_t)(q[j + 4] & 0xFF) << (8 * j);
-    }
-    *reinterpret_cast<uint2*>(out_row_chunk) = make_uint2(w0, w1);
-  }
-}
 
 // ---- per-row scales: one workgroup per row, row resident in registers ------
 
@@ -538,6 +458,33 @@ int luq_pair_impl(const void* qw, int64_t rows, int64_t kp, void* out, hipStream
   const int64_t n = rows * (kp / 16);
   hipLaunchKernelGGL(luq_pair_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const int8_t*)qw, rows, kp, (int8_t*)out);
   return check_launch("luq_pair_kernel");
+}
+
+int hq_job_impl(HqArgs& a, const void* in, int64_t M, int64_t K, int n, int bits, int rounding, uint64_t seed, uint32_t rng_stream,
+                int scale_mode, void* codes_out, int64_t ld_codes, float* scales_out, const float* stat, int nstat, int stat_stride,
+                int64_t groups) {
+  const char* who = "row-wise quantiser";
+  if (M <= 0 || K <= 0 || K % 8 || K % n || n < 1 || n > 16 || groups < 1 || M % groups) return fail(HOT_ERR_INVALID, "%s: bad shape M=%lld K=%lld", who, (long long)M, (long long)K);
+  const int64_t nch = K / EPL, chunks = M / groups * nch;
+  if (chunks >= (1ll << 31)) return fail(HOT_ERR_UNSUPPORTED, "%s: %lld x %lld elements", who, (long long)M, (long long)K);
+  a.in = in; a.codes = (int8_t*)codes_out; a.scales = scales_out;
+  a.M = M; a.K = K; a.ld = ld_codes;
+  a.nch_row = (uint32_t)nch;
+  a.div_m = 0; a.div_s = 0;
+  if (nch > 1) {
+    int s = 0;
+    while ((1ll << s) < nch) ++s;
+    a.div_m = (uint32_t)((1ull << (31 + s)) / (uint64_t)nch + 1);
+    a.div_s = (uint32_t)(s - 1);
+  }
+  a.chunks = (uint32_t)chunks;
+  a.wgs = (uint32_t)((chunks + 256 * HQ_UNROLL - 1) / (256 * HQ_UNROLL));
+  a.rows = M / groups;
+  a.n = n; a.bits = bits; a.rounding = rounding; a.per_row = scale_mode == HOT_SCALE_ROW ? 1 : 0; a.groups = a.per_row ? 1 : (int32_t)groups;
+  a.stat = stat; a.nstat = nstat; a.stat_stride = stat_stride;
+  a.seed = seed; a.stream = rng_stream;
+  if (hq_body_blocks(a) >= (1ll << 31)) return fail(HOT_ERR_UNSUPPORTED, "%s: M too large", who);
+  return HOT_OK;
 }
 
 int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int bits, int rounding,

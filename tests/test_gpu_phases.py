@@ -1,0 +1,81 @@
+"""The shared launches of a backward pass (both phases of the transforms, both products) at the sizes where they can
+go wrong: short Hadamard blocks with ragged tails, rows on either side of what a wave holds, jobs that round differently,
+the edges of the paired products' tiles, values on and beside the boundary between two codes.  Bit-exact against the
+oracle: integers, then the same fp32 operations in the same order."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import hot_oracle as orc
+from test_gpu_backward import make_case, run_both
+from test_gpu_random_cases import _options
+
+pytestmark = pytest.mark.gpu
+
+STOCH = dict(gx_round=orc.ROUND_STOCH, gw_round=orc.ROUND_STOCH, seed=21)
+
+
+def check(gpu, L, O, I, dt, seed=3, **variant):
+    x, w, gy = make_case(L, O, I, seed=seed, dtype=dt)
+    ocfg = orc.HotConfig.python_rule(L, **variant)
+    gx, gw, tr = run_both(x, w, gy, ocfg, _options(ocfg), gpu)
+    assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
+
+
+@pytest.mark.parametrize("n_o,O", [(1, 24), (2, 72), (4, 104), (8, 40), (8, 1000), (16, 272)])
+@pytest.mark.parametrize("variant", [dict(), dict(gx_scale=orc.SCALE_ROW), dict(w_round=orc.ROUND_STOCH, seed=4), dict(w_scale=orc.SCALE_SAWB),
+                                     dict(gx_bits=8, w_bits=8, **STOCH), dict(gx_round=orc.ROUND_STOCH, seed=9)])
+def test_short_hadamard_blocks(gpu, n_o, O, variant):
+    """W and the row-wise quantiser with blocks of 1 .. 16 along the out-features, the last group of 16 rows of W cut
+    short; a last variant in which the two quantisers of g_y round differently."""
+    check(gpu, 66, O, 40, torch.bfloat16 if O % 48 else torch.float32, n_o=n_o, **variant)
+
+
+@pytest.mark.parametrize("L", [2, 6, 12, 24, 40, 48, 160, 320])
+@pytest.mark.parametrize("variant", [dict(), dict(gw_scale=orc.SCALE_ROW, act_scale=orc.SCALE_SAWB), STOCH])
+def test_short_token_blocks(gpu, L, variant):
+    """Token blocks of 2 .. 64, the short ones sixteen rows at a time with a tail."""
+    check(gpu, L, 64, 264, torch.float32, **variant)
+
+
+@pytest.mark.parametrize("O", [4096, 4112, 16384, 16400])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_row_quantiser_widths(gpu, O, dt):
+    """A step per token: rows of a wave (up to 4096), of a workgroup (up to 16384) and of the kernel of their own."""
+    check(gpu, 5, O, 8, dt, gx_scale=orc.SCALE_ROW)
+
+
+@pytest.mark.parametrize("L,O,I", [(1, 16, 8), (127, 64, 128), (129, 80, 136), (64, 3072, 2048), (64, 3056, 2048), (192, 192, 128),
+                                   (200, 400, 264)])
+@pytest.mark.parametrize("dt,bits", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 4)])
+def test_paired_products(gpu, L, O, I, dt, bits):
+    """Tile edges of the paired products, either side of the line between their two tilings (256 tiles of 192 x 128 of
+    g_W: 3072 x 2048), K shorter than the ring."""
+    check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
+
+
+@pytest.mark.parametrize("scale", [1.0, 3.1e-3, 7.7e4])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_codes_on_the_boundary(gpu, scale, bits):
+    """Values whose quotient by the step lies on a half-integer, or one ulp beside it: the code is that of the IEEE
+    quotient rounded to even (np.rint), wherever the fast path cannot decide."""
+    from hot_amd import ops
+    qmax = 2 ** (bits - 1) - 1
+    step = np.float32(scale)
+    half = (np.arange(-qmax, qmax, dtype=np.float32) + np.float32(0.5)) * step
+    v = np.concatenate([half, np.nextafter(half, np.float32(np.inf)), np.nextafter(half, np.float32(-np.inf))]).astype(np.float32)
+    v = np.concatenate([v, np.full((-v.size - 8) % 16, 0, np.float32), np.full(8, step * np.float32(qmax), np.float32)])
+    t = torch.from_numpy(np.tile(v, (4, 1)))
+    codes, steps = ops.hq_rowwise(t.to(gpu), n=1, bits=bits, scale="row")
+    d = np.float32(np.float32(np.max(np.abs(v))) / np.float32(qmax))
+    assert np.array_equal(steps.cpu().numpy(), np.full(4, d))
+    ref = np.rint(v / np.float32(d + np.float32(1e-11))).astype(np.int64)
+    got = codes.cpu().numpy().astype(np.int64)
+    if bits == 4:
+        lo, hi = got & 15, (got >> 4) & 15
+        got = np.stack([lo, hi], -1).reshape(4, -1)
+        got = np.where(got > 7, got - 16, got)
+    assert np.array_equal(got, np.tile(ref, (4, 1)))
+    # the same values along the tokens (blocks of one): the column-wise body
+    col, sc, kout = ops.hla_tokenwise(torch.from_numpy(np.tile(v[:, None], (1, 8))).to(gpu), 1, (0,), bits=bits)
+    assert np.array_equal(col.cpu().numpy()[:, :kout].astype(np.int64), np.tile(ref, (8, 1)))
