@@ -312,6 +312,16 @@ static int dispatch_sawb(const ColJob& job, int pass, hipStream_t st) {
   return fail(HOT_ERR_INVALID, "colwise: bad selection %d", (int)job.sel);
 }
 
+// Whether the workgroups of a token-wise quantise pass run the row-wise quantiser of the same tensor too: from three of
+// them per CU on, where they fill the chip alone (us of the quantise phase, joined / as a job of its own: 12608 x 3072
+// bf16 39 / 46.5, 12608 x 2304 fp32 47.5 / 55, 8192 x 11008 bf16 101 / 130; below that the separate workgroups are what
+// fills it: 3003 x 1000 fp16 13.6 / 12.9).
+static bool row_job_joins(const ColJob& g, const HqArgs& h) {
+  if (col_job_blocks(g, 1) < 768) return false;
+  if (g.sel == COL_RT32 || g.sel == COL_RT64 || g.sel == COL_RT128) return false;   // (no registers to spare)
+  return !h.per_row && h.groups == 1 && g.a.groups == 1 && g.a.in == h.in && g.a.R == h.M && g.a.C == h.K;
+}
+
 int phase_launch(int pass, int dtype, const ColJob* g, const ColJob* w, const HqArgs* h, const ColsumArgs* s, hipStream_t st) {
   if (g && g->a.mode == HOT_SCALE_SAWB) {
     // a SAWB token-wise job has kernels of its own and comes alone
@@ -333,7 +343,11 @@ int phase_launch(int pass, int dtype, const ColJob* g, const ColJob* w, const Hq
   size_t lds = 0;
   if (g) { p.g = col_job_args(*g, pass); p.g_blocks = col_job_blocks(*g, pass); lds = g->lds[pass]; }
   if (w) { p.w = col_job_args(*w, pass); p.w_blocks = col_job_blocks(*w, pass); if (w->lds[pass] > lds) lds = w->lds[pass]; }
-  if (h) { p.h = *h; p.h_blocks = (uint32_t)hq_body_blocks(*h); }
+  if (h) {
+    p.h = *h;
+    if (g && row_job_joins(*g, *h)) p.h_in_g = 1;
+    else p.h_blocks = (uint32_t)hq_body_blocks(*h);
+  }
   if (s) { p.s = *s; p.s_blocks = (uint32_t)((s->C + CS_CHANS - 1) / CS_CHANS); if (lds < CS_GROUPS * CS_CHANS * 4) lds = CS_GROUPS * CS_CHANS * 4; }
   const ColSel sel = g ? g->sel : COL_SHORT;
   switch (dtype) {

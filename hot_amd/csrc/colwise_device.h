@@ -3,8 +3,7 @@
 // the data moves is described in colwise.hip.
 #pragma once
 
-#include "hot_device.h"
-#include "hot_host.h"
+#include "hq_device.h"
 
 #include <type_traits>
 
@@ -210,9 +209,14 @@ __device__ __forceinline__ void rs_column(const uint8_t* wave_buf, int lane, flo
 // needs no statistics pass of its own.  Adjacent lanes hold adjacent channels, hence the row-wise
 // butterflies run across lanes.
 // ROUND and SAWB: 0 / 1, or 2 = as the arguments say.
+// HQ (quantise pass): with `hq` the pass is the row-wise quantiser of the same input as well (one step per tensor,
+// Hadamard blocks of up to 16, the rounding of this pass): a wave takes the rows of a step a second time from its
+// slice of the ring, lane = 16 channels of one row, instead of the input being read again by workgroups of their own
+// (quantise phase at 12608 x 3072 bf16 46.5 -> 39 us, at 8192 x 11008 130 -> 101 us; 19 vector instructions per element
+// and the K-major stores bound it now: without the stores 34 and 84 us).
 constexpr int RUNTIME = 2;
-template <typename T, int N, int PASS, int ROUND, int SAWB, typename SEL, bool RS = false>
-__device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, uint8_t* lds) {
+template <typename T, int N, int PASS, int ROUND, int SAWB, typename SEL, bool RS = false, bool HQ = false>
+__device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, uint8_t* lds, const HqArgs* hq = nullptr) {
   constexpr bool SHORT = std::is_same<SEL, SelShort>::value || std::is_same<SEL, SelShortFull>::value;
   static_assert(!SHORT || N == CW_ROWS, "short blocks are handled 16 rows at a time");
   constexpr int SPB = N >= CW_ROWS ? N / CW_ROWS : 1;        // steps per token block
@@ -355,6 +359,75 @@ __device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, u
   }
   const float rcpk = rcp * 65536.0f;       // stochastic rounding works in units of 2^-16
 
+  // row-wise quantiser: lane = 16 channels (two chunks) of row lane / 4 of a step
+  constexpr bool HQP = PASS == 1 && HQ;
+  float hd = 1.f, hrcp = 1.f;
+  int8_t* hout = nullptr;
+  int64_t hstep = 0;
+  uint64_t hoct = 0;
+  int hvalid = 0, hpad = 0, hcb = 0;   // chunks of this lane that exist; bytes to clear behind a row (the last strip's); bytes of a chunk
+  if constexpr (HQP) {
+    if (hq) {
+      __shared__ float s_hq[CW / 64];
+      float m = wave_max(part_max(hq->stat, hq->nstat, hq->stat_stride, tid));
+      if (lane == 0) s_hq[wave] = m;
+      __syncthreads();
+      m = fmaxf(fmaxf(s_hq[0], s_hq[1]), fmaxf(s_hq[2], s_hq[3]));
+      const float sc = m / (float)((1 << (hq->bits - 1)) - 1);
+      hd = sc + 1e-11f;
+      hrcp = 1.0f / hd;
+      if (wg_lin == 0 && tid == 0) hq->scales[0] = sc;
+      const int64_t row = row0 + (lane >> 2), ch = cg0 + 64 * wave + (lane & 3) * 16;
+      const int64_t left = (a.C - ch) / EPL;
+      hvalid = left <= 0 ? 0 : left == 1 ? 1 : 2;
+      hcb = hq->bits;
+      hout = hq->codes + row * hq->ld + ch / EPL * hcb;
+      hstep = CW_ROWS * hq->ld;
+      hoct = ((uint64_t)row * (uint64_t)a.C + (uint64_t)ch) >> 3;
+      if (bx + 1 == a.gx && wave == 0) hpad = (int)(hq->ld - a.C / EPL * hcb);
+    }
+  }
+  auto row_quant = [&](int s) {
+    const T* p = reinterpret_cast<const T*>(my + (s % CW_DEPTH) * BUF) + (lane >> 2) * 64 + (lane & 3) * 16;
+    float y[16];
+    load_chunk<T>(p, y);
+    load_chunk<T>(p + EPL, y + EPL);
+    fwht_short(y, hq->n, 1);
+    uint32_t q[16];
+    if constexpr (ROUND == HOT_ROUND_NEAREST) {
+      const rint_rcp hb = rint_bounds(hrcp);
+      uint32_t unsure = 0;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) q[j] = rint_div_bits(y[j], hb, unsure);
+      if (__builtin_expect(unsure != 0, 0)) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) q[j] = rint_div_exact(y[j], hd, hrcp);
+      }
+    } else {
+      const int hmax = (1 << (hq->bits - 1)) - 1;
+      quant_stoch(y, hrcp, hoct << 3, hq->seed, hq->stream, hmax, q);
+      quant_stoch(y + EPL, hrcp, (hoct + 1) << 3, hq->seed, hq->stream, hmax, q + EPL);
+      hoct += (uint64_t)a.C * (CW_ROWS / EPL);
+    }
+    const bool row_in = s * CW_ROWS + (lane >> 2) < rows_wg;
+    if (hcb == 4) {
+      uint2 w;
+      w.x = pack_codes4(q);
+      w.y = pack_codes4(q + EPL);
+      if (row_in && hvalid == 2) *reinterpret_cast<uint2*>(hout) = w;
+      else if (row_in && hvalid == 1) *reinterpret_cast<uint32_t*>(hout) = w.x;
+    } else {
+      const uint2 w0 = pack_codes8(q), w1 = pack_codes8(q + EPL);
+      if (row_in && hvalid == 2) *reinterpret_cast<uint4*>(hout) = make_uint4(w0.x, w0.y, w1.x, w1.y);
+      else if (row_in && hvalid == 1) *reinterpret_cast<uint2*>(hout) = w0;
+    }
+    if (hpad && row_in) {
+      int8_t* const tail = hout + (a.C - cg0) / EPL * hcb - (lane & 3) * 2 * hcb;
+      for (int b = (lane & 3) * 4; b < hpad; b += 16) *reinterpret_cast<uint32_t*>(tail + b) = 0u;
+    }
+    hout += hstep;
+  };
+
   float cmax = 0.f, rmax = 0.f, csum = 0.f;
   double ssq = 0.0, sab = 0.0;
   float x[XL];
@@ -393,13 +466,21 @@ __device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, u
       if (nearest) {
         // |v / d| <= qmax (1 + 2^-22) by construction of d (absmax) or of the clip (SAWB): the rounded code cannot
         // leave [-qmax, qmax]
-        float dev = 0.f;
+        const rint_rcp b = rint_bounds(rcp);
+        uint32_t unsure = 0;
+        if constexpr (N >= 64 && SEL::STATIC) {
+          // the coefficients are complete here: the compiler would sink the last butterfly stage into both
+          // branches and hold its inputs until then (half as many registers again)
+#pragma unroll
+          for (int i = 0; i < N; ++i)
+            if (SEL::slot(i) >= 0) asm volatile("" : "+v"(x[base + i]));
+        }
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           const int sl = place(i);
-          if (sl >= 0) row[sl] = (uint8_t)rint_div_bits(x[base + i], rcp, dev);
+          if (sl >= 0) row[sl] = (uint8_t)rint_div_bits(x[base + i], b, unsure);
         }
-        if (__builtin_expect(rint_unsure(dev), 0)) {
+        if (__builtin_expect(unsure != 0, 0)) {
 #pragma unroll
           for (int i = 0; i < N; ++i) {
             const int sl = place(i);
@@ -500,7 +581,8 @@ __device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, u
   const float sg4 = (chan & 4) ? -1.f : 1.f, sg8 = (chan & 8) ? -1.f : 1.f;
   auto step = [&](int s, float* dst) {
     // this wave's rows of step s have landed, and its LDS reads of step s-1 are complete: the
-    // slice that held step s-1 may be refilled.  Steps s+1 .. s+CW_DEPTH-2 may still be in flight.
+    // slice that held step s-1 may be refilled.  Steps s+1 .. s+CW_DEPTH-2 may still be in flight.  (Row stores sit
+    // among them and only make the wait a little stricter: counting them in changed nothing measurable.)
     if (CW_DEPTH >= 4 && s + 2 < nsteps) wait_stream<2 * LPW>();
     else if (CW_DEPTH >= 3 && s + 1 < nsteps) wait_stream<LPW>();
     else wait_stream<0>();
@@ -567,6 +649,10 @@ __device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, u
           if (i < valid) rmax = fmaxf(rmax, fabsf(t[i]));
       }
       return;
+    }
+    if constexpr (HQP) {
+      if (hq) row_quant(s);
+      __builtin_amdgcn_sched_barrier(0);     // (its registers are free again before the columns are read)
     }
     rs_column<T>(my + (s % CW_DEPTH) * BUF, lane, dst);
   };

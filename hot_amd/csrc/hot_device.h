@@ -229,17 +229,19 @@ __device__ __forceinline__ float part_max(const float* p, int n, int stride, int
 }
 
 // rint(x / d) with rcp = 1 / d (correctly rounded) for |x / d| <= 128, in three instructions, almost always: adding
-// 1.5 * 2^23 in the fused multiply-add rounds x * rcp to an integer, whose two's complement stands in the low bits of
-// the sum.  x * rcp is within 2^-17 of x / d and the fp32 quotient within 2^-18, so both round to the same
-// integer unless x * rcp lies within 2^-16 of a half-integer: `dev` collects the largest distance from the chosen
-// integer, and where rint_unsure(dev) says so the caller takes rint_div_exact for the values it covers.
+// 1.5 * 2^23 in the fused multiply-add rounds a product to an integer, whose two's complement stands in the low bits of
+// the sum.  It is done with a reciprocal 2^-22 too small and with one 2^-22 too large: the fp32 quotient lies between the
+// two products (rcp and the quotient are each within 2^-24), so where both round to the same integer the quotient does
+// too.  `unsure` is zero while they do; otherwise (two quotients in a million) the caller takes rint_div_exact for the
+// values it covers.  (Each difference is below 2^24: up to 256 values to an `unsure`.)
 constexpr float RINT_MAGIC = 12582912.0f;
-__device__ __forceinline__ uint32_t rint_div_bits(float x, float rcp, float& dev) {
-  const float t = __builtin_fmaf(x, rcp, RINT_MAGIC);
-  dev = fmaxf(dev, fabsf(__builtin_fmaf(x, rcp, -(t - RINT_MAGIC))));
-  return as_u(t);
+struct rint_rcp { float lo, hi; };
+__device__ __forceinline__ rint_rcp rint_bounds(float rcp) { return {rcp * (1.0f - 2.384185791015625e-07f), rcp * (1.0f + 2.384185791015625e-07f)}; }
+__device__ __forceinline__ uint32_t rint_div_bits(float x, const rint_rcp& r, uint32_t& unsure) {
+  const uint32_t lo = as_u(__builtin_fmaf(x, r.lo, RINT_MAGIC)), hi = as_u(__builtin_fmaf(x, r.hi, RINT_MAGIC));
+  unsure = (lo ^ hi) + unsure;
+  return lo;
 }
-__device__ __forceinline__ bool rint_unsure(float dev) { return dev > 0.5f - 1.52587890625e-05f; }
 // The same with the IEEE quotient, without a division: two residual corrections of x * rcp.  The first leaves a
 // quotient within an ulp, from which the second gives the correctly rounded one (Markstein: its residual is exact and
 // rcp is the rounded reciprocal).

@@ -59,10 +59,11 @@ __device__ __forceinline__ void fwht_lanes(float* x, int lane, int nrt) {
 // Codes of a chunk, in the low bits of q.
 __device__ __forceinline__ void quant_nearest(const float* x, float d, float rcp, uint32_t* q) {
   // |x / d| <= qmax (1 + 2^-22) because d comes from the absmax: no clamp needed
-  float dev = 0.f;
+  const rint_rcp r = rint_bounds(rcp);
+  uint32_t unsure = 0;
 #pragma unroll
-  for (int j = 0; j < EPL; ++j) q[j] = rint_div_bits(x[j], rcp, dev);
-  if (__builtin_expect(rint_unsure(dev), 0)) {
+  for (int j = 0; j < EPL; ++j) q[j] = rint_div_bits(x[j], r, unsure);
+  if (__builtin_expect(unsure != 0, 0)) {
 #pragma unroll
     for (int j = 0; j < EPL; ++j) q[j] = rint_div_exact(x[j], d, rcp);
   }
@@ -79,13 +80,15 @@ __device__ __forceinline__ uint32_t pack_bytes(uint32_t a, uint32_t b, uint32_t 
   const uint32_t lo = __builtin_amdgcn_perm(b, a, 0x0C0C0400u), hi = __builtin_amdgcn_perm(d, c, 0x04000C0Cu);
   return lo | hi;
 }
-__device__ __forceinline__ void store_codes4(const uint32_t* q, int8_t* out) {
+__device__ __forceinline__ uint32_t pack_codes4(const uint32_t* q) {
   const uint32_t ev = pack_bytes(q[0], q[2], q[4], q[6]), od = pack_bytes(q[1], q[3], q[5], q[7]);
-  *reinterpret_cast<uint32_t*>(out) = (ev & 0x0F0F0F0Fu) | ((od << 4) & 0xF0F0F0F0u);
+  return (ev & 0x0F0F0F0Fu) | ((od << 4) & 0xF0F0F0F0u);
 }
-__device__ __forceinline__ void store_codes8(const uint32_t* q, int8_t* out) {
-  *reinterpret_cast<uint2*>(out) = make_uint2(pack_bytes(q[0], q[1], q[2], q[3]), pack_bytes(q[4], q[5], q[6], q[7]));
+__device__ __forceinline__ uint2 pack_codes8(const uint32_t* q) {
+  return make_uint2(pack_bytes(q[0], q[1], q[2], q[3]), pack_bytes(q[4], q[5], q[6], q[7]));
 }
+__device__ __forceinline__ void store_codes4(const uint32_t* q, int8_t* out) { *reinterpret_cast<uint32_t*>(out) = pack_codes4(q); }
+__device__ __forceinline__ void store_codes8(const uint32_t* q, int8_t* out) { *reinterpret_cast<uint2*>(out) = pack_codes8(q); }
 
 template <int BITS, int ROUND>
 __device__ __forceinline__ void quant_store_chunk(const float* x, float d, float rcp, uint64_t e0, uint64_t seed,

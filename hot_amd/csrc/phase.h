@@ -59,6 +59,7 @@ struct PhaseArgs {
   ColsumArgs s;         // the bias gradient (quantise phase only)
   uint32_t g_blocks, w_blocks, h_blocks, s_blocks;   // workgroups of each; 0 = absent (g and w: multiples of 8, so that
                                                      // a job's workgroup number modulo 8 stays its XCD)
+  int32_t h_in_g;       // quantise phase: g's workgroups run the row-wise job too (h_blocks = 0)
 };
 
 // Which instance a block length and selection takes; the caller has filled a.slot.

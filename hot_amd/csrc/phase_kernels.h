@@ -16,8 +16,13 @@ __device__ __forceinline__ const PhaseArgs& phase_args() {
   return *(const PhaseArgs*)k;
 }
 
+// Wavefronts per SIMD that the registers leave room for: three (what the LDS allows in the quantise pass) wherever a
+// thread's block and its selection are small enough to be held without spilling.
+template <int N, typename SEL> constexpr int phase_waves() {
+  return !std::is_same<SEL, SelRuntime>::value ? 3 : N <= 32 ? 3 : N == 64 ? 2 : 1;
+}
 template <typename T, int N, int PASS, int ROUND, typename SEL, bool RS>
-__global__ void __launch_bounds__(CW) phase_kernel(const PhaseArgs p) {
+__global__ void __launch_bounds__(CW, (phase_waves<N, SEL>())) phase_kernel(const PhaseArgs p) {
   extern __shared__ __align__(16) uint8_t lds[];
   unsigned b = blockIdx.x;
   // the short jobs first: they end early and the long one's workgroups fill in behind them
@@ -27,7 +32,7 @@ __global__ void __launch_bounds__(CW) phase_kernel(const PhaseArgs p) {
   }
   b -= p.w_blocks;
   if (PASS == 0 || b < p.g_blocks) {
-    colwise_body<T, N, PASS, ROUND, 0, SEL, RS>(phase_args().g, b, lds);
+    colwise_body<T, N, PASS, ROUND, 0, SEL, RS, PASS == 1 && !std::is_same<SEL, SelRuntime>::value>(phase_args().g, b, lds, p.h_in_g ? &phase_args().h : nullptr);
     return;
   }
   if constexpr (PASS == 1) {

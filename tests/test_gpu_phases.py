@@ -31,6 +31,15 @@ def test_short_hadamard_blocks(gpu, n_o, O, variant):
     check(gpu, 66, O, 40, torch.bfloat16 if O % 48 else torch.float32, n_o=n_o, **variant)
 
 
+@pytest.mark.parametrize("L,O,I", [(2999, 2056, 24), (3006, 2064, 16), (6416, 2048, 8), (6464, 2056, 8), (13952, 2064, 8)])
+@pytest.mark.parametrize("dt,variant", [(torch.bfloat16, dict()), (torch.float32, dict(gx_bits=8, w_bits=8, **STOCH)),
+                                        (torch.float16, dict(gw_scale=orc.SCALE_ROW)), (torch.float32, dict())])
+def test_row_quantiser_in_the_token_pass(gpu, L, O, I, dt, variant):
+    """Tensors of 768 workgroups and more, whose token-wise pass runs the row-wise quantiser too: token blocks of 1, 2, 16, 64
+    and 128, a last strip of 8 or 16 channels, row tails to clear, row groups cut short."""
+    check(gpu, L, O, I, dt, n_o=min(16, O & -O), **variant)
+
+
 @pytest.mark.parametrize("L", [2, 6, 12, 24, 40, 48, 160, 320])
 @pytest.mark.parametrize("variant", [dict(), dict(gw_scale=orc.SCALE_ROW, act_scale=orc.SCALE_SAWB), STOCH])
 def test_short_token_blocks(gpu, L, variant):
