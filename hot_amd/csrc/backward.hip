@@ -377,7 +377,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
                           cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, I};
   const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
                           1.0f / (float)cfg->hla_n, gw, I};
-  if (!split && cfg->streams != 2 && gemm_pair_possible(pw, px)) {
+  if (!split && cfg->streams != 2 && gemm_pair_possible(pw, px) && gemm_pair_pays(pw, px)) {
     rc = gemm_pair_impl(pw, px, out_dtype, st);
     if (!rc && marks) mark(STAGE_GEMM);
     return rc;

@@ -1476,6 +1476,18 @@ bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
   return w.bits == 8 && fits(w) && fits(x);
 }
 
+// A g_x product of few tiles with a long K is a chain of stages that nothing else in the pair covers (0.9 us for each
+// 256 codes of a 128 x 128 INT4 tile): such a product goes by itself, cut into K ranges or into shorter tiles by its own
+// plan.  The line is where 168 shapes of 49 .. 16383 tokens and 64 .. 10624 channels are at most 14 % and on average 0.4 %
+// slower than the better of the two; us of both products, pair / apart: 2758 x 128 x 8520 INT4 32.0 / 26.2, 197 x 1024 x
+// 10624 45.1 / 29.3, INT8 63.7 / 34.1, 1001 x 768 x 3072 INT8 23.8 / 19.0; 2758 x 768 x 3072 INT4 20.6 / 28.5,
+// 4583 x 128 x 4096 21.4 / 27.6, 8191 x 128 x 8520 35.4 / 45.2.
+bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
+  auto stages = [](const GemmProduct& p) { return round_up(p.K, GEMM_KTILE) * p.bits / 8 / 128; };
+  const int64_t x_tiles = ((x.M + 127) / 128) * ((x.N + 127) / 128);
+  return x_tiles > 192 || stages(x) < 14 || stages(x) < 2 * stages(w);
+}
+
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
   PairArgs p;
   if (int rc = gemm_fill(p.w, w, out_dtype, nullptr)) return rc;

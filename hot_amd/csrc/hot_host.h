@@ -122,6 +122,7 @@ struct GemmProduct {
   void* out; int64_t ldo;
 };
 bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x);
+bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x);   // and where they are faster in one launch
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st);
 int gemm_bf16_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N, int64_t K,
                    const void* bias, void* out, int out_dtype, int64_t ldo, hipStream_t st, int variant);

@@ -55,11 +55,12 @@ def test_row_quantiser_widths(gpu, O, dt):
 
 
 @pytest.mark.parametrize("L,O,I", [(1, 16, 8), (127, 64, 128), (129, 80, 136), (64, 3072, 2048), (64, 3056, 2048), (192, 192, 128),
-                                   (200, 400, 264)])
+                                   (200, 400, 264), (40, 3328, 136), (40, 3584, 136), (1800, 1792, 16), (300, 1664, 16)])
 @pytest.mark.parametrize("dt,bits", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 4)])
 def test_paired_products(gpu, L, O, I, dt, bits):
     """Tile edges of the paired products, either side of the line between their two tilings (256 tiles of 192 x 128 of
-    g_W: 3072 x 2048), K shorter than the ring."""
+    g_W: 3072 x 2048), K shorter than the ring; g_x products of few tiles on either side of the length of K (14 stages, twice
+    those of g_W) from which the two go apart."""
     check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
 
 
