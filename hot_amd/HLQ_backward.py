@@ -27,6 +27,7 @@ gx_rounding = "stoch"
 other_rounding = "nearest"
 hla_max_block = 8192     # see hot_amd.args.hla_max_block
 seed = 0
+_OPTIONS: dict = {}      # options() per token count and setting
 
 
 def _check(t: torch.Tensor, name: str) -> None:
@@ -39,14 +40,21 @@ def _check(t: torch.Tensor, name: str) -> None:
 
 
 def options(L: int, H_size: int, per_token: bool) -> ops.HotOptions:
+    key = (L, H_size, per_token, gx_bits, gw_bits, gx_rounding, other_rounding, hla_max_block, seed)
+    hit = _OPTIONS.get(key)
+    if hit is not None:
+        return hit
     n, rows = hla_rows(L)
     if n > hla_max_block:
         n, rows = hla_rows(hla_max_block)
-    return ops.HotOptions(
+    if len(_OPTIONS) >= 4096:
+        _OPTIONS.clear()
+    opt = _OPTIONS[key] = ops.HotOptions(
         n_o=int(H_size), hla_n=int(n), hla_rows=tuple(int(v) for v in rows),
         gx_bits=gx_bits, w_bits=gx_bits, gw_bits=gw_bits, act_bits=gw_bits,
         gx_round=gx_rounding, w_round=other_rounding, gw_round=other_rounding, act_round=other_rounding,
         gx_scale="row" if per_token else "tensor", seed=seed)
+    return opt
 
 
 def backward(Go: torch.Tensor, W: torch.Tensor, X: torch.Tensor, reorder_idx_go=0, reorder_idx_X=0,

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
-from dataclasses import dataclass, field, replace
+from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -41,12 +41,27 @@ def _need_gpu_2d(t: torch.Tensor, name: str) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # (the handle alone: building a torch.cuda.Stream around it takes 3 us, a fifth of a small call)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _ws(nbytes: int, device) -> torch.Tensor:
     # torch allocations are at least 512-byte aligned
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
+
+
+def _size(opt: "HotOptions", entry: str, *shape: int) -> int:
+    """A size query of the library (hot_<entry>), which is a pure function of the options and the shape: kept per options."""
+    sizes = opt.__dict__.setdefault("_ws_bytes", {})
+    key = (entry,) + shape
+    n = sizes.get(key)
+    if n is None:
+        if len(sizes) >= 4096:
+            sizes.clear()
+        n = int(getattr(_lib.lib(), "hot_" + entry)(*shape, C.byref(opt.to_c())))
+        if n > 0:
+            sizes[key] = n
+    return n
 
 
 @functools.lru_cache(maxsize=4096)
@@ -88,8 +103,10 @@ class HotOptions:
         seed = int(seed)
         if seed == self.seed:
             return self
-        other = replace(self, seed=seed)
         base = self.to_c()
+        self.__dict__.setdefault("_ws_bytes", {})     # (shared: no size depends on the seed)
+        other = object.__new__(HotOptions)
+        other.__dict__.update(self.__dict__, seed=seed)
         c = _lib.HotConfig.from_buffer_copy(base)
         c.seed = seed & 0xFFFFFFFFFFFFFFFF
         object.__setattr__(other, "_c", c)
@@ -289,7 +306,7 @@ def abc_forward(x: torch.Tensor, opt: HotOptions, side: Optional["torch.cuda.Str
     with _on_stream(side):
         xq = torch.empty((I, kpad(opt.lprime(L))), dtype=torch.int8, device=x.device)
         sx = torch.empty((1,), dtype=torch.float32, device=x.device)
-        ws = _ws(_lib.lib().hot_abc_workspace_bytes(L, I, C.byref(cfg)), x.device)
+        ws = _ws(_size(opt, "abc_workspace_bytes", L, I), x.device)
     try:
         _lib.check(_lib.lib().hot_abc_forward(x.data_ptr(), _dt(x), L, I, C.byref(cfg), xq.data_ptr(), sx.data_ptr(),
                                               ws.data_ptr(), ws.numel(), _launch_stream(side)))
@@ -318,13 +335,9 @@ def linear_backward(gy: torch.Tensor, w: torch.Tensor, xq: torch.Tensor, sx: tor
     lp = opt.lprime(L)
     if tuple(xq.shape) != (I, kpad(lp)) or xq.dtype != torch.int8:
         raise RuntimeError("xq must be the int8 [I, kpad(L')] buffer written by abc_forward")
-    sizes = opt.__dict__.setdefault("_ws_bytes", {})      # per options object: the query is a pure function of these
-    need = sizes.get((L, O, I))
-    if need is None:
-        need = _lib.lib().hot_backward_workspace_bytes(L, O, I, C.byref(cfg))
-        if need == 0:
-            raise HotError("bad configuration: %s" % _lib.lib().hot_last_error().decode())
-        sizes[(L, O, I)] = need
+    need = _size(opt, "backward_workspace_bytes", L, O, I)
+    if need == 0:
+        raise HotError("bad configuration: %s" % _lib.lib().hot_last_error().decode())
     if workspace is None or workspace.numel() < need:
         workspace = _ws(need, gy.device)
     gx = torch.empty((L, I), dtype=out_dtype, device=gy.device)
@@ -355,7 +368,7 @@ def backward_streams(L: int, O: int, I: int, opt: HotOptions) -> int:
 
 def kpad_group(T: int, opt: HotOptions) -> int:
     """Code bytes every sample takes in the K dimension of the batched g_W operands."""
-    return int(_lib.lib().hot_kpad_group(int(T), C.byref(opt.to_c())))
+    return _size(opt, "kpad_group", int(T))
 
 
 def backward_batched_ranges(B: int, T: int, O: int, I: int, opt: HotOptions) -> int:
@@ -375,7 +388,7 @@ def abc_forward_batched(x: torch.Tensor, opt: HotOptions, side: Optional["torch.
     with _on_stream(side):
         xq = torch.empty((I, B * kg), dtype=torch.int8, device=x.device)
         sx = torch.empty((B,), dtype=torch.float32, device=x.device)
-        ws = _ws(_lib.lib().hot_abc_batched_workspace_bytes(B, T, I, C.byref(cfg)), x.device)
+        ws = _ws(_size(opt, "abc_batched_workspace_bytes", B, T, I), x.device)
     try:
         _lib.check(_lib.lib().hot_abc_forward_batched(x.data_ptr(), _dt(x), B, T, I, C.byref(cfg), xq.data_ptr(),
                                                       sx.data_ptr(), ws.data_ptr(), ws.numel(), _launch_stream(side)))
@@ -400,7 +413,7 @@ def linear_backward_batched(gy: torch.Tensor, w: torch.Tensor, xq: torch.Tensor,
     kg = kpad_group(T, opt)
     if tuple(xq.shape) != (I, B * kg) or xq.dtype != torch.int8 or sx.numel() != B:
         raise RuntimeError("xq / sx must be the buffers written by abc_forward_batched")
-    need = _lib.lib().hot_backward_batched_workspace_bytes(B, T, O, I, C.byref(cfg))
+    need = _size(opt, "backward_batched_workspace_bytes", B, T, O, I)
     if need == 0:
         raise HotError("bad configuration: %s" % _lib.lib().hot_last_error().decode())
     if workspace is None or workspace.numel() < need:

@@ -1108,6 +1108,13 @@ def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_arg
         qm.overlap_buffer_write = True
 
 
+def test_hq_linear_small_inputs_beside_the_product(gpu, fresh_args, monkeypatch):
+    """The same with the side stream taken by inputs of every size (by default it begins at 24 MiB)."""
+    from hot_amd import quant_matmul as qm
+    monkeypatch.setattr(qm, "OVERLAP_MIN_BYTES", 0)
+    test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_args)
+
+
 @pytest.mark.parametrize("gw_bits,act_bits", [(4, 8), (4, 4), (8, 4)])
 @pytest.mark.parametrize("path", ["luq", "low_rank"])
 def test_hq_linear_gw_widths_on_the_separate_gx_paths(gpu, fresh_args, path, gw_bits, act_bits):
