@@ -40,7 +40,7 @@ def _check(t: torch.Tensor, name: str) -> None:
 
 
 def options(L: int, H_size: int, per_token: bool) -> ops.HotOptions:
-    key = (L, H_size, per_token, gx_bits, gw_bits, gx_rounding, other_rounding, hla_max_block, seed)
+    key = (int(L), int(H_size), bool(per_token), gx_bits, gw_bits, gx_rounding, other_rounding, hla_max_block, seed)
     hit = _OPTIONS.get(key)
     if hit is not None:
         return hit

@@ -200,6 +200,14 @@ def test_hlq_backward_checks_like_the_reference():
         HLQ_backward.backward(z, z, z, 0, 0, 16, True)
 
 
+def test_hlq_options_follow_the_value_of_the_block_size():
+    from hot_amd import HLQ_backward
+    size = torch.tensor(16)
+    assert HLQ_backward.options(48, size, True).n_o == 16
+    size.fill_(8)
+    assert HLQ_backward.options(48, size, True).n_o == 8
+
+
 # --------------------------------------------------------------- the C ABI
 
 def _declared():
