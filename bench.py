@@ -130,13 +130,13 @@ def kernel_table(w, sets, bufs, opt, ws, iters, warm, traffic=None):
             acc = [a + b for a, b in zip(acc, t)]
     us = [a / iters * 1e6 for a in acc]
     spec = [
-        ("clear", "hot::clear3_kernel", us[0], "hbm", 0.0),
-        ("gy_stats", "hot::colwise_kernel<.., PASS 0, RS 16> (g_y: token-wise + row-wise absmax)", us[1], "hbm", L * O * e),
-        ("gy_hla_quant", "hot::colwise_kernel<.., PASS 1> (g_y: HLA + INT8, transposed)", us[2], "hbm", L * O * e + lp * O),
-        ("gy_hq_quant", "hot::hq_tensor_kernel (g_y: Hadamard-16 + INT%d)" % opt.gx_bits, us[3], "hbm",
+        ("clear", "clear of the statistics that are updated by atomics (no launch for most calls)", us[0], "hbm", 0.0),
+        ("gy_stats", "hot::phase_kernel<.., PASS 0, RS> (g_y: token-wise + row-wise absmax)", us[1], "hbm", L * O * e),
+        ("gy_hla_quant", "hot::phase_kernel<.., PASS 1> (g_y: HLA + INT8, transposed)", us[2], "hbm", L * O * e + lp * O),
+        ("gy_hq_quant", "hot::phase_kernel, row-wise job (g_y: Hadamard-16 + INT%d)" % opt.gx_bits, us[3], "hbm",
          L * O * e + L * O * opt.gx_bits // 8),
-        ("w_stats", "hot::colwise_kernel<.., PASS 0> (W)", us[4], "hbm", O * I * e),
-        ("w_quant", "hot::colwise_kernel<.., PASS 1> (W: Hadamard-16 + INT%d, transposed)" % opt.w_bits, us[5], "hbm",
+        ("w_stats", "hot::phase_kernel<.., PASS 0>, column-wise job (W)", us[4], "hbm", O * I * e),
+        ("w_quant", "hot::phase_kernel<.., PASS 1>, column-wise job (W: Hadamard-16 + INT%d, transposed)" % opt.w_bits, us[5], "hbm",
          O * I * e + O * I * opt.w_bits // 8),
         ("gemm_gx", "hot::%s INT%d (g_x)" % (gemm_kernel_name(L, I, O, opt.gx_bits), opt.gx_bits), us[6], "mfma", 2.0 * L * O * I),
         ("gemm_gw", "hot::%s INT8 (g_W)" % gemm_kernel_name(O, I, lp, 8, with_ws=True)
@@ -388,8 +388,8 @@ def scheme_table(dev):
 def host_cost(dev, calls=300):
     """Host time of one backward call: the C entry point through ctypes with prepared arguments, and
     ops.linear_backward, at a shape whose kernels are short (64 tokens, O = I = 64), issued back to back
-    without waiting for the GPU, in the one-stream order (what the library picks for short calls) and
-    with the two-stream order forced (three event record / wait pairs more)."""
+    without waiting for the GPU, in the order that the library picks for short calls and with the
+    products forced apart, g_x on the side stream (two event record / wait pairs more)."""
     import ctypes as C
     import time
     import torch
@@ -647,8 +647,8 @@ def main():
             out["ceilings"] = {"error": repr(e)[:200]}
         # Roofline entry: the single launch with the longest duration inside the step, measured with
         # HIP events on the launch stream around every kernel group, the groups launched one after
-        # the other (the timed steps above overlap independent kernels on two streams, which
-        # stretches each of them; a kernel's own duration is the serial one).  A group of two
+        # the other (in the timed steps above independent jobs share launches; a job's own
+        # duration is the serial one).  A group of two
         # launches, the split-K GEMM and its reduce kernel, is not one kernel and stands in the
         # table only.  The same two GEMMs launched back to back, without the neighbouring
         # kernels, are reported beside it.

@@ -89,7 +89,7 @@ class HotOptions:
     gw_scale: int = SCALE_TENSOR
     act_scale: int = SCALE_TENSOR
     seed: int = 0
-    streams: int = 0      # launch order of the backward: 0 = the library's rule, 1 = one stream, 2 = with its side stream
+    streams: int = 0      # launch order of the backward: 0 = the library's rule, 1 = one stream, 2 = products apart, with its side stream
 
     @property
     def hla_r(self) -> int:

@@ -102,16 +102,18 @@ typedef struct hot_config {
                                   they take a two-level transform through an fp32
                                   workspace (launches only: capturable)          */
   int32_t streams;  /* launch order of hot_linear_backward(_bias): 0 = the library's rule
-                       (hot_backward_streams), 1 = every kernel on the caller's stream, 2 =
-                       independent kernels also on the library's side stream (forked and joined by
-                       events).  The results do not depend on it.                               */
+                       (both products in one launch where their operands allow it, else
+                       hot_backward_streams), 1 = every kernel on the caller's stream, 2 =
+                       the products apart, g_x on the library's side stream when g_W cannot fill
+                       the chip (forked and joined by events).  The results do not depend on it. */
   int32_t reserved; /* 0 */
 } hot_config;
 
 HOT_API const char* hot_last_error(void);
-/* 1 or 2: the launch order hot_linear_backward takes for this shape (cfg->streams when it is 1 or 2).
- * Short calls, whose kernels take less time than the host needs for the event operations that fork
- * and join the side stream, run on one stream; long ones overlap their independent kernels. */
+/* 1 or 2: the launch order hot_linear_backward takes for this shape when its two products do not share a
+ * launch (cfg->streams when it is 1 or 2).  Short calls, whose kernels take less time than the host needs
+ * for the event operations that fork and join the side stream, run on one stream; in long ones the g_x
+ * product may run beside the g_W product. */
 HOT_API int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_abi_version(void);
 
@@ -229,12 +231,12 @@ HOT_API int hot_abc_forward(const void* x, int dtype, int64_t L, int64_t I, cons
  *               GEMMs, 0: dequantisation is the GEMMs' epilogue}; non-NULL makes
  *               the call synchronise the stream and run its kernels one after the
  *               other on `hip_stream`
- * Without timing, independent kernels of the call (the two W kernels, the row-wise
- * quantise pass of g_y and, for products too small to fill the chip, the g_x GEMM) run
- * on a side stream of the library (one per device, created on first use, default
- * priority) between events recorded on `hip_stream` and a wait on it, so they overlap
- * the token-wise g_y kernels and the g_W GEMM; everything is ordered after earlier
- * work on `hip_stream` and before later work on it.
+ * Without timing the transforms take two launches (statistics, then everything that needs a
+ * step), each a grid of independent jobs, and the two products one.  Products that cannot share
+ * a launch follow one another, or, when the g_W product is too small to fill the chip, the g_x
+ * product runs on a side stream of the library (one per device, created on first use, default
+ * priority) between events recorded on `hip_stream` and a wait on it; everything is ordered
+ * after earlier work on `hip_stream` and before later work on it.
  */
 HOT_API size_t hot_backward_workspace_bytes(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_linear_backward(const void* gy, const void* w, int dtype, const void* xq,
