@@ -33,7 +33,8 @@ EXPORTS = (
     "hot_gemm_plan", "hot_gemm_workspace_bytes", "hot_gemm_i8_variant", "hot_gemm_bf16",
     "hot_hla_tokenwise_static", "hot_measure_ceilings",
     "hot_kpad_group", "hot_abc_batched_workspace_bytes", "hot_abc_forward_batched",
-    "hot_backward_batched_workspace_bytes", "hot_linear_backward_batched", "hot_backward_batched_ranges",
+    "hot_backward_batched_workspace_bytes", "hot_linear_backward_batched", "hot_linear_backward_batched_bias",
+    "hot_backward_batched_ranges",
     "hot_gx_lowrank_workspace_bytes", "hot_gx_lowrank", "hot_gx_luq_workspace_bytes", "hot_gx_luq",
     "hot_gw_luq_workspace_bytes", "hot_gw_luq",
 )
@@ -133,6 +134,8 @@ def _declare(lib):
     lib.hot_backward_batched_ranges.argtypes = [i64, i64, i64, i64, cfgp]
     lib.hot_linear_backward_batched.restype = i32
     lib.hot_linear_backward_batched.argtypes = [vp, vp, i32, vp, vp, i64, i64, i64, i64, cfgp, vp, vp, i32, vp, sz, vp]
+    lib.hot_linear_backward_batched_bias.restype = i32
+    lib.hot_linear_backward_batched_bias.argtypes = [vp, vp, i32, vp, vp, i64, i64, i64, i64, cfgp, vp, vp, vp, i32, vp, sz, vp]
     lib.hot_measure_ceilings.restype = i32
     lib.hot_measure_ceilings.argtypes = [vp, sz, C.POINTER(C.c_float), C.POINTER(C.c_float), vp]
     lib.hot_linear_backward_bias.restype = i32

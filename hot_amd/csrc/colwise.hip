@@ -367,7 +367,7 @@ static int64_t colsum_strip_rows_big(int64_t R, int64_t C) {
   return rows < 64 ? 64 : rows;
 }
 
-int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes) {
+int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes, int64_t groups) {
   if (R <= 0 || C <= 0 || n < 1 || r < 1) return 0;
   if (n > COL_MAX_N) {
     const int64_t rows = colsum_strip_rows_big(R, C);
@@ -375,7 +375,7 @@ int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int m
   }
   const int64_t NB = R / n;
   const ColPartition part = col_partition(n, r, store4, mode, C, NB, elem_bytes);
-  return (NB + part.tb0 - 1) / part.tb0;
+  return (NB / groups + part.tb0 - 1) / part.tb0 * groups;
 }
 
 int colsum_finish_impl(const ColsumArgs& a, hipStream_t st) {

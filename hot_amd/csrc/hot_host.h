@@ -88,7 +88,7 @@ size_t colwise_group_workspace_bytes_impl(int64_t C, int groups);
 // colsum_strips_impl(...) rows of C partial sums (fp32; elem_bytes = size of an input element, on which the
 // partition of the passes depends), one row per run of token blocks of its statistics pass, which holds the sum of
 // every block as coefficient 0; colsum_finish_impl adds the rows in a fixed order and rounds once to the output type.
-int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes);
+int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes, int64_t groups = 1);
 struct ColsumArgs;
 int colsum_finish_impl(const ColsumArgs& a, hipStream_t st);
 size_t colwise_workspace_bytes_impl(int64_t C);

@@ -398,9 +398,10 @@ def abc_forward_batched(x: torch.Tensor, opt: HotOptions, side: Optional["torch.
 
 
 def linear_backward_batched(gy: torch.Tensor, w: torch.Tensor, xq: torch.Tensor, sx: torch.Tensor, opt: HotOptions,
-                            out_dtype=None, workspace: Optional[torch.Tensor] = None):
+                            out_dtype=None, workspace: Optional[torch.Tensor] = None, bias_grad: bool = False):
     """g_x [B, T, I] and g_W [O, I] (summed over the samples) for g_y [B, T, O] with one set of steps per
-    sample (hot_linear_backward_batched)."""
+    sample (hot_linear_backward_batched); with bias_grad=True also g_b [O], the sum of g_y over samples and
+    tokens (hot_linear_backward_batched_bias)."""
     if not gy.is_cuda or gy.dim() != 3 or not gy.is_contiguous():
         raise RuntimeError("Go must be a contiguous CUDA tensor [B, T, O]!")
     _need_gpu_2d(w, "Wt")
@@ -420,6 +421,12 @@ def linear_backward_batched(gy: torch.Tensor, w: torch.Tensor, xq: torch.Tensor,
         workspace = _ws(need, gy.device)
     gx = torch.empty((B, T, I), dtype=out_dtype, device=gy.device)
     gw = torch.empty((O, I), dtype=out_dtype, device=gy.device)
+    if bias_grad:
+        gb = torch.empty((O,), dtype=out_dtype, device=gy.device)
+        _lib.check(_lib.lib().hot_linear_backward_batched_bias(
+            gy.data_ptr(), w.data_ptr(), _dt(gy), xq.data_ptr(), sx.data_ptr(), B, T, O, I, C.byref(cfg), gx.data_ptr(),
+            gw.data_ptr(), gb.data_ptr(), _DTYPES[out_dtype], workspace.data_ptr(), workspace.numel(), _stream()))
+        return gx, gw, gb
     _lib.check(_lib.lib().hot_linear_backward_batched(gy.data_ptr(), w.data_ptr(), _dt(gy), xq.data_ptr(), sx.data_ptr(), B, T,
                                                       O, I, C.byref(cfg), gx.data_ptr(), gw.data_ptr(), _DTYPES[out_dtype],
                                                       workspace.data_ptr(), workspace.numel(), _stream()))

@@ -360,6 +360,14 @@ class FLinearQ(Function):
             grad_w = gw.to(wc.dtype)
             grad_input = torch.stack(gxs) if per_sample else gxs[0].reshape(ctx.x_shape)
         elif go.dim() == 3 and args.batched_mode == "per_sample" and ctx.batched:
+            if ctx.has_bias and ctx.needs_input_grad[5] and go.dtype == grad_output.dtype and go.dtype != torch.float32:
+                # out of the statistics pass, in fp32, rounded once to 16 bits: the error is the rounding's, 1.6e-3 in bf16 with either
+                # order of the sum.  fp32 gradients keep the reduction, whose order is up to twice as accurate (4 x 49 tokens
+                # 5.8e-8 against 1.2e-7); gradients of another type than the weights' are summed as they came in.
+                gx, grad_w, gb = ops.linear_backward_batched(_pad8(go), wc, xq, sx, opt, bias_grad=True)
+                if O % 8 or I % 8:
+                    grad_w = grad_w[:O, :I]
+                return gx[..., :I], grad_w, None, None, None, gb[:O]
             gx, grad_w = ops.linear_backward_batched(_pad8(go), wc, xq, sx, opt)
             grad_input = gx[..., :I]
         elif go.dim() == 3 and args.batched_mode == "per_sample":

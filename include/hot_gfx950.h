@@ -293,6 +293,13 @@ HOT_API int hot_linear_backward_batched(const void* gy, const void* w, int dtype
                                 const hot_config* cfg, void* gx, void* gw, int out_dtype,
                                 void* workspace, size_t workspace_bytes, void* hip_stream);
 
+/* The same with the bias gradient gb[O] of out_dtype: the sum of g_y over samples and tokens, as in
+ * hot_linear_backward_bias (fp32 in a fixed order, rounded once; no pass over g_y).  Same workspace. */
+HOT_API int hot_linear_backward_batched_bias(const void* gy, const void* w, int dtype, const void* xq,
+                                const float* sx, int64_t B, int64_t T, int64_t O, int64_t I,
+                                const hot_config* cfg, void* gx, void* gw, void* gb, int out_dtype,
+                                void* workspace, size_t workspace_bytes, void* hip_stream);
+
 /*
  * g_x of the schemes that project g_y to low rank along the TOKENS for that product
  * (utils/quant_matmul.py, transform_scheme "low_rank" and "gilr_gwh": :229-233 g_y <- P g_y,

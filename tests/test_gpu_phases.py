@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import hot_oracle as orc
-from test_gpu_backward import make_case, run_both
+from test_gpu_backward import fresh_args, make_case, run_both  # noqa: F401 (a fixture)
 from test_gpu_random_cases import _options
 
 pytestmark = pytest.mark.gpu
@@ -89,3 +89,45 @@ def test_codes_on_the_boundary(gpu, scale, bits):
     # the same values along the tokens (blocks of one): the column-wise body
     col, sc, kout = ops.hla_tokenwise(torch.from_numpy(np.tile(v[:, None], (1, 8))).to(gpu), 1, (0,), bits=bits)
     assert np.array_equal(col.cpu().numpy()[:, :kout].astype(np.int64), np.tile(ref, (8, 1)))
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,T,O,variant", [(5, 197, 208, dict()), (3, 64, 192, dict(gx_scale=orc.SCALE_ROW, gw_scale=orc.SCALE_ROW)),
+                                           (4, 196, 96, STOCH), (7, 6, 8, dict()), (2, 48, 264, dict()), (1, 128, 40, STOCH),
+                                           (3, 640, 16, dict()), (130, 197, 128, dict()), (64, 2, 2056, dict(gx_scale=orc.SCALE_ROW))])
+def test_batched_bias_gradient(gpu, dt, B, T, O, variant):
+    """The column sums that leave the statistics pass of a batched backward: token blocks of 1 .. 128, the last strip of a
+    sample cut short, strips of many samples.  Integers (below 2^24): every order gives the exact sum, a block dropped, doubled or
+    misplaced shows.  Random values: within the fp32 accumulation bound of the 64-bit sum.  g_x and g_W stay as without it."""
+    from hot_amd import ops
+    ocfg = orc.HotConfig.python_rule(T, n_o=min(16, O & -O), **variant)
+    opt = _options(ocfg)
+    g = torch.Generator().manual_seed(B * T + O)
+    w = ((torch.rand(O, 24, generator=g) * 2 - 1) / 5).to(dt).to(gpu)
+    xq, sx = ops.abc_forward_batched(torch.randn(B, T, 24, generator=g).to(dt).to(gpu), opt)
+    gy = torch.randn(B, T, O, generator=g).to(dt)
+    gx, gw, gb = ops.linear_backward_batched(gy.to(gpu), w, xq, sx, opt, out_dtype=torch.float32, bias_grad=True)
+    gx0, gw0 = ops.linear_backward_batched(gy.to(gpu), w, xq, sx, opt, out_dtype=torch.float32)
+    assert torch.equal(gx, gx0) and torch.equal(gw, gw0)
+    d = gy.double().reshape(-1, O)
+    assert torch.all((gb.cpu().double() - d.sum(0)).abs() <= B * T * 2.0 ** -24 * d.abs().sum(0))
+    gi = torch.randint(-8, 9, (B, T, O), generator=g).to(dt)
+    gb = ops.linear_backward_batched(gi.to(gpu), w, xq, sx, opt, out_dtype=torch.float32, bias_grad=True)[2]
+    assert torch.equal(gb.cpu(), gi.double().reshape(-1, O).sum(0).float())
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("O", [96, 100])
+def test_layer_bias_gradient_per_sample(gpu, fresh_args, dt, O):
+    """The bias gradient of a layer on 3-D activations with steps per sample, widths with and without padding: the 64-bit
+    sum within the fp32 accumulation bound and one rounding of the type."""
+    from hot_amd.quant_matmul import HQ_Linear
+    fresh_args.hot_recipe()
+    fresh_args.batched_mode = "per_sample"
+    g = torch.Generator().manual_seed(O)
+    lin = HQ_Linear(64, O).to(gpu).to(dt)
+    gy = torch.randn(6, 197, O, generator=g).to(dt)
+    lin(torch.randn(6, 197, 64, generator=g).to(dt).to(gpu)).backward(gy.to(gpu))
+    d = gy.double().reshape(-1, O)
+    bound = 6 * 197 * 2.0 ** -24 * d.abs().sum(0) + (2.0 ** -8 * d.sum(0).abs() if dt == torch.bfloat16 else 0)
+    assert lin.bias.grad.dtype == dt and torch.all((lin.bias.grad.double().cpu() - d.sum(0)).abs() <= bound)
