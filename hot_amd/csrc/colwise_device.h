@@ -722,7 +722,8 @@ __device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, u
       // untransposed store: coefficient row (blk0 + b) r + k takes one code of every channel; a
       // wave writes 64 adjacent bytes (INT8) or, two channels to a byte, 32 (packed INT4: the even
       // channel in bits 3:0)
-      const int krun = nblk * a.r;
+      // (short blocks: nblk counts groups of 16 rows and a.r the codes of a group; the last group may be cut short)
+      const int krun = SHORT ? (rows_wg >> a.nrt_log) * (a.r >> (4 - a.nrt_log)) : nblk * a.r;
       int8_t* orow = a.out + blk0 * a.r * a.ld_out;
       for (int k = 0; k < krun; ++k, orow += a.ld_out) {
         const int code = stage[tid * pitch + k];

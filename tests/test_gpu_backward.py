@@ -833,6 +833,30 @@ def test_gx_lowrank_matches_oracle(gpu, dtype, L, O, I, rule, variant):
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dtype))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("kept", ["low", "all"])
+@pytest.mark.parametrize("L,n,O", [(2, 2, 4096), (50, 2, 264), (34, 2, 64), (12, 4, 520), (196, 4, 264), (200, 8, 264), (24, 8, 4096), (48, 16, 64)])
+def test_gx_lowrank_stays_in_its_workspace(gpu, L, n, O, kept, bits):
+    """Blocks of 2, 4 and 8 tokens with a last group of 16 rows cut short: the untransposed store ends with row NB r - 1.
+    Guard bytes lie behind the workspace; with 8 and 16 inputs W's operand is smaller than a group of surplus rows."""
+    import ctypes as C
+    from hot_amd import _lib, ops
+    rows = tuple(range(n)) if kept == "all" else tuple(range(n // 2))
+    opt = ops.HotOptions(hla_n=n, hla_rows=rows, gx_bits=bits, w_bits=bits)
+    ocfg = orc.HotConfig(hla_n=n, hla_rows=rows, gx_bits=bits, w_bits=bits)
+    lib, cfg = _lib.lib(), opt.to_c()
+    for I in (8, 16):
+        x, w, gy = make_case(L, O, I, seed=L + I)
+        gyd, wd = gy.to(gpu), w.to(gpu)
+        gx = torch.empty((L, I), device=gpu)
+        need = lib.hot_gx_lowrank_workspace_bytes(L, O, I, C.byref(cfg))
+        ws = torch.full((need + (1 << 20),), 0xA5, dtype=torch.uint8, device=gpu)
+        _lib.check(lib.hot_gx_lowrank(gyd.data_ptr(), wd.data_ptr(), _lib.F32, L, O, I, C.byref(cfg), gx.data_ptr(), _lib.F32,
+                                      ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+        assert bool((ws[need:] == 0xA5).all()), "bytes past the workspace were written"
+        assert np.array_equal(gx.cpu().numpy(), orc.gx_lowrank(gy.numpy(), w.numpy(), ocfg).g_x)
+
+
 def test_gx_lowrank_refuses_what_it_cannot_do(gpu):
     from hot_amd import ops
     x, w, gy = make_case(256, 64, 32, seed=0)
