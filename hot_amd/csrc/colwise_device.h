@@ -216,7 +216,10 @@ __device__ __forceinline__ void rs_column(const uint8_t* wave_buf, int lane, flo
 // and the K-major stores bound it now: without the stores 34 and 84 us).
 constexpr int RUNTIME = 2;
 template <typename T, int N, int PASS, int ROUND, int SAWB, typename SEL, bool RS = false, bool HQ = false>
-__device__ __forceinline__ void colwise_body(const ColArgs& a, unsigned block, uint8_t* lds, const HqArgs* hq = nullptr) {
+__device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block, uint8_t* lds, const HqArgs* hq = nullptr) {
+  // A copy, so that every argument is loaded once: read through the reference they would be loaded again at each use behind
+  // the memory clobber of a DMA instruction, 59 scalar loads and waits in the loop of <bf16, 1, 1, stochastic>.
+  const ColArgs a = args;
   constexpr bool SHORT = std::is_same<SEL, SelShort>::value || std::is_same<SEL, SelShortFull>::value;
   static_assert(!SHORT || N == CW_ROWS, "short blocks are handled 16 rows at a time");
   constexpr int SPB = N >= CW_ROWS ? N / CW_ROWS : 1;        // steps per token block
