@@ -140,17 +140,19 @@ static bool matches(const ColArgs& a) {
   return true;
 }
 
-// The instance for a.slot of a block of n rows with r kept ones; blocks of 2 .. 16 rows without an instance of
-// their own become SelShort: 16 rows at a time.
+// The instance for a.slot of a block of n rows with r kept ones.
 static ColSel pick_sel(ColArgs& a, int n, bool as_short) {
   const int r = a.r;
   if (!as_short) {
     switch (n) {
       case 1: return COL_ONE;
+      case 2: return COL_RT2;
+      case 4: return COL_RT4;
+      case 8: return COL_RT8;
       case 16:
         if (r == 16 && matches<SelFull<16>, 16>(a)) return COL_FULL16;
         if (r == 8 && matches<SelPaper16, 16>(a)) return COL_PAPER16;
-        break;
+        return COL_RT16;
       case 32: return r == 32 && matches<SelFull<32>, 32>(a) ? COL_FULL32 : COL_RT32;
       case 64:
         if (r == 36 && matches<SelPy64, 64>(a)) return COL_PY64;
@@ -192,7 +194,7 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
   a.in = in; a.R = R; a.C = C; a.NB = R / n; a.Kout = a.NB * r; a.Rs = R / groups;
   a.out = (int8_t*)codes_out; a.ld_out = ld_out;
   a.seed = seed; a.stream = rng_stream;
-  a.r = r; a.rpad = r == 1 ? 0 : (r + 7) & ~7; a.bits = bits; a.rounding = rounding; a.mode = scale_mode;
+  a.r = r; a.rpad = (r + 7) & ~7; a.bits = bits; a.rounding = rounding; a.mode = scale_mode;
   for (int i = 0; i < COL_MAX_N; ++i) a.slot[i] = -1;
   for (int k = 0; k < r; ++k) {
     if (rows[k] < 0 || rows[k] >= n) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d outside [0, %d)", who, k, rows[k], n);
@@ -235,11 +237,6 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
     // 16 rows at a time (the partition takes whole groups of them)
     const int per = CW_ROWS / n;
     a.nrt = n;
-    for (a.nrt_log = 0; (1 << a.nrt_log) < n; ++a.nrt_log) {}
-    for (int i = CW_ROWS - 1; i >= 0; --i) {
-      const int sl = a.slot[i % n];
-      a.slot[i] = (int8_t)(sl < 0 ? -1 : (i / n) * r + sl);
-    }
     a.r = per * r;
     a.NBs = (a.NBs + per - 1) / per;
     job.tb[0] /= per; job.tb[1] /= per;
@@ -298,7 +295,11 @@ template <typename T>
 static int dispatch_sawb(const ColJob& job, int pass, hipStream_t st) {
   switch (job.sel) {
     case COL_ONE: return launch_sawb<T, 1, SelFull<1>>(job, pass, st);
-    case COL_SHORT: return launch_sawb<T, 16, SelShort>(job, pass, st);
+    case COL_SHORT: break;      // (W's slot of a phase)
+    case COL_RT2: return launch_sawb<T, 2, SelRuntime>(job, pass, st);
+    case COL_RT4: return launch_sawb<T, 4, SelRuntime>(job, pass, st);
+    case COL_RT8: return launch_sawb<T, 8, SelRuntime>(job, pass, st);
+    case COL_RT16: return launch_sawb<T, 16, SelRuntime>(job, pass, st);
     case COL_PAPER16: return launch_sawb<T, 16, SelPaper16>(job, pass, st);
     case COL_FULL16: return launch_sawb<T, 16, SelFull<16>>(job, pass, st);
     case COL_RT32: return launch_sawb<T, 32, SelRuntime>(job, pass, st);

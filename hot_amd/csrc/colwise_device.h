@@ -37,7 +37,7 @@ struct ColArgs {
   uint64_t seed;
   uint32_t stream;
   int32_t r, rpad, bits, store4, rounding, mode, tb;
-  int32_t nrt, nrt_log;  // SelShort: the block length (1 .. 16) and its logarithm
+  int32_t nrt;         // SelShortFull: the block length (1 .. 16)
   uint32_t gx, gy;     // logical grid: channel strips x runs of token blocks
   // Sample groups (3-D activations: one step per sample).  The R rows are `groups` samples of NBs
   // token blocks each; a workgroup's run of blocks never leaves its sample (`runs` runs per sample),
@@ -51,7 +51,7 @@ struct ColArgs {
   // rowmajor: the codes are stored untransposed, [NB r, C] with ld_out bytes per coefficient row
   // (the A operand of a product whose K runs along the channels), instead of [C, NB r]
   int32_t rowmajor;
-  int8_t slot[COL_MAX_N];  // output position of natural row i, -1 = dropped (SelShort: of row i of 16 rows)
+  int8_t slot[COL_MAX_N];  // output position of natural row i, -1 = dropped
 };
 
 // Which coefficients of a block are kept and where they go.  The generic policy reads the table
@@ -59,11 +59,9 @@ struct ColArgs {
 // per-coefficient scalar branches and lets the compiler drop the butterflies that only feed
 // discarded coefficients.
 struct SelRuntime { static constexpr bool STATIC = false; };
-// Blocks of 1 .. 16 rows, whatever their length and selection: 16 rows at a time, the butterfly stages and the
-// places of the kept coefficients taken from the arguments (r, tb, NB and slot count whole groups of 16 rows then,
-// the last one may be cut short).  Stochastic rounding with it: blocks of 2 .. 16.
-struct SelShort { static constexpr bool STATIC = false; };
-struct SelShortFull {  // every row kept, in order
+// Blocks of 1 .. 16 rows, their length known at run time, every row kept in order (W): 16 rows at a time, r, tb, NBs and
+// runs count whole groups of 16 rows then, the last one may be cut short.  Stochastic rounding with it: blocks of 16.
+struct SelShortFull {
   static constexpr bool STATIC = true;
   static constexpr int slot(int i) { return i; }
 };
@@ -220,7 +218,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   // A copy, so that every argument is loaded once: read through the reference they would be loaded again at each use behind
   // the memory clobber of a DMA instruction, 59 scalar loads and waits in the loop of <bf16, 1, 1, stochastic>.
   const ColArgs a = args;
-  constexpr bool SHORT = std::is_same<SEL, SelShort>::value || std::is_same<SEL, SelShortFull>::value;
+  constexpr bool SHORT = std::is_same<SEL, SelShortFull>::value;
   static_assert(!SHORT || N == CW_ROWS, "short blocks are handled 16 rows at a time");
   constexpr int SPB = N >= CW_ROWS ? N / CW_ROWS : 1;        // steps per token block
   constexpr int BPS = N >= CW_ROWS ? 1 : CW_ROWS / N;        // token blocks per step
@@ -258,8 +256,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   const int run = (int)by - sample * a.runs;
   const int64_t blk_in = (int64_t)run * a.tb;                    // first block of the run within its sample
   const int64_t blk0 = (int64_t)sample * a.NBs + blk_in;
-  const int64_t row0 = SHORT ? (int64_t)sample * a.Rs + blk_in * N : blk0 * N;
-  const int64_t sblk0 = SHORT ? ((int64_t)sample * a.Rs + blk_in * N) >> a.nrt_log : 0;   // first short block
+  const int64_t row0 = blk0 * N;
   int nblk = (int)((a.NBs - blk_in) < a.tb ? (a.NBs - blk_in) : a.tb);
   const int nsteps = (nblk * N + CW_ROWS - 1) / CW_ROWS;
   // (short blocks: the last group of 16 rows may be cut short; what its missing rows deliver is not consumed)
@@ -490,31 +487,13 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
             if (sl >= 0) row[sl] = (uint8_t)rint_div_exact(x[base + i], d, rcp);
           }
         }
-      } else if constexpr (SHORT && SEL::STATIC) {
-        // whole blocks of 16 (shorter ones with stochastic rounding take SelShort): eight coefficients to a generator call
+      } else if constexpr (SHORT) {
+        // whole blocks of 16: eight coefficients to a generator call
         uint32_t u[8];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          if ((i & 7) == 0) sr_bits8(((uint64_t)c * (uint64_t)a.NB + (uint64_t)(sblk0 + blk)) * (uint64_t)(N / 8) + (uint64_t)(i >> 3), a.seed, a.stream, u);
+          if ((i & 7) == 0) sr_bits8(((uint64_t)c * (uint64_t)a.NB + (uint64_t)(blk0 + blk)) * (uint64_t)(N / 8) + (uint64_t)(i >> 3), a.seed, a.stream, u);
           if (place(i) >= 0) row[i] = (uint8_t)q_stoch_fix(x[base + i], rcpk, u[i & 7], qmax);
-        }
-      } else if constexpr (SHORT) {
-        // counter of element e: e = (channel * NB + block) * rpad + visit index (block of its own for every short block)
-        philox_words us = {0u, 0u, 0u, 0u};
-        int visited = 0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          if ((i & (a.nrt - 1)) == 0) visited = 0;           // a short block begins
-          const int sl = place(i);
-          if (sl >= 0) {
-            if ((visited & 7) == 0) {
-              const uint64_t e = (uint64_t)c * (uint64_t)a.NB + (uint64_t)(sblk0 + (blk << (4 - a.nrt_log)) + (i >> a.nrt_log));
-              if (a.rpad == 0) { us = sr_octet_words(e >> 3, a.seed, a.stream); visited = (int)(e & 7u); }   // one kept per block
-              else us = sr_octet_words(e * (uint64_t)(a.rpad >> 3) + (uint64_t)(visited >> 3), a.seed, a.stream);
-            }
-            row[sl] = (uint8_t)q_stoch_fix(x[base + i], rcpk, sr_bits_of(us, (uint32_t)visited), qmax);
-            ++visited;
-          }
         }
       } else {
         int visited = 0;      // kept coefficients of this block quantised so far
@@ -553,17 +532,10 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
     }
   };
   auto consume = [&](int bl) {
-    if constexpr (SHORT) fwht_short(x, a.nrt, RSP ? 2 : 1);
+    if constexpr (SHORT) fwht_short(x, a.nrt, 1);
     else fwht_regs<N, XL, (RSP && N >= 2) ? 2 : 1>(x);   // the fused statistics pass runs stage h = 1 while loading
     if constexpr (SHORT) {
       const int valid = rows_wg - bl * N;
-      if constexpr (PASS == 0)
-        if (a.colsum) {
-          // coefficient 0 of a block is the sum of its tokens (row 0 of H is all ones)
-#pragma unroll
-          for (int i = 0; i < N; ++i)
-            if ((i & (a.nrt - 1)) == 0 && i < valid) csum += x[i];
-        }
       if (valid >= N) block_body(std::false_type{}, 0, bl, N);
       else block_body(std::true_type{}, 0, bl, valid);
     } else {
@@ -571,7 +543,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       for (int g = 0; g < BPS; ++g) {
         const int blk = bl + g;
         if (blk < nblk) {
-          if constexpr (PASS == 0) csum += x[g * N];     // (coefficient 0 of a block: the sum of its tokens)
+          if constexpr (PASS == 0) csum += x[g * N];     // (coefficient 0 of a block: the sum of its tokens, row 0 of H is all ones)
           block_body(std::false_type{}, g * N, blk, N);
         }
       }
@@ -604,7 +576,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       static_assert(CW_ROWS == 16, "the operand list below names sixteen rows");
       float t[CW_ROWS];
       rs_column<T>(my + (s % CW_DEPTH) * BUF, chan & 63, t);
-      if (N >= 2 && (!SHORT || a.nrt >= 2)) {
+      if (N >= 2) {
 #pragma unroll
         for (int j = 0; j < CW_ROWS; j += 2) { dst[j] = t[j] + t[j + 1]; dst[j + 1] = t[j] - t[j + 1]; }
       } else {
@@ -725,8 +697,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       // untransposed store: coefficient row (blk0 + b) r + k takes one code of every channel; a
       // wave writes 64 adjacent bytes (INT8) or, two channels to a byte, 32 (packed INT4: the even
       // channel in bits 3:0)
-      // (short blocks: nblk counts groups of 16 rows and a.r the codes of a group; the last group may be cut short)
-      const int krun = SHORT ? (rows_wg >> a.nrt_log) * (a.r >> (4 - a.nrt_log)) : nblk * a.r;
+      const int krun = nblk * a.r;      // (groups of short blocks, whose last one may hold fewer, are never stored this way)
       int8_t* orow = a.out + blk0 * a.r * a.ld_out;
       for (int k = 0; k < krun; ++k, orow += a.ld_out) {
         const int code = stage[tid * pitch + k];

@@ -54,7 +54,7 @@ __device__ __forceinline__ void colsum_finish_body(const ColsumArgs& a, unsigned
 
 struct PhaseArgs {
   ColArgs g;            // the token-wise job (its n and selection pick the kernel)
-  ColArgs w;            // the column-wise job with short blocks (W): SelShort
+  ColArgs w;            // the column-wise job with short blocks (W): SelShortFull
   HqArgs h;             // the row-wise job and
   ColsumArgs s;         // the bias gradient (quantise phase only)
   uint32_t g_blocks, w_blocks, h_blocks, s_blocks;   // workgroups of each; 0 = absent (g and w: multiples of 8, so that
@@ -63,7 +63,7 @@ struct PhaseArgs {
 };
 
 // Which instance a block length and selection takes; the caller has filled a.slot.
-enum ColSel { COL_SHORT, COL_ONE, COL_PAPER16, COL_FULL16, COL_RT32, COL_FULL32, COL_RT64, COL_PY64, COL_FULL64, COL_RT128, COL_PY128 };
+enum ColSel { COL_SHORT, COL_ONE, COL_RT2, COL_RT4, COL_RT8, COL_RT16, COL_PAPER16, COL_FULL16, COL_RT32, COL_FULL32, COL_RT64, COL_PY64, COL_FULL64, COL_RT128, COL_PY128 };
 
 // A column-wise job: the arguments of both passes, and what differs between them.
 struct ColJob {

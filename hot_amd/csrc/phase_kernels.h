@@ -32,7 +32,8 @@ __global__ void __launch_bounds__(CW, (phase_waves<N, SEL>())) phase_kernel(cons
   }
   b -= p.w_blocks;
   if (PASS == 0 || b < p.g_blocks) {
-    colwise_body<T, N, PASS, ROUND, 0, SEL, RS, PASS == 1 && !std::is_same<SEL, SelRuntime>::value>(phase_args().g, b, lds, p.h_in_g ? &phase_args().h : nullptr);
+    constexpr bool HQ = PASS == 1 && (N <= CW_ROWS || !std::is_same<SEL, SelRuntime>::value);      // (row_job_joins)
+    colwise_body<T, N, PASS, ROUND, 0, SEL, RS, HQ>(phase_args().g, b, lds, p.h_in_g ? &phase_args().h : nullptr);
     return;
   }
   if constexpr (PASS == 1) {
@@ -73,7 +74,11 @@ template <typename T>
 int phase_launch_impl(int pass, ColSel sel, const PhaseArgs& p, size_t lds, hipStream_t st) {
   switch (sel) {
     case COL_ONE: return launch_phase_sel<T, 1, SelFull<1>>(pass, p, lds, st);
-    case COL_SHORT: return launch_phase_sel<T, 16, SelShort>(pass, p, lds, st);
+    case COL_RT2: return launch_phase_sel<T, 2, SelRuntime>(pass, p, lds, st);
+    case COL_RT4: return launch_phase_sel<T, 4, SelRuntime>(pass, p, lds, st);
+    case COL_RT8: return launch_phase_sel<T, 8, SelRuntime>(pass, p, lds, st);
+    case COL_RT16: return launch_phase_sel<T, 16, SelRuntime>(pass, p, lds, st);
+    case COL_SHORT:                     // (no token-wise job: any instance runs the others)
     case COL_PAPER16: return launch_phase_sel<T, 16, SelPaper16>(pass, p, lds, st);
     case COL_FULL16: return launch_phase_sel<T, 16, SelFull<16>>(pass, p, lds, st);
     case COL_RT32: return launch_phase_sel<T, 32, SelRuntime>(pass, p, lds, st);
