@@ -110,7 +110,7 @@ class HotOptions:
         c = _lib.HotConfig.from_buffer_copy(base)
         c.seed = seed & 0xFFFFFFFFFFFFFFFF
         object.__setattr__(other, "_c", c)
-        object.__setattr__(other, "_keep", base)     # owner of what hla_rows_big points to
+        object.__setattr__(other, "_keep", self.__dict__.get("_keep", base))     # owner of what hla_rows_big points to
         return other
 
     def to_c(self) -> _lib.HotConfig:

@@ -208,6 +208,21 @@ def test_hlq_options_follow_the_value_of_the_block_size():
     assert HLQ_backward.options(48, size, True).n_o == 8
 
 
+def test_options_keep_the_row_list_through_a_chain_of_keys():
+    """hla_rows_big is a host pointer: whichever ancestor built the array, the last of a chain of with_seed() owns it."""
+    import gc
+    from hot_amd import ops
+    rows = tuple(range(2048))
+    first = ops.HotOptions(hla_n=2048, hla_rows=rows)
+    second = first.with_seed(1)
+    last = second.with_seed(2).with_seed(3)
+    del first, second
+    gc.collect()
+    noise = [(C.c_int32 * 2048)(*([7777] * 2048)) for _ in range(64)]
+    c = last.to_c()
+    assert c.seed == 3 and [c.hla_rows_big[i] for i in range(2048)] == list(rows) and len(noise) == 64
+
+
 # --------------------------------------------------------------- the C ABI
 
 def _declared():
