@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
-from dataclasses import dataclass, field
+from dataclasses import dataclass, field, replace
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -105,8 +105,12 @@ class HotOptions:
             return self
         base = self.to_c()
         self.__dict__.setdefault("_ws_bytes", {})     # (shared: no size depends on the seed)
-        other = object.__new__(HotOptions)
-        other.__dict__.update(self.__dict__, seed=seed)
+        if type(self) is HotOptions:
+            other = object.__new__(HotOptions)
+            other.__dict__.update(self.__dict__, seed=seed)
+        else:
+            other = replace(self, seed=seed)         # (a subclass: its own __init__ and __post_init__ run)
+            other.__dict__["_ws_bytes"] = self.__dict__["_ws_bytes"]
         c = _lib.HotConfig.from_buffer_copy(base)
         c.seed = seed & 0xFFFFFFFFFFFFFFFF
         object.__setattr__(other, "_c", c)

@@ -223,6 +223,15 @@ def test_options_keep_the_row_list_through_a_chain_of_keys():
     assert c.seed == 3 and [c.hla_rows_big[i] for i in range(2048)] == list(rows) and len(noise) == 64
 
 
+def test_options_under_another_key_keep_their_class():
+    from hot_amd import ops
+
+    class Options(ops.HotOptions):
+        pass
+
+    assert type(Options(seed=1).with_seed(2)) is Options
+
+
 # --------------------------------------------------------------- the C ABI
 
 def _declared():
