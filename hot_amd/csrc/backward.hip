@@ -47,6 +47,15 @@ static int check_cfg(const hot_config* c, const char* who) {
   return HOT_OK;
 }
 
+// The quantiser of g_y for the g_x product and the results' type, whichever kernels will serve them: refused before anything
+// is launched (the quantisers of the column-wise passes are checked where their jobs are filled).
+static int check_gx_modes(const hot_config* c, int out_dtype, const char* who) {
+  if (c->gx_round != HOT_ROUND_NEAREST && c->gx_round != HOT_ROUND_STOCH) return fail(HOT_ERR_INVALID, "%s: bad rounding %d", who, c->gx_round);
+  if (c->gx_scale != HOT_SCALE_TENSOR && c->gx_scale != HOT_SCALE_ROW) return fail(HOT_ERR_UNSUPPORTED, "%s: g_y scale mode %d (tensor or row)", who, c->gx_scale);
+  if (out_dtype != HOT_F32 && out_dtype != HOT_BF16 && out_dtype != HOT_F16) return fail(HOT_ERR_INVALID, "%s: bad out dtype %d", who, out_dtype);
+  return HOT_OK;
+}
+
 struct BwdLayout {
   int64_t ld_g, ld_w, ld_gp;                       // code pitches in bytes
   size_t off_hq, off_colw, off_colg, off_sg, off_sw, off_sgp, off_qg, off_qw, off_qgp, off_split, off_colsum, total;
@@ -271,6 +280,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   if (cfg->w_scale == HOT_SCALE_ROW) return fail(HOT_ERR_UNSUPPORTED, "%s: W uses one step per tensor", who);
   if (cfg->gw_scale == HOT_SCALE_SAWB) return fail(HOT_ERR_UNSUPPORTED, "%s: SAWB applies to W and x only", who);
   // limits of the stages, checked here so that nothing has been launched when one of them refuses
+  if (int e = check_gx_modes(cfg, out_dtype, who)) return e;
   if (O % 8 || I % 8) return fail(HOT_ERR_UNSUPPORTED, "%s: O=%lld and I=%lld must be multiples of 8", who, (long long)O, (long long)I);
   if (O * I * 4 >= (1ll << 32)) return fail(HOT_ERR_UNSUPPORTED, "%s: W of %lld x %lld elements exceeds the 32-bit offsets of the loader", who, (long long)O, (long long)I);
   if (cfg->hla_n <= COL_MAX_N && L * O * 4 >= (1ll << 32)) return fail(HOT_ERR_UNSUPPORTED, "%s: g_y of %lld x %lld elements exceeds the 32-bit offsets of the loader", who, (long long)L, (long long)O);
@@ -842,6 +852,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
   if (cfg->gx_bits != cfg->w_bits) return fail(HOT_ERR_UNSUPPORTED, "%s: gx_bits (%d) and w_bits (%d) must match", who, cfg->gx_bits, cfg->w_bits);
   if (cfg->gx_scale == HOT_SCALE_SAWB || cfg->gw_scale == HOT_SCALE_SAWB) return fail(HOT_ERR_UNSUPPORTED, "%s: SAWB applies to W and x only", who);
   if (cfg->w_scale == HOT_SCALE_ROW) return fail(HOT_ERR_UNSUPPORTED, "%s: W uses one step per tensor", who);
+  if (int e = check_gx_modes(cfg, out_dtype, who)) return e;
   const int64_t L = B * T;
   if (L * O * 4 >= (1ll << 32) || O * I * 4 >= (1ll << 32)) return fail(HOT_ERR_UNSUPPORTED, "%s: tensors exceed the 32-bit offsets of the loader", who);
   const BatchedLayout b = batched_layout(B, T, O, I, cfg);

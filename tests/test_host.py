@@ -303,6 +303,30 @@ def test_library_argument_checks_need_no_gpu():
         _lib.check(-2)
 
 
+@pytest.mark.parametrize("field,value,message", [("gx_scale", 7, b"scale mode"), ("gx_scale", -1, b"scale mode"), ("gx_round", 5, b"rounding"),
+                                                 ("out_dtype", 9, b"dtype")])
+@pytest.mark.parametrize("hla_n", [1, 64, 256])
+def test_backward_refuses_unknown_modes_before_any_launch(field, value, message, hla_n):
+    """Fields outside their enums, in the fused entry points: an error from the host, nothing launched."""
+    from hot_amd import _lib, ops
+    lib = _lib.lib()
+    one = C.c_void_p(4096)  # never dereferenced: every call below fails validation first
+    cfg = ops.HotOptions(hla_n=hla_n, hla_rows=tuple(range(max(1, hla_n // 2)))).to_c()
+    out = _lib.F32
+    if field == "out_dtype":
+        out = value
+    else:
+        setattr(cfg, field, value)
+    big = 1 << 40
+    assert lib.hot_linear_backward(one, one, 0, one, one, 256, 64, 64, C.byref(cfg), one, one, out, one, big, None, None) < 0
+    assert message in lib.hot_last_error()
+    assert lib.hot_linear_backward_bias(one, one, 0, one, one, 256, 64, 64, C.byref(cfg), one, one, one, out, one, big, None) < 0
+    assert message in lib.hot_last_error()
+    if hla_n <= 128:
+        assert lib.hot_linear_backward_batched_bias(one, one, 0, one, one, 2, 128, 64, 64, C.byref(cfg), one, one, one, out, one, big, None) < 0
+        assert message in lib.hot_last_error()
+
+
 def test_bench_refuses_more_than_one_gpu():
     """Every box has one GPU: the benchmark says so instead of running a second rank."""
     import subprocess
