@@ -383,9 +383,9 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   if (marks && !split) mark(STAGE_QUANT);
 
   // the products: g_x = (qG . qW^T) sG sW / n_o and g_W = (qGp . xq^T) sGp sx / hla_n
-  const GemmProduct px = {ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, b.ld_g * 8 / cfg->gx_bits, sg,
+  const GemmProduct px = {ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, b.ld_g * 8 / cfg->gx_bits, O, sg,
                           cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, I};
-  const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
+  const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
                           1.0f / (float)cfg->hla_n, gw, I};
   if (!split && cfg->streams != 2 && gemm_pair_possible(pw, px) && gemm_pair_pays(pw, px)) {
     rc = gemm_pair_impl(pw, px, out_dtype, st);
@@ -394,8 +394,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   }
   auto run_gemm = [&](const GemmProduct& p, hipStream_t s2) {
     // (no split on the side stream: the split workspace belongs to the g_W product)
-    return gemm_i8_impl(p.A, p.lda, p.B, p.ldb, p.bits, p.M, p.N, p.K, p.scale_a, p.a_per_row, p.scale_b, p.post_scale, p.out, out_dtype,
-                        p.ldo, nullptr, s2, s2 == st && b.split_bytes ? ws + b.off_split : nullptr, s2 == st ? b.split_bytes : 0);
+    return gemm_i8_impl(p, out_dtype, nullptr, s2, s2 == st && b.split_bytes ? ws + b.off_split : nullptr, s2 == st ? b.split_bytes : 0);
   };
   // Beside the g_W product when that has fewer tiles than the chip has CUs and cannot fill it alone (two large
   // products only get in each other's way).

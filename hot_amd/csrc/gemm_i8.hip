@@ -1376,8 +1376,8 @@ static int gemm_fill(GemmArgs& g, const GemmProduct& p, int out_dtype, int32_t* 
     return fail(HOT_ERR_INVALID, "hot_gemm_i8: row pitches (%lld, %lld) must be multiples of 16 and >= %lld bytes", (long long)p.lda, (long long)p.ldb, (long long)need);
   if (((uintptr_t)p.A & 15) || ((uintptr_t)p.B & 15)) return fail(HOT_ERR_INVALID, "hot_gemm_i8: operands must be 16-byte aligned");
   if (p.ldo < p.N) return fail(HOT_ERR_INVALID, "hot_gemm_i8: ldo=%lld < N", (long long)p.ldo);
-  if (p.bits == 4 && p.K > (int64_t)(0x7FFFFFFF / (112 * 112))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for the scaled INT4 accumulator");
-  if (p.bits == 8 && p.K > (int64_t)(0x7FFFFFFF / (127 * 127))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for int32 accumulation");
+  if (p.bits == 4 && p.codes > (int64_t)(0x7FFFFFFF / (112 * 112))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for the scaled INT4 accumulator");
+  if (p.bits == 8 && p.codes > (int64_t)(0x7FFFFFFF / (127 * 127))) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: K too large for int32 accumulation");
   memset(&g, 0, sizeof(g));
   g.A = (const uint8_t*)p.A; g.B = (const uint8_t*)p.B; g.lda = p.lda; g.ldb = p.ldb; g.M = p.M; g.N = p.N;
   g.ktiles = (int)(kpad / G_BK);
@@ -1393,8 +1393,14 @@ int gemm_i8_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int bit
                  int64_t K, const float* scale_a, int a_per_row, const float* scale_b, float post_scale,
                  void* out, int out_dtype, int64_t ldo, int32_t* acc_out, hipStream_t st, void* split_ws,
                  size_t split_ws_bytes, int variant) {
+  const GemmProduct p = {A, lda, B, ldb, bits, M, N, K, K, scale_a, a_per_row, scale_b, post_scale, out, ldo};
+  return gemm_i8_impl(p, out_dtype, acc_out, st, split_ws, split_ws_bytes, variant);
+}
+
+int gemm_i8_impl(const GemmProduct& p, int out_dtype, int32_t* acc_out, hipStream_t st, void* split_ws, size_t split_ws_bytes, int variant) {
+  const int64_t M = p.M, N = p.N, K = p.K, lda = p.lda, ldb = p.ldb;
+  const int bits = p.bits;
   GemmArgs g;
-  const GemmProduct p = {A, lda, B, ldb, bits, M, N, K, scale_a, a_per_row, scale_b, post_scale, out, ldo};
   if (int rc = gemm_fill(g, p, out_dtype, acc_out)) return rc;
   if (variant < HOT_GEMM_AUTO || variant >= HOT_GEMM_VARIANTS) return fail(HOT_ERR_INVALID, "hot_gemm_i8: unknown kernel variant %d", variant);
   if (M == 0 || N == 0) return HOT_OK;

@@ -117,10 +117,12 @@ struct GemmProduct {
   const void* B; int64_t ldb;
   int bits;
   int64_t M, N, K;
+  int64_t codes;       // of K, those that may be other than zero (the rest pads the rows to whole lines): bounds the accumulator
   const float* scale_a; int a_per_row;
   const float* scale_b; float post_scale;
   void* out; int64_t ldo;
 };
+int gemm_i8_impl(const GemmProduct& p, int out_dtype, int32_t* acc_out, hipStream_t st, void* split_ws = nullptr, size_t split_ws_bytes = 0, int variant = HOT_GEMM_AUTO);
 bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x);
 bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x);   // and where they are faster in one launch
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st);

@@ -64,6 +64,12 @@ def test_paired_products(gpu, L, O, I, dt, bits):
     check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
 
 
+@pytest.mark.parametrize("bits,O", [(8, 133144), (4, 171192)])
+def test_longest_rows(gpu, bits, O):
+    """As many out-features as an int32 accumulator takes: the zero codes that pad a row to whole lines do not count."""
+    check(gpu, 3, O, 8, torch.bfloat16, n_o=8, gx_bits=bits, w_bits=bits)
+
+
 @pytest.mark.parametrize("scale", [1.0, 3.1e-3, 7.7e4])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_codes_on_the_boundary(gpu, scale, bits):
