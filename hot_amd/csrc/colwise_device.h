@@ -396,10 +396,10 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
     uint32_t q[16];
     if constexpr (ROUND == HOT_ROUND_NEAREST) {
       const rint_rcp hb = rint_bounds(hrcp);
-      uint32_t unsure = 0;
+      uint32_t unsure = 0, any = 0;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) q[j] = rint_div_bits(y[j], hb, unsure);
-      if (__builtin_expect(unsure != 0, 0)) {
+      for (int j = 0; j < 16; ++j) q[j] = rint_div_bits(y[j], hb, unsure, any);
+      if (__builtin_expect((unsure | rint_nan<T>(any)) != 0, 0)) {
 #pragma unroll
         for (int j = 0; j < 16; ++j) q[j] = rint_div_exact(y[j], hd, hrcp);
       }
@@ -467,7 +467,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
         // |v / d| <= qmax (1 + 2^-22) by construction of d (absmax) or of the clip (SAWB): the rounded code cannot
         // leave [-qmax, qmax]
         const rint_rcp b = rint_bounds(rcp);
-        uint32_t unsure = 0;
+        uint32_t unsure = 0, any = 0;
         if constexpr (N >= 64 && SEL::STATIC) {
           // the coefficients are complete here: the compiler would sink the last butterfly stage into both
           // branches and hold its inputs until then (half as many registers again)
@@ -478,9 +478,9 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
 #pragma unroll
         for (int i = 0; i < N; ++i) {
           const int sl = place(i);
-          if (sl >= 0) row[sl] = (uint8_t)rint_div_bits(x[base + i], b, unsure);
+          if (sl >= 0) row[sl] = (uint8_t)rint_div_bits(x[base + i], b, unsure, any);
         }
-        if (__builtin_expect(unsure != 0, 0)) {
+        if (__builtin_expect((unsure | rint_nan<T>(any)) != 0, 0)) {
 #pragma unroll
           for (int i = 0; i < N; ++i) {
             const int sl = place(i);

@@ -234,12 +234,17 @@ __device__ __forceinline__ float part_max(const float* p, int n, int stride, int
 // two products (rcp and the quotient are each within 2^-24), so where both round to the same integer the quotient does
 // too.  `unsure` is zero while they do; otherwise (two quotients in a million) the caller takes rint_div_exact for the
 // values it covers.  (Each difference is below 2^24: up to 256 values to an `unsure`.)
+// A NaN is coded 0, in the exact form.  It passes through both products unchanged, so fp32 inputs ask the exponents as
+// well (rint_nan): the low byte of a sum is then the low byte of the NaN's payload.  16-bit inputs have no payload there.
 constexpr float RINT_MAGIC = 12582912.0f;
+constexpr uint32_t RINT_NAN = 0x30000000u;     // no bit of it is set in a sum of an integer and RINT_MAGIC
+template <typename T> __device__ __forceinline__ uint32_t rint_nan(uint32_t any) { return sizeof(T) == 4 ? any & RINT_NAN : 0u; }
 struct rint_rcp { float lo, hi; };
 __device__ __forceinline__ rint_rcp rint_bounds(float rcp) { return {rcp * (1.0f - 2.384185791015625e-07f), rcp * (1.0f + 2.384185791015625e-07f)}; }
-__device__ __forceinline__ uint32_t rint_div_bits(float x, const rint_rcp& r, uint32_t& unsure) {
+__device__ __forceinline__ uint32_t rint_div_bits(float x, const rint_rcp& r, uint32_t& unsure, uint32_t& any) {
   const uint32_t lo = as_u(__builtin_fmaf(x, r.lo, RINT_MAGIC)), hi = as_u(__builtin_fmaf(x, r.hi, RINT_MAGIC));
   unsure = (lo ^ hi) + unsure;
+  any |= lo;
   return lo;
 }
 // The same with the IEEE quotient, without a division: two residual corrections of x * rcp.  The first leaves a
@@ -249,7 +254,7 @@ __device__ __forceinline__ uint32_t rint_div_exact(float x, float d, float rcp) 
   float q = x * rcp;
   q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
   q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
-  return as_u(rintf(q) + RINT_MAGIC);
+  return q == q ? as_u(rintf(q) + RINT_MAGIC) : 0u;
 }
 
 // rint(x / d) with rcp = 1 / d precomputed: the product x * rcp is within 1.5 * 2^-23 |x/d| of

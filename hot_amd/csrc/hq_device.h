@@ -56,14 +56,15 @@ __device__ __forceinline__ void fwht_lanes(float* x, int lane, int nrt) {
   }
 }
 
-// Codes of a chunk, in the low bits of q.
+// Codes of a chunk of an input of type T, in the low bits of q.
+template <typename T>
 __device__ __forceinline__ void quant_nearest(const float* x, float d, float rcp, uint32_t* q) {
   // |x / d| <= qmax (1 + 2^-22) because d comes from the absmax: no clamp needed
   const rint_rcp r = rint_bounds(rcp);
-  uint32_t unsure = 0;
+  uint32_t unsure = 0, any = 0;
 #pragma unroll
-  for (int j = 0; j < EPL; ++j) q[j] = rint_div_bits(x[j], r, unsure);
-  if (__builtin_expect(unsure != 0, 0)) {
+  for (int j = 0; j < EPL; ++j) q[j] = rint_div_bits(x[j], r, unsure, any);
+  if (__builtin_expect((unsure | rint_nan<T>(any)) != 0, 0)) {
 #pragma unroll
     for (int j = 0; j < EPL; ++j) q[j] = rint_div_exact(x[j], d, rcp);
   }
@@ -90,11 +91,11 @@ __device__ __forceinline__ uint2 pack_codes8(const uint32_t* q) {
 __device__ __forceinline__ void store_codes4(const uint32_t* q, int8_t* out) { *reinterpret_cast<uint32_t*>(out) = pack_codes4(q); }
 __device__ __forceinline__ void store_codes8(const uint32_t* q, int8_t* out) { *reinterpret_cast<uint2*>(out) = pack_codes8(q); }
 
-template <int BITS, int ROUND>
+template <typename T, int BITS, int ROUND>
 __device__ __forceinline__ void quant_store_chunk(const float* x, float d, float rcp, uint64_t e0, uint64_t seed,
                                                   uint32_t stream, int8_t* out_row_chunk) {
   uint32_t q[EPL];
-  if constexpr (ROUND == 0) quant_nearest(x, d, rcp, q);
+  if constexpr (ROUND == 0) quant_nearest<T>(x, d, rcp, q);
   else quant_stoch(x, rcp, e0, seed, stream, (1 << (BITS - 1)) - 1, q);
   if constexpr (BITS == 4) store_codes4(q, out_row_chunk);
   else store_codes8(q, out_row_chunk);
@@ -140,10 +141,10 @@ __device__ __forceinline__ void fwht_lanes_short(float* x, int lane, int n) {
   }
 }
 
-template <int ROUND>
+template <typename T, int ROUND>
 __device__ __forceinline__ void hq_store_chunk(const HqArgs& a, const float* x, float d, float rcp, uint64_t e0, int8_t* out) {
   uint32_t q[EPL];
-  if constexpr (ROUND == HOT_ROUND_NEAREST) quant_nearest(x, d, rcp, q);
+  if constexpr (ROUND == HOT_ROUND_NEAREST) quant_nearest<T>(x, d, rcp, q);
   else quant_stoch(x, rcp, e0, a.seed, a.stream, (1 << (a.bits - 1)) - 1, q);
   if (a.bits == 4) store_codes4(q, out);
   else store_codes8(q, out);
@@ -202,7 +203,7 @@ __device__ __forceinline__ void hq_row_body(const HqArgs& a, int64_t row, int la
   for (int c = 0; c < C; ++c) {
     if (t0 + c * lanes >= nch) break;
     const int ch = t + c * lanes;
-    if (ch < nch) hq_store_chunk<ROUND>(a, x[c], d, rcp, (uint64_t)row * (uint64_t)a.K + (uint64_t)ch * EPL, orow + (int64_t)ch * cb);
+    if (ch < nch) hq_store_chunk<T, ROUND>(a, x[c], d, rcp, (uint64_t)row * (uint64_t)a.K + (uint64_t)ch * EPL, orow + (int64_t)ch * cb);
   }
   const int pad0 = nch * cb, pad = (int)(a.ld - pad0) / 4;
   for (int i = t; i < pad; i += lanes) *reinterpret_cast<uint32_t*>(orow + pad0 + i * 4) = 0u;
@@ -261,14 +262,14 @@ __device__ __forceinline__ void hq_body(const HqArgs& a, unsigned block) {
     if (ch >= a.chunks) continue;
     const uint64_t cht = (uint64_t)g * a.chunks + ch;
     if (dense) {
-      hq_store_chunk<ROUND>(a, x, d, rcp, cht * EPL, a.codes + (int64_t)cht * cb);
+      hq_store_chunk<T, ROUND>(a, x, d, rcp, cht * EPL, a.codes + (int64_t)cht * cb);
       continue;
     }
     const uint32_t row = hq_row_of(a, ch), col = ch - row * a.nch_row;
     const int64_t grow = (int64_t)g * a.rows + row;
     int8_t* orow = a.codes + grow * a.ld;
     if (a.groups > 1 && col == 0) a.scales[grow] = s;
-    hq_store_chunk<ROUND>(a, x, d, rcp, cht * EPL, orow + (int64_t)col * cb);
+    hq_store_chunk<T, ROUND>(a, x, d, rcp, cht * EPL, orow + (int64_t)col * cb);
     if (col + 1 == a.nch_row)
       for (int64_t p = (int64_t)a.nch_row * cb; p < a.ld; p += 4) *reinterpret_cast<uint32_t*>(orow + p) = 0u;
   }

@@ -75,7 +75,7 @@ __global__ void hq_row_kernel(const T* __restrict__ in, int64_t K, int8_t* __res
   for (int c = 0; c < C; ++c) {
     const int ch = tid + c * team;
     if (ch < nch) {
-      quant_store_chunk<BITS, ROUND>(x[c], d, rcp, (uint64_t)row * (uint64_t)K + (uint64_t)ch * EPL, seed,
+      quant_store_chunk<T, BITS, ROUND>(x[c], d, rcp, (uint64_t)row * (uint64_t)K + (uint64_t)ch * EPL, seed,
                                      stream, orow + (int64_t)ch * (EPL * BITS / 8));
     }
   }
@@ -128,7 +128,7 @@ __global__ void hq_tensor_kernel(const T* __restrict__ in, int64_t nchunks, int6
       const int64_t row = ch / nch_row;
       off = row * ld + (ch - row * nch_row) * (EPL * BITS / 8);
     }
-    quant_store_chunk<BITS, ROUND>(x, d, rcp, (uint64_t)ch * EPL, seed, stream, codes + off);
+    quant_store_chunk<T, BITS, ROUND>(x, d, rcp, (uint64_t)ch * EPL, seed, stream, codes + off);
   }
 }
 
@@ -184,7 +184,7 @@ __global__ void hq_group_quant_kernel(const T* __restrict__ in, int64_t chunks_p
     fwht_lanes<N>(x, lane, nrt);
     const int64_t row = ch / nch_row, col = ch - row * nch_row;
     if (col == 0) scales_out[row] = s;
-    quant_store_chunk<BITS, ROUND>(x, d, rcp, (uint64_t)ch * EPL, seed, stream, codes + row * ld + col * (EPL * BITS / 8));
+    quant_store_chunk<T, BITS, ROUND>(x, d, rcp, (uint64_t)ch * EPL, seed, stream, codes + row * ld + col * (EPL * BITS / 8));
   }
 }
 

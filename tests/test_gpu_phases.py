@@ -137,3 +137,60 @@ def test_layer_bias_gradient_per_sample(gpu, fresh_args, dt, O):
     d = gy.double().reshape(-1, O)
     bound = 6 * 197 * 2.0 ** -24 * d.abs().sum(0) + (2.0 ** -8 * d.sum(0).abs() if dt == torch.bfloat16 else 0)
     assert lin.bias.grad.dtype == dt and torch.all((lin.bias.grad.double().cpu() - d.sum(0)).abs() <= bound)
+
+
+# An fp32 NaN with a payload (its low byte is no code), quiet and negative.
+NAN = np.array([0x7FC12345, 0xFFC0007F], np.uint32).view(np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 2, 8, 16, 32, 64, 128, 256])
+@pytest.mark.parametrize("rounding", ["nearest", "stoch"])
+def test_nan_and_infinity_in_the_quantisers(gpu, n, rounding):
+    """A NaN spoils the Hadamard block that holds it and nothing else: its codes are 0, like those of a block of zeros, whatever
+    its payload.  An infinity makes the step infinite and every code 0."""
+    from hot_amd import ops
+    L, C = 512, 264
+    x = np.random.default_rng(n).standard_normal((L, C)).astype(np.float32)
+    x[300, 17] = 1000.0                                        # the absmax, in a block of its own
+    bad, zeroed = x.copy(), x.copy()
+    bad[70, 40], bad[511, 263] = NAN
+    zeroed[70 // n * n:70 // n * n + n, 40] = zeroed[511 // n * n:, 263] = 0.0
+    tok = lambda v: ops.hla_tokenwise(torch.from_numpy(v).to(gpu), n, tuple(range(n)), bits=8, rounding=rounding, seed=3)
+    for got, ref in zip(tok(bad)[:2], tok(zeroed)[:2]):
+        assert torch.equal(got, ref)
+    bad[70, 40] = np.inf
+    bad[511, 263] = 0.0
+    q, step = tok(bad)[:2]
+    assert torch.isinf(step).all() and not q.any()
+    if n > 64:
+        return
+    for scale in ("tensor", "row"):
+        w = x[:, :256].copy()
+        bad, zeroed = w.copy(), w.copy()
+        bad[70, 40], bad[511, 255] = NAN
+        zeroed[70, 40 // n * n:40 // n * n + n] = zeroed[511, 255 // n * n:] = 0.0
+        row = lambda v: ops.hq_rowwise(torch.from_numpy(v).to(gpu), n=n, bits=4, rounding=rounding, scale=scale, seed=3)
+        for got, ref in zip(row(bad), row(zeroed)):
+            assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("L,O", [(66, 272), (2999, 2064), (6464, 2064)])
+@pytest.mark.parametrize("scale", ["tensor", "row"])
+def test_nan_in_the_gradient(gpu, L, O, scale):
+    """The same through the backward: g_x misses the row-wise block that holds the NaN, g_W the token-wise one.  The last two
+    shapes join the row-wise quantiser to the token-wise pass (steps per tensor)."""
+    from hot_amd import ops
+    x, w, gy = make_case(L, O, 24, seed=5, dtype=torch.float32)
+    ocfg = orc.HotConfig.python_rule(L, gx_scale=orc.SCALE_ROW if scale == "row" else orc.SCALE_TENSOR)
+    opt, n = _options(ocfg), ocfg.hla_n
+    gy = gy.numpy()
+    gy[1, 3] = 100 * np.abs(gy).max()
+    t, o = L - 1, O - 20                                        # (a Hadamard block other than the one of the absmax)
+    bad, zero_row, zero_tok = gy.copy(), gy.copy(), gy.copy()
+    bad[t, o] = NAN[0]
+    zero_row[t, o // 16 * 16:o // 16 * 16 + 16] = 0.0
+    zero_tok[t // n * n:t // n * n + n, o] = 0.0
+    xq, sx = ops.abc_forward(x.to(gpu), opt)
+    back = lambda v: ops.linear_backward(torch.from_numpy(v).to(gpu), w.to(gpu), xq, sx, opt)
+    gx, gw = back(bad)[:2]
+    assert torch.equal(gx, back(zero_row)[0]) and torch.equal(gw, back(zero_tok)[1])
