@@ -1096,12 +1096,21 @@ def test_hq_linear_3d_per_sample_on_the_separate_gx_paths(gpu, fresh_args, path,
     assert np.array_equal(lin.weight.grad.cpu().numpy(), gw)
 
 
-def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_args):
+def _watch_buffer_streams(qm, monkeypatch):
+    """The stream of every buffer write from here on (None: in line)."""
+    taken, pick = [], qm._buffer_stream
+    monkeypatch.setattr(qm, "_buffer_stream", lambda x: taken.append(pick(x)) or taken[-1])
+    return taken
+
+
+def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_args, monkeypatch):
     """The reference trains under autocast (ViT_main.py:386): x stays fp32, F.linear makes and releases
     a bf16 copy of it while the buffer kernels run on the side stream.  Their outputs and workspace come
     from the side stream's own pool, so the released copy cannot be handed to them; the buffer, g_x and
     g_W equal those of the same step with the buffer written in line, over several layers in a row."""
     from hot_amd import quant_matmul as qm
+    monkeypatch.setattr(qm, "OVERLAP_MIN_BYTES", 0)         # (layers this small are written in line by themselves)
+    taken = _watch_buffer_streams(qm, monkeypatch)
     L, I, O = 3200, 256, 512
     torch.manual_seed(4)
     lins = [qm.HQ_Linear(I, O).to(gpu), qm.HQ_Linear(O, I).to(gpu), qm.HQ_Linear(I, O).to(gpu)]
@@ -1124,19 +1133,39 @@ def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_arg
 
     try:
         ref = run(False)
+        assert taken == [None] * 3
         for _ in range(3):
             got = run(True)
             for a, b in zip(got, ref):
                 assert torch.equal(a, b)
+        assert len(taken) == 12 and None not in taken[3:]
     finally:
         qm.overlap_buffer_write = True
 
 
-def test_hq_linear_small_inputs_beside_the_product(gpu, fresh_args, monkeypatch):
-    """The same with the side stream taken by inputs of every size (by default it begins at 24 MiB)."""
+@pytest.mark.parametrize("rows,beside", [(24 * 1024, True), (24 * 1024 - 1, False)])
+def test_hq_linear_buffer_write_beside_the_product_from_24_mib(gpu, fresh_args, monkeypatch, rows, beside):
+    """The side stream is taken by inputs of 24 MiB and more, smaller ones are written in line; the gradients are those of
+    the in-line write."""
     from hot_amd import quant_matmul as qm
-    monkeypatch.setattr(qm, "OVERLAP_MIN_BYTES", 0)
-    test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_args)
+    taken = _watch_buffer_streams(qm, monkeypatch)
+    torch.manual_seed(4)
+    lin = qm.HQ_Linear(512, 64).to(gpu, torch.bfloat16)
+    x0 = torch.randn(rows, 512, device=gpu).bfloat16()
+    gy = (torch.randn(rows, 64, device=gpu) * 1e-3).bfloat16()
+
+    def run(overlap):
+        monkeypatch.setattr(qm, "overlap_buffer_write", overlap)
+        fresh_args.sr_step = 0
+        lin.zero_grad(set_to_none=True)
+        x = x0.clone().requires_grad_(True)
+        lin(x).backward(gy)
+        return x.grad, lin.weight.grad.clone(), lin.bias.grad.clone()
+
+    ref, got = run(False), run(True)
+    assert [t is not None for t in taken] == [False, beside]
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("gw_bits,act_bits", [(4, 8), (4, 4), (8, 4)])
