@@ -374,7 +374,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   }
   if (!hq_job) {
     rc = hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg,
-                         b.ld_g, sg, slots, STAT_SLOT_BYTES, st, false);
+                         b.ld_g, sg, slots, STAT_SLOT_BYTES, st);
     if (rc) return rc;
   }
   if (split) mark(K_GY_HQ);
@@ -895,7 +895,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
   if (!rc && !w_short) rc = phase_launch(1, dtype, &wj, nullptr, nullptr, nullptr, st);
   if (!rc && !hq_job)
     rc = hq_rowwise_impl(gy, dtype, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale,
-                         ws + b.off_qg, b.ld_g, sg, ws + b.off_hq, b.off_sg - b.off_hq, st, false, row_tensor ? T : 0, nullptr);
+                         ws + b.off_qg, b.ld_g, sg, ws + b.off_hq, b.off_sg - b.off_hq, st, row_tensor ? T : 0);
   if (rc) return rc;
   rc = gemm_i8_impl(ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, O, sg, cfg->gx_scale == HOT_SCALE_ROW || B > 1 || !hq_job, sw,
                     1.0f / (float)cfg->n_o, gx, out_dtype, I, nullptr, st);   // (one sample: one step for the whole operand)

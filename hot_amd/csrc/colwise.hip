@@ -49,7 +49,7 @@ __global__ void colwise_clear_kernel(float* colmax, int64_t ncolmax, float* gsta
 // ---- column sums ------------------------------------------------------------------
 
 // Sums of a strip of rows per channel, thread = channel: the stand-alone form of what the statistics
-// pass of colwise_kernel delivers for free (used when the token blocks take the two-level path).
+// pass of the phase kernels delivers for free (used when the token blocks take the two-level path).
 template <typename T>
 __global__ void __launch_bounds__(256) colsum_strip_kernel(const void* in, int64_t R, int64_t C, int64_t rows_per_wg,
                                                             float* partial) {
@@ -85,16 +85,16 @@ size_t hla_workspace_bytes_impl(int64_t R, int64_t C, int n, int r) {
 
 constexpr int64_t COL_MAX_WGS = 65536;   // workgroups of a pass
 size_t colwise_workspace_bytes_impl(int64_t C) {
-  // head | per-channel max | a statistic per workgroup: two doubles (SAWB), or an absmax and a row-wise absmax
-  return COL_STAT_BYTES + (size_t)round_up(C * 4 * COLMAX_COPIES, 256) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
+  // per-channel max | a statistic per workgroup: two doubles (SAWB), or an absmax and a row-wise absmax
+  return (size_t)round_up(C * 4 * COLMAX_COPIES, 256) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
 }
 
-// with sample groups: head | per-sample per-channel max | per-sample statistics | partial sums
+// with sample groups: per-sample per-channel max | per-sample statistics | partial sums
 static size_t group_colmax_bytes(int64_t C, int groups) { return (size_t)round_up(C * 4 * (int64_t)groups, 256); }
 static size_t group_gstat_bytes(int groups) { return (size_t)round_up((int64_t)groups * GS * 4, 256); }
 size_t colwise_group_workspace_bytes_impl(int64_t C, int groups) {
   if (groups <= 1) return colwise_workspace_bytes_impl(C);
-  return COL_STAT_BYTES + group_colmax_bytes(C, groups) + group_gstat_bytes(groups) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
+  return group_colmax_bytes(C, groups) + group_gstat_bytes(groups) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
 }
 
 // Token blocks per workgroup of the quantise pass (tb) and of an absmax statistics pass (tb0).
@@ -210,11 +210,11 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
   if ((uintptr_t)workspace & 255) return fail(HOT_ERR_INVALID, "%s: workspace must be 256-byte aligned", who);
   a.store4 = store4;
   uint8_t* ws = (uint8_t*)workspace;
-  a.colmax = (float*)(ws + COL_STAT_BYTES);
-  uint8_t* part = ws + COL_STAT_BYTES + (groups > 1 ? group_colmax_bytes(C, groups) + group_gstat_bytes(groups) : (size_t)round_up(C * 4 * COLMAX_COPIES, 256));
+  a.colmax = (float*)ws;
+  uint8_t* part = ws + (groups > 1 ? group_colmax_bytes(C, groups) + group_gstat_bytes(groups) : (size_t)round_up(C * 4 * COLMAX_COPIES, 256));
   a.partial = (double*)part;
   a.pmax = (float*)part;
-  if (groups > 1) a.gstat = (float*)(ws + COL_STAT_BYTES + group_colmax_bytes(C, groups));
+  if (groups > 1) a.gstat = (float*)(ws + group_colmax_bytes(C, groups));
   a.rowmajor = rowmajor ? 1 : 0;
   a.groups = groups; a.NBs = a.NB / groups; a.Kpad = groups > 1 ? kpad_group : ld_out;
   a.scales_out = scales_out;
@@ -426,13 +426,13 @@ int colwise_quant_impl(const void* in, int dtype, int64_t R, int64_t C, int n, c
 
 // ---- the entry point that allocates nothing ---------------------------------------
 //
-// hot_hla_tokenwise needs a workspace (statistics words, per-channel maxima, per-workgroup sums).
+// hot_hla_tokenwise needs a workspace (per-channel maxima, a statistic per workgroup).
 // For callers that cannot allocate one, the same kernels run on a fixed array in device memory
 // that is part of the library's code object: every GPU that loads the library holds one copy of
 // it until the process ends.  Its size fixes the largest channel count the entry point takes.
 constexpr int64_t STATIC_MAX_C = HOT_STATIC_MAX_CHANNELS;
 constexpr size_t STATIC_SCRATCH_BYTES =
-    COL_STAT_BYTES + (size_t)STATIC_MAX_C * 4 * COLMAX_COPIES + (size_t)(2 * sizeof(double)) * 65536;
+    (size_t)STATIC_MAX_C * 4 * COLMAX_COPIES + (size_t)(2 * sizeof(double)) * 65536;
 static_assert((STATIC_MAX_C * 4 * COLMAX_COPIES) % 256 == 0, "the per-channel maxima end on a 256-byte boundary");
 static __device__ __align__(256) uint8_t scratch[STATIC_SCRATCH_BYTES];
 
@@ -471,8 +471,7 @@ extern "C" int hot_hla_tokenwise_static(const void* in, int dtype, int64_t R, in
                 (long long)C, (long long)STATIC_MAX_C);
   uint8_t* ws = nullptr;
   if (int rc = static_scratch_ptr(&ws, who)) return rc;
-  // the statistics words at the head of the array are cleared by the first kernel of the call
-  // (stats_cleared = false), everything else is written before it is read
+  // (per-channel maxima are cleared by the first kernel of the call, everything else is written before it is read)
   return colwise_quant_impl(in, dtype, R, C, n, rows, r, bits, rounding, seed, rng_stream, scale_mode, codes_out,
                             ld_out, /*store4=*/0, scales_out, ws, STATIC_SCRATCH_BYTES, (hipStream_t)hip_stream, who);
 }

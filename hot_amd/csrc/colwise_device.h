@@ -11,7 +11,6 @@
 namespace hot {
 
 constexpr int CW = 256;        // threads per workgroup = channels per workgroup
-constexpr size_t COL_STAT_BYTES = 256 + STAT_SLOT_BYTES;   // head of the workspace, ahead of the per-channel maxima
 constexpr int COLMAX_COPIES = 8;  // per-channel maxima: workgroup row y folds into copy y % 8 (fewer atomics per line)
 constexpr int CW_ROWS = 16;    // rows staged per step
 
@@ -290,7 +289,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
 
   float d = 1.f, rcp = 1.f, clip = 0.f;
   if constexpr (PASS == 1) {
-    // the steps come from the statistics themselves (no finalize kernel in between), read behind the first
+    // the steps come from the statistics themselves (no kernel in between), read behind the first
     // rows' way here; the first workgroup publishes them
     if (sawb) {
       // sums of the statistics pass, added in a fixed order: 256 strided chains, then a tree
@@ -679,7 +678,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       }
       return;
     }
-    // SAWB: per-workgroup partial sums, reduced in a fixed order by the finalize kernel
+    // SAWB: per-workgroup partial sums, reduced in a fixed order by every workgroup of the quantise pass
     ssq = wave_sum(active ? ssq : 0.0);
     sab = wave_sum(active ? sab : 0.0);
     if (lane == 0) { s_sum[0][wave] = ssq; s_sum[1][wave] = sab; }

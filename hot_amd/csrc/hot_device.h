@@ -98,12 +98,6 @@ __device__ __forceinline__ void unpack_vec<f16_t>(const uint4& raw, float* out) 
   }
 }
 
-// Scalar element load -> fp32 (used by the column-wise kernels).
-template <typename T> __device__ __forceinline__ float load_scalar(const T* p);
-template <> __device__ __forceinline__ float load_scalar<float>(const float* p) { return *p; }
-template <> __device__ __forceinline__ float load_scalar<bf16_t>(const bf16_t* p) { return as_f((uint32_t)p->v << 16); }
-template <> __device__ __forceinline__ float load_scalar<f16_t>(const f16_t* p) { return (float)p->v; }
-
 // round-to-nearest-even; gfx950 converts in hardware (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
@@ -187,11 +181,6 @@ __device__ __forceinline__ int q_stoch_fix(float x, float rcpk, uint32_t r, int 
   const uint32_t m = min(((uint32_t)p + r) >> 16, (uint32_t)qmax);
   return x < 0.f ? -(int)m : (int)m;
 }
-
-// y = x / d already divided.  Nearest: ties to even.
-__device__ __forceinline__ int q_nearest(float y) { return (int)rintf(y); }
-
-__device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
 // non-negative float max through an integer atomic (bit patterns of
 // non-negative floats are ordered like unsigned integers).  The plain read

@@ -33,10 +33,10 @@ constexpr size_t STAT_SLOT_BYTES = (size_t)STAT_SLOTS * STAT_SLOT_STRIDE * 4;   
 int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int bits, int rounding,
                     uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_codes,
                     float* scales_out, void* workspace, size_t workspace_bytes, hipStream_t st,
-                    bool absmax_ready = false, int64_t group_rows = 0, float* group_steps = nullptr);
+                    int64_t group_rows = 0);
 // group_rows > 0 (per-tensor steps only): every run of group_rows rows is a sample with a step of its
 // own; scales_out then holds M entries (the step of each row's sample, the form the GEMM epilogue
-// reads), group_steps (may be null) the M / group_rows steps, and the workspace 128 bytes per sample.
+// reads), and the workspace takes 128 bytes per sample.
 
 // The row-wise quantiser (blocks of up to 16; per-row steps: K <= HQ_ROW_MAX_K) as a job of a quantise phase (phase.h).
 // stat: nstat absmax values stat_stride floats apart; with groups > 1 one per sample, stat_stride apart, and scales_out [M].

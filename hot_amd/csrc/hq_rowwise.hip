@@ -162,20 +162,17 @@ __global__ void hq_group_absmax_kernel(const T* __restrict__ in, int64_t chunks_
   }
 }
 
-// scales_out [M]: the step of every row (= of its group), the form the GEMM epilogue reads;
-// group_steps [groups] (may be null): the steps themselves
+// scales_out [M]: the step of every row (= of its group), the form the GEMM epilogue reads
 template <typename T, int N, int BITS, int ROUND>
 __global__ void hq_group_quant_kernel(const T* __restrict__ in, int64_t chunks_per_group, int64_t nch_row, int64_t ld,
                                       const float* __restrict__ gmax, int8_t* __restrict__ codes,
-                                      float* __restrict__ scales_out, float* __restrict__ group_steps, uint64_t seed,
-                                      uint32_t stream, int nrt) {
+                                      float* __restrict__ scales_out, uint64_t seed, uint32_t stream, int nrt) {
   const int lane = threadIdx.x & 63;
   const int64_t g = blockIdx.y;
   constexpr float QMAXF = (float)((1 << (BITS - 1)) - 1);
   const float s = gmax[g * GROUP_STAT_STRIDE] / QMAXF;
   const float d = s + 1e-11f;
   const float rcp = 1.0f / d;
-  if (group_steps && blockIdx.x == 0 && threadIdx.x == 0) group_steps[g] = s;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t c0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c0 < chunks_per_group; c0 += stride) {
     const int64_t ch = g * chunks_per_group + c0;
@@ -331,17 +328,15 @@ static int launch_row(const void* in, int64_t M, int64_t K, void* codes, int64_t
 
 template <typename T, int N, int BITS, int ROUND>
 static int launch_tensor(const void* in, int64_t M, int64_t K, void* codes, int64_t ld, float* scales, float* absmax,
-                         uint64_t seed, uint32_t stream_id, hipStream_t st, bool absmax_ready, int nrt) {
+                         uint64_t seed, uint32_t stream_id, hipStream_t st, int nrt) {
   const int64_t nch = M * K / EPL;
   const int block = 256;
   int64_t blocks = (nch + block - 1) / block;
   const int64_t cap = 256 * 16;  // 16 workgroups per CU, grid-stride beyond
   if (blocks > cap) blocks = cap;
   if (blocks < 1) blocks = 1;
-  if (!absmax_ready) {
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(2), dim3(256), 0, st, (uint32_t*)absmax, 0u, (int)(STAT_SLOT_BYTES / 4));
-    hipLaunchKernelGGL((hq_absmax_kernel<T, N>), dim3((unsigned)blocks), dim3(block), 0, st, (const T*)in, nch, absmax, nrt);
-  }
+  hipLaunchKernelGGL(fill_u32_kernel, dim3(2), dim3(256), 0, st, (uint32_t*)absmax, 0u, (int)(STAT_SLOT_BYTES / 4));
+  hipLaunchKernelGGL((hq_absmax_kernel<T, N>), dim3((unsigned)blocks), dim3(block), 0, st, (const T*)in, nch, absmax, nrt);
   hipLaunchKernelGGL((hq_tensor_kernel<T, N, BITS, ROUND>), dim3((unsigned)blocks), dim3(block), 0, st,
                      (const T*)in, nch, K / EPL, ld, absmax, (int8_t*)codes, scales, seed, stream_id, nrt);
   return check_launch("hq_tensor_kernel");
@@ -349,7 +344,7 @@ static int launch_tensor(const void* in, int64_t M, int64_t K, void* codes, int6
 
 template <typename T, int N, int BITS, int ROUND>
 static int launch_groups(const void* in, int64_t M, int64_t K, void* codes, int64_t ld, float* scales, float* gmax,
-                         float* group_steps, int64_t group_rows, uint64_t seed, uint32_t stream_id, hipStream_t st, int nrt) {
+                         int64_t group_rows, uint64_t seed, uint32_t stream_id, hipStream_t st, int nrt) {
   const int64_t groups = M / group_rows, cpg = group_rows * (K / EPL);
   int64_t bx = (cpg + 255) / 256;
   const int64_t cap = (256 * 16 + groups - 1) / groups;    // about 16 workgroups per CU in all
@@ -360,49 +355,48 @@ static int launch_groups(const void* in, int64_t M, int64_t K, void* codes, int6
   hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((groups * GROUP_STAT_STRIDE + 255) / 256)), dim3(256), 0, st, (uint32_t*)gmax, 0u, (int)(groups * GROUP_STAT_STRIDE));
   hipLaunchKernelGGL((hq_group_absmax_kernel<T, N>), grid, dim3(256), 0, st, (const T*)in, cpg, gmax, nrt);
   hipLaunchKernelGGL((hq_group_quant_kernel<T, N, BITS, ROUND>), grid, dim3(256), 0, st, (const T*)in, cpg, K / EPL, ld, gmax,
-                     (int8_t*)codes, scales, group_steps, seed, stream_id, nrt);
+                     (int8_t*)codes, scales, seed, stream_id, nrt);
   return check_launch("hq_group_quant_kernel");
 }
 
 template <typename T, int N, int BITS, int ROUND>
 static int dispatch_mode(int scale_mode, const void* in, int64_t M, int64_t K, void* codes, int64_t ld, float* scales,
-                         float* absmax, uint64_t seed, uint32_t stream_id, hipStream_t st, bool absmax_ready, int nrt,
-                         int64_t group_rows, float* group_steps) {
+                         float* absmax, uint64_t seed, uint32_t stream_id, hipStream_t st, int nrt, int64_t group_rows) {
   const int64_t row_bytes = K * BITS / 8;
   if (ld > row_bytes) {
     const int64_t n = M * ((ld - row_bytes) / 4);
     hipLaunchKernelGGL(zero_pad_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (int8_t*)codes, M, row_bytes, ld);
   }
   if (scale_mode == HOT_SCALE_TENSOR && group_rows > 0)
-    return launch_groups<T, N, BITS, ROUND>(in, M, K, codes, ld, scales, absmax, group_steps, group_rows, seed, stream_id, st, nrt);
+    return launch_groups<T, N, BITS, ROUND>(in, M, K, codes, ld, scales, absmax, group_rows, seed, stream_id, st, nrt);
   if (scale_mode == HOT_SCALE_ROW) return launch_row<T, N, BITS, ROUND>(in, M, K, codes, ld, scales, seed, stream_id, st, nrt);
-  return launch_tensor<T, N, BITS, ROUND>(in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, nrt);
+  return launch_tensor<T, N, BITS, ROUND>(in, M, K, codes, ld, scales, absmax, seed, stream_id, st, nrt);
 }
 
 template <typename T, int N>
 static int dispatch_bits(int bits, int rounding, int scale_mode, const void* in, int64_t M, int64_t K,
                          void* codes, int64_t ld, float* scales, float* absmax, uint64_t seed, uint32_t stream_id,
-                         hipStream_t st, bool absmax_ready, int nrt, int64_t group_rows, float* group_steps) {
+                         hipStream_t st, int nrt, int64_t group_rows) {
   if (bits == 4) {
     return rounding == HOT_ROUND_NEAREST
-               ? dispatch_mode<T, N, 4, 0>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, nrt, group_rows, group_steps)
-               : dispatch_mode<T, N, 4, 1>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, nrt, group_rows, group_steps);
+               ? dispatch_mode<T, N, 4, 0>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, nrt, group_rows)
+               : dispatch_mode<T, N, 4, 1>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, nrt, group_rows);
   }
   return rounding == HOT_ROUND_NEAREST
-             ? dispatch_mode<T, N, 8, 0>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, nrt, group_rows, group_steps)
-             : dispatch_mode<T, N, 8, 1>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, nrt, group_rows, group_steps);
+             ? dispatch_mode<T, N, 8, 0>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, nrt, group_rows)
+             : dispatch_mode<T, N, 8, 1>(scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, nrt, group_rows);
 }
 
 template <typename T>
 static int dispatch_n(int n, int bits, int rounding, int scale_mode, const void* in, int64_t M, int64_t K,
                       void* codes, int64_t ld, float* scales, float* absmax, uint64_t seed, uint32_t stream_id,
-                      hipStream_t st, bool absmax_ready, int64_t group_rows, float* group_steps) {
+                      hipStream_t st, int64_t group_rows) {
   switch (n) {
     case 1: case 2: case 4: case 8:
-      return dispatch_bits<T, 8>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, n, group_rows, group_steps);
-    case 16: return dispatch_bits<T, 16>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, n, group_rows, group_steps);
-    case 32: return dispatch_bits<T, 32>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, n, group_rows, group_steps);
-    default: return dispatch_bits<T, 64>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, absmax_ready, n, group_rows, group_steps);
+      return dispatch_bits<T, 8>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, n, group_rows);
+    case 16: return dispatch_bits<T, 16>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, n, group_rows);
+    case 32: return dispatch_bits<T, 32>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, n, group_rows);
+    default: return dispatch_bits<T, 64>(bits, rounding, scale_mode, in, M, K, codes, ld, scales, absmax, seed, stream_id, st, n, group_rows);
   }
 }
 
@@ -489,8 +483,8 @@ int hq_job_impl(HqArgs& a, const void* in, int64_t M, int64_t K, int n, int bits
 
 int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int bits, int rounding,
                     uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_codes,
-                    float* scales_out, void* workspace, size_t workspace_bytes, hipStream_t st, bool absmax_ready,
-                    int64_t group_rows, float* group_steps) {
+                    float* scales_out, void* workspace, size_t workspace_bytes, hipStream_t st,
+                    int64_t group_rows) {
   if (M != 0 && (!in || !codes_out || !scales_out)) return fail(HOT_ERR_INVALID, "hot_hq_rowwise: null pointer");
   if (M < 0 || K <= 0) return fail(HOT_ERR_INVALID, "hot_hq_rowwise: bad shape M=%lld K=%lld", (long long)M, (long long)K);
   if (n < 1 || n > 64 || (n & (n - 1))) return fail(HOT_ERR_UNSUPPORTED, "hot_hq_rowwise: Hadamard block %d (a power of two up to 64)", n);
@@ -511,9 +505,9 @@ int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int 
   }
   if (M == 0) return HOT_OK;
   switch (dtype) {
-    case HOT_F32: return dispatch_n<float>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, absmax_ready, group_rows, group_steps);
-    case HOT_BF16: return dispatch_n<bf16_t>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, absmax_ready, group_rows, group_steps);
-    case HOT_F16: return dispatch_n<f16_t>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, absmax_ready, group_rows, group_steps);
+    case HOT_F32: return dispatch_n<float>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, group_rows);
+    case HOT_BF16: return dispatch_n<bf16_t>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, group_rows);
+    case HOT_F16: return dispatch_n<f16_t>(n, bits, rounding, scale_mode, in, M, K, codes_out, ld_codes, scales_out, absmax, seed, rng_stream, st, group_rows);
     default: return fail(HOT_ERR_INVALID, "hot_hq_rowwise: bad dtype %d", dtype);
   }
 }
