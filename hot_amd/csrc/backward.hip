@@ -94,10 +94,10 @@ static BwdLayout bwd_layout(int64_t L, int64_t O, int64_t I, const hot_config* c
   return b;
 }
 
-// One stream or two.  The transform + quantise work is two launches either way; the second stream carries the g_x
-// product beside the g_W product.  Forking and joining it costs the host two event record / wait pairs, 21 us
-// (measured), which only long calls hide: calls with little arithmetic (both products together below 30 GOP, e.g.
-// ViT-B proj at 12608 tokens) keep everything on the caller's stream.
+// One stream or two, for products that cannot share a launch.  The transform + quantise work is two launches either way; the
+// second stream carries the g_x product beside the g_W product.  Forking and joining it costs the host two event record /
+// wait pairs, 21 us (measured), which only long calls hide: calls with little arithmetic (both products together below
+// 30 GOP, e.g. ViT-B proj at 12608 tokens) keep everything on the caller's stream.
 static int backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* c) {
   if (c->streams == 1 || c->streams == 2) return c->streams;
   const double lp = (double)((L / c->hla_n) * c->hla_r);
@@ -387,7 +387,8 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
                           cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, I};
   const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
                           1.0f / (float)cfg->hla_n, gw, I};
-  if (!split && cfg->streams != 2 && gemm_pair_possible(pw, px) && gemm_pair_pays(pw, px)) {
+  const bool pairable = gemm_pair_possible(pw, px);
+  if (!split && cfg->streams != 2 && pairable && gemm_pair_pays(pw, px)) {
     rc = gemm_pair_impl(pw, px, out_dtype, st);
     if (!rc && marks) mark(STAGE_GEMM);
     return rc;
@@ -396,11 +397,14 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
     // (no split on the side stream: the split workspace belongs to the g_W product)
     return gemm_i8_impl(p, out_dtype, nullptr, s2, s2 == st && b.split_bytes ? ws + b.off_split : nullptr, s2 == st ? b.split_bytes : 0);
   };
-  // Beside the g_W product when that has fewer tiles than the chip has CUs and cannot fill it alone (two large
-  // products only get in each other's way).
+  // Beside the g_W product when that has fewer tiles than the chip has CUs and cannot fill it alone (two large products
+  // only get in each other's way), and only where the caller asks for it or an operand is too large for the paired kernel.  A
+  // g_x product that could pair but is better off alone has few tiles and a long K: the fork is 10 us of GPU time and as much
+  // of the host's that its neighbour does not cover, and the split workspace stays behind (us of the whole backward, INT8,
+  // forked / one after the other: 3904 x 10496 x 384 113 / 101, 8128 x 9984 x 320 182 / 172, 4032 x 5120 x 640 82 / 69).
   std::unique_lock<std::mutex> side_guard(g_side_mutex, std::defer_lock);
   SideLane* side = nullptr;
-  if (!marks && backward_streams(L, O, I, cfg) == 2 && ((O + 127) / 128) * ((I + 127) / 128) < 256) {
+  if (!marks && (cfg->streams == 2 || !pairable) && backward_streams(L, O, I, cfg) == 2 && ((O + 127) / 128) * ((I + 127) / 128) < 256) {
     side_guard.lock();
     side = side_lane_locked();
     if (!side) side_guard.unlock();

@@ -102,18 +102,19 @@ typedef struct hot_config {
                                   they take a two-level transform through an fp32
                                   workspace (launches only: capturable)          */
   int32_t streams;  /* launch order of hot_linear_backward(_bias): 0 = the library's rule
-                       (both products in one launch where their operands allow it, else
-                       hot_backward_streams), 1 = every kernel on the caller's stream, 2 =
-                       the products apart, g_x on the library's side stream when g_W cannot fill
-                       the chip (forked and joined by events).  The results do not depend on it. */
+                       (both products in one launch where that is the faster order, else one
+                       after the other; with an operand of 4 GiB or more hot_backward_streams),
+                       1 = every kernel on the caller's stream, 2 = the products apart, g_x on
+                       the library's side stream when g_W cannot fill the chip (forked and
+                       joined by events).  The results do not depend on it.             */
   int32_t reserved; /* 0 */
 } hot_config;
 
 HOT_API const char* hot_last_error(void);
-/* 1 or 2: the launch order hot_linear_backward takes for this shape when its two products do not share a
- * launch (cfg->streams when it is 1 or 2).  Short calls, whose kernels take less time than the host needs
- * for the event operations that fork and join the side stream, run on one stream; in long ones the g_x
- * product may run beside the g_W product. */
+/* 1 or 2: the launch order hot_linear_backward takes for this shape when its two products cannot share a
+ * launch (an operand of 4 GiB or more; cfg->streams when it is 1 or 2).  Short calls, whose kernels take less
+ * time than the host needs for the event operations that fork and join the side stream, run on one stream;
+ * in long ones the g_x product may run beside the g_W product. */
 HOT_API int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_abi_version(void);
 
@@ -232,11 +233,13 @@ HOT_API int hot_abc_forward(const void* x, int dtype, int64_t L, int64_t I, cons
  *               the call synchronise the stream and run its kernels one after the
  *               other on `hip_stream`
  * Without timing the transforms take two launches (statistics, then everything that needs a
- * step), each a grid of independent jobs, and the two products one.  Products that cannot share
- * a launch follow one another, or, when the g_W product is too small to fill the chip, the g_x
- * product runs on a side stream of the library (one per device, created on first use, default
- * priority) between events recorded on `hip_stream` and a wait on it; everything is ordered
- * after earlier work on `hip_stream` and before later work on it.
+ * step), each a grid of independent jobs, behind a clear when g_W has a step per channel, and the
+ * two products one.  Products that are faster apart (a g_x of few tiles and a long K, two products
+ * that fill their rounds of large tiles) follow one another.  With cfg->streams = 2, or by the rule
+ * of hot_backward_streams when an operand of 4 GiB or more rules the shared launch out, and a g_W
+ * product too small to fill the chip, the g_x product runs on a side stream of the library (one per
+ * device, created on first use, default priority) between events recorded on `hip_stream` and a
+ * wait on it.  Everything is ordered after earlier work on `hip_stream` and before later work on it.
  */
 HOT_API size_t hot_backward_workspace_bytes(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_linear_backward(const void* gy, const void* w, int dtype, const void* xq,

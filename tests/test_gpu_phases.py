@@ -194,3 +194,21 @@ def test_nan_in_the_gradient(gpu, L, O, scale):
     back = lambda v: ops.linear_backward(torch.from_numpy(v).to(gpu), w.to(gpu), xq, sx, opt)
     gx, gw = back(bad)[:2]
     assert torch.equal(gx, back(zero_row)[0]) and torch.equal(gw, back(zero_tok)[1])
+
+
+@pytest.mark.parametrize("L,O,I,bits", [(4032, 5120, 640, 8), (4672, 11008, 256, 4)])
+def test_long_products_that_leave_the_paired_launch(gpu, L, O, I, bits):
+    """Few g_x tiles with a long K in a call long enough for a side stream: the default order keeps both products on the
+    caller's stream (shorter INT8 tiles; INT4 in K ranges through the split workspace) and gives the bits of the forced orders."""
+    from dataclasses import replace
+    from hot_amd import ops
+    x, w, gy = make_case(L, O, I, seed=6, dtype=torch.bfloat16)
+    ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits)
+    opt = _options(ocfg)
+    assert ops.backward_streams(L, O, I, opt) == 2
+    gx, gw, tr = run_both(x, w, gy, ocfg, opt, gpu)
+    assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(gx.dtype)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(gw.dtype))
+    xq, sx = ops.abc_forward(x.to(gpu), opt)
+    for streams in (1, 2):
+        other = ops.linear_backward(gy.to(gpu), w.to(gpu), xq, sx, replace(opt, streams=streams))
+        assert torch.equal(gx, other[0]) and torch.equal(gw, other[1])
