@@ -1433,7 +1433,8 @@ int gemm_i8_impl(const GemmProduct& p, int out_dtype, int32_t* acc_out, hipStrea
 //     x 3072 + 3072 x 768 x 7092: 69.1 / 86.1; 3003 x 520 x 1000 + 1000 x 520 x 3003: 11.8 / 19.3; 128 tokens: 5.3 / 10.0
 //   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008 INT4 + 11008 x 4096 x 4096: 409 / 456;
 //     8192 x 11008 x 4096 + 4096 x 11008 x 2080: 348 / 424; 8192 x 4096 x 4096 + 4096^3: 174 / 187
-// (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174).
+// (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174; the products
+// alone, launched over and over: inside a step the 256 x 256 tiles that have their rounds full come out ahead, gemm_pair_pays).
 struct PairArgs {
   GemmArgs w, x;
   uint32_t w_blocks;      // a multiple of 8: blockIdx % 8 stays the XCD of the second product's tiles
@@ -1488,10 +1489,24 @@ bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
 // slower than the better of the two; us of both products, pair / apart: 2758 x 128 x 8520 INT4 32.0 / 26.2, 197 x 1024 x
 // 10624 45.1 / 29.3, INT8 63.7 / 34.1, 1001 x 768 x 3072 INT8 23.8 / 19.0; 2758 x 768 x 3072 INT4 20.6 / 28.5,
 // 4583 x 128 x 4096 21.4 / 27.6, 8191 x 128 x 8520 35.4 / 45.2.
+//
+// What the pair gains is idle CUs filled and stores hidden; what it gives up is the 256 x 256 tile, which asks the L2 for 0.6
+// of the operand bytes per operation.  Two products that take that tile, fill its rounds and have few stores for their
+// operations (K of g_x no shorter than 2/3 of its width, 14 stages and more in g_W) have nothing to gain.  us of the whole
+// backward bf16, pair / apart: INT4 8192 x 11008 x 4096 576 / 560 (the first 20 calls of an idle GPU 672 / 645), 8192 x 4096
+// x 4096 231 / 224; INT8 the same 685 / 635, 263 / 240, 9216 x 8704 x 3584 708 / 675; on the other side of the lines INT4
+// 4608 x 4608 x 10624 357 / 393, 8192 x 4096 x 11008 523 / 550, INT8 2048 x 8192 x 8064 323 / 342, 3200 x 8576 x 9856 568 / 610.
+// Of 70 shapes of both products in such tiles one that goes apart is slower for it by more than 1 % (4096 x 9984 x 8192
+// INT4 553 / 567; cold 636 / 616).
 bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
   auto stages = [](const GemmProduct& p) { return round_up(p.K, GEMM_KTILE) * p.bits / 8 / 128; };
   const int64_t x_tiles = ((x.M + 127) / 128) * ((x.N + 127) / 128);
-  return x_tiles > 192 || stages(x) < 14 || stages(x) < 2 * stages(w);
+  if (x_tiles <= 192 && stages(x) >= 14 && stages(x) >= 2 * stages(w)) return false;
+  auto tile256 = [](const GemmProduct& p) { return gemm_plan_impl(p.M, p.N, p.K, p.bits, p.lda, p.ldb, 0) == HOT_GEMM_SLOT_256; };
+  if (3 * x.K < 2 * x.N || stages(w) < 14 || !tile256(w) || !tile256(x)) return true;
+  auto rounds = [](const GemmProduct& p) { return (double)((((p.M + 255) / 256) * ((p.N + 255) / 256) + 255) / 256) * (double)p.K; };
+  const double done = ((double)w.M * w.N * w.K + (double)x.M * x.N * x.K) / (256.0 * 65536.0);
+  return done < (x.bits == 4 ? 0.96 : 0.94) * (rounds(w) + rounds(x));
 }
 
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
