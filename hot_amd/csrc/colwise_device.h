@@ -215,8 +215,10 @@ constexpr int RUNTIME = 2;
 template <typename T, int N, int PASS, int ROUND, int SAWB, typename SEL, bool RS = false, bool HQ = false>
 __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block, uint8_t* lds, const HqArgs* hq = nullptr) {
   // A copy, so that every argument is loaded once: read through the reference they would be loaded again at each use behind
-  // the memory clobber of a DMA instruction, 59 scalar loads and waits in the loop of <bf16, 1, 1, stochastic>.
-  const ColArgs a = args;
+  // the memory clobber of a DMA instruction, 59 scalar loads and waits in the loop of <bf16, 1, 1, stochastic>.  Blocks of
+  // 128 leave no registers for it (a copy costs the pass 30 spilled ones), and the selection of the other lengths is read
+  // where it is used: as a part of the copy it overflows the scalar registers (500 of them spilled).
+  typename std::conditional<(N < COL_MAX_N), const ColArgs, const ColArgs&>::type a = args;
   constexpr bool SHORT = std::is_same<SEL, SelShortFull>::value;
   static_assert(!SHORT || N == CW_ROWS, "short blocks are handled 16 rows at a time");
   constexpr int SPB = N >= CW_ROWS ? N / CW_ROWS : 1;        // steps per token block
@@ -440,7 +442,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
     auto place = [&](int i) -> int {
       if constexpr (PARTIAL) if (i >= valid) return -1;
       if constexpr (SEL::STATIC) return SEL::slot(i);
-      else return a.slot[i];
+      else return args.slot[i];
     };
     if constexpr (PASS == 0) {
       if (!sawb) {

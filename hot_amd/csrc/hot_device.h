@@ -243,7 +243,9 @@ __device__ __forceinline__ uint32_t rint_div_exact(float x, float d, float rcp) 
   float q = x * rcp;
   q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
   q = __builtin_fmaf(__builtin_fmaf(-q, d, x), rcp, q);
-  return q == q ? as_u(rintf(q) + RINT_MAGIC) : 0u;
+  // (a NaN becomes -256, whose low byte is 0: a maximum instead of a comparison, whose masks would crowd the scalar registers
+  // out of a pass that unrolls this over a block)
+  return as_u(rintf(fmaxf(q, -256.0f)) + RINT_MAGIC);
 }
 
 // rint(x / d) with rcp = 1 / d precomputed: the product x * rcp is within 1.5 * 2^-23 |x/d| of

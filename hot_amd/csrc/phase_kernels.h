@@ -17,12 +17,15 @@ __device__ __forceinline__ const PhaseArgs& phase_args() {
 }
 
 // Wavefronts per SIMD that the registers leave room for: three (what the LDS allows in the quantise pass) wherever a
-// thread's block and its selection are small enough to be held without spilling.
-template <int N, typename SEL> constexpr int phase_waves() {
+// thread's block and its selection are small enough to be held.  The quantise pass over blocks of 128 rounding to nearest is at
+// the edge: 16-bit inputs spill 6 registers and are faster so than with two waves (the backward of 25216 x 3072 -> 768 bf16
+// 155 / 170 us), fp32 inputs would spill 21 (25216 x 2304 207 / 181 with 51 spilled / two waves).
+template <typename T, int N, int PASS, int ROUND, typename SEL> constexpr int phase_waves() {
+  if (sizeof(T) == 4 && N == 128 && PASS == 1 && ROUND == HOT_ROUND_NEAREST && SEL::STATIC) return 2;
   return !std::is_same<SEL, SelRuntime>::value ? 3 : N <= 32 ? 3 : N == 64 ? 2 : 1;
 }
 template <typename T, int N, int PASS, int ROUND, typename SEL, bool RS>
-__global__ void __launch_bounds__(CW, (phase_waves<N, SEL>())) phase_kernel(const PhaseArgs p) {
+__global__ void __launch_bounds__(CW, (phase_waves<T, N, PASS, ROUND, SEL>())) phase_kernel(const PhaseArgs p) {
   extern __shared__ __align__(16) uint8_t lds[];
   unsigned b = blockIdx.x;
   // the short jobs first: they end early and the long one's workgroups fill in behind them
