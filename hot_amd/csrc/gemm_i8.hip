@@ -1434,7 +1434,7 @@ int gemm_i8_impl(const GemmProduct& p, int out_dtype, int32_t* acc_out, hipStrea
 //   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008 INT4 + 11008 x 4096 x 4096: 409 / 456;
 //     8192 x 11008 x 4096 + 4096 x 11008 x 2080: 348 / 424; 8192 x 4096 x 4096 + 4096^3: 174 / 187
 // (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174; the products
-// alone, launched over and over: inside a step the 256 x 256 tiles that have their rounds full come out ahead, gemm_pair_pays).
+// alone, launched over and over: inside a step INT8 products with full rounds of 256 x 256 tiles come out ahead, gemm_pair_pays).
 struct PairArgs {
   GemmArgs w, x;
   uint32_t w_blocks;      // a multiple of 8: blockIdx % 8 stays the XCD of the second product's tiles
@@ -1491,22 +1491,22 @@ bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
 // 4583 x 128 x 4096 21.4 / 27.6, 8191 x 128 x 8520 35.4 / 45.2.
 //
 // What the pair gains is idle CUs filled and stores hidden; what it gives up is the 256 x 256 tile, which asks the L2 for 0.6
-// of the operand bytes per operation.  Two products that take that tile, fill its rounds and have few stores for their
-// operations (K of g_x no shorter than 2/3 of its width, 14 stages and more in g_W) have nothing to gain.  us of the whole
-// backward bf16, pair / apart: INT4 8192 x 11008 x 4096 576 / 560 (the first 20 calls of an idle GPU 672 / 645), 8192 x 4096
-// x 4096 231 / 224; INT8 the same 685 / 635, 263 / 240, 9216 x 8704 x 3584 708 / 675; on the other side of the lines INT4
-// 4608 x 4608 x 10624 357 / 393, 8192 x 4096 x 11008 523 / 550, INT8 2048 x 8192 x 8064 323 / 342, 3200 x 8576 x 9856 568 / 610.
-// Of 70 shapes of both products in such tiles one that goes apart is slower for it by more than 1 % (4096 x 9984 x 8192
-// INT4 553 / 567; cold 636 / 616).
+// of the operand bytes per operation.  With INT8 operands of g_x two products that take that tile, fill 94 % of its rounds and
+// have few stores for their operations (K of g_x no shorter than 2/3 of its width, 14 stages and more in g_W) have nothing to
+// gain.  us of the whole backward, bf16, gradients with outliers, pair / apart: 3584 x 10752 x 8960 652 / 624, 9216 x 8704 x
+// 3584 688 / 661, 11264 x 4096 x 4096 340 / 324, 8192 x 11008 x 4096 in blocks of 8192 tokens 734 / 704; beside the lines
+// 2048 x 8192 x 8064 313 / 329, 3200 x 8576 x 9856 540 / 587, 9472 x 5760 x 4992 472 / 484.  (Of 70 shapes none that goes apart
+// is slower for it by more than 1 %.)  INT4 operands halve the bytes in question and stay in the pair: 8192 x 11008 x 4096
+// 551 / 560 at work, 639 / 623 over the first 20 calls of an idle GPU.
 bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
   auto stages = [](const GemmProduct& p) { return round_up(p.K, GEMM_KTILE) * p.bits / 8 / 128; };
   const int64_t x_tiles = ((x.M + 127) / 128) * ((x.N + 127) / 128);
   if (x_tiles <= 192 && stages(x) >= 14 && stages(x) >= 2 * stages(w)) return false;
   auto tile256 = [](const GemmProduct& p) { return gemm_plan_impl(p.M, p.N, p.K, p.bits, p.lda, p.ldb, 0) == HOT_GEMM_SLOT_256; };
-  if (3 * x.K < 2 * x.N || stages(w) < 14 || !tile256(w) || !tile256(x)) return true;
+  if (x.bits == 4 || 3 * x.K < 2 * x.N || stages(w) < 14 || !tile256(w) || !tile256(x)) return true;
   auto rounds = [](const GemmProduct& p) { return (double)((((p.M + 255) / 256) * ((p.N + 255) / 256) + 255) / 256) * (double)p.K; };
   const double done = ((double)w.M * w.N * w.K + (double)x.M * x.N * x.K) / (256.0 * 65536.0);
-  return done < (x.bits == 4 ? 0.96 : 0.94) * (rounds(w) + rounds(x));
+  return done < 0.94 * (rounds(w) + rounds(x));
 }
 
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
