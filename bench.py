@@ -12,13 +12,15 @@ written beforehand by the forward-side kernel.  Four input sets (> 256 MiB in
 total) are rotated so that g_y is not served from the Infinity Cache.
 
 Prints ONE JSON line.  Besides the contract fields it carries
-  roofline      the dominant kernel of the step, timed live inside the fused
-                step with HIP events on the launch stream
-                (hot_linear_backward_kernels), against the chip's published peak
+  roofline      the longest of the step's three launches, timed live inside the
+                step with HIP events on the launch stream (the stage times of
+                hot_linear_backward), against the chip's published peak
+  launches      the three launches of the step: statistics, transform + quantise, both products
   cpu_baseline  the op-for-op CPU port of the reference's fake-quant path
                 (oracle/fakequant_port.py) on the same layer, on the host cores
   ceilings      what this box reaches with a plain copy kernel and a loop of INT8 MFMAs
-  kernels       per-kernel microseconds and achieved rates for this layer
+  kernels       microseconds and achieved rates of every job of the step launched on its own
+                (hot_linear_backward_kernels)
   layers        the same step at every ViT-B and Llama-7B layer shape, bf16 and fp32
   llama_gate_up per-kernel pass at the Llama-7B gate/up shape
   llama_gate_up_python_rule  the same layer with the reference's own low-rank rule (n = 8192, r = 2080)
@@ -152,6 +154,40 @@ def kernel_table(w, sets, bufs, opt, ws, iters, warm, traffic=None):
                          traffic=(round(traffic[key]) if traffic and key in traffic else None),
                          work=("%.0f bytes" % alg if bound == "hbm" else "%.0f ops" % alg),
                          launches=launches.get(key, 1)))
+    return rows
+
+
+def launch_table(w, sets, bufs, opt, ws, iters, warm, traffic=None):
+    """The three launches of the step as it runs (independent jobs share a grid), from the stage times of
+    hot_linear_backward: an event on the launch stream behind each.  Bytes: every input read once, codes written
+    once; operations: 2 M N K of both products."""
+    from hot_amd import ops
+    L, O = sets[0][1].shape
+    I = w.shape[1]
+    e = sets[0][1].element_size()
+    lp = opt.lprime(L)
+    acc = [0.0] * 4
+    for it in range(warm + iters):
+        i = it % len(sets)
+        _, _, t = ops.linear_backward(sets[i][1], w, bufs[i][0], bufs[i][1], opt, timing=True, workspace=ws)
+        if it >= warm:
+            acc = [a + b for a, b in zip(acc, t)]
+    us = [a / iters * 1e6 for a in acc]
+    read = (L * O + O * I) * e
+    spec = [
+        ("statistics", "hot::phase_kernel<.., PASS 0> (g_y token-wise and row-wise, W)", us[0], "hbm", read),
+        ("quantise", "hot::phase_kernel<.., PASS 1> (g_y: HLA + INT8, Hadamard + INT%d; W: Hadamard + INT%d)" % (opt.gx_bits, opt.w_bits), us[1],
+         "hbm", read + lp * O + L * O * opt.gx_bits // 8 + O * I * opt.w_bits // 8),
+        ("products", "hot::gemm_pair_kernel (g_x INT%d and g_W INT8)" % opt.gx_bits, us[2], "mfma", 2.0 * O * I * (L + lp)),
+    ]
+    rows = []
+    for key, name, t, bound, alg in spec:
+        peak = HBM_PEAK_GBS if bound == "hbm" else INT8_PEAK_TOPS
+        ach = (alg / t / 1e3 if bound == "hbm" else alg / t / 1e6) if t > 0 else 0.0
+        rows.append(dict(key=key, kernel=name, us=round(t, 2), bound=bound, achieved=round(ach, 1), peak=peak,
+                         unit="GB/s" if bound == "hbm" else "TOP/s", frac=round(ach / peak, 4),
+                         traffic=(round(traffic[key]) if traffic and key in traffic else None),
+                         work=("%.0f bytes" % alg if bound == "hbm" else "%.0f ops" % alg)))
     return rows
 
 
@@ -562,8 +598,8 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-extras", action="store_true", help="skip the per-kernel table and the Llama shape")
     ap.add_argument("--table-only", action="store_true",
-                    help="of the extras keep only the per-kernel table (kernels launched one after the other, as "
-                         "the roofline entry measures them); the profiling runs use this")
+                    help="of the extras keep only the tables of the step's launches and of its jobs launched "
+                         "one by one; the profiling runs use this")
     ap.add_argument("--copy-calibration", action="store_true",
                     help="also run three 512 MiB device-to-device copies (a kernel of known traffic, for scaling "
                          "the FETCH_SIZE / WRITE_SIZE counters of a profiler run)")
@@ -645,27 +681,19 @@ def main():
                                        "loop of independent v_mfma_i32_32x32x32_i8, one wave per SIMD"}
         except Exception as e:
             out["ceilings"] = {"error": repr(e)[:200]}
-        # Roofline entry: the single launch with the longest duration inside the step, measured with
-        # HIP events on the launch stream around every kernel group, the groups launched one after
-        # the other (in the timed steps above independent jobs share launches; a job's own
-        # duration is the serial one).  A group of two
-        # launches, the split-K GEMM and its reduce kernel, is not one kernel and stands in the
-        # table only.  The same two GEMMs launched back to back, without the neighbouring
-        # kernels, are reported beside it.
-        rows = {r["key"]: r for r in table}
-        key = max((k for k in rows if rows[k]["launches"] == 1), key=lambda k: rows[k]["us"])
-        dom = rows[key]
+        # Roofline entry: the longest of the three launches the step consists of, an event on the launch stream behind
+        # each.  (In the table above every job is launched on its own.)  The two products launched back to back, one at
+        # a time and without the neighbouring launches, are reported beside it.
+        launches = launch_table(w, sets, bufs, opt, ws, iters=20, warm=4, traffic=traffic)
+        out["launches"] = launches
+        dom = max(launches, key=lambda r: r["us"])
         def entry(r):
             return {"kernel": r["kernel"], "bound": r["bound"], "achieved": r["achieved"], "peak": r["peak"],
                     "unit": r["unit"], "frac": r["frac"], "traffic": r["traffic"], "us_per_launch": r["us"],
                     "per_launch": r["work"]}
         out["roofline"] = entry(dom)
-        # At this workload the g_x GEMM and the token-wise quantise pass of g_y take the same time to
-        # within a microsecond, and either may come out on top of a run: the longest launch of each
-        # bound class is reported as well.
         out["roofline_by_bound"] = {
-            b: entry(max((r for r in table if r["bound"] == b and r["launches"] == 1), key=lambda r: r["us"]))
-            for b in ("mfma", "hbm")}
+            b: entry(max((r for r in launches if r["bound"] == b), key=lambda r: r["us"])) for b in ("mfma", "hbm")}
         if not a.table_only:
             us_gx, us_gw = gemm_launch_times(w, sets, bufs, opt)
             out["roofline"]["back_to_back_us"] = {"gemm_gx": round(us_gx, 2), "gemm_gw": round(us_gw, 2)}
