@@ -17,7 +17,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libhot_gfx950.so")
-SOURCES = ["phase_bf16.hip", "phase_f16.hip", "phase_f32.hip", "colwise.hip", "gemm_i8.hip", "hq_rowwise.hip", "hla_big.hip", "backward.hip", "ceilings.hip", "hla_expand.hip"]
+SOURCES = ["phase_bf16.hip", "phase_f16.hip", "phase_f32.hip", "colwise.hip", "gemm_i8.hip", "gemm_pair.hip", "hq_rowwise.hip", "hla_big.hip", "backward.hip", "ceilings.hip", "hla_expand.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
