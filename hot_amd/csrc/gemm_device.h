@@ -122,7 +122,8 @@ __device__ __forceinline__ void load_row_scales(const GemmArgs& g, int64_t row_b
 // fp32 sum itself, and `bias` (the column's bias, 0 without one) is added.
 // FOLD (post_scale is a power of two): the caller passes s_b * post_scale, and with INT4 s_a / 256.  Powers of two commute
 // with the rounding of the two products, and float(acc) of 256 x a sum below 2^24 is exact, so the value is the same with
-// two vector instructions less per output, three with INT4 (of 5.5; the epilogue issues little else).
+// two vector instructions less per output, three with INT4 (of 5.5; the epilogue issues little else).  (The smaller factors
+// stay normal numbers: the quantisers divide by the step + 1e-11, so an operand whose step is below 1e-17 has zero codes.)
 template <int BITS, bool FOLD, typename OutT>
 __device__ __forceinline__ float acc_value(int a, float sa, float sb, float post, float bias) {
   if constexpr (BITS == 16) return __builtin_bit_cast(float, a) + bias;

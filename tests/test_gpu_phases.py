@@ -64,6 +64,21 @@ def test_paired_products(gpu, L, O, I, dt, bits):
     check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("L,O,I", [(384, 144, 256), (64, 3088, 2176)])
+@pytest.mark.parametrize("size", [1.0, 2.0 ** -12])
+def test_epilogues_of_paired_products(gpu, dt, bits, L, O, I, size):
+    """Whole tiles (stored through LDS) and cut ones (stored directly) in one product, in both tilings, with the powers of two
+    folded into the steps: the values of the unfolded form, also where fp16 results are subnormal (gradients of 2^-12 size)
+    and are rounded to fp32 first."""
+    x, w, gy = make_case(L, O, I, seed=5, dtype=torch.float32)
+    ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits, n_o=16)
+    x, w, gy = x.to(dt), w.to(dt), (gy * size).to(dt)
+    gx, gw, tr = run_both(x, w, gy, ocfg, _options(ocfg), gpu)
+    assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
+
+
 @pytest.mark.parametrize("bits,O", [(8, 133144), (4, 171192)])
 def test_longest_rows(gpu, bits, O):
     """As many out-features as an int32 accumulator takes: the zero codes that pad a row to whole lines do not count."""
