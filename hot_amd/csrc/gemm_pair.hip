@@ -18,6 +18,7 @@ namespace hot {
 //     x 3072 + 3072 x 768 x 7092: 69.1 / 86.1; 3003 x 520 x 1000 + 1000 x 520 x 3003: 11.8 / 19.3; 128 tokens: 5.3 / 10.0
 //   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008 INT4 + 11008 x 4096 x 4096: 409 / 456;
 //     8192 x 11008 x 4096 + 4096 x 11008 x 2080: 348 / 424; 8192 x 4096 x 4096 + 4096^3: 174 / 187
+// (Taken with ordinary stores on both sides; the streaming ones take another 3 to 19 % off the pair, gemm_epilogue_staged.)
 // (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174; the products
 // alone, launched over and over: inside a step INT8 products with full rounds of 256 x 256 tiles come out ahead, gemm_pair_pays).
 struct PairArgs {
