@@ -66,7 +66,7 @@ bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
   auto fits = [](const GemmProduct& p) {
     int e;
     return p.M > 0 && p.N > 0 && p.K > 0 && (round_up(p.K, GEMM_KTILE) * p.bits / 8) % 128 == 0 && p.M * p.lda < (1ll << 32) && p.N * p.ldb < (1ll << 32) &&
-           frexpf(p.post_scale, &e) == 0.5f;                   // (a power of two: acc_value)
+           frexpf(p.post_scale, &e) == 0.5f && p.post_scale <= 1.f && p.post_scale >= FOLD_POST_MIN;   // (a power of two: acc_value, fold_exact)
   };
   return w.bits == 8 && fits(w) && fits(x);
 }

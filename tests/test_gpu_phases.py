@@ -79,6 +79,58 @@ def test_epilogues_of_paired_products(gpu, dt, bits, L, O, I, size):
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("L,O,I", [(384, 144, 256), (208, 1552, 4104)])
+@pytest.mark.parametrize("case,dt", [(c, d) for c in ("g_x overflows", "g_w overflows", "g_w subnormal", "row steps")
+                                     for d in (torch.float32, torch.bfloat16)] + [("row steps", torch.float16)])
+def test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, case):
+    """Steps so large that a product of them overflows before the scale of the transform brings it back, and so small that
+    results are subnormal (rounded once more): the paired launch, in both tilings, gives the values of the unfolded form there
+    too, on whole tiles as on cut ones, and those of the products launched apart.  Last: rows whose steps lie on either side of
+    what the folded form takes (2^-48, 2^47), and rows of zeros."""
+    from dataclasses import replace
+    from hot_amd import ops
+    x, w, gy = make_case(L, O, I, seed=8)
+    by_row = dict(gx_scale=orc.SCALE_ROW, gw_scale=orc.SCALE_ROW) if case == "row steps" else {}
+    ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits, n_o=16, **by_row)
+    opt = _options(ocfg)
+    xq_ref, sx_ref = orc.abc_forward(x.numpy(), ocfg)
+    ref = lambda sx: orc.linear_backward(gy.to(dt).float().numpy(), w.to(dt).float().numpy(), xq_ref, sx, ocfg)
+    top = lambda v: int(np.ceil(np.log2(np.abs(v).max())))
+    tr = ref(sx_ref)
+    sx = sx_ref
+    if case == "g_x overflows":                     # the largest sum of scaled products reaches 2^129, the result 2^125
+        k = 129 - top(tr.g_x) - 4
+        gy, w = gy * 2.0 ** (k // 2), w * 2.0 ** (k - k // 2)
+    elif case == "g_w overflows":                   # (a step of the caller's: 2^129 again, divided by the token block)
+        sx = sx_ref * np.float32(2.0 ** (129 - top(tr.g_w) - int(np.log2(ocfg.hla_n))))
+    elif case == "g_w subnormal":                   # results of at most 2^-124
+        gy = gy * 2.0 ** -20
+        sx = sx_ref * np.float32(2.0 ** (-124 - top(ref(sx_ref).g_w)))
+    elif case == "row steps":
+        e = torch.tensor([0, 50, 55, 60, -10, -20, -30, -48]) // (5 if dt == torch.float16 else 1)
+        gy = gy * 2.0 ** e.repeat(L // 8)[:, None]
+        gy[3::16] = 0.0
+    with np.errstate(over="ignore"):
+        tr = ref(sx)
+    if case == "g_x overflows":
+        assert np.isinf(tr.g_x).any() and np.isfinite(tr.g_x).mean() > 0.9
+    elif case == "g_w overflows":
+        assert np.isinf(tr.g_w).any() and np.isfinite(tr.g_w).mean() > 0.9
+    args = (gy.to(dt).to(gpu), w.to(dt).to(gpu), torch.from_numpy(np.ascontiguousarray(_buffer(xq_ref))).to(gpu), torch.from_numpy(sx).to(gpu))
+    gx, gw = ops.linear_backward(*args, opt)
+    apart = ops.linear_backward(*args, replace(opt, streams=2))
+    assert torch.equal(gx, apart[0]) and torch.equal(gw, apart[1])
+    assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
+
+
+def _buffer(xq):
+    """The oracle's codes [L', I] as the activation buffer holds them: [I, L' rounded up to whole lines of 128 codes]."""
+    out = np.zeros((xq.shape[1], -(-xq.shape[0] // 128) * 128), np.int8)
+    out[:, :xq.shape[0]] = xq.T
+    return out
+
+
 @pytest.mark.parametrize("bits,O", [(8, 133144), (4, 171192)])
 def test_longest_rows(gpu, bits, O):
     """As many out-features as an int32 accumulator takes: the zero codes that pad a row to whole lines do not count."""
