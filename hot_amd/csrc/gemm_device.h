@@ -92,7 +92,7 @@ inline int pick_group_m(int tiles_m, int tiles_n, int wgs_per_cu) {
 }
 
 
-// Fused dequantisation epilogue, shared by both kernels.  The MFMAs are issued with the operands
+// Fused dequantisation epilogue, shared by all kernels but the grouped ones.  The MFMAs are issued with the operands
 // swapped (B fragment first), so a 32x32 accumulator tile holds the TRANSPOSED product: lane l owns
 // output row l % 32 and, in registers 4 q .. 4 q + 3, the four adjacent output columns
 // 8 q + 4 (l / 32) .. + 3.  Each lane therefore stores four adjacent outputs at a time (8 bytes of
@@ -300,7 +300,7 @@ __device__ __forceinline__ uint32_t lds_offset(const uint8_t* p) {
 }
 
 // ---------------------------------------------------------------------------
-// Slot-scheduled variant.  Same data path as the pipelined kernel above (operand tiles HBM -> LDS by
+// Slot-scheduled variant.  Same data path as the pipelined kernel (gemm_i8_pipe_kernel: operand tiles HBM -> LDS by
 // DMA through a ring of S stages, packed INT4 expanded after the fragment read), but the K loop is
 // laid out by hand as a sequence of "slots", one MFMA each, fenced from one another, so that
 // everything else rides in the shadow of the matrix pipe instead of between its blocks:
@@ -310,10 +310,10 @@ __device__ __forceinline__ uint32_t lds_offset(const uint8_t* p) {
 //     current round, the high-nibble operands (in place) in the first half of their own round;
 //   * the DMA instructions that refill a stage go out one per slot behind the barrier;
 //   * a stage is refilled as soon as its second round is in registers (S - 1 tiles in flight).
-// The wave grid is GM x GN (four or eight waves), a wave owns (32 WM) x (32 WN) outputs, so
+// The wave grid is GM x GN (2 x 2, 1 x 4 or 4 x 1), a wave owns (32 WM) x (32 WN) outputs, so
 // block tiles of any multiple of 32 rows exist (160 x 256 gives ViT-B's 12608 tokens x 768 one
 // balanced round of 237 tiles on 256 CUs).  A stage's KiB chunks (1024 / RB rows each) are dealt round-
-// robin to the waves; when they do not come out even the spare DMA slots fetch into a
+// robin to the four waves; when they do not come out even the spare DMA slots fetch into a
 // spare KiB, so that every wave issues the same number of loads and one vmcnt serves all.
 // ---------------------------------------------------------------------------
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -323,20 +323,19 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 template <int WM, int WN, int GM, int GN, int S, int RB>
 constexpr int slot_ring_bytes() {
   const int rows = 32 * (WM * GM + WN * GN), chunks = rows * RB / 1024;
-  return S * rows * RB + (chunks % (GM * GN) ? 1024 : 0);
+  return S * rows * RB + (chunks % 4 ? 1024 : 0);
 }
 
 template <int WM, int WN, int GM, int GN, int BITS, int S, int RB, typename OutT, bool FOLD = false>
 __device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uint8_t* ring) {
-  constexpr int NW = GM * GN;
-  static_assert(NW == 4 || NW == 8, "four or eight waves");
+  static_assert(64 * GM * GN == G_THREADS, "the waves of a workgroup of the kernels' launch bounds, four");
   static_assert(RB == 64 || RB == 128, "stage rows of 64 or 128 bytes");
   constexpr int BM = 32 * WM * GM, BN = 32 * WN * GN;
   constexpr int SPR = RB / 16;                      // 16-byte slots per stage row
   constexpr int RPC = 1024 / RB;                    // rows per KiB chunk (one DMA instruction)
   constexpr int RPS = RB / 32;                      // rounds per stage: a round consumes 32 bytes of every row
-  constexpr int ROWS = BM + BN, CHUNKS = ROWS / RPC, LPW = (CHUNKS + NW - 1) / NW;
-  constexpr bool SPARE = LPW * NW != CHUNKS;
+  constexpr int ROWS = BM + BN, CHUNKS = ROWS / RPC, LPW = (CHUNKS + 3) / 4;
+  constexpr bool SPARE = LPW * 4 != CHUNKS;
   constexpr int STAGE_BYTES = ROWS * RB;
   constexpr int RING_BYTES = slot_ring_bytes<WM, WN, GM, GN, S, RB>();
   static_assert(S >= 2 && RING_BYTES <= 160 * 1024, "two or more LDS stages within 160 KiB");
@@ -376,7 +375,7 @@ __device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uin
   uint32_t is_b = 0;                                // bit i: instruction i reads B
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
-    int c = NW * i + wave;
+    int c = 4 * i + wave;
     const bool spare = SPARE && c >= CHUNKS;
     ldst[i] = spare ? (uint32_t)(S * STAGE_BYTES) : (uint32_t)c * 1024u;
     if (spare) c = 0;
@@ -563,7 +562,7 @@ __device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uin
     exact = __all(exact);
   }
   constexpr int AREA = 32 * (WN * 32 * (int)sizeof(OutT) + 16);
-  if (NW * AREA <= S * STAGE_BYTES && g.vec16 && !g.acc_out && row0 + BM <= g.M && col0 + BN <= g.N) {
+  if (4 * AREA <= S * STAGE_BYTES && g.vec16 && !g.acc_out && row0 + BM <= g.M && col0 + BN <= g.N) {
     __syncthreads();                                     // every wave is done with the ring
     if (exact) {
       gemm_epilogue_staged<WM, WN, BITS, OutT, FOLD>(acc, g, row0 + wm * WM * 32, col0 + wn * WN * 32, lane, sa_fold, sb_fold,
