@@ -94,6 +94,16 @@ static BwdLayout bwd_layout(int64_t L, int64_t O, int64_t I, const hot_config* c
   return b;
 }
 
+// The two products, g_x = (qG . qW^T) sG sW / n_o and g_W = (qGp . xq^T) sGp sx / hla_n: their sizes, without operands.
+static GemmProduct gx_product(const BwdLayout& b, int64_t L, int64_t O, int64_t I, const hot_config* c) {
+  return {nullptr, b.ld_g, nullptr, b.ld_w, c->gx_bits, L, I, b.ld_g * 8 / c->gx_bits, O, nullptr, c->gx_scale == HOT_SCALE_ROW, nullptr,
+          1.0f / (float)c->n_o, nullptr, I};
+}
+static GemmProduct gw_product(const BwdLayout& b, int64_t L, int64_t O, int64_t I, const hot_config* c) {
+  const int64_t lp = (L / c->hla_n) * c->hla_r;
+  return {nullptr, b.ld_gp, nullptr, b.ld_gp, 8, O, I, lp, lp, nullptr, c->gw_scale == HOT_SCALE_ROW, nullptr, 1.0f / (float)c->hla_n, nullptr, I};
+}
+
 // One stream or two, for products that cannot share a launch.  The transform + quantise work is two launches either way; the
 // second stream carries the g_x product beside the g_W product.  Forking and joining it costs the host two event record /
 // wait pairs, 21 us (measured), which only long calls hide: calls with little arithmetic (both products together below
@@ -103,6 +113,11 @@ static int backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* c
   const double lp = (double)((L / c->hla_n) * c->hla_r);
   const double ops = 2.0 * (double)O * (double)I * ((double)L + lp);
   return ops < 3.0e10 ? 1 : 2;
+}
+
+// Whether the products share a launch (calls that time every kernel on its own aside).
+static bool pairs(const GemmProduct& w, const GemmProduct& x, const hot_config* c) {
+  return c->streams != 2 && gemm_pair_possible(w, x) && gemm_pair_pays(w, x);
 }
 
 static const int32_t* identity_rows() {
@@ -125,6 +140,13 @@ int hot_abi_version(void) { return HOT_ABI_VERSION; }
 int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg) {
   if (check_cfg(cfg, "hot_backward_streams") || L <= 0 || O <= 0 || I <= 0) return 0;
   return backward_streams(L, O, I, cfg);
+}
+int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg) {
+  if (check_cfg(cfg, "hot_backward_products") || L <= 0 || O <= 0 || I <= 0 || L % cfg->hla_n || O % cfg->n_o) return 0;
+  const BwdLayout b = bwd_layout(L, O, I, cfg);
+  const GemmProduct px = gx_product(b, L, O, I, cfg), pw = gw_product(b, L, O, I, cfg);
+  if (!pairs(pw, px, cfg)) return HOT_PRODUCTS_APART;
+  return gemm_pair_large(pw) ? HOT_PRODUCTS_PAIR_192 : HOT_PRODUCTS_PAIR_128;
 }
 int64_t hot_kpad(int64_t k) { return round_up(k, GEMM_KTILE); }
 
@@ -293,7 +315,6 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   float* sg = (float*)(ws + b.off_sg);
   float* sw = (float*)(ws + b.off_sw);
   float* sgp = (float*)(ws + b.off_sgp);
-  const int64_t lp = (L / cfg->hla_n) * cfg->hla_r;
   if (marks) (void)hipEventRecord(marks->ev[0], st);
   auto mark = [&](int slot) {
     if (!marks) return;
@@ -382,13 +403,11 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   if (split) mark(K_W_QUANT);
   if (marks && !split) mark(STAGE_QUANT);
 
-  // the products: g_x = (qG . qW^T) sG sW / n_o and g_W = (qGp . xq^T) sGp sx / hla_n
-  const GemmProduct px = {ws + b.off_qg, b.ld_g, ws + b.off_qw, b.ld_w, cfg->gx_bits, L, I, b.ld_g * 8 / cfg->gx_bits, O, sg,
-                          cfg->gx_scale == HOT_SCALE_ROW, sw, 1.0f / (float)cfg->n_o, gx, I};
-  const GemmProduct pw = {ws + b.off_qgp, b.ld_gp, xq, b.ld_gp, 8, O, I, lp, lp, sgp, cfg->gw_scale == HOT_SCALE_ROW, sx,
-                          1.0f / (float)cfg->hla_n, gw, I};
-  const bool pairable = gemm_pair_possible(pw, px);
-  if (!split && cfg->streams != 2 && pairable && gemm_pair_pays(pw, px)) {
+  // the products
+  GemmProduct px = gx_product(b, L, O, I, cfg), pw = gw_product(b, L, O, I, cfg);
+  px.A = ws + b.off_qg; px.B = ws + b.off_qw; px.scale_a = sg; px.scale_b = sw; px.out = gx;
+  pw.A = ws + b.off_qgp; pw.B = xq; pw.scale_a = sgp; pw.scale_b = sx; pw.out = gw;
+  if (!split && pairs(pw, px, cfg)) {
     rc = gemm_pair_impl(pw, px, out_dtype, st);
     if (!rc && marks) mark(STAGE_GEMM);
     return rc;
@@ -404,7 +423,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   // forked / one after the other: 3904 x 10496 x 384 113 / 101, 8128 x 9984 x 320 182 / 172, 4032 x 5120 x 640 82 / 69).
   std::unique_lock<std::mutex> side_guard(g_side_mutex, std::defer_lock);
   SideLane* side = nullptr;
-  if (!marks && (cfg->streams == 2 || !pairable) && backward_streams(L, O, I, cfg) == 2 && ((O + 127) / 128) * ((I + 127) / 128) < 256) {
+  if (!marks && (cfg->streams == 2 || !gemm_pair_possible(pw, px)) && backward_streams(L, O, I, cfg) == 2 && ((O + 127) / 128) * ((I + 127) / 128) < 256) {
     side_guard.lock();
     side = side_lane_locked();
     if (!side) side_guard.unlock();

@@ -97,12 +97,14 @@ bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
   return done < 0.94 * (rounds(w) + rounds(x));
 }
 
+bool gemm_pair_large(const GemmProduct& w) { return ((w.M + 191) / 192) * ((w.N + 127) / 128) >= 256; }
+
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
   PairArgs p;
   if (int rc = gemm_fill(p.w, w, out_dtype, nullptr)) return rc;
   if (int rc = gemm_fill(p.x, x, out_dtype, nullptr)) return rc;
   if (!gemm_pair_possible(w, x)) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: the paired kernel takes rows of whole 128-byte lines");
-  const bool large = ((w.M + 191) / 192) * ((w.N + 127) / 128) >= 256;
+  const bool large = gemm_pair_large(w);
 #define HOT_PAIR_CASE(OUT)                                                                                          \
   return x.bits == 4 ? (large ? launch_pair<4, true, OUT>(p, st) : launch_pair<4, false, OUT>(p, st))               \
                      : (large ? launch_pair<8, true, OUT>(p, st) : launch_pair<8, false, OUT>(p, st))

@@ -370,6 +370,14 @@ def backward_streams(L: int, O: int, I: int, opt: HotOptions) -> int:
     return int(_lib.lib().hot_backward_streams(int(L), int(O), int(I), C.byref(opt.to_c())))
 
 
+PRODUCTS_APART, PRODUCTS_PAIR_128, PRODUCTS_PAIR_192 = 1, 2, 3
+
+
+def backward_products(L: int, O: int, I: int, opt: HotOptions) -> int:
+    """PRODUCTS_*: how linear_backward launches its two products at this shape (hot_backward_products)."""
+    return int(_lib.lib().hot_backward_products(int(L), int(O), int(I), C.byref(opt.to_c())))
+
+
 def kpad_group(T: int, opt: HotOptions) -> int:
     """Code bytes every sample takes in the K dimension of the batched g_W operands."""
     return _size(opt, "kpad_group", int(T))

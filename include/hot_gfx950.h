@@ -116,6 +116,14 @@ HOT_API const char* hot_last_error(void);
  * time than the host needs for the event operations that fork and join the side stream, run on one stream;
  * in long ones the g_x product may run beside the g_W product. */
 HOT_API int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
+/* How hot_linear_backward(_bias) launches its two products at this shape (0: the arguments are refused), so that tests and
+ * measurements know which kernel they cover. */
+enum hot_products_launch {
+  HOT_PRODUCTS_APART = 1,     /* one after the other (or beside one another: cfg->streams), each by hot_gemm_plan     */
+  HOT_PRODUCTS_PAIR_128 = 2,  /* in one launch: g_x in tiles of 128 x 128, g_W in tiles of 64 x 128                   */
+  HOT_PRODUCTS_PAIR_192 = 3   /* in one launch: both in tiles of 192 x 128                                            */
+};
+HOT_API int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_abi_version(void);
 
 /* Bytes of the leading dimension (row pitch) the library uses for a K-major

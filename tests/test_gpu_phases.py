@@ -54,36 +54,55 @@ def test_row_quantiser_widths(gpu, O, dt):
     check(gpu, 5, O, 8, dt, gx_scale=orc.SCALE_ROW)
 
 
-@pytest.mark.parametrize("L,O,I", [(1, 16, 8), (127, 64, 128), (129, 80, 136), (64, 3072, 2048), (64, 3056, 2048), (192, 192, 128),
-                                   (200, 400, 264), (40, 3328, 136), (40, 3584, 136), (1800, 1792, 16), (300, 1664, 16)])
+# How the products of a shape are launched, with INT4 and with INT8 operands of g_x: apart, or together with g_x / g_W in tiles of
+# 128 x 128 / 64 x 128, or of 192 x 128 both (ops.PRODUCTS_*).
+APART, P128, P192 = 1, 2, 3
+
+
+def launched(L, O, I, ocfg, launches):
+    from hot_amd import ops
+    assert (APART, P128, P192) == (ops.PRODUCTS_APART, ops.PRODUCTS_PAIR_128, ops.PRODUCTS_PAIR_192)
+    return ops.backward_products(L, O, I, _options(ocfg)) == launches[ocfg.gx_bits == 8]
+
+
+@pytest.mark.parametrize("L,O,I,launches", [
+    (1, 16, 8, (P128, P128)), (127, 64, 128, (P128, P128)), (129, 80, 136, (P128, P128)), (192, 192, 128, (P128, P128)),
+    (200, 400, 264, (P128, P128)), (300, 1664, 16, (P128, P128)),
+    (64, 3072, 2048, (P192, APART)), (64, 3056, 2048, (P192, APART)), (64, 2880, 2048, (P128, APART)),
+    (64, 1536, 4096, (P192, P192)), (64, 1536, 3968, (P128, P128)),
+    (40, 3328, 136, (P128, APART)), (40, 3584, 136, (APART, APART)), (1800, 1792, 16, (P128, APART))])
 @pytest.mark.parametrize("dt,bits", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 4)])
-def test_paired_products(gpu, L, O, I, dt, bits):
-    """Tile edges of the paired products, either side of the line between their two tilings (256 tiles of 192 x 128 of
-    g_W: 3072 x 2048), K shorter than the ring; g_x products of few tiles on either side of the length of K (14 stages, twice
+def test_paired_products(gpu, L, O, I, launches, dt, bits):
+    """Tile edges of the paired products, K shorter than the ring, either side of the line between their two tilings (256 tiles of
+    192 x 128 of g_W: 1536 x 4096, 3072 x 2048); g_x products of few tiles on either side of the length of K (14 stages, twice
     those of g_W) from which the two go apart."""
+    assert launched(L, O, I, orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits), launches)
     check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("L,O,I", [(384, 144, 256), (64, 3088, 2176)])
+@pytest.mark.parametrize("L,O,I,launches", [(200, 144, 264, (P128, P128)), (384, 144, 256, (P128, P128)),
+                                            (208, 1552, 4104, (P192, P192)), (64, 3088, 2176, (P192, APART))])
 @pytest.mark.parametrize("size", [1.0, 2.0 ** -12])
-def test_epilogues_of_paired_products(gpu, dt, bits, L, O, I, size):
-    """Whole tiles (stored through LDS) and cut ones (stored directly) in one product, in both tilings, with the powers of two
-    folded into the steps: the values of the unfolded form, also where fp16 results are subnormal (gradients of 2^-12 size)
-    and are rounded to fp32 first."""
+def test_epilogues_of_paired_products(gpu, dt, bits, L, O, I, launches, size):
+    """Whole tiles (stored through LDS) and cut ones (stored directly) of both products in both tilings (first and third shape; the
+    second has no cut tile of g_x, the last no whole one), with the powers of two folded into the steps: the values of the
+    unfolded form, also where fp16 results are subnormal (gradients of 2^-12 size) and are rounded to fp32 first.  With INT8
+    operands the last shape runs the products one after the other, unfolded."""
     x, w, gy = make_case(L, O, I, seed=5, dtype=torch.float32)
     ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits, n_o=16)
+    assert launched(L, O, I, ocfg, launches)
     x, w, gy = x.to(dt), w.to(dt), (gy * size).to(dt)
     gx, gw, tr = run_both(x, w, gy, ocfg, _options(ocfg), gpu)
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("L,O,I", [(384, 144, 256), (208, 1552, 4104)])
+@pytest.mark.parametrize("L,O,I,launches", [(200, 144, 264, (P128, P128)), (208, 1552, 4104, (P192, P192))])
 @pytest.mark.parametrize("case,dt", [(c, d) for c in ("g_x overflows", "g_w overflows", "g_w subnormal", "row steps")
                                      for d in (torch.float32, torch.bfloat16)] + [("row steps", torch.float16)])
-def test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, case):
+def test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, launches, case):
     """Steps so large that a product of them overflows before the scale of the transform brings it back, and so small that
     results are subnormal (rounded once more): the paired launch, in both tilings, gives the values of the unfolded form there
     too, on whole tiles as on cut ones, and those of the products launched apart.  Last: rows whose steps lie on either side of
@@ -94,6 +113,7 @@ def test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, case):
     by_row = dict(gx_scale=orc.SCALE_ROW, gw_scale=orc.SCALE_ROW) if case == "row steps" else {}
     ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits, n_o=16, **by_row)
     opt = _options(ocfg)
+    assert launched(L, O, I, ocfg, launches)
     xq_ref, sx_ref = orc.abc_forward(x.numpy(), ocfg)
     ref = lambda sx: orc.linear_backward(gy.to(dt).float().numpy(), w.to(dt).float().numpy(), xq_ref, sx, ocfg)
     top = lambda v: int(np.ceil(np.log2(np.abs(v).max())))
@@ -272,7 +292,7 @@ def test_long_products_that_leave_the_paired_launch(gpu, L, O, I, bits):
     x, w, gy = make_case(L, O, I, seed=6, dtype=torch.bfloat16)
     ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits)
     opt = _options(ocfg)
-    assert ops.backward_streams(L, O, I, opt) == 2
+    assert ops.backward_streams(L, O, I, opt) == 2 and launched(L, O, I, ocfg, (APART, APART))
     gx, gw, tr = run_both(x, w, gy, ocfg, opt, gpu)
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(gx.dtype)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(gw.dtype))
     xq, sx = ops.abc_forward(x.to(gpu), opt)

@@ -333,3 +333,21 @@ def test_bench_refuses_more_than_one_gpu():
     import sys
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0 and "ONE GPU" in r.stderr and r.stdout.strip() == ""
+
+
+def test_launch_of_the_products():
+    """hot_backward_products: refused arguments, the order that the caller asks for, and both widths on either side of the lines
+    between the launches (few tiles of g_x with a long K; 256 tiles of 192 x 128 of g_W; full rounds of 256 x 256 tiles)."""
+    from hot_amd import ops
+
+    def launch(L, O, I, bits=4, n=16, **kw):
+        rows = orc.paper_rows(n, n // 2)[1] if n > 1 else (0,)
+        return ops.backward_products(L, O, I, ops.HotOptions(n_o=16, hla_n=n, hla_rows=tuple(int(r) for r in rows), gx_bits=bits, w_bits=bits, **kw))
+
+    assert launch(100, 64, 64) == 0 and launch(0, 64, 64) == 0 and launch(64, 72, 64) == 0      # blocks of 16 tokens and channels
+    assert launch(64, 64, 64) == ops.PRODUCTS_PAIR_128 == launch(64, 64, 64, streams=1)
+    assert launch(64, 64, 64, streams=2) == ops.PRODUCTS_APART
+    for bits, longest in ((4, 3328), (8, 1664)):
+        assert launch(64, longest, 64, bits) == ops.PRODUCTS_PAIR_128 and launch(64, longest + 16, 64, bits) == ops.PRODUCTS_APART
+        assert launch(64, 1536, 3968, bits) == ops.PRODUCTS_PAIR_128 and launch(64, 1536, 4096, bits) == ops.PRODUCTS_PAIR_192
+    assert launch(8192, 11008, 4096) == ops.PRODUCTS_PAIR_192
