@@ -83,8 +83,8 @@ def profiled_traffic(workload="vit_b_fc1"):
     """HBM bytes per launch of the kernels of the step at a workload ("vit_b_fc1", "llama_gate_up"), as
     the committed counter summary gives them (profiles/hot_linear_backward_<workload>_bf16.hbm_traffic.txt:
     lines `traffic_bytes <kernel key> <bytes>` and `measured_at <commit>`), or (None, None) when the
-    summary is absent or carries no such lines.  The figures belong to the commit named there: kernels
-    changed since then are listed without traffic."""
+    summary is absent or carries no such lines.  The figures belong to the commit named there: where a kernel
+    has changed since, they are its traffic of then."""
     path = os.path.join(ROOT, "profiles", "hot_linear_backward_%s_bf16.hbm_traffic.txt" % workload)
     table, commit = {}, None
     try:

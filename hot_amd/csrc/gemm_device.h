@@ -203,15 +203,19 @@ __device__ __forceinline__ void gemm_epilogue(const v16i (&acc)[WM][WN], const G
 
 // Epilogue through LDS for tiles that lie fully inside the output: a wave turns one row of its
 // fragments (32 output rows x WN * 32 columns) into output values, parks them row-major in a
-// wave-private LDS area and writes them back out 16 bytes per lane along the rows, so every store
-// instruction covers whole 128-byte lines (the direct epilogue hands the memory system 16-byte
-// pieces of 32 different rows per instruction).  Wave-private, and a wave's LDS accesses are carried out in the order
+// wave-private LDS area and writes them back out 16 bytes per lane along the rows, so a store
+// instruction covers whole 128-byte lines (with one fragment column of 16-bit results, the 64 x 128 tiles of g_W and the
+// 32 .. 96 x 128 ones, half lines, whose other half a neighbouring wave stores), where the direct epilogue hands the memory
+// system 16-byte pieces of 32 different rows per instruction.  Wave-private, and a wave's LDS accesses are carried out in the order
 // in which it issues them: a read finds what the writes before it left, the next fragment row may overwrite the area
 // behind the reads, and nothing waits between them but a store for its own data.
 // The stores are marked as streaming: nothing in the launch reads a result again, and as ordinary stores they push the
-// operands that other workgroups share out of the L2.  us of both products in one launch, ordinary / streaming: 25216 x 3072
-// x 768 INT4 + 768 x 3072 x 7092 (155 MB of results) 98 / 79, 12608 x 768 x 3072 + 3072 x 768 x 7092 48.5 / 46.2, 8192 x
-// 4096 x 4096 + 4096^3 160 / 156; no shape was slower.
+// operands that other workgroups share out of the L2.  MiB fetched by a launch of both products, ordinary / streaming: 25216
+// tokens, 768 -> 3072 INT4 (155 MB of results) 123 / 100, 12608 tokens INT8 133 / 126, fp32 107 / 95, 3072 -> 768 137 / 134.
+// (That last one writes 0.6 MiB more for its half lines.)  us of the whole backward, bf16: 25216 tokens, 768 -> 3072 128 / 116,
+// 12608 80.7 / 76.5, INT8 86.6 / 83.5, 3072 -> 768 106.9 / 107.7, 8192 tokens, 11008 -> 4096 537 / 529, INT8 674 / 664; fp32:
+// 25216 173 / 151, 12608 105 / 90, 3072 -> 768 136.5 / 133.1, 11008 -> 4096 653 / 634.  Single products launched over and over:
+// 0 to 7 % faster (hot_gemm_bf16 0 to 15 %), the slowest 12608 x 3072 x 768 INT4 to fp32 at 41.0 / 41.5.
 // `area` must hold 32 * (WN * 32 * sizeof(OutT) + 16) bytes.
 template <int WM, int WN, int BITS, typename OutT, bool FOLD = false>
 __device__ __forceinline__ void gemm_epilogue_staged(const v16i (&acc)[WM][WN], const GemmArgs& g, int64_t row_base,

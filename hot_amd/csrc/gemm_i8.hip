@@ -769,7 +769,8 @@ GemmSplit gemm_split_plan(int64_t M, int64_t N, int64_t K, int bits) {
 //   256 x 256, slot-scheduled:                    INT4 9 + 0.0108 K,     INT8 9 + 0.0122 K
 //   256 x 256, pipelined:                         INT4 10 + 0.0131 K,    INT8 10 + 0.0136 K
 //   160 x 256, slot-scheduled (INT4):             14.3 + 0.0064 K
-// times the rounds a launch needs.  The 9-14 us of the large tiles are fill and epilogue that a lone
+// times the rounds a launch needs (measured with ordinary stores of the results; streaming ones are 0 to 7 % faster, the large
+// tiles most).  The 9-14 us of the large tiles are fill and epilogue that a lone
 // workgroup per CU cannot overlap: INT8 operands take them from K of about 1100 on, packed INT4
 // operands only from about 7000 on, and a product of exactly 256 large tiles beats 1024 small ones.
 // Products of at most 256 small tiles with a long K take the slot-scheduled small kernel (one

@@ -11,16 +11,15 @@ namespace hot {
 // idle in its last round, and a lone workgroup per CU leaves the matrix cores idle while it fills its ring and while it
 // stores; here both share a grid and two workgroups share a CU (at most 80 KiB of LDS and 256 registers each), so that
 // one's loads and stores lie under the other's MFMAs.  The g_W tiles come first: they run longest, and g_x tiles fill
-// in behind them.  Two tilings, g_x / g_W:
+// in behind them.  Two tilings, g_x / g_W (us of the whole backward, tokens x out x in, bf16, INT4 unless noted: first tiling /
+// second / one after the other by gemm_plan_impl):
 //   128 x 128 (2 stages) / 64 x 128 (3 stages): while the g_W product makes fewer than 256 tiles of 192 x 128, i.e.
-//     one long tile per CU would be its latency.  Measured against one after the other by gemm_plan_impl (us,
-//     bf16 results): 12608 x 768 x 3072 INT4 + 3072 x 768 x 7092: 50.2 / 57.5; 768 wide (proj): 21.4 / 31.0; 25216 x 768
-//     x 3072 + 3072 x 768 x 7092: 69.1 / 86.1; 3003 x 520 x 1000 + 1000 x 520 x 3003: 11.8 / 19.3; 128 tokens: 5.3 / 10.0
-//   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008 INT4 + 11008 x 4096 x 4096: 409 / 456;
-//     8192 x 11008 x 4096 + 4096 x 11008 x 2080: 348 / 424; 8192 x 4096 x 4096 + 4096^3: 174 / 187
-// (Taken with ordinary stores on both sides; the streaming ones take another 3 to 19 % off the pair, gemm_epilogue_staged.)
-// (the tilings the other way round: 49.1 for qkv at 12608 tokens against 42.4, 183 for the last pair against 174; the products
-// alone, launched over and over: inside a step INT8 products with full rounds of 256 x 256 tiles come out ahead, gemm_pair_pays).
+//     one long tile per CU would be its latency.  12608 x 3072 x 768: 106 / 114 / 116; 2304 wide: 88 / 95 / 92; 768 wide:
+//     45 / 69 / 53; 3003 x 1000 x 520: 29 / 39 / 37; 128 x 768 x 768: 27 / 32 / 30.  (g_x products of many tiles would rather
+//     have the second one: 12608 x 768 x 3072 76.6 / 74.2 / 79.2, INT8 82.8 / 78.6 / 91.6; 25216 tokens 115 / 109 / 114, INT8
+//     127 / 119 / 137; 25216 x 3072 x 768 153 / 152 / 165, INT8 180 / 172 / 199: the line does not look at them.)
+//   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008: 542 / 466 / 508; 8192 x 11008 x 4096: 618 / 594 / 582,
+//     in blocks of 16 tokens 575 / 536 / 522; 8192 x 4096 x 4096: 266 / 250 / 247 (the last three: gemm_pair_pays)
 struct PairArgs {
   GemmArgs w, x;
   uint32_t w_blocks;      // a multiple of 8: blockIdx % 8 stays the XCD of the second product's tiles
@@ -73,19 +72,23 @@ bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x) {
 
 // A g_x product of few tiles with a long K is a chain of stages that nothing else in the pair covers (0.9 us for each
 // 256 codes of a 128 x 128 INT4 tile): such a product goes by itself, cut into K ranges or into shorter tiles by its own
-// plan.  The line is where 168 shapes of 49 .. 16383 tokens and 64 .. 10624 channels are at most 14 % and on average 0.4 %
-// slower than the better of the two; us of both products, pair / apart: 2758 x 128 x 8520 INT4 32.0 / 26.2, 197 x 1024 x
-// 10624 45.1 / 29.3, INT8 63.7 / 34.1, 1001 x 768 x 3072 INT8 23.8 / 19.0; 2758 x 768 x 3072 INT4 20.6 / 28.5,
-// 4583 x 128 x 4096 21.4 / 27.6, 8191 x 128 x 8520 35.4 / 45.2.
+// plan.  Over 170 shapes of 49 .. 16383 tokens and 64 .. 10624 channels, INT4 and INT8, the choice is on average 0.35 % slower
+// than the better of the two and at most 4 %, but for INT4 products of 14 or 15 stages and a handful of tiles, where the launches
+// that going apart adds cost more than the chain (240 x 3808 x 160 30.5 / 38.6, 80 x 3392 x 64 31.9 / 40.2).  us of the whole
+// backward, tokens x out x in, bf16, pair / apart: 2758 x 8520 x 128 INT4 86.6 / 82.2, 197 x 10624 x 1024 66.9 / 50.9, INT8
+// 90.0 / 57.9, 1001 x 3072 x 768 INT8 39.7 / 35.1; beside the line 2758 x 3072 x 768 INT4 47.1 / 55.1, 4583 x 4096 x 128
+// 58.2 / 65.9, 8191 x 8520 x 128 147 / 162.
 //
 // What the pair gains is idle CUs filled and stores hidden; what it gives up is the 256 x 256 tile, which asks the L2 for 0.6
 // of the operand bytes per operation.  With INT8 operands of g_x two products that take that tile, fill 94 % of its rounds and
 // have few stores for their operations (K of g_x no shorter than 2/3 of its width, 14 stages and more in g_W) have nothing to
-// gain.  us of the whole backward, bf16, gradients with outliers, pair / apart: 3584 x 10752 x 8960 652 / 624, 9216 x 8704 x
-// 3584 688 / 661, 11264 x 4096 x 4096 340 / 324, 8192 x 11008 x 4096 in blocks of 8192 tokens 734 / 704; beside the lines
-// 2048 x 8192 x 8064 313 / 329, 3200 x 8576 x 9856 540 / 587, 9472 x 5760 x 4992 472 / 484.  (Of 70 shapes none that goes apart
-// is slower for it by more than 1 %.)  INT4 operands halve the bytes in question and stay in the pair: 8192 x 11008 x 4096
-// 551 / 560 at work, 639 / 623 over the first 20 calls of an idle GPU.
+// gain.  us of the whole backward, tokens x out x in, blocks of 16 tokens, bf16, gradients with outliers, half a second of each,
+// pair / apart: 3584 x 10752 x 8960 632 / 581, 9216 x 8704 x 3584 510 / 478, 11264 x 4096 x 4096 335 / 310, 8192 x 11008 x 4096
+// 657 / 602, in one block of 8192 tokens 723 / 670; beside the lines 2048 x 8192 x 8064 292 / 305, 3200 x 8576 x 9856 518 / 555,
+// 9472 x 5760 x 4992 467 / 463.  (Of 60 more shapes the one that goes apart gains 8 %; of those that stay in the pair 1792 x 9728
+// x 2048 would gain 7 %, 3584 x 5632 x 9216 and 11008 x 5120 x 5632 4 %, three others 2 to 3 %.)  INT4 operands halve the bytes
+// in question and stay in the pair, which was the faster order there while its results were stored through the L2: now
+// 8192 x 11008 x 4096 537 / 523, in one block 620 / 597, 8192 x 4096 x 4096 223 / 215, but 8192 x 4096 x 11008 488 / 532.
 bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
   auto stages = [](const GemmProduct& p) { return round_up(p.K, GEMM_KTILE) * p.bits / 8 / 128; };
   const int64_t x_tiles = ((x.M + 127) / 128) * ((x.N + 127) / 128);
