@@ -140,8 +140,8 @@ __device__ __forceinline__ float acc_value(int a, float sa, float sb, float post
 // Whether a step leaves the folded form exact, whatever the other step and the sum: with the magnitudes of both in [2^-48, 2^47)
 // and a post_scale in [2^-30, 1] (FOLD_POST_MIN, checked by the host) every nonzero |acc| < 2^31 keeps each factor, product and
 // result between 2^-126 and 2^126.  A step of 0 (a row of zeros) gives zeros in either form.  Infinite and NaN steps are not
-// admitted.  (On the bits: a few instructions a tile and no branches.  Without / with the check, us of the whole backward:
-// 12608 x 3072 x 768 103.6 / 104.4, 12608 x 2304 x 768 fp32 111.4 / 112.5, 12608 x 768 x 3072 INT8 91.1 / 91.3.)
+// admitted.  (On the bits: a few instructions a tile and no branches.  A build without the check / with it, us of the whole
+// backward: 12608 x 3072 x 768 104.0 / 104.5, 12608 x 2304 x 768 fp32 112.5 / 112.6, 12608 x 768 x 3072 INT8 91.7 / 91.7.)
 constexpr float FOLD_POST_MIN = 0x1p-30f;
 __device__ __forceinline__ bool fold_exact(float step) {
   const uint32_t lo = (127u - 48u) << 23, hi = (127u + 47u) << 23;
