@@ -142,7 +142,7 @@ int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg)
   return backward_streams(L, O, I, cfg);
 }
 int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg) {
-  if (check_cfg(cfg, "hot_backward_products") || L <= 0 || O <= 0 || I <= 0 || L % cfg->hla_n || O % cfg->n_o) return 0;
+  if (check_cfg(cfg, "hot_backward_products") || L <= 0 || O <= 0 || I <= 0 || L % cfg->hla_n || O % cfg->n_o || O % 8 || I % 8 || cfg->gx_bits != cfg->w_bits) return 0;
   const BwdLayout b = bwd_layout(L, O, I, cfg);
   const GemmProduct px = gx_product(b, L, O, I, cfg), pw = gw_product(b, L, O, I, cfg);
   if (!pairs(pw, px, cfg)) return HOT_PRODUCTS_APART;

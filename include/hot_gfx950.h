@@ -116,7 +116,7 @@ HOT_API const char* hot_last_error(void);
  * time than the host needs for the event operations that fork and join the side stream, run on one stream;
  * in long ones the g_x product may run beside the g_W product. */
 HOT_API int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
-/* How hot_linear_backward(_bias) launches its two products at this shape (0: the arguments are refused), so that tests and
+/* How hot_linear_backward(_bias) launches its two products at this shape (0: a size or width that it refuses), so that tests and
  * measurements know which kernel they cover. */
 enum hot_products_launch {
   HOT_PRODUCTS_APART = 1,     /* one after the other (or beside one another: cfg->streams), each by hot_gemm_plan     */

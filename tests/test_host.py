@@ -345,6 +345,7 @@ def test_launch_of_the_products():
         return ops.backward_products(L, O, I, ops.HotOptions(n_o=16, hla_n=n, hla_rows=tuple(int(r) for r in rows), gx_bits=bits, w_bits=bits, **kw))
 
     assert launch(100, 64, 64) == 0 and launch(0, 64, 64) == 0 and launch(64, 72, 64) == 0      # blocks of 16 tokens and channels
+    assert launch(64, 64, 20) == 0
     assert launch(64, 64, 64) == ops.PRODUCTS_PAIR_128 == launch(64, 64, 64, streams=1)
     assert launch(64, 64, 64, streams=2) == ops.PRODUCTS_APART
     for bits, longest in ((4, 3328), (8, 1664)):
