@@ -141,7 +141,8 @@ __device__ __forceinline__ float acc_value(int a, float sa, float sb, float post
 // and a post_scale in [2^-30, 1] (FOLD_POST_MIN, checked by the host) every nonzero |acc| < 2^31 keeps each factor, product and
 // result between 2^-126 and 2^126.  A step of 0 (a row of zeros) gives zeros in either form.  Infinite and NaN steps are not
 // admitted.  (On the bits: a few instructions a tile and no branches.  A build without the check / with it, us of the whole
-// backward: 12608 x 3072 x 768 104.0 / 104.5, 12608 x 2304 x 768 fp32 112.5 / 112.6, 12608 x 768 x 3072 INT8 91.7 / 91.7.)
+// backward: 12608 x 3072 x 768 104.0 / 104.5, 12608 x 2304 x 768 fp32 112.5 / 112.6, 12608 x 768 x 3072 INT8 91.7 / 91.7, both
+// before the direct epilogue formed its values once.)
 constexpr float FOLD_POST_MIN = 0x1p-30f;
 __device__ __forceinline__ bool fold_exact(float step) {
   const uint32_t lo = (127u - 48u) << 23, hi = (127u + 47u) << 23;
@@ -158,7 +159,12 @@ template <> __device__ __forceinline__ float bias_at<f16_t>(const void* bias, in
   return bias ? (float)reinterpret_cast<const _Float16*>(bias)[col] : 0.f;
 }
 
-template <int WM, int WN, int BITS, typename OutT>
+// FOLD: the tiles of a paired launch that do not take the folded epilogue (cut ones, and steps that fold_exact does not admit):
+// post_scale stays apart; with INT4 the caller passes s_a / 256 (exact: a step below 2^-118 has no codes but zeros).  The values
+// are formed once, before the choice between a store of four and four single ones: code that is rarely run, but its length is
+// felt by the code beside it (us of the whole backward, formed for either store / once: 12608 x 3072 x 768 106.0 / 105.3, 12608 x
+// 2304 x 768 fp32 113.8 / 113.0, 12608 x 768 x 3072 INT8 96.3 / 95.7).
+template <int WM, int WN, int BITS, typename OutT, bool FOLD = false>
 __device__ __forceinline__ void gemm_epilogue(const v16i (&acc)[WM][WN], const GemmArgs& g, int64_t row_base,
                                               int64_t col_base, int lane, const float (&sa_row)[WM], float sb) {
   OutT* out = reinterpret_cast<OutT*>(g.out);
@@ -186,15 +192,27 @@ __device__ __forceinline__ void gemm_epilogue(const v16i (&acc)[WM][WN], const G
           for (int t = 0; t < 4; ++t)
             if (col + t < g.N) g.acc_out[row * g.N + col + t] = BITS == 4 ? a[t] >> 8 : a[t];
         }
+        float once[4];
+        if constexpr (FOLD) {
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            once[t] = acc_value<8, false, OutT>(a[t], sa, sb, g.post_scale, 0.f);
+            asm volatile("" : "+v"(once[t]));
+          }
+        }
+        auto value = [&](int t) {
+          if constexpr (FOLD) return once[t];
+          else return acc_value<BITS, false, OutT>(a[t], sa, sb, g.post_scale, bv[t]);
+        };
         if (g.vec_out && col + 3 < g.N) {
           typename Quad<OutT>::type v;
 #pragma unroll
-          for (int t = 0; t < 4; ++t) quad_set<OutT>(v, t, acc_value<BITS, false, OutT>(a[t], sa, sb, g.post_scale, bv[t]));
+          for (int t = 0; t < 4; ++t) quad_set<OutT>(v, t, value(t));
           *reinterpret_cast<typename Quad<OutT>::type*>(out + row * g.ldo + col) = v;
         } else {
 #pragma unroll
           for (int t = 0; t < 4; ++t)
-            if (col + t < g.N) store_scalar<OutT>(out + row * g.ldo + col + t, acc_value<BITS, false, OutT>(a[t], sa, sb, g.post_scale, bv[t]));
+            if (col + t < g.N) store_scalar<OutT>(out + row * g.ldo + col + t, value(t));
         }
       }
     }
@@ -574,7 +592,7 @@ __device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uin
       return;
     }
   }
-  gemm_epilogue<WM, WN, BITS, OutT>(acc, g, row0 + wm * WM * 32, col0 + wn * WN * 32, lane, sa_row, sb);
+  gemm_epilogue<WM, WN, BITS, OutT, FOLD>(acc, g, row0 + wm * WM * 32, col0 + wn * WN * 32, lane, sa_fold, sb);
 }
 
 // Checks a product and fills the arguments that every kernel takes.
