@@ -328,9 +328,12 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   // the launches of the two phases (phase.h); larger ones have kernels of their own.
   const bool big = cfg->hla_n > COL_MAX_N, w_short = w_joins_phase(cfg);
   ColJob gj, wj;
+  const int elem = dtype == HOT_F32 ? 4 : 2;
+  const int64_t want = col_jobs_want(col_job_workgroups(O, I, cfg->n_o, cfg->n_o, cfg->w_bits == 4, cfg->w_scale, elem) +
+                                     (big ? 0 : col_job_workgroups(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, elem)) + L * O / 8192);
   rc = col_job_impl(wj, w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed, HOT_STREAM_W,
                     cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw, colwise_workspace_bytes_impl(I), who,
-                    1, 0, false, w_short);
+                    1, 0, false, w_short, want);
   if (rc) return rc;
   // With one step per tensor both quantisers of g_y need the absmax of their transform first: the statistics pass of
   // the token-wise job delivers both from a single read of g_y.
@@ -341,7 +344,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   if (!big) {
     rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
                       HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg, colwise_workspace_bytes_impl(O), who,
-                      1, 0, false, false);
+                      1, 0, false, false, want, gb != nullptr);
     if (rc) return rc;
     if (row_fused) col_job_row_stat(gj, cfg->n_o);
     if (gb) gj.a.colsum = (float*)(ws + b.off_colsum);

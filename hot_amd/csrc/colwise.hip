@@ -109,27 +109,46 @@ size_t colwise_group_workspace_bytes_impl(int64_t C, int groups) {
 // g_y statistics pass it runs beside: the step came out 2 us slower.)  Absmax statistics stage nothing: while the grid has fewer than 2048
 // workgroups they take shorter workgroups, down to 64 rows (measured 1 us faster at 12608 x 3072).
 // The SAWB sums are order-sensitive and keep the partition of the quantise pass.
+// With fewer workgroups than `want` the runs go below 32 bytes, down to one step or one output word: a workgroup's time is then
+// a chain (rows on their way, transform, store), and two workgroups on two CUs take half of it each (col_jobs_want).
+// col_ring_bytes: a workgroup of one or two steps has a ring of as many buffers, which is what lets more of them share a CU.
 struct ColPartition { int tb, tb0; };
-static ColPartition col_partition(int n, int r, int store4, int mode, int64_t C, int64_t NB, int elem_bytes) {
+static ColPartition col_partition(int n, int r, int store4, int mode, int64_t C, int64_t NB, int elem_bytes, int64_t want, bool keep_stat) {
   const int BPS = n >= CW_ROWS ? 1 : CW_ROWS / n;
   const int64_t gx = (C + CW - 1) / CW;
-  const size_t ring = (size_t)(elem_bytes == 4 ? 3 : 4) * CW_ROWS * CW * elem_bytes;
   auto run_bytes = [&](int t) { return store4 ? t * r / 2 : t * r; };   // t * r is a multiple of 8 when store4
   auto wgs = [&](int t) { return gx * ((NB + t - 1) / t); };
   auto resident = [&](int t) {   // workgroups of the quantise pass per CU, as far as LDS decides (three are enough)
-    const size_t per = ring + (size_t)CW * (t * r + 4) + 256;
+    const size_t per = col_ring_bytes(t * n, elem_bytes) + (size_t)CW * (t * r + 4) + 256;
     const int k = (int)((160u * 1024u) / per);
     return k > 3 ? 3 : k;
   };
-  int tb = BPS;
-  while ((tb * r) % (store4 ? 8 : 4) != 0 || run_bytes(tb) < 32) tb <<= 1;
+  int least = BPS;
+  while ((least * r) % (store4 ? 8 : 4) != 0) least <<= 1;
+  int tb = least;
+  while (run_bytes(tb) < 32) tb <<= 1;
   while (run_bytes(tb) < 128 && wgs(2 * tb) >= 1024 && resident(2 * tb) >= resident(tb)) tb <<= 1;
-  int tb0 = tb;
+  const int whole = tb;
+  if (mode != HOT_SCALE_SAWB)
+    while (tb > least && wgs(tb) < want) tb >>= 1;
+  int tb0 = keep_stat ? whole : tb;
   if (mode != HOT_SCALE_SAWB)
     while (tb0 > BPS && (tb0 & 1) == 0 && tb0 * n > 64 && wgs(tb0) < 2048) tb0 >>= 1;
   return {tb, tb0};
 }
 
+// The fewest workgroups that each column-wise job of a launch should have, given how many all jobs of the launch have while none
+// is cut up.  us of the whole backward, runs of 32 bytes and more / cut, bf16, tokens x out x in: 272 x 128 x 80 23.1 / 19.0,
+// 197 x 632 x 2048 27.2 / 23.5, 4334 x 640 x 72 31.9 / 27.6, 2048 x 1024 x 1024 48.9 / 45.2, 779 x 7504 x 448 52.9 / 49.9, 4096 x 720 x
+// 6528 fp32 76.2 / 72.0.  A launch that is full without it only gets more starts and ends of workgroups: 4137 x 7808 x 64 129.5 /
+// 131.3; on the wrong side 323 x 3456 x 6144 INT8 67.8 / 70.7, 1505 x 1056 x 3200 38.9 / 40.1, 5216 x 384 x 784 26.0 / 26.4.
+// (48 shapes of 64 .. 16384 tokens and 64 .. 11008 channels: 4.5 % on average, with the shorter rings.)
+int64_t col_jobs_want(int64_t workgroups) { return workgroups < 2048 ? 256 : 128; }
+
+int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes) {
+  const ColPartition cp = col_partition(n, r, store4, mode, C, R / n, elem_bytes, 0, false);
+  return (C + CW - 1) / CW * ((R / n + cp.tb - 1) / cp.tb);
+}
 
 // ---- jobs -----------------------------------------------------------------------
 
@@ -167,7 +186,7 @@ static ColSel pick_sel(ColArgs& a, int n, bool as_short) {
 int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, int n, const int32_t* rows, int r, int bits,
                  int rounding, uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_out, int store4,
                  float* scales_out, void* workspace, size_t workspace_bytes, const char* who, int groups, int64_t kpad_group,
-                 bool rowmajor, bool as_short) {
+                 bool rowmajor, bool as_short, int64_t want, bool keep_stat) {
   if (!in || !codes_out || !scales_out || !rows) return fail(HOT_ERR_INVALID, "%s: null pointer", who);
   if (rowmajor && (groups > 1 || scale_mode == HOT_SCALE_ROW))
     return fail(HOT_ERR_UNSUPPORTED, "%s: the untransposed store takes one step for the tensor", who);
@@ -221,13 +240,12 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
 
   // grids: strips of channels x runs of token blocks, per sample group (a run never leaves its sample)
   const int elem = dtype == HOT_F32 ? 4 : 2;
-  const ColPartition cp = col_partition(n, r, store4, scale_mode, C, a.NB, elem);
+  const ColPartition cp = col_partition(n, r, store4, scale_mode, C, a.NB, elem, groups > 1 ? 0 : want, keep_stat);
   const int64_t gx = (C + CW - 1) / CW, runs = (a.NBs + cp.tb - 1) / cp.tb, runs0 = (a.NBs + cp.tb0 - 1) / cp.tb0;
   if (runs * groups > 65535 || gx * runs * groups > COL_MAX_WGS || gx * runs0 * groups > COL_MAX_WGS)
     return fail(HOT_ERR_UNSUPPORTED, "%s: grid %lld x %lld too large", who, (long long)gx, (long long)(runs * groups));
-  const size_t ring = (size_t)(elem == 4 ? 3 : 4) * CW_ROWS * CW * elem;
-  job.lds[0] = ring;
-  job.lds[1] = ring + (size_t)CW * (cp.tb * r + 4);
+  job.lds[0] = col_ring_bytes(cp.tb0 * n, elem);
+  job.lds[1] = col_ring_bytes(cp.tb * n, elem) + (size_t)CW * (cp.tb * r + 4);
   if (job.lds[1] > 150 * 1024) return fail(HOT_ERR_UNSUPPORTED, "colwise: staging does not fit LDS");
   job.sel = pick_sel(a, n, as_short);
   a.gx = (uint32_t)gx;
@@ -375,7 +393,7 @@ int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int m
     return (R + rows - 1) / rows;
   }
   const int64_t NB = R / n;
-  const ColPartition part = col_partition(n, r, store4, mode, C, NB, elem_bytes);
+  const ColPartition part = col_partition(n, r, store4, mode, C, NB, elem_bytes, 0, true);
   return (NB / groups + part.tb0 - 1) / part.tb0 * groups;
 }
 
@@ -418,7 +436,8 @@ int colwise_quant_impl(const void* in, int dtype, int64_t R, int64_t C, int n, c
   if (row16_absmax_out || colsum_partial) return fail(HOT_ERR_INVALID, "%s: fused statistics of short blocks belong to a phase", who);
   ColJob job;
   if (int rc = col_job_impl(job, in, dtype, R, C, n, rows, r, bits, rounding, seed, rng_stream, scale_mode, codes_out, ld_out, store4,
-                            scales_out, workspace, workspace_bytes, who, groups, kpad_group, rowmajor, false)) return rc;
+                            scales_out, workspace, workspace_bytes, who, groups, kpad_group, rowmajor, false,
+                            col_jobs_want(0), false)) return rc;
   col_job_clear(job, st);
   if (int rc = phase_launch(0, dtype, &job, nullptr, nullptr, nullptr, st)) return rc;
   return phase_launch(1, dtype, &job, nullptr, nullptr, nullptr, st);

@@ -137,6 +137,11 @@ __device__ __forceinline__ void fwht_short(float (&v)[16], int n, int h0) {
 // LDS buffers in the ring (steps in flight behind the one in use = depth - 1): four for 16-bit
 // inputs; 32-bit rows are twice as large, and three buffers keep a second workgroup on the CU.
 template <typename T> constexpr int ring_depth() { return sizeof(T) == 4 ? 3 : 4; }
+// ... and the bytes of the ring of a workgroup that covers `rows` rows: no more buffers than it has steps
+__host__ __device__ inline int col_ring_bytes(int rows, int elem_bytes) {
+  const int depth = elem_bytes == 4 ? 3 : 4, steps = (rows + CW_ROWS - 1) / CW_ROWS;
+  return (steps < depth ? steps : depth) * CW_ROWS * CW * elem_bytes;
+}
 
 template <typename T>
 struct RowStream {
@@ -228,7 +233,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   __shared__ float s_max[CW / 64];
   __shared__ double s_sum[2][CW / 64];
   constexpr int CW_DEPTH = ring_depth<T>();
-  uint8_t* const stage = lds + CW_DEPTH * BUF;               // PASS 1: codes [channel][k]
+  uint8_t* const stage = lds;                                // PASS 1: codes [channel][k], before the ring
   const bool sawb = SAWB == RUNTIME ? a.mode == HOT_SCALE_SAWB : SAWB != 0;
   const bool nearest = ROUND == RUNTIME ? a.rounding == HOT_ROUND_NEAREST : ROUND == HOT_ROUND_NEAREST;
 
@@ -265,6 +270,8 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   const int qmax = (1 << (a.bits - 1)) - 1;
   const int sb = a.tb * a.r;        // staged code bytes per channel
   const int pitch = sb + 4;
+  // (the ring behind it: as many buffers as col_ring_bytes says)
+  uint8_t* const ring = lds + (PASS == 1 ? CW * pitch : 0) + wave * RowStream<T>::WAVE_BYTES;       // this wave's slice of buffer 0
 
   RowStream<T> rs;
   rs.pitch = (uint32_t)(a.C * (int64_t)sizeof(T));
@@ -282,9 +289,9 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   }
 
   // ring of CW_DEPTH LDS buffers: steps s+1 .. s+CW_DEPTH-1 are in flight while step s is consumed
-  constexpr int LPW = RowStream<T>::LPW, WB = RowStream<T>::WAVE_BYTES;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)lds + wave * WB;
-  const uint8_t* const my = lds + wave * WB;               // this wave's slice of ring buffer 0
+  constexpr int LPW = RowStream<T>::LPW;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)ring;
+  const uint8_t* const my = ring;
 #pragma unroll
   for (int s = 0; s < CW_DEPTH - 1; ++s)
     if (s < nsteps) rs_issue<T>(rs, lds0 + s * BUF, s, lane);

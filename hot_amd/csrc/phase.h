@@ -77,7 +77,12 @@ struct ColJob {
 int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, int n, const int32_t* rows, int r, int bits,
                  int rounding, uint64_t seed, uint32_t rng_stream, int scale_mode, void* codes_out, int64_t ld_out, int store4,
                  float* scales_out, void* workspace, size_t workspace_bytes, const char* who, int groups, int64_t kpad_group,
-                 bool rowmajor, bool as_short);
+                 bool rowmajor, bool as_short, int64_t want = 0, bool keep_stat = false);
+// want: the fewest workgroups it should have (one group, absmax steps; 0: as many as long runs give).  keep_stat: the statistics
+// pass keeps the partition of want = 0, on which the order of the column sums depends.
+int64_t col_jobs_want(int64_t workgroups);
+// Workgroups of the quantise pass with want = 0.
+int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes);
 // The statistics pass also delivers the absmax of the row-wise Hadamard of blocks of n_o (1 .. 16) of the same input.
 void col_job_row_stat(ColJob& job, int n_o);
 // Zeroes what the statistics pass updates by atomics (nothing for most jobs).

@@ -103,6 +103,27 @@ def test_backward_matches_oracle(gpu, dtype, shape, variant):
         assert torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dtype))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("variant", [dict(), dict(gx_bits=8, w_bits=8, gw_scale=orc.SCALE_ROW),
+                                     dict(gx_round=orc.ROUND_STOCH, w_round=orc.ROUND_STOCH, gw_round=orc.ROUND_STOCH, seed=5)])
+@pytest.mark.parametrize("L,O,I", [
+    (17, 32, 40),        # blocks of one token, the last run of one row
+    (130, 48, 264),      # blocks of two, a strip of eight channels
+    (276, 208, 24),      # blocks of four, W in groups of sixteen rows
+    (48, 528, 72),       # blocks of sixteen: three steps
+    (96, 272, 520),      # blocks of 32
+    (16 * 67, 32, 16),   # enough runs of sixteen tokens that some workgroups take several
+    (3001, 144, 16),     # blocks of one token, many of them: the last run of nine rows
+])
+def test_backward_small_grids(gpu, L, O, I, dtype, variant):
+    """Problems whose column-wise jobs are cut into short runs of token blocks (col_partition): rings of one to four
+    buffers, runs of 4 bytes and more, ends that fill no run.  Bit-exact."""
+    x, w, gy = make_case(L, O, I, seed=L + O, dtype=dtype)
+    ocfg, opt = both_configs(L, max_block=128, **variant)
+    gx, gw, tr = run_both(x, w, gy, ocfg, opt, gpu)
+    assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dtype)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dtype))
+
+
 @pytest.mark.parametrize("variant", [dict(), dict(gw_scale=orc.SCALE_ROW, gx_bits=8, w_bits=8)])
 def test_backward_split_k(gpu, variant):
     """Few output tiles and a long reduction (L' = 2304): the g_W GEMM cuts K into ranges that meet
