@@ -700,7 +700,8 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       a.partial[2 * wg + 1] = b;
     }
   } else {
-    __syncthreads();
+    // the codes that a lane reads below are its wave's, which carries out its LDS accesses in order
+    asm volatile("" ::: "memory");
     if (a.rowmajor) {
       // untransposed store: coefficient row (blk0 + b) r + k takes one code of every channel; a
       // wave writes 64 adjacent bytes (INT8) or, two channels to a byte, 32 (packed INT4: the even
@@ -718,17 +719,23 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       }
       return;
     }
-    // flush: each channel's staged run is one contiguous global segment
+    // flush: each channel's staged run is one contiguous global segment; a wave writes those of its own 64 channels, without waiting
+    // for the others, and what has to be zero behind the last run in a loop of its own that reads nothing (through the same loop as
+    // the codes it was 0.35 us a round: 64 x 512 x 512, one block of tokens and 92 bytes of zeros to a channel, 23.3 / 21.4 us).  Two or
+    // four units under way at once are slower (fc2's buffer 39.6 / 40.3 / 40.8): these passes feel the length of their code.
     const bool last = blk_in + a.tb >= a.NBs;       // the run that ends its sample also zeroes the sample's tail
     const int out_sb = a.store4 ? sb / 2 : sb;
     const int64_t seg0 = (int64_t)sample * a.Kpad + (int64_t)run * out_sb;      // byte offset in the output row
     const int64_t seg_end = last ? (int64_t)(sample + 1) * a.Kpad : seg0 + out_sb;
     const int ndw = (int)((seg_end - seg0) / 4);            // output dwords per channel
-    const int sdw = out_sb / 4;                             // of which staged
-    const int nch = (int)((a.C - cg0) < CW ? (a.C - cg0) : CW);
+    const int sdw = out_sb / 4 < ndw ? out_sb / 4 : ndw;    // of which staged
+    const int64_t ch0 = cg0 + 64 * wave;                    // this wave's first channel
+    const int nch = (int)(a.C - ch0 < 64 ? a.C - ch0 : 64);
+    if (nch <= 0) return;
+    const uint8_t* const wstage = stage + 64 * wave * pitch;
+    int8_t* const wout = a.out + ch0 * a.ld_out + seg0;
     // output dword jd of a staged channel row (packing two codes per byte when store4)
     auto word = [&](const uint32_t* row, int jd) -> uint32_t {
-      if (jd >= sdw) return 0u;
       if (a.store4) {
         const uint32_t lo = row[2 * jd], hi = row[2 * jd + 1];
         // bytes b0..b7 -> nibbles: byte j of the result = (b[2j+1] << 4) | (b[2j] & 15)
@@ -738,26 +745,41 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       }
       return row[jd];
     };
-    // consecutive threads walk along K within a channel, then on to the next channel; (ch, jd) of
-    // position p = tid + k CW advance by a fixed step, so the loop carries them instead of dividing.
-    // Units of 8 bytes when the segments allow it (half the store instructions), else of 4.
+    // consecutive lanes walk along K within a channel, then on to the next channel; (ch, jd) of position p = lane + 64 k advance by a
+    // fixed step, so the loop carries them instead of dividing.  Units of 8 bytes when the segments allow it (half the store
+    // instructions), else of 4.
     const int unit = ((out_sb & 7) == 0 && (ndw & 1) == 0) ? 2 : 1;      // dwords per store
-    const int nun = ndw / unit;                                          // units per channel
-    const int total = nch * nun;
-    const int step_ch = CW / nun, step_jd = CW - step_ch * nun;
-    int ch = tid / nun, jd = tid - ch * nun;
-    int8_t* dst = a.out + (cg0 + ch) * a.ld_out + seg0 + (int64_t)jd * 4 * unit;
-    const int64_t step_dst = step_ch * a.ld_out + (int64_t)step_jd * 4 * unit, wrap_dst = a.ld_out - (int64_t)nun * 4 * unit;
-    for (int p = tid; p < total; p += CW, ch += step_ch, jd += step_jd, dst += step_dst) {
-      if (jd >= nun) { jd -= nun; ++ch; dst += wrap_dst; }
-      const uint32_t* row = reinterpret_cast<const uint32_t*>(stage + ch * pitch);
-      if (unit == 2) {
-        uint2 w2;
-        w2.x = word(row, 2 * jd);
-        w2.y = word(row, 2 * jd + 1);
-        *reinterpret_cast<uint2*>(dst) = w2;
-      } else {
-        *reinterpret_cast<uint32_t*>(dst) = word(row, jd);
+    {
+      const int nun = sdw / unit;                                        // units per channel
+      const int total = nch * nun;
+      const int step_ch = 64 / nun, step_jd = 64 - step_ch * nun;
+      int ch = lane / nun, jd = lane - ch * nun;
+      int8_t* at = wout + ch * a.ld_out + (int64_t)jd * (4 * unit);
+      const int64_t step_at = step_ch * a.ld_out + (int64_t)step_jd * (4 * unit), wrap_at = a.ld_out - (int64_t)nun * (4 * unit);
+      for (int p = lane; p < total; p += 64, ch += step_ch, jd += step_jd, at += step_at) {
+        if (jd >= nun) { jd -= nun; ++ch; at += wrap_at; }
+        const uint32_t* row = reinterpret_cast<const uint32_t*>(wstage + ch * pitch);
+        if (unit == 2) {
+          uint2 w2;
+          w2.x = word(row, 2 * jd);
+          w2.y = word(row, 2 * jd + 1);
+          *reinterpret_cast<uint2*>(at) = w2;
+        } else {
+          *reinterpret_cast<uint32_t*>(at) = word(row, jd);
+        }
+      }
+    }
+    if (ndw > sdw) {
+      const int nun = (ndw - sdw) / unit, total = nch * nun;
+      const int step_ch = 64 / nun, step_jd = 64 - step_ch * nun;
+      const int ch = lane / nun;
+      int jd = lane - ch * nun;
+      int8_t* at = wout + 4 * sdw + ch * a.ld_out + (int64_t)jd * (4 * unit);
+      const int64_t step_at = step_ch * a.ld_out + (int64_t)step_jd * (4 * unit), wrap_at = a.ld_out - (int64_t)nun * (4 * unit);
+      for (int p = lane; p < total; p += 64, jd += step_jd, at += step_at) {
+        if (jd >= nun) { jd -= nun; at += wrap_at; }
+        if (unit == 2) *reinterpret_cast<uint2*>(at) = make_uint2(0u, 0u);
+        else *reinterpret_cast<uint32_t*>(at) = 0u;
       }
     }
   }
