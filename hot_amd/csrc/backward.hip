@@ -141,12 +141,17 @@ int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_config* cfg)
   if (check_cfg(cfg, "hot_backward_streams") || L <= 0 || O <= 0 || I <= 0) return 0;
   return backward_streams(L, O, I, cfg);
 }
+int hot_backward_pair_rows(int64_t L, int64_t O, int64_t I, const hot_config* cfg) {
+  if (hot_backward_products(L, O, I, cfg) <= HOT_PRODUCTS_APART) return 0;
+  const BwdLayout b = bwd_layout(L, O, I, cfg);
+  return gemm_pair_tile_rows(gw_product(b, L, O, I, cfg), gx_product(b, L, O, I, cfg));
+}
 int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg) {
   if (check_cfg(cfg, "hot_backward_products") || L <= 0 || O <= 0 || I <= 0 || L % cfg->hla_n || O % cfg->n_o || O % 8 || I % 8 || cfg->gx_bits != cfg->w_bits) return 0;
   const BwdLayout b = bwd_layout(L, O, I, cfg);
   const GemmProduct px = gx_product(b, L, O, I, cfg), pw = gw_product(b, L, O, I, cfg);
   if (!pairs(pw, px, cfg)) return HOT_PRODUCTS_APART;
-  return gemm_pair_large(pw) ? HOT_PRODUCTS_PAIR_192 : HOT_PRODUCTS_PAIR_128;
+  return gemm_pair_tile_rows(pw, px) == 192 ? HOT_PRODUCTS_PAIR_192 : HOT_PRODUCTS_PAIR_128;
 }
 int64_t hot_kpad(int64_t k) { return round_up(k, GEMM_KTILE); }
 

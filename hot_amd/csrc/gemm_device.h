@@ -366,8 +366,8 @@ __device__ __forceinline__ void gemm_slot_body(const GemmArgs& g, int block, uin
   constexpr int NR = WM + WN;                       // fragment reads per round
   constexpr int H = NM / 2;                         // slots per half round
   constexpr int DPS = (LPW + NM - 1) / NM;          // DMA instructions per slot of the refilling round
-  constexpr int RPSL = (NR + NM - 1) / NM;          // fragment reads per slot (1 unless NR > NM)
-  static_assert(NR <= H || BITS != 4, "the reads of a round fit the first half of the round before");
+  constexpr int RS_ = BITS == 4 ? H : NM;           // slots the fragment reads go out in (INT4: the second half expands them)
+  constexpr int RPSL = (NR + RS_ - 1) / RS_;        // fragment reads per slot
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -11,25 +11,29 @@ namespace hot {
 // idle in its last round, and a lone workgroup per CU leaves the matrix cores idle while it fills its ring and while it
 // stores; here both share a grid and two workgroups share a CU (at most 80 KiB of LDS and 256 registers each), so that
 // one's loads and stores lie under the other's MFMAs.  The g_W tiles come first: they run longest, and g_x tiles fill
-// in behind them.  Two tilings, g_x / g_W (us of the whole backward, tokens x out x in, bf16, INT4 unless noted: first tiling /
-// second / one after the other by gemm_plan_impl):
-//   128 x 128 (2 stages) / 64 x 128 (3 stages): while the g_W product makes fewer than 256 tiles of 192 x 128, i.e.
-//     one long tile per CU would be its latency.  12608 x 3072 x 768: 106 / 114 / 116; 2304 wide: 88 / 95 / 92; 768 wide:
-//     45 / 69 / 53; 3003 x 1000 x 520: 29 / 39 / 37; 128 x 768 x 768: 27 / 32 / 30.  (g_x products of many tiles would rather
-//     have the second one: 12608 x 768 x 3072 76.6 / 74.2 / 79.2, INT8 82.8 / 78.6 / 91.6; 25216 tokens 115 / 109 / 114, INT8
-//     127 / 119 / 137; 25216 x 3072 x 768 153 / 152 / 165, INT8 180 / 172 / 199: the line does not look at them.)
-//   192 x 128 / 192 x 128 (2 stages): from there on.  8192 x 4096 x 11008: 542 / 466 / 508; 8192 x 11008 x 4096: 618 / 594 / 582,
-//     in blocks of 16 tokens 575 / 536 / 522; 8192 x 4096 x 4096: 266 / 250 / 247 (the last three: gemm_pair_pays)
+// in behind them.  Three tilings, g_x / g_W (us of the whole backward, tokens x out x in, bf16, INT4 unless noted: the three tilings in
+// this order / one after the other by gemm_plan_impl; gemm_pair_tiling chooses):
+//   64 x 64 both (4 stages): products that leave CUs idle in larger tiles, where the time is a chain of stages: a stage of
+//     64 x 64 is 0.2 us of it, one of 128 x 128 0.45 (half the operands to wait for, and four of them under way instead of two).
+//     112 x 896 x 1912 19.4 / 23.2 / 26.0 / 31.0; 15360 x 128 x 824 INT8 30.5 / 37.0 / 63.5 / 42.0; 49 x 3072 x 768 fp32 26.6 / 29.8 / 32.8 /
+//     36.2; 3003 x 1000 x 520 fp16 25.7 / 26.9 / 38.0 / 34.5
+//   128 x 128 (2 stages) / 64 x 128 (3 stages): what fills the chip but would make few tiles of 192 x 128.  12608 x 3072 x 768
+//     118 / 105 / 114 / 117; 2304 wide fp32 121 / 111 / 129 / 119; 999 x 720 x 3696 fp16 32.4 / 30.9 / 31.8 / 35.0
+//   192 x 128 both (2 stages): many tiles.  12608 x 768 x 3072 INT8 112 / 83.5 / 80.3 / 91.6; 25216 x 768 x 3072 179 / 117 / 110 / 114;
+//     5376 x 4736 x 10240 666 / 514 / 464 / 527; 8192 x 11008 x 4096, blocks of 16 tokens 757 / 578 / 529 / 520 (the last one: gemm_pair_pays)
 struct PairArgs {
   GemmArgs w, x;
   uint32_t w_blocks;      // a multiple of 8: blockIdx % 8 stays the XCD of the second product's tiles
 };
 
-template <int XBITS, bool LARGE, typename OutT>
+enum { PAIR_64, PAIR_128, PAIR_192 };   // tilings of the launch
+template <int XBITS, int TILING, typename OutT>
 __global__ void __launch_bounds__(G_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_pair_kernel(const PairArgs p) {
-  constexpr int XM = LARGE ? 3 : 2, WM = LARGE ? 3 : 2, WN = LARGE ? 2 : 1, WGM = LARGE ? 2 : 1, WGN = LARGE ? 2 : 4, WS = LARGE ? 2 : 3;
-  constexpr int LX = slot_ring_bytes<XM, 2, 2, 2, 2, 128>(), LW = slot_ring_bytes<WM, WN, WGM, WGN, WS, 128>();
+  constexpr bool LARGE = TILING == PAIR_192, SMALL = TILING == PAIR_64;
+  constexpr int XM = LARGE ? 3 : SMALL ? 1 : 2, XN = SMALL ? 1 : 2, XS = SMALL ? 4 : 2;
+  constexpr int WM = LARGE ? 3 : SMALL ? 1 : 2, WN = LARGE ? 2 : 1, WGM = LARGE || SMALL ? 2 : 1, WGN = LARGE || SMALL ? 2 : 4, WS = LARGE ? 2 : SMALL ? 4 : 3;
+  constexpr int LX = slot_ring_bytes<XM, XN, 2, 2, XS, 128>(), LW = slot_ring_bytes<WM, WN, WGM, WGN, WS, 128>();
   static_assert(LX <= 80 * 1024 && LW <= 80 * 1024, "two workgroups per CU");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[LX > LW ? LX : LW];
   // (the arguments are read inside the branch that uses them: both products' would overflow the scalar registers)
@@ -40,7 +44,7 @@ gemm_pair_kernel(const PairArgs p) {
   if (blockIdx.x < p.w_blocks) {
     if ((int)blockIdx.x < q.w.tiles_m * q.w.tiles_n) gemm_slot_body<WM, WN, WGM, WGN, 8, WS, 128, OutT, true>(q.w, (int)blockIdx.x, ring);
   } else {
-    gemm_slot_body<XM, 2, 2, 2, XBITS, 2, 128, OutT, true>(q.x, (int)(blockIdx.x - p.w_blocks), ring);
+    gemm_slot_body<XM, XN, 2, 2, XBITS, XS, 128, OutT, true>(q.x, (int)(blockIdx.x - p.w_blocks), ring);
   }
 }
 
@@ -50,14 +54,14 @@ static void pair_tiles(GemmArgs& g, int bm, int bn) {
   g.group_m = pick_group_m(g.tiles_m, g.tiles_n, 2);
 }
 
-template <int XBITS, bool LARGE, typename OutT>
+template <int XBITS, int TILING, typename OutT>
 static int launch_pair(PairArgs& p, hipStream_t st) {
-  pair_tiles(p.w, LARGE ? 192 : 64, 128);
-  pair_tiles(p.x, LARGE ? 192 : 128, 128);
+  pair_tiles(p.w, TILING == PAIR_192 ? 192 : 64, TILING == PAIR_64 ? 64 : 128);
+  pair_tiles(p.x, TILING == PAIR_192 ? 192 : TILING == PAIR_64 ? 64 : 128, TILING == PAIR_64 ? 64 : 128);
   p.w_blocks = (uint32_t)round_up((int64_t)p.w.tiles_m * p.w.tiles_n, 8);
   const int64_t total = (int64_t)p.w_blocks + (int64_t)p.x.tiles_m * p.x.tiles_n;
   if (total > (1 << 30)) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: too many tiles");
-  hipLaunchKernelGGL((gemm_pair_kernel<XBITS, LARGE, OutT>), dim3((unsigned)total), dim3(G_THREADS), 0, st, p);
+  hipLaunchKernelGGL((gemm_pair_kernel<XBITS, TILING, OutT>), dim3((unsigned)total), dim3(G_THREADS), 0, st, p);
   return check_launch("gemm_pair_kernel");
 }
 
@@ -100,17 +104,47 @@ bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
   return done < 0.94 * (rounds(w) + rounds(x));
 }
 
-bool gemm_pair_large(const GemmProduct& w) { return ((w.M + 191) / 192) * ((w.N + 127) / 128) >= 256; }
+// The tiling: from 256 tiles of 192 x 128 of g_W on that one, below them the one of the least time by this model.  A launch takes as
+// long as the work of all tiles on the 512 places there are for them (two to a CU), or as the stages of one tile one after the other,
+// whichever is longer, and a quarter of the other.  us for each stage of 128 bytes a row in that chain and with the chip full, and for the
+// start and end of a tile, g_x and g_W; with INT8 operands a stage of g_x has half the multiplications: x_int8 of it.  Fitted to
+// 157 shapes of 49 .. 25216 tokens and 64 .. 11008 channels, INT4 and INT8, all types, each timed in all three tilings: the choice is on
+// average 0.3 % slower than the best of the three (two tilings and the line alone: 5.1 %).  On the wrong side of the line 128 x 2304 x 5248
+// 49.0 / 46.5 / 52.0 and 512 x 4352 x 7336 127 / 118 / 127.
+static int gemm_pair_tiling(const GemmProduct& w, const GemmProduct& x) {
+  struct Tiling { int xm, xn, wm, wn; double chain_x, chain_w, full_x, full_w, ends_x, ends_w, x_int8; };
+  static const Tiling tilings[3] = {{64, 64, 64, 64, 0.20, 0.16, 0.22, 0.18, 2.0, 1.5, 0.8},
+                                    {128, 128, 64, 128, 0.45, 0.24, 0.95, 0.37, 3.3, 1.7, 0.7},
+                                    {192, 128, 192, 128, 0.60, 0.48, 1.08, 1.00, 3.9, 4.8, 0.8}};
+  auto tiles = [](const GemmProduct& p, int m, int n) { return (double)((p.M + m - 1) / m) * (double)((p.N + n - 1) / n); };
+  auto stages = [](const GemmProduct& p) { return (double)(round_up(p.K, GEMM_KTILE) * p.bits / 8 / 128); };
+  if (tiles(w, 192, 128) >= 256) return PAIR_192;
+  int best = PAIR_128;
+  double least = 0.0;
+  for (int k = PAIR_64; k <= PAIR_192; ++k) {
+    const Tiling& t = tilings[k];
+    const double sx = stages(x) * (x.bits == 8 ? t.x_int8 : 1.0), sw = stages(w);
+    const double full = (tiles(x, t.xm, t.xn) * (sx * t.full_x + t.ends_x) + tiles(w, t.wm, t.wn) * (sw * t.full_w + t.ends_w)) / 512.0;
+    const double chain = fmax(sx * t.chain_x + t.ends_x, sw * t.chain_w + t.ends_w);
+    const double us = fmax(full, chain) + 0.25 * fmin(full, chain);
+    if (k == PAIR_64 || us < least) { best = k; least = us; }
+  }
+  return best;
+}
+int gemm_pair_tile_rows(const GemmProduct& w, const GemmProduct& x) {
+  const int t = gemm_pair_tiling(w, x);
+  return t == PAIR_192 ? 192 : t == PAIR_128 ? 128 : 64;
+}
 
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st) {
   PairArgs p;
   if (int rc = gemm_fill(p.w, w, out_dtype, nullptr)) return rc;
   if (int rc = gemm_fill(p.x, x, out_dtype, nullptr)) return rc;
   if (!gemm_pair_possible(w, x)) return fail(HOT_ERR_UNSUPPORTED, "hot_gemm_i8: the paired kernel takes rows of whole 128-byte lines");
-  const bool large = gemm_pair_large(w);
-#define HOT_PAIR_CASE(OUT)                                                                                          \
-  return x.bits == 4 ? (large ? launch_pair<4, true, OUT>(p, st) : launch_pair<4, false, OUT>(p, st))               \
-                     : (large ? launch_pair<8, true, OUT>(p, st) : launch_pair<8, false, OUT>(p, st))
+  const int tiling = gemm_pair_tiling(w, x);
+#define HOT_PAIR_TILING(BITS, OUT) \
+  (tiling == PAIR_64 ? launch_pair<BITS, PAIR_64, OUT>(p, st) : tiling == PAIR_128 ? launch_pair<BITS, PAIR_128, OUT>(p, st) : launch_pair<BITS, PAIR_192, OUT>(p, st))
+#define HOT_PAIR_CASE(OUT) return x.bits == 4 ? HOT_PAIR_TILING(4, OUT) : HOT_PAIR_TILING(8, OUT)
   switch (out_dtype) {
     case HOT_F32: HOT_PAIR_CASE(float);
     case HOT_BF16: HOT_PAIR_CASE(bf16_t);
@@ -118,6 +152,7 @@ int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hi
     default: return fail(HOT_ERR_INVALID, "hot_gemm_i8: bad out dtype %d", out_dtype);
   }
 #undef HOT_PAIR_CASE
+#undef HOT_PAIR_TILING
 }
 
 }  // namespace hot

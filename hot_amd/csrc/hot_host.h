@@ -125,7 +125,7 @@ struct GemmProduct {
 int gemm_i8_impl(const GemmProduct& p, int out_dtype, int32_t* acc_out, hipStream_t st, void* split_ws = nullptr, size_t split_ws_bytes = 0, int variant = HOT_GEMM_AUTO);
 bool gemm_pair_possible(const GemmProduct& w, const GemmProduct& x);
 bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x);   // and where they are faster in one launch
-bool gemm_pair_large(const GemmProduct& w);                        // in which of its two tilings
+int gemm_pair_tile_rows(const GemmProduct& w, const GemmProduct& x);   // rows of g_x in a tile of that launch: 64, 128 or 192
 int gemm_pair_impl(const GemmProduct& w, const GemmProduct& x, int out_dtype, hipStream_t st);
 int gemm_bf16_impl(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N, int64_t K,
                    const void* bias, void* out, int out_dtype, int64_t ldo, hipStream_t st, int variant);

@@ -378,6 +378,11 @@ def backward_products(L: int, O: int, I: int, opt: HotOptions) -> int:
     return int(_lib.lib().hot_backward_products(int(L), int(O), int(I), C.byref(opt.to_c())))
 
 
+def backward_pair_rows(L: int, O: int, I: int, opt: HotOptions) -> int:
+    """Rows of g_x in a tile of the launch that both products share: 64, 128 or 192 (hot_backward_pair_rows; 0 when they share none)."""
+    return int(_lib.lib().hot_backward_pair_rows(int(L), int(O), int(I), C.byref(opt.to_c())))
+
+
 def kpad_group(T: int, opt: HotOptions) -> int:
     """Code bytes every sample takes in the K dimension of the batched g_W operands."""
     return _size(opt, "kpad_group", int(T))

@@ -120,10 +120,13 @@ HOT_API int hot_backward_streams(int64_t L, int64_t O, int64_t I, const hot_conf
  * measurements know which kernel they cover. */
 enum hot_products_launch {
   HOT_PRODUCTS_APART = 1,     /* one after the other (or beside one another: cfg->streams), each by hot_gemm_plan     */
-  HOT_PRODUCTS_PAIR_128 = 2,  /* in one launch: g_x in tiles of 128 x 128, g_W in tiles of 64 x 128                   */
+  HOT_PRODUCTS_PAIR_128 = 2,  /* in one launch: g_x in tiles of 128 x 128, g_W in tiles of 64 x 128, or both of 64 x 64
+                                 (hot_backward_pair_rows)                                                             */
   HOT_PRODUCTS_PAIR_192 = 3   /* in one launch: both in tiles of 192 x 128                                            */
 };
 HOT_API int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
+/* Rows of g_x in a tile of that launch, 64, 128 or 192 (0: the products do not share one, or the size is refused). */
+HOT_API int hot_backward_pair_rows(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 HOT_API int hot_abi_version(void);
 
 /* Bytes of the leading dimension (row pitch) the library uses for a K-major

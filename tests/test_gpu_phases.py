@@ -144,6 +144,33 @@ def test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, launches, cas
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dt)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dt))
 
 
+@pytest.mark.parametrize("L,O,I,rows", [
+    (1, 16, 8, 64), (63, 64, 64, 64), (65, 80, 72, 64), (128, 128, 128, 64), (449, 16, 72, 64),
+    (64, 784, 128, 64), (64, 1040, 72, 64), (64, 1296, 64, 64), (64, 1808, 64, 64), (1153, 2048, 64, 64),
+    (771, 80, 4104, 128), (1001, 64, 3992, 128), (896, 64, 4096, 128), (6304, 16, 3080, 128),
+    (208, 1552, 4104, 192)])
+@pytest.mark.parametrize("dt,bits", [(torch.float32, 4), (torch.bfloat16, 8), (torch.float16, 4)])
+def test_tilings_of_paired_products(gpu, L, O, I, rows, dt, bits):
+    """The three tilings of the paired launch: edges of their tiles, and with 64 x 64 as many stages of g_x and g_W as leave the
+    ring of four unfilled, fill it, and take every remainder of its rounds."""
+    from hot_amd import ops
+    ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits)
+    if not (bits == 8 and O > 1664):                # (those go apart)
+        assert ops.backward_pair_rows(L, O, I, _options(ocfg)) == rows
+    check(gpu, L, O, I, dt, gx_bits=bits, w_bits=bits)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("case,dt", [("g_x overflows", torch.float32), ("g_w subnormal", torch.bfloat16), ("row steps", torch.float16)])
+def test_ends_of_the_range_in_wide_tiles(gpu, dt, bits, case):
+    """The same in tiles of 128 x 128 / 64 x 128, whole ones and cut ones."""
+    from hot_amd import ops
+    L, O, I = 776, 80, 4104
+    ocfg = orc.HotConfig.python_rule(L, gx_bits=bits, w_bits=bits, n_o=16)
+    assert ops.backward_pair_rows(L, O, I, _options(ocfg)) == 128
+    test_products_at_the_ends_of_the_range(gpu, dt, bits, L, O, I, (P128, P128), case)
+
+
 def _buffer(xq):
     """The oracle's codes [L', I] as the activation buffer holds them: [I, L' rounded up to whole lines of 128 codes]."""
     out = np.zeros((xq.shape[1], -(-xq.shape[0] // 128) * 128), np.int8)

@@ -352,3 +352,17 @@ def test_launch_of_the_products():
         assert launch(64, longest, 64, bits) == ops.PRODUCTS_PAIR_128 and launch(64, longest + 16, 64, bits) == ops.PRODUCTS_APART
         assert launch(64, 1536, 3968, bits) == ops.PRODUCTS_PAIR_128 and launch(64, 1536, 4096, bits) == ops.PRODUCTS_PAIR_192
     assert launch(8192, 11008, 4096) == ops.PRODUCTS_PAIR_192
+
+
+def test_tiling_of_the_paired_products():
+    """hot_backward_pair_rows: small products in tiles of 64, those that fill the chip in larger ones, 0 where none is shared."""
+    from hot_amd import ops
+
+    def rows(L, O, I, bits=4, **kw):
+        n, r = orc.hla_rows(min(L & -L, 64) or 1)
+        return ops.backward_pair_rows(L, O, I, ops.HotOptions(n_o=8, hla_n=n, hla_rows=tuple(int(v) for v in r), gx_bits=bits, w_bits=bits, **kw))
+
+    assert rows(49, 3072, 768) == rows(64, 64, 64) == rows(3003, 1000, 520) == 64
+    assert rows(12608, 3072, 768) == rows(12608, 2304, 768) == rows(12608, 3072, 768, 8) == 128
+    assert rows(12608, 768, 3072, 8) == rows(8192, 11008, 4096) == 192
+    assert rows(64, 64, 64, streams=2) == rows(64, 8192, 64) == rows(0, 64, 64) == rows(64, 64, 20) == 0
