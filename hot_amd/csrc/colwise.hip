@@ -259,7 +259,15 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
     a.NBs = (a.NBs + per - 1) / per;
     job.tb[0] /= per; job.tb[1] /= per;
   }
-  // per-sample statistics and per-channel maxima are kept by atomics, everything else by workgroup
+  // per-sample statistics and the per-channel maxima of many runs are kept by atomics, everything else by workgroup.  The maxima of a
+  // few runs have the second half of the statistics for themselves (us of the whole backward, cleared and updated / own: 197 x 632 x 2048
+  // 24.7 / 21.9, 49 x 3072 x 768 fp32 26.5 / 24.5, 192 x 640 x 1400 25.3 / 21.9; more of them would be a long chain of loads for each reader).
+  a.ncolmax = COLMAX_COPIES;
+  if (scale_mode == HOT_SCALE_ROW && groups == 1 && runs0 <= COLMAX_OWN && runs0 * C <= 2 * COL_MAX_WGS) {
+    a.colmax = a.pmax + 2 * COL_MAX_WGS;
+    a.ncolmax = (int32_t)runs0;
+    a.colmax_own = 1;
+  }
   a.npart = (int32_t)(scale_mode == HOT_SCALE_SAWB ? gx * runs : gx * runs0);
   return HOT_OK;
 }
@@ -283,7 +291,7 @@ ColArgs col_job_args(const ColJob& job, int pass) {
 
 void col_job_clear(const ColJob& job, hipStream_t st) {
   const ColArgs& a = job.a;
-  const int64_t ncolmax = a.mode == HOT_SCALE_ROW ? (a.groups > 1 ? a.C * a.groups : a.C * COLMAX_COPIES) : 0;
+  const int64_t ncolmax = a.mode == HOT_SCALE_ROW ? (a.groups > 1 ? a.C * a.groups : a.colmax_own ? 0 : a.C * COLMAX_COPIES) : 0;
   const int64_t ngstat = a.groups > 1 && (a.mode == HOT_SCALE_TENSOR || a.row_absmax) ? GS * (int64_t)a.groups : 0;
   const int64_t n = ncolmax > ngstat ? ncolmax : ngstat;
   if (n > 0)

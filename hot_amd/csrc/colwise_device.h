@@ -11,7 +11,8 @@
 namespace hot {
 
 constexpr int CW = 256;        // threads per workgroup = channels per workgroup
-constexpr int COLMAX_COPIES = 8;  // per-channel maxima: workgroup row y folds into copy y % 8 (fewer atomics per line)
+constexpr int COLMAX_COPIES = 8;  // per-channel maxima: workgroup row y folds into copy y % 8 (fewer atomics per line) ...
+constexpr int COLMAX_OWN = 64;    // ... or, up to that many workgroup rows, each has a copy of its own: nothing to clear, a launch less
 constexpr int CW_ROWS = 16;    // rows staged per step
 
 constexpr int GS = 32;   // floats between the statistics of two sample groups (one 128-byte line each)
@@ -28,7 +29,9 @@ struct ColArgs {
   float* pmax;        // TENSOR: absmax per workgroup, npart of them
   double* partial;    // SAWB: 2 doubles per workgroup, npart of them (per sample group)
   int32_t npart;
-  float* colmax;      // ROW: per-channel absmax, COLMAX_COPIES arrays of C floats
+  float* colmax;      // ROW: per-channel absmax, ncolmax arrays of C floats
+  int32_t ncolmax;    // COLMAX_COPIES of them, updated by atomics, or (own) one per run of token blocks of the statistics pass
+  int32_t colmax_own;
   float* scales_out;
   float* row_absmax;  // statistics pass with RS: absmax of the row-wise block Hadamard, one per workgroup (sample groups: row_absmax[GS g])
   int32_t rs_n;       // ... its block along the channels (1, 2, 4, 8 or 16)
@@ -335,8 +338,13 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
         if (a.groups > 1) {
           cm = a.colmax[(int64_t)sample * a.C + c];
         } else {
+          for (int k0 = 0; k0 < a.ncolmax; k0 += COLMAX_COPIES) {      // (that many loads under way at a time)
+            float v[COLMAX_COPIES];
 #pragma unroll
-          for (int k = 0; k < COLMAX_COPIES; ++k) cm = fmaxf(cm, a.colmax[k * a.C + c]);
+            for (int k = 0; k < COLMAX_COPIES; ++k) v[k] = a.colmax[(k0 + k < a.ncolmax ? k0 + k : a.ncolmax - 1) * a.C + c];
+#pragma unroll
+            for (int k = 0; k < COLMAX_COPIES; ++k) cm = fmaxf(cm, v[k]);
+          }
         }
       }
       const float sc = cm / (float)qmax;
@@ -671,6 +679,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
     if (a.mode == HOT_SCALE_ROW) {
       if (active) {
         if (a.groups > 1) atomic_max_nonneg(a.colmax + (int64_t)sample * a.C + c, cmax);
+        else if (a.colmax_own) a.colmax[by * a.C + c] = cmax;
         else atomic_max_nonneg(a.colmax + (by % COLMAX_COPIES) * a.C + c, cmax);
       }
       return;

@@ -114,6 +114,9 @@ def test_backward_matches_oracle(gpu, dtype, shape, variant):
     (96, 272, 520),      # blocks of 32
     (16 * 67, 32, 16),   # enough runs of sixteen tokens that some workgroups take several
     (3001, 144, 16),     # blocks of one token, many of them: the last run of nine rows
+    (1023, 32, 16),      # 64 runs: with a step per channel each has maxima of its own
+    (1025, 32, 16),      # 65: they share eight copies
+    (1023, 2064, 8),     # 64 runs of more channels than there is room for
 ])
 def test_backward_small_grids(gpu, L, O, I, dtype, variant):
     """Problems whose column-wise jobs are cut into short runs of token blocks (col_partition): rings of one to four
