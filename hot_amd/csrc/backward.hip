@@ -358,7 +358,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   if (hq_job) {
     const float* stat = !row_tensor ? nullptr : big ? slots : gj.a.row_absmax;
     rc = hq_job_impl(hj, gy, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg, b.ld_g, sg,
-                     stat, big ? STAT_SLOTS : row_tensor ? gj.a.npart : 0, big ? STAT_SLOT_STRIDE : 1, 1);
+                     stat, big ? 1 : row_tensor ? gj.a.npart : 0, 1, 1);
     if (rc) return rc;
   }
   ColsumArgs sj;

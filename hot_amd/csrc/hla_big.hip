@@ -15,10 +15,13 @@
 //   transpose codes [L', C] -> [C, ld] (K-major for the GEMM), padding zeroed
 // Only the coefficients a kept row needs make the round trip: natural row i of a block is coefficient
 // k = i % 64 of run i / 64, so a k that no kept row has is never written by stage 1 nor read by stage 2
-// (the make_WHT selections keep no odd row: half the traffic).  The row table lives in the workspace
-// and is written by kernels whose arguments carry the rows by value, so the whole call is a sequence
+// (the make_WHT selections keep no odd row: half the traffic).  Which rows are kept travels in the kernel
+// arguments, as bit masks; a list that is not run-major also needs a table of them, which lives in the workspace
+// and is written by kernels whose arguments carry the rows by value.  So the whole call is a sequence
 // of launches: no host-to-device copy, nothing read from host memory after the call returns, and a
-// stream under graph capture records it like any other call.
+// stream under graph capture records it like any other call.  Stage 1 clears what stage 2 updates by atomics (us of the
+// whole backward with a launch that clears and writes the table before it / without: 1024 x 1024 x 1024 39.8 / 34.8, 8192 x
+// 4096 x 11008 489.7 / 478.9).
 // This is the exactness path for large blocks, not a tuned one: the input is read with scalar loads
 // and the coefficients make a round trip through HBM in fp32.
 #include <string.h>
@@ -41,22 +44,27 @@ struct BigArgs {
   float* T;            // [R, C] fp32 coefficients of the 64-point stage
   int8_t* tmp;         // [Kout, tmp_ld] codes before the transpose (or the untransposed destination itself)
   int64_t tmp_ld;
-  const int32_t* tab;  // per natural row of a block: slot | visit << 16, or -1 when dropped
+  const int32_t* tab;  // lists that are not run-major: per natural row of a block, its slot | visit << 16, or -1 when dropped
   int64_t R, C, NB;    // NB = R / n blocks
   int32_t n, r, rpad, bits, rounding, mode;
   int32_t nk;          // coefficients of a 64-run that some kept row needs
   uint64_t kmask;      // bit k: coefficient k is one of them
   uint8_t klist[64];   // the nk set bits of kmask in increasing order
-  // run-major row lists only (big_stage2_runs_kernel): which runs keep needed coefficient index kc
-  // (bit j of keep[kc]: natural row 64 j + klist[kc] is kept), and the output coefficient of its first
-  // kept row (kbase[kc]; kbase[nk] = r): its other kept rows follow in run order
+  // which runs keep needed coefficient index kc (bit j of keep[kc]: natural row 64 j + klist[kc] is kept); for run-major lists
+  // (big_stage2_runs_kernel) the output coefficient of its first kept row (kbase[kc]; kbase[nk] = r): its other kept rows
+  // follow in run order; and for the visits of stochastic rounding (ranks among the kept rows in natural order) which
+  // coefficient indices run j keeps and how many rows the runs before it do
   uint32_t keep[64][4];
   uint16_t kbase[65];
+  uint64_t run_keep[128];
+  uint16_t run_base[128];
   float* stat;         // [0] absmax, [1] step, [2] clip; the absmax slots from word 64
   float* colmax;       // per-channel absmax (ROW)
   double* partial;     // SAWB: 2 doubles per workgroup
   float* scales_out;
-  float* row_absmax;   // stage 1 with RS: absmax of the row-wise 16-point Hadamard (STAT_SLOTS partial maxima), or null
+  float* row_part;     // stage 1 with RS: absmax of the row-wise 16-point Hadamard, one per workgroup, or null; the statistics pass
+  int64_t row_nparts;  // of stage 2 takes the maximum of all of them ...
+  float* row_absmax;   // ... to this word
   uint64_t seed;
   uint32_t stream;
 };
@@ -96,6 +104,12 @@ __global__ void __launch_bounds__(BT) big_stage1_kernel(const BigArgs a) {
   const int chan = RS ? (tid ^ ((tid & 4) ? 0xB : 0)) : tid;
   const int64_t c = (int64_t)blockIdx.x * BT + chan;
   const bool active = c < a.C;
+  // what stage 2 updates by atomics is cleared here, a launch before it
+  if (blockIdx.y == 0) {
+    if (active) a.colmax[c] = 0.f;
+    if (blockIdx.x == 0)
+      for (int i = tid; i < (int)(STAT_BYTES / 4); i += BT) a.stat[i] = 0.f;
+  }
   if (!RS && !active) return;
   const int64_t row0 = (int64_t)blockIdx.y * 64;
   const T* in = reinterpret_cast<const T*>(a.in) + row0 * a.C + (active ? c : 0);
@@ -138,7 +152,7 @@ __global__ void __launch_bounds__(BT) big_stage1_kernel(const BigArgs a) {
     if (tid == 0) {
       float mm = s_max[0];
       for (int i = 1; i < BT / 64; ++i) mm = fmaxf(mm, s_max[i]);
-      stat_slot_update(a.row_absmax, blockIdx.y * gridDim.x + blockIdx.x, mm);
+      a.row_part[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = mm;
     }
     if (!active) return;
   }
@@ -169,9 +183,17 @@ __global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
   // The table entries of this coefficient index (one per run) go through LDS: read from global memory
   // inside the quantise loop they would sit between the loop's byte stores, and every such load then
   // waits for the store before it (one memory round trip per kept row).
-  __shared__ int32_t s_tab[M];
-  if (tid < M) s_tab[tid] = a.tab[tid * 64 + k];
-  __syncthreads();
+  __shared__ int32_t s_tab[PASS == 1 ? M : 1];
+  if constexpr (PASS == 1) {
+    if (tid < M) s_tab[tid] = a.tab[tid * 64 + k];
+    __syncthreads();
+  } else if (a.row_part && blockIdx.x == 0 && blockIdx.y == 0) {
+    const float m = wave_max(part_max(a.row_part, (int)a.row_nparts, 1, tid));
+    if (lane == 0) s_max[wave] = m;
+    __syncthreads();
+    if (tid == 0) a.row_absmax[0] = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+    __syncthreads();
+  }
   float v[M];
   if (active) {
     const float* t = a.T + ((blk * M) * a.nk + kc) * a.C + c;
@@ -194,7 +216,7 @@ __global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
     double ssq = 0.0, sab = 0.0;
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-      if (s_tab[j] >= 0) {
+      if ((a.keep[kc][j >> 5] >> (j & 31)) & 1u) {
         cmax = fmaxf(cmax, fabsf(v[j]));
         if constexpr (SAWB) { ssq += (double)v[j] * (double)v[j]; sab += (double)fabsf(v[j]); }
       }
@@ -324,7 +346,7 @@ __global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigAr
       if constexpr (ROUND == HOT_ROUND_NEAREST) {
         q = (int)rint_div_fast(x, d, rcp);      // bit for bit rintf(x / d)
       } else {
-        const int visit = a.tab[j * 64 + k] >> 16;
+        const int visit = a.run_base[j] + __popcll(a.run_keep[j] & ((1ull << k) - 1ull));
         const uint64_t idx = ((uint64_t)c * (uint64_t)a.NB + (uint64_t)blk) * (uint64_t)a.rpad + (uint64_t)visit;
         q = q_stoch_fix(x, rcp * 65536.0f, bits_of(idx, a.seed, a.stream), qmax);
       }
@@ -392,14 +414,6 @@ int dispatch_runs(int m, const BigArgs& a, void* out, int64_t ld_out, hipStream_
   }
 }
 
-__global__ void big_clear_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n, float* row_absmax) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < (int64_t)(STAT_BYTES / 4)) stat[i] = 0.f;
-  if (row_absmax && i < (int64_t)(STAT_SLOT_BYTES / 4)) row_absmax[i] = 0.f;
-  if (i < C) colmax[i] = 0.f;
-  if (i < n) tab[i] = -1;
-}
-
 // The row table, built by ONE launch whose arguments carry the kept rows by value: up to 2304 rows
 // of 13 bits each (3744 bytes of the 4 KiB a launch may carry; larger selections go in pieces of that
 // size).  Entry of natural row i: its output coefficient (the position of i in the caller's list) in
@@ -445,11 +459,10 @@ __global__ void __launch_bounds__(256) big_table_kernel(int32_t* tab, const TabR
   const int rank = (int)(s_below[row >> 5] + (uint32_t)__popc(s_map[row >> 5] & ((1u << (row & 31)) - 1u)));
   tab[row] = k | (rank << 16);
 }
-// Clear and table in one launch (selections of up to TAB_ROWS rows): every workgroup marks the kept
-// rows in its own LDS bitmap; thread i of the grid clears word i of the statistics and of the
-// per-channel maxima, writes -1 for natural row i when it is dropped, and the entry of the i-th row of
-// the caller's list.  Dropped and kept rows are disjoint, so the two writes never meet.
-__global__ void __launch_bounds__(256) big_prepare_kernel(float* stat, float* colmax, int64_t C, int32_t* tab, int n, float* row_absmax, const TabRows p) {
+// The whole table in one launch (selections of up to TAB_ROWS rows): every workgroup marks the kept rows in its own LDS bitmap;
+// thread i of the grid writes -1 for natural row i when it is dropped, and the entry of the i-th row of the caller's list.
+// Dropped and kept rows are disjoint, so the two writes never meet.
+__global__ void __launch_bounds__(256) big_prepare_kernel(int32_t* tab, int n, const TabRows p) {
   __shared__ uint32_t s_map[8192 / 32];
   __shared__ uint32_t s_below[8192 / 32];
   const int tid = threadIdx.x;
@@ -467,9 +480,6 @@ __global__ void __launch_bounds__(256) big_prepare_kernel(float* stat, float* co
   }
   __syncthreads();
   const int64_t i = (int64_t)blockIdx.x * 256 + tid;
-  if (i < (int64_t)(STAT_BYTES / 4)) stat[i] = 0.f;
-  if (row_absmax && i < (int64_t)(STAT_SLOT_BYTES / 4)) row_absmax[i] = 0.f;
-  if (i < C) colmax[i] = 0.f;
   if (i < n && !((s_map[i >> 5] >> (i & 31)) & 1u)) tab[i] = -1;
   if (i < p.count) {
     const int row = tab_row_get(p.packed, (int)i);
@@ -679,13 +689,14 @@ int dispatch_stage2(int m, const BigArgs& a, dim3 grid, int pass, hipStream_t st
 }
 
 
-struct BigLayout { size_t off_colmax, off_partial, off_tab, off_T, off_tmp, total; };
+struct BigLayout { size_t off_colmax, off_partial, off_rows, off_tab, off_T, off_tmp, total; };
 
 BigLayout big_layout(int64_t R, int64_t C, int n, int r) {
   BigLayout b;
   size_t o = STAT_BYTES;
   b.off_colmax = o;  o += (size_t)round_up(C * 4, 256);
   b.off_partial = o; o += (size_t)(2 * sizeof(double)) * 65536;
+  b.off_rows = o;    o += (size_t)round_up((C + BT - 1) / BT * (R / 64) * 4, 256);
   b.off_tab = o;     o += (size_t)round_up((int64_t)n * 4, 256);
   b.off_T = o;       o += (size_t)round_up(R * C * 4, 256);
   b.off_tmp = o;     o += (size_t)round_up((R / n) * r * C, 256);
@@ -725,42 +736,61 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
   a.mode = scale_mode; a.stat = (float*)ws; a.colmax = (float*)(ws + b.off_colmax);
   a.partial = (double*)(ws + b.off_partial); a.scales_out = scales_out; a.seed = seed; a.stream = rng_stream;
   a.tmp_ld = C;
-  // the row table (and with it the check of the row list), after the clear kernel below
   uint64_t kmask = 0;
-  for (int k = 0; k < r; ++k)
-    if (rows[k] >= 0 && rows[k] < n) kmask |= 1ull << (rows[k] & 63);
+  for (int k = 0; k < r; ++k) {
+    if (rows[k] < 0 || rows[k] >= n) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d outside [0, %d)", who, k, rows[k], n);
+    kmask |= 1ull << (rows[k] & 63);
+  }
   a.kmask = kmask; a.nk = 0;
+  int kc_of[64];
   for (int k = 0; k < 64; ++k) {
     a.klist[k] = 0;
+    kc_of[k] = a.nk;
     if ((kmask >> k) & 1ull) a.klist[a.nk++] = (uint8_t)k;
   }
   if (NB * a.nk > 65535) return fail(HOT_ERR_UNSUPPORTED, "%s: %lld blocks of %d tokens exceed the grid of the large-block path", who, (long long)NB, n);
-
-  // statistics and table cleared, then the table written piece by piece (rows in natural order, so
-  // the visit number of a piece's entry i is its position in the sorted list)
-  const int64_t nclr = std::max<int64_t>(std::max<int64_t>(C, n), (int64_t)(STAT_BYTES / 4));
-  if (r <= TAB_ROWS) {
-    // the row list is checked here, the table written by the clear launch itself
-    std::unique_ptr<uint8_t[]> seen(new uint8_t[(size_t)n]());
-    TabRows tr;
-    memset(&tr, 0, sizeof(tr));
-    tr.count = r;
-    for (int k = 0; k < r; ++k) {
-      if (rows[k] < 0 || rows[k] >= n) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d outside [0, %d)", who, k, rows[k], n);
-      if (seen[(size_t)rows[k]]) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d listed twice", who, k, rows[k]);
-      seen[(size_t)rows[k]] = 1;
-      tab_row_put(tr.packed, k, rows[k]);
-    }
-    hipLaunchKernelGGL(big_prepare_kernel, dim3((unsigned)((nclr + 255) / 256)), dim3(256), 0, st, a.stat, a.colmax, C,
-                       (int32_t*)(ws + b.off_tab), n, row16_absmax_out, tr);
-    if (int rc = check_launch("big_prepare_kernel")) return rc;
+  memset(a.keep, 0, sizeof(a.keep));
+  memset(a.run_keep, 0, sizeof(a.run_keep));
+  for (int i = 0; i < r; ++i) {
+    const int k = rows[i] & 63, j = rows[i] >> 6;
+    if ((a.run_keep[j] >> k) & 1ull) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d listed twice", who, i, rows[i]);
+    a.run_keep[j] |= 1ull << k;
+    a.keep[kc_of[k]][j >> 5] |= 1u << (j & 31);
+  }
+  for (int j = 0, below = 0; j < 128; ++j) {
+    a.run_base[j] = (uint16_t)below;
+    below += __builtin_popcountll(a.run_keep[j]);
+  }
+  // rows listed run-major (sorted by (row % 64, row / 64)): the quantise pass stores K-major itself
+  bool run_major = !rowmajor && NB * ((a.nk + KG - 1) / KG) <= 65535;
+  for (int k = 1; k < r && run_major; ++k) {
+    const int prev = (rows[k - 1] & 63) * m + (rows[k - 1] >> 6), cur = (rows[k] & 63) * m + (rows[k] >> 6);
+    run_major = cur > prev;
+  }
+  memset(a.kbase, 0, sizeof(a.kbase));
+  if (run_major) {
+    int kc = -1, last_k = -1;
+    for (int i = 0; i < r; ++i)
+      if ((rows[i] & 63) != last_k) { last_k = rows[i] & 63; a.kbase[++kc] = (uint16_t)i; }
+    for (int q = kc + 1; q <= 64; ++q) a.kbase[q] = (uint16_t)r;
   } else {
-    hipLaunchKernelGGL(big_clear_kernel, dim3((unsigned)((nclr + 255) / 256)), dim3(256), 0, st, a.stat, a.colmax, C,
-                       (int32_t*)(ws + b.off_tab), n, row16_absmax_out);
-    if (int rc = build_row_table((int32_t*)(ws + b.off_tab), n, rows, r, nullptr, st, who)) return rc;
+    // the quantise pass of any other list reads a table of its rows, written piece by piece when it is long
+    if (r <= TAB_ROWS) {
+      TabRows tr;
+      memset(&tr, 0, sizeof(tr));
+      tr.count = r;
+      for (int k = 0; k < r; ++k) tab_row_put(tr.packed, k, rows[k]);
+      hipLaunchKernelGGL(big_prepare_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (int32_t*)(ws + b.off_tab), n, tr);
+      if (int rc = check_launch("big_prepare_kernel")) return rc;
+    } else {
+      hipLaunchKernelGGL(tab_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (int32_t*)(ws + b.off_tab), n);
+      if (int rc = build_row_table((int32_t*)(ws + b.off_tab), n, rows, r, nullptr, st, who)) return rc;
+    }
   }
   const dim3 g1((unsigned)gx, (unsigned)(R / 64));
   a.row_absmax = row16_absmax_out;
+  a.row_part = row16_absmax_out ? (float*)(ws + b.off_rows) : nullptr;
+  a.row_nparts = gx * (R / 64);
   if (row16_absmax_out && (C % 16 || scale_mode == HOT_SCALE_SAWB))
     return fail(HOT_ERR_UNSUPPORTED, "%s: fused row statistic unavailable for this configuration", who);
   switch (dtype) {
@@ -781,12 +811,6 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
   if (int rc = check_launch("big_stage1_kernel")) return rc;
   const dim3 g2((unsigned)gx, (unsigned)(NB * a.nk));
   if (int rc = dispatch_stage2(m, a, g2, 0, st)) return rc;
-  // rows listed run-major (sorted by (row % 64, row / 64)): the quantise pass stores K-major itself
-  bool run_major = !rowmajor && NB * ((a.nk + KG - 1) / KG) <= 65535;
-  for (int k = 1; k < r && run_major; ++k) {
-    const int prev = (rows[k - 1] & 63) * m + (rows[k - 1] >> 6), cur = (rows[k] & 63) * m + (rows[k] >> 6);
-    run_major = cur > prev;
-  }
   // (with absmax steps the run-major quantise pass reads the statistic itself and publishes the steps)
   if (!(run_major && scale_mode != HOT_SCALE_SAWB))
     hipLaunchKernelGGL(big_finalize_kernel, dim3(1), dim3(256), 0, st, a, (int64_t)gx * NB * a.nk, kout);
@@ -802,18 +826,7 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
     }
     return HOT_OK;
   }
-  if (run_major) {
-    memset(a.keep, 0, sizeof(a.keep));
-    memset(a.kbase, 0, sizeof(a.kbase));
-    int kc = -1, last_k = -1;
-    for (int i = 0; i < r; ++i) {
-      const int k = rows[i] & 63, j = rows[i] >> 6;
-      if (k != last_k) { ++kc; last_k = k; a.kbase[kc] = (uint16_t)i; }
-      a.keep[kc][j >> 5] |= 1u << (j & 31);
-    }
-    for (int q = kc + 1; q <= 64; ++q) a.kbase[q] = (uint16_t)r;
-    return dispatch_runs(m, a, codes_out, ld_out, st);
-  }
+  if (run_major) return dispatch_runs(m, a, codes_out, ld_out, st);
   if (int rc = dispatch_stage2(m, a, g2, 1, st)) return rc;
   const dim3 gt((unsigned)((ld_out + 63) / 64), (unsigned)((C + 63) / 64));
   hipLaunchKernelGGL(transpose_i8_kernel, gt, dim3(256), 0, st, a.tmp, kout, C, (int8_t*)codes_out, ld_out);

@@ -101,7 +101,7 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
                  float* row16_absmax_out = nullptr, bool rowmajor = false, int store4 = 0);
 // rowmajor: the codes are stored untransposed, [NB r, C] with ld_out bytes per coefficient row (store4:
 // two channels to a byte).
-// row16_absmax_out (STAT_SLOTS partial maxima, cleared by the call's first launch; C a multiple of 16, absmax steps):
+// row16_absmax_out (one word; C a multiple of 16, absmax steps):
 // stage 1 also delivers the absmax of the row-wise 16-point Hadamard of the input.
 size_t hla_big_workspace_bytes_impl(int64_t R, int64_t C, int n, int r);
 // Workspace of a token-wise transform of [R, C] with blocks of n tokens and r kept rows, either path.
