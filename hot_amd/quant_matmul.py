@@ -191,26 +191,32 @@ def _pad8(t: Tensor) -> Tensor:
 _PLAIN_APPLY = hasattr(torch._C, "_are_functorch_transforms_active")
 
 
-# The activation buffer is written beside the forward GEMM, not behind it: the two read the same x and
-# neither needs the other (the GEMM is bound by the matrix cores, the buffer kernels by memory).
+# The activation buffer can be written beside the forward GEMM: the two read the same x and neither needs the other.
 # forward() records an event on the current stream before it launches the GEMM; setup_context, which
 # autograd calls right after forward on the same thread, lets a side stream wait for that event, runs
 # the buffer kernels there and makes the current stream wait for them.  One side stream per device,
 # default priority.  Not under stream capture (a capture must not be forked behind its back).
 #
-# Only for inputs above 24 MiB: the fork and the join cost the host 30 us (an event, two stream waits, the side
-# stream's pool), about what the buffer kernels take for 24 MiB.  Smaller layers run at the pace of the host, and
-# in line the kernels cost it two launches (a training step of 12608 tokens 768 -> 768, 19 MB: 306 us forked; 128
-# tokens: 325 us).
+# It pays only for fp32 products of 2^35 multiply-adds and more.  A product in 16 bits leaves the buffer kernels one workgroup per
+# CU (124 KB of LDS), loses what it gives them, and the fork and the join cost the host 30 us; us of a training step of one
+# layer, canonical recipe, tokens x in -> out, beside / in line: bf16 25216 x 3072 -> 768 376 / 359, 8191 x 3072 -> 1024 235 / 203,
+# 12608 x 3072 -> 768 267 / 196, 8192 x 4096 -> 11008 1475 / 1448, 16384 x 4096 -> 4096 1029 / 999, the MLP of 25216 x 768 886 / 873;
+# fp32 16000 x 1024 -> 1024 (2^34) 414 / 390, 12608 x 1024 -> 3072 (2^35.2) 859 / 871.
+#
+# overlap_buffer_write: None = that rule; True = beside from OVERLAP_MIN_BYTES of input on, whatever the product; False = in line.
 _FWD = threading.local()
 _SIDE_STREAMS: dict = {}
-overlap_buffer_write = True
+overlap_buffer_write = None
 OVERLAP_MIN_BYTES = 24 << 20
+OVERLAP_MIN_MACS_FP32 = 1 << 35
 
 
-def _mark_input_ready(x: Tensor) -> None:
+def _mark_input_ready(x: Tensor, w: Tensor) -> None:
     _FWD.event = None
-    if not (overlap_buffer_write and x.is_cuda) or x.numel() * x.element_size() < OVERLAP_MIN_BYTES:
+    if overlap_buffer_write is False or not x.is_cuda or x.numel() * x.element_size() < OVERLAP_MIN_BYTES:
+        return
+    if overlap_buffer_write is None and (x.dtype != torch.float32 or x.numel() * w.shape[0] < OVERLAP_MIN_MACS_FP32
+                                         or torch.is_autocast_enabled()):
         return
     if hot_switched_off() or torch.cuda.is_current_stream_capturing():
         return
@@ -250,7 +256,7 @@ class FLinearQ(Function):
         # `bias` is an addition to the reference's five arguments (which adds the bias after the
         # Function, utils/quant_matmul.py:419-420): inside, it rides in the GEMM epilogue instead of
         # costing a pass over the output
-        _mark_input_ready(x)
+        _mark_input_ready(x, w)
         return F.linear(x, w, bias)
 
     @staticmethod

@@ -1192,6 +1192,35 @@ def test_hq_linear_buffer_write_beside_the_product_from_24_mib(gpu, fresh_args, 
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype,rows,autocast,beside", [(torch.float32, 512, False, True), (torch.float32, 511, False, False),
+                                                        (torch.bfloat16, 1024, False, False), (torch.float32, 512, True, False)])
+def test_hq_linear_buffer_write_rule(gpu, fresh_args, monkeypatch, dtype, rows, autocast, beside):
+    """Left to the rule, the buffer is written beside fp32 products from the line on and in line everywhere else; the gradients are
+    those of the in-line write."""
+    from hot_amd import quant_matmul as qm
+    monkeypatch.setattr(qm, "OVERLAP_MIN_BYTES", 0)
+    monkeypatch.setattr(qm, "OVERLAP_MIN_MACS_FP32", 512 * 64 * 128)
+    taken = _watch_buffer_streams(qm, monkeypatch)
+    torch.manual_seed(4)
+    lin = qm.HQ_Linear(64, 128).to(gpu, dtype)
+    x0, gy = torch.randn(rows, 64, device=gpu).to(dtype), (torch.randn(rows, 128, device=gpu) * 1e-3).to(dtype)
+
+    def run(overlap):
+        monkeypatch.setattr(qm, "overlap_buffer_write", overlap)
+        fresh_args.sr_step = 0
+        lin.zero_grad(set_to_none=True)
+        x = x0.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+            y = lin(x)
+        y.backward(gy.to(y.dtype))
+        return x.grad, lin.weight.grad.clone(), lin.bias.grad.clone()
+
+    ref, got = run(False), run(None)
+    assert [t is not None for t in taken] == [False, beside]
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("gw_bits,act_bits", [(4, 8), (4, 4), (8, 4)])
 @pytest.mark.parametrize("path", ["luq", "low_rank"])
 def test_hq_linear_gw_widths_on_the_separate_gx_paths(gpu, fresh_args, path, gw_bits, act_bits):
