@@ -910,7 +910,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
   if (hq_job) {
     if (row_tensor) col_job_row_stat(gj, cfg->n_o);
     rc = hq_job_impl(hj, gy, L, O, cfg->n_o, cfg->gx_bits, cfg->gx_round, cfg->seed, HOT_STREAM_GX, cfg->gx_scale, ws + b.off_qg, b.ld_g, sg,
-                     gj.a.row_absmax, B > 1 ? 1 : gj.a.npart, B > 1 ? GS : 1, B);
+                     gj.a.row_absmax, gj.a.npart, 1, B);
     if (rc) return rc;
   }
   ColsumArgs sj;

@@ -39,11 +39,10 @@ __global__ void __launch_bounds__(CW) colwise_sawb_kernel(const ColArgs a) {
   colwise_body<T, N, PASS, ROUND, 1, SEL>(a, blockIdx.x, lds);
 }
 
-// Per-channel maxima and per-sample statistics: what the atomics of a statistics pass need zeroed
-__global__ void colwise_clear_kernel(float* colmax, int64_t ncolmax, float* gstat, int64_t ngstat) {
+// Per-channel maxima that the atomics of a statistics pass need zeroed
+__global__ void colwise_clear_kernel(float* colmax, int64_t ncolmax) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < ncolmax) colmax[i] = 0.f;
-  if (i < ngstat) gstat[i] = 0.f;
 }
 
 // ---- column sums ------------------------------------------------------------------
@@ -89,12 +88,11 @@ size_t colwise_workspace_bytes_impl(int64_t C) {
   return (size_t)round_up(C * 4 * COLMAX_COPIES, 256) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
 }
 
-// with sample groups: per-sample per-channel max | per-sample statistics | partial sums
-static size_t group_colmax_bytes(int64_t C, int groups) { return (size_t)round_up(C * 4 * (int64_t)groups, 256); }
-static size_t group_gstat_bytes(int groups) { return (size_t)round_up((int64_t)groups * GS * 4, 256); }
+// with sample groups: per-sample per-channel max | a statistic per workgroup
+static size_t colmax_bytes(int64_t C, int groups) { return (size_t)round_up(C * 4 * (groups > 1 ? (int64_t)groups : COLMAX_COPIES), 256); }
 size_t colwise_group_workspace_bytes_impl(int64_t C, int groups) {
   if (groups <= 1) return colwise_workspace_bytes_impl(C);
-  return group_colmax_bytes(C, groups) + group_gstat_bytes(groups) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
+  return colmax_bytes(C, groups) + (size_t)(2 * sizeof(double)) * COL_MAX_WGS;
 }
 
 // Token blocks per workgroup of the quantise pass (tb) and of an absmax statistics pass (tb0).
@@ -230,10 +228,8 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
   a.store4 = store4;
   uint8_t* ws = (uint8_t*)workspace;
   a.colmax = (float*)ws;
-  uint8_t* part = ws + (groups > 1 ? group_colmax_bytes(C, groups) + group_gstat_bytes(groups) : (size_t)round_up(C * 4 * COLMAX_COPIES, 256));
-  a.partial = (double*)part;
-  a.pmax = (float*)part;
-  if (groups > 1) a.gstat = (float*)(ws + group_colmax_bytes(C, groups));
+  a.partial = (double*)(ws + colmax_bytes(C, groups));
+  a.pmax = (float*)a.partial;
   a.rowmajor = rowmajor ? 1 : 0;
   a.groups = groups; a.NBs = a.NB / groups; a.Kpad = groups > 1 ? kpad_group : ld_out;
   a.scales_out = scales_out;
@@ -241,15 +237,23 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
   // grids: strips of channels x runs of token blocks, per sample group (a run never leaves its sample)
   const int elem = dtype == HOT_F32 ? 4 : 2;
   const ColPartition cp = col_partition(n, r, store4, scale_mode, C, a.NB, elem, groups > 1 ? 0 : want, keep_stat);
-  const int64_t gx = (C + CW - 1) / CW, runs = (a.NBs + cp.tb - 1) / cp.tb, runs0 = (a.NBs + cp.tb0 - 1) / cp.tb0;
+  const int64_t gx = (C + CW - 1) / CW, runs = (a.NBs + cp.tb - 1) / cp.tb;
+  int tb0 = cp.tb0;
+  int64_t runs0 = (a.NBs + tb0 - 1) / tb0;
   if (runs * groups > 65535 || gx * runs * groups > COL_MAX_WGS || gx * runs0 * groups > COL_MAX_WGS)
     return fail(HOT_ERR_UNSUPPORTED, "%s: grid %lld x %lld too large", who, (long long)gx, (long long)(runs * groups));
-  job.lds[0] = col_ring_bytes(cp.tb0 * n, elem);
+  const int64_t tall_gx = (C + 63) / 64, room = (int64_t)colmax_bytes(C, groups) / 4 + 3 * COL_MAX_WGS;
+  // (the tall statistics pass below: longer runs while it keeps 2048 waves, or 1024 to get below 32 arrays of maxima, which every
+  // workgroup of the quantise pass reads: us of the whole backward, runs of 64 rows / these: 12608 x 768 x 3072 INT8 89.7 / 88.1,
+  // 16383 x 512 x 512 fp32 69.1 / 67.5)
+  if (scale_mode == HOT_SCALE_ROW && groups == 1 && (runs0 > COLMAX_OWN || runs0 * C > room) && !keep_stat)
+    for (; runs0 > 32 && tall_gx * runs0 >= (runs0 > 128 ? 2048 : 4096); runs0 = (a.NBs + tb0 - 1) / tb0) tb0 *= 2;
+  job.lds[0] = col_ring_bytes(tb0 * n, elem);
   job.lds[1] = col_ring_bytes(cp.tb * n, elem) + (size_t)CW * (cp.tb * r + 4);
   if (job.lds[1] > 150 * 1024) return fail(HOT_ERR_UNSUPPORTED, "colwise: staging does not fit LDS");
   job.sel = pick_sel(a, n, as_short);
   a.gx = (uint32_t)gx;
-  job.tb[0] = cp.tb0; job.tb[1] = cp.tb;
+  job.tb[0] = tb0; job.tb[1] = cp.tb;
   job.runs[0] = (int)runs0; job.runs[1] = (int)runs;
   if (job.sel == COL_SHORT) {
     // 16 rows at a time (the partition takes whole groups of them)
@@ -259,26 +263,36 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
     a.NBs = (a.NBs + per - 1) / per;
     job.tb[0] /= per; job.tb[1] /= per;
   }
-  // per-sample statistics and the per-channel maxima of many runs are kept by atomics, everything else by workgroup.  The maxima of a
-  // few runs have the second half of the statistics for themselves (us of the whole backward, cleared and updated / own: 197 x 632 x 2048
-  // 24.7 / 21.9, 49 x 3072 x 768 fp32 26.5 / 24.5, 192 x 640 x 1400 25.3 / 21.9; more of them would be a long chain of loads for each reader).
-  a.ncolmax = COLMAX_COPIES;
-  if (scale_mode == HOT_SCALE_ROW && groups == 1 && runs0 <= COLMAX_OWN && runs0 * C <= 2 * COL_MAX_WGS) {
-    a.colmax = a.pmax + 2 * COL_MAX_WGS;
-    a.ncolmax = (int32_t)runs0;
-    a.colmax_own = 1;
+  // Per-channel maxima: every row of workgroups of the statistics pass has an array of its own, up to COLMAX_OWN of them (every
+  // workgroup of the quantise pass reads them all) and as far as they find room beside the row-wise maxima; where there are more
+  // runs a workgroup takes four of them and 64 channels (tall).  Else atomics update a few copies, which a launch clears.
+  // us of the whole backward, cleared and updated / own: 197 x 632 x 2048 24.7 / 21.9, 49 x 3072 x 768 fp32 26.5 / 24.5, 4096 x 768 x 768
+  // 27.4 / 24.6, 1505 x 1056 x 3200 38.8 / 36.0; tall: 12608 x 768 x 3072 INT8 92.0 / 88.1, 16383 x 512 x 512 fp32 75.2 / 67.5.
+  a.ncolmax = groups > 1 ? 1 : COLMAX_COPIES;
+  job.tall_gx = job.tall_gy = 0;
+  if (scale_mode == HOT_SCALE_ROW) {
+    const int64_t tall_gy = (runs0 + 3) / 4;
+    if (runs0 <= COLMAX_OWN && runs0 * groups * C <= room) {
+      a.ncolmax = (int32_t)runs0;
+      a.colmax_own = 1;
+    } else if (groups == 1 && tall_gy <= COLMAX_OWN && tall_gy * C <= room && tall_gx * tall_gy <= COL_MAX_WGS) {
+      a.ncolmax = (int32_t)tall_gy;
+      a.colmax_own = 1;
+      job.tall_gx = (uint32_t)tall_gx; job.tall_gy = (uint32_t)tall_gy;
+    }
   }
-  a.npart = (int32_t)(scale_mode == HOT_SCALE_SAWB ? gx * runs : gx * runs0);
+  a.npart = (int32_t)(scale_mode == HOT_SCALE_SAWB ? gx * runs : job.tall_gx ? (int64_t)job.tall_gx * job.tall_gy : gx * runs0);
   return HOT_OK;
 }
 
 void col_job_row_stat(ColJob& job, int n_o) {
   ColArgs& a = job.a;
   a.rs_n = n_o;
-  a.row_absmax = a.groups > 1 ? a.gstat + 1 : a.pmax + COL_MAX_WGS;
+  a.row_absmax = a.pmax + 3 * COL_MAX_WGS;
 }
 
 uint32_t col_job_blocks(const ColJob& job, int pass) {
+  if (pass == 0 && job.tall_gx) return (uint32_t)round_up((int64_t)job.tall_gx * job.tall_gy, 8);
   return (uint32_t)round_up((int64_t)job.a.gx * job.runs[pass] * job.a.groups, 8);
 }
 
@@ -286,16 +300,14 @@ ColArgs col_job_args(const ColJob& job, int pass) {
   ColArgs a = job.a;
   a.tb = job.tb[pass]; a.runs = job.runs[pass];
   a.gy = (uint32_t)(job.runs[pass] * a.groups);
+  if (pass == 0 && job.tall_gx) { a.tall = 1; a.gx = job.tall_gx; a.gy = job.tall_gy; }
   return a;
 }
 
 void col_job_clear(const ColJob& job, hipStream_t st) {
   const ColArgs& a = job.a;
-  const int64_t ncolmax = a.mode == HOT_SCALE_ROW ? (a.groups > 1 ? a.C * a.groups : a.colmax_own ? 0 : a.C * COLMAX_COPIES) : 0;
-  const int64_t ngstat = a.groups > 1 && (a.mode == HOT_SCALE_TENSOR || a.row_absmax) ? GS * (int64_t)a.groups : 0;
-  const int64_t n = ncolmax > ngstat ? ncolmax : ngstat;
-  if (n > 0)
-    hipLaunchKernelGGL(colwise_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.colmax, ncolmax, a.gstat, ngstat);
+  const int64_t n = a.mode == HOT_SCALE_ROW && !a.colmax_own ? a.C * a.ncolmax * a.groups : 0;
+  if (n > 0) hipLaunchKernelGGL(colwise_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.colmax, n);
 }
 
 template <typename T, int N, typename SEL>

@@ -12,10 +12,8 @@ namespace hot {
 
 constexpr int CW = 256;        // threads per workgroup = channels per workgroup
 constexpr int COLMAX_COPIES = 8;  // per-channel maxima: workgroup row y folds into copy y % 8 (fewer atomics per line) ...
-constexpr int COLMAX_OWN = 64;    // ... or, up to that many workgroup rows, each has a copy of its own: nothing to clear, a launch less
+constexpr int COLMAX_OWN = 64;    // ... or, up to that many workgroup rows (per sample), each has a copy of its own: nothing to clear, a launch less
 constexpr int CW_ROWS = 16;    // rows staged per step
-
-constexpr int GS = 32;   // floats between the statistics of two sample groups (one 128-byte line each)
 
 struct ColArgs {
   const void* in;
@@ -26,14 +24,15 @@ struct ColArgs {
   int64_t ld_out;     // bytes
   // Statistics of the whole tensor: every workgroup of the statistics pass leaves its own value (nothing to
   // clear beforehand, no updates queueing on one address) and every workgroup of the quantise pass reduces them.
-  float* pmax;        // TENSOR: absmax per workgroup, npart of them
+  float* pmax;        // TENSOR: absmax per workgroup, npart of them (per sample group)
   double* partial;    // SAWB: 2 doubles per workgroup, npart of them (per sample group)
   int32_t npart;
-  float* colmax;      // ROW: per-channel absmax, ncolmax arrays of C floats
-  int32_t ncolmax;    // COLMAX_COPIES of them, updated by atomics, or (own) one per run of token blocks of the statistics pass
+  float* colmax;      // ROW: per-channel absmax, ncolmax arrays of C floats per sample group
+  int32_t ncolmax;    // own: one per row of workgroups of the statistics pass; else updated by atomics, COLMAX_COPIES (sample groups: 1)
   int32_t colmax_own;
+  int32_t tall;       // statistics pass: a workgroup is 64 channels x four runs of token blocks, a run to a wave, instead of 256 channels x one
   float* scales_out;
-  float* row_absmax;  // statistics pass with RS: absmax of the row-wise block Hadamard, one per workgroup (sample groups: row_absmax[GS g])
+  float* row_absmax;  // statistics pass with RS: absmax of the row-wise block Hadamard, one per workgroup
   int32_t rs_n;       // ... its block along the channels (1, 2, 4, 8 or 16)
   float* colsum;      // statistics pass: NULL or per-channel sums of the input, one row of C floats per run of token blocks
   uint64_t seed;
@@ -44,12 +43,10 @@ struct ColArgs {
   // Sample groups (3-D activations: one step per sample).  The R rows are `groups` samples of NBs
   // token blocks each; a workgroup's run of blocks never leaves its sample (`runs` runs per sample),
   // the codes of a sample take Kpad bytes of every output row (the tail zeroed), and the statistics
-  // are kept per sample: gstat[GS g] (absmax, TENSOR) -- a 128-byte line per sample, since every workgroup of
-  // a sample updates its absmax and updates of one line queue up behind each other at the memory side --,
-  // colmax[g * C + c] (ROW).  groups == 1: the whole input is one group with Kpad = ld_out.
+  // are kept per sample: its workgroups are neighbours in pmax, and it has ncolmax arrays of maxima per channel.
+  // groups == 1: the whole input is one group with Kpad = ld_out.
   int32_t groups, runs;
   int64_t NBs, Kpad, Rs;  // Rs: rows per sample
-  float* gstat;
   // rowmajor: the codes are stored untransposed, [NB r, C] with ld_out bytes per coefficient row
   // (the A operand of a product whose K runs along the channels), instead of [C, NB r]
   int32_t rowmajor;
@@ -253,20 +250,23 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   const unsigned wg_id = by * a.gx + bx;     // the numbering the ordered reductions use
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t cg0 = (int64_t)bx * CW;
+  const bool tall = PASS == 0 && !SHORT && SAWB != 1 && a.tall;
+  const int64_t cg0 = (int64_t)bx * (tall ? 64 : CW);
+  const int64_t cw0 = tall ? cg0 : cg0 + 64 * wave;        // first channel of this wave
   // Fused row statistic: within each group of 16 lanes the channels are dealt out so that the four
   // stages of the 16-point row transform pair lanes at the distances a single DPP operand reaches
   // (channel bit 0 <-> lane xor 1, bit 1 <-> xor 2, bit 2 <-> xor 15, bit 3 <-> xor 8).
   constexpr bool RSP = PASS == 0 && RS;
   const int chan = RSP ? (tid ^ ((tid & 4) ? 0xB : 0)) : tid;   // channel of this thread within the workgroup
-  const int64_t c = cg0 + chan;
+  const int64_t c = cw0 + (chan & 63);
   const bool active = c < a.C;
   const int sample = a.groups > 1 ? (int)(by / (unsigned)a.runs) : 0;
-  const int run = (int)by - sample * a.runs;
+  const int run = tall ? (int)by * (CW / 64) + wave : (int)by - sample * a.runs;
   const int64_t blk_in = (int64_t)run * a.tb;                    // first block of the run within its sample
   const int64_t blk0 = (int64_t)sample * a.NBs + blk_in;
   const int64_t row0 = blk0 * N;
   int nblk = (int)((a.NBs - blk_in) < a.tb ? (a.NBs - blk_in) : a.tb);
+  if (tall && nblk < 0) nblk = 0;                          // (a wave past the last run: no steps, maxima of 0)
   const int nsteps = (nblk * N + CW_ROWS - 1) / CW_ROWS;
   // (short blocks: the last group of 16 rows may be cut short; what its missing rows deliver is not consumed)
   const int rows_wg = SHORT && a.Rs - blk_in * N < (int64_t)nblk * N ? (int)(a.Rs - blk_in * N) : nblk * N;
@@ -283,11 +283,11 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   {
     // channels of this wave that exist; a wave past the end streams the workgroup's first
     // channels instead (valid addresses, never consumed)
-    int64_t cw0 = cg0 + 64 * wave;
-    int64_t chans = a.C - cw0;
-    if (chans <= 0) { cw0 = cg0; chans = a.C - cg0; }
+    int64_t first = cw0;
+    int64_t chans = a.C - first;
+    if (chans <= 0) { first = cg0; chans = a.C - cg0; }
     if (chans > 64) chans = 64;
-    rs.base = reinterpret_cast<const uint8_t*>(a.in) + cw0 * (int64_t)sizeof(T);
+    rs.base = reinterpret_cast<const uint8_t*>(a.in) + first * (int64_t)sizeof(T);
     rs.nvec_row = (int)(chans * (int64_t)sizeof(T) / 16);
   }
 
@@ -335,31 +335,28 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
     } else if (a.mode == HOT_SCALE_ROW) {
       float cm = 0.f;
       if (active) {
-        if (a.groups > 1) {
-          cm = a.colmax[(int64_t)sample * a.C + c];
-        } else {
-          for (int k0 = 0; k0 < a.ncolmax; k0 += COLMAX_COPIES) {      // (that many loads under way at a time)
-            float v[COLMAX_COPIES];
+        const float* cmx = a.colmax + (int64_t)sample * a.ncolmax * a.C + c;
+        auto fold = [&](auto under_way) {                            // (that many loads at a time)
+          constexpr int W = decltype(under_way)::value;
+          for (int k0 = 0; k0 < a.ncolmax; k0 += W) {
+            float v[W];
 #pragma unroll
-            for (int k = 0; k < COLMAX_COPIES; ++k) v[k] = a.colmax[(k0 + k < a.ncolmax ? k0 + k : a.ncolmax - 1) * a.C + c];
+            for (int k = 0; k < W; ++k) v[k] = cmx[(k0 + k < a.ncolmax ? k0 + k : a.ncolmax - 1) * a.C];
 #pragma unroll
-            for (int k = 0; k < COLMAX_COPIES; ++k) cm = fmaxf(cm, v[k]);
+            for (int k = 0; k < W; ++k) cm = fmaxf(cm, v[k]);
           }
-        }
+        };
+        if (a.ncolmax <= 8) fold(std::integral_constant<int, 8>{});
+        else fold(std::integral_constant<int, 32>{});
       }
       const float sc = cm / (float)qmax;
       d = active ? sc + 1e-11f : 1.f;
       if (active && run == 0) a.scales_out[(int64_t)sample * a.C + c] = sc;
     } else {
-      float m;
-      if (a.groups > 1) {
-        m = a.gstat[GS * sample];
-      } else {
-        m = wave_max(part_max(a.pmax, a.npart, 1, tid));
-        if (lane == 0) s_max[wave] = m;
-        __syncthreads();
-        m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-      }
+      float m = wave_max(part_max(a.pmax + (int64_t)sample * a.npart, a.npart, 1, tid));
+      if (lane == 0) s_max[wave] = m;
+      __syncthreads();
+      m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
       const float sc = m / (float)qmax;
       d = sc + 1e-11f;
       if (bx == 0 && run == 0 && tid == 0) a.scales_out[sample] = sc;
@@ -661,7 +658,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
   }
 
   if constexpr (PASS == 0) {
-    if (a.colsum && active) a.colsum[(int64_t)by * a.C + c] = csum;
+    if (a.colsum && active && nblk > 0) a.colsum[(tall ? (int64_t)run : (int64_t)by) * a.C + c] = csum;
     if constexpr (RS) {
       // rows past the end of the input were redirected to real rows and channels past C form whole
       // inactive blocks, so only the latter need masking
@@ -671,15 +668,23 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       if (tid == 0) {
         float mm = s_max[0];
         for (int i = 1; i < CW / 64; ++i) mm = fmaxf(mm, s_max[i]);
-        if (a.groups > 1) atomic_max_nonneg(a.row_absmax + GS * sample, mm);
-        else a.row_absmax[wg_id] = mm;
+        a.row_absmax[wg_id] = mm;
       }
       __syncthreads();
     }
     if (a.mode == HOT_SCALE_ROW) {
+      if (tall) {
+        // the four runs meet in the ring, whose rows every wave has read
+        float* const s_cm = reinterpret_cast<float*>(lds);
+        __syncthreads();
+        s_cm[tid] = cmax;
+        __syncthreads();
+        if (wave == 0 && active) a.colmax[by * a.C + c] = fmaxf(fmaxf(cmax, s_cm[lane + 64]), fmaxf(s_cm[lane + 128], s_cm[lane + 192]));
+        return;
+      }
       if (active) {
-        if (a.groups > 1) atomic_max_nonneg(a.colmax + (int64_t)sample * a.C + c, cmax);
-        else if (a.colmax_own) a.colmax[by * a.C + c] = cmax;
+        if (a.colmax_own) a.colmax[by * a.C + c] = cmax;
+        else if (a.groups > 1) atomic_max_nonneg(a.colmax + (int64_t)sample * a.C + c, cmax);
         else atomic_max_nonneg(a.colmax + (by % COLMAX_COPIES) * a.C + c, cmax);
       }
       return;
@@ -691,8 +696,7 @@ __device__ __forceinline__ void colwise_body(const ColArgs& args, unsigned block
       if (tid == 0) {
         float mm = s_max[0];
         for (int i = 1; i < CW / 64; ++i) mm = fmaxf(mm, s_max[i]);
-        if (a.groups > 1) atomic_max_nonneg(a.gstat + GS * sample, mm);
-        else a.pmax[wg_id] = mm;
+        a.pmax[wg_id] = mm;
       }
       return;
     }

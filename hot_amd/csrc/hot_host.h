@@ -39,7 +39,7 @@ int hq_rowwise_impl(const void* in, int dtype, int64_t M, int64_t K, int n, int 
 // reads), and the workspace takes 128 bytes per sample.
 
 // The row-wise quantiser (blocks of up to 16; per-row steps: K <= HQ_ROW_MAX_K) as a job of a quantise phase (phase.h).
-// stat: nstat absmax values stat_stride floats apart; with groups > 1 one per sample, stat_stride apart, and scales_out [M].
+// stat: nstat absmax values stat_stride floats apart; with groups > 1 that many per sample, one sample after the other, and scales_out [M].
 struct HqArgs;
 int hq_job_impl(HqArgs& a, const void* in, int64_t M, int64_t K, int n, int bits, int rounding, uint64_t seed, uint32_t rng_stream,
                 int scale_mode, void* codes_out, int64_t ld_codes, float* scales_out, const float* stat, int nstat, int stat_stride,

@@ -120,7 +120,7 @@ struct HqArgs {
   uint32_t wgs;           // workgroups per sample
   int64_t rows;           // per sample
   int32_t n, bits, rounding, per_row, groups;
-  const float* stat;      // absmax: nstat values stat_stride floats apart (per sample: one, at stat[GS g])
+  const float* stat;      // absmax: nstat values stat_stride floats apart (per sample, those of one after the other)
   int32_t nstat, stat_stride;
   uint64_t seed;
   uint32_t stream;
@@ -239,15 +239,10 @@ __device__ __forceinline__ void hq_body(const HqArgs& a, unsigned block) {
     const uint32_t ch = c0 + u * 256u;
     raw[u] = load_raw<T>(in + (int64_t)(ch < a.chunks ? ch : a.chunks - 1) * EPL);   // (the last chunk again past the end: never stored)
   }
-  float m = 0.f;
-  if (a.groups > 1) {
-    m = a.stat[(int64_t)g * a.stat_stride];
-  } else {
-    m = wave_max(part_max(a.stat, a.nstat, a.stat_stride, tid));
-    if (lane == 0) s_red[tid >> 6] = m;
-    __syncthreads();
-    m = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-  }
+  float m = wave_max(part_max(a.stat + (int64_t)g * a.nstat * a.stat_stride, a.nstat, a.stat_stride, tid));
+  if (lane == 0) s_red[tid >> 6] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
   const float s = m / (float)((1 << (a.bits - 1)) - 1);
   const float d = s + 1e-11f, rcp = 1.0f / d;
   if (a.groups == 1 && b == 0 && tid == 0) a.scales[0] = s;

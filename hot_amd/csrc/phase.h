@@ -71,6 +71,7 @@ struct ColJob {
   ColSel sel;
   int tb[2], runs[2];
   size_t lds[2];
+  uint32_t tall_gx, tall_gy;   // grid of the statistics pass in its tall form, else 0
 };
 // Fills a job (blocks of up to 128 rows) and checks everything a pass would refuse.  as_short: for the w slot of a
 // phase (blocks of up to 16 rows).

@@ -115,7 +115,9 @@ def test_backward_matches_oracle(gpu, dtype, shape, variant):
     (16 * 67, 32, 16),   # enough runs of sixteen tokens that some workgroups take several
     (3001, 144, 16),     # blocks of one token, many of them: the last run of nine rows
     (1023, 32, 16),      # 64 runs: with a step per channel each has maxima of its own
-    (1025, 32, 16),      # 65: they share eight copies
+    (1025, 32, 16),      # 65: a workgroup takes four of them, the last one a single run
+    (4163, 80, 16),      # 66 runs of 64 tokens, the last of three, a second strip of sixteen channels
+    (16411, 16, 16),     # 257 runs: eight copies that the workgroups share
     (1023, 2064, 8),     # 64 runs of more channels than there is room for
 ])
 def test_backward_small_grids(gpu, L, O, I, dtype, variant):
@@ -125,6 +127,20 @@ def test_backward_small_grids(gpu, L, O, I, dtype, variant):
     ocfg, opt = both_configs(L, max_block=128, **variant)
     gx, gw, tr = run_both(x, w, gy, ocfg, opt, gpu)
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dtype)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dtype))
+
+
+@pytest.mark.parametrize("L", [4096 + 16, 4163, 16411])
+def test_bias_gradient_of_many_runs(gpu, L):
+    """A step per channel and the bias gradient from one statistics pass of more than 64 runs of token blocks: every run leaves its own
+    partial sum (integers below 2^24: any order gives the same sum), and no other bytes change."""
+    from hot_amd import ops
+    x, w, _ = make_case(L, 80, 16, seed=L)
+    gy = torch.randint(-50, 51, (L, 80), generator=torch.Generator().manual_seed(L)).float()
+    _, opt = both_configs(L, max_block=128, gx_scale=orc.SCALE_ROW, gw_scale=orc.SCALE_ROW)
+    xq, sx = ops.abc_forward(x.to(gpu), opt)
+    gx, gw, gb = ops.linear_backward(gy.to(gpu), w.to(gpu), xq, sx, opt, bias_grad=True)
+    gx1, gw1 = ops.linear_backward(gy.to(gpu), w.to(gpu), xq, sx, opt)
+    assert torch.equal(gb.cpu(), gy.sum(0)) and torch.equal(gx, gx1) and torch.equal(gw, gw1)
 
 
 @pytest.mark.parametrize("variant", [dict(), dict(gw_scale=orc.SCALE_ROW, gx_bits=8, w_bits=8)])
