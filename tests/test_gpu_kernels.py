@@ -61,6 +61,19 @@ def test_hq_rowwise_widths(gpu, K, scale):
     assert np.array_equal(np_codes(codes, 4, K), q_ref)
 
 
+@pytest.mark.parametrize("chunks", [1, 1024, 1025, 512 * 1024, 512 * 1024 + 1, 4 * 512 * 1024 + 3])
+def test_hq_rowwise_absmax_grid(gpu, chunks):
+    """One step per tensor at the edges of the absmax pass: one workgroup of 1024 chunks, all 512 of them, a chunk of a second load and of a
+    second sweep.  The largest value stands in the last chunk, on a dirty workspace of the allocator."""
+    from hot_amd import ops
+    g = torch.Generator().manual_seed(chunks)
+    x = torch.rand(chunks, 8, generator=g) - 0.5
+    x[-1, -1] = 100.0
+    codes, s = ops.hq_rowwise(x.to(gpu), n=8, bits=8, scale="tensor")
+    q_ref, s_ref = orc.quant(orc.fwht_blocks_last(x.numpy(), 8), 8, orc.SCALE_TENSOR)
+    assert np.array_equal(s.cpu().numpy(), s_ref) and np.array_equal(np_codes(codes, 8, 8), q_ref)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("scale", ["tensor", "row"])
