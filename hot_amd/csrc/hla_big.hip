@@ -168,57 +168,64 @@ __device__ __forceinline__ uint32_t bits_of(uint64_t e, uint64_t seed, uint32_t 
   return sr_bits_of(sr_octet_words(e >> 3, seed, stream), (uint32_t)e);
 }
 
-// blockIdx.y = block * nk + (index of k among the needed coefficients)
+// Item = block * nk + (index of k among the needed coefficients).  A workgroup of the statistics pass takes `per` consecutive items,
+// as many as make 32 loads of a thread where that leaves two workgroups per CU (items_per): with one item of a block of 256 tokens it
+// was four loads and an update per channel, and the updates of one channel queue up at the memory side (21760 x 232, a step per
+// channel: 68 us of a 190 us backward).
+template <int M> constexpr int items_most() { return M >= 32 ? 1 : 32 / M; }
+int items_per(int m, int64_t C, int64_t items) {
+  int per = m >= 32 ? 1 : 32 / m;
+  while (per > 1 && (C + BT - 1) / BT * ((items + per - 1) / per) < 512) --per;
+  return per;
+}
 template <int M, int PASS, int ROUND, bool SAWB>
-__global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
+__global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a, int per) {
   __shared__ float s_max[BT / 64];
   __shared__ double s_sum[2][BT / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t c = (int64_t)blockIdx.x * BT + tid;
   const bool active = c < a.C;
-  const int64_t blk = blockIdx.y / a.nk;
-  const int kc = (int)(blockIdx.y - blk * a.nk);
-  const int k = a.klist[kc];
   const int qmax = (1 << (a.bits - 1)) - 1;
-  // The table entries of this coefficient index (one per run) go through LDS: read from global memory
-  // inside the quantise loop they would sit between the loop's byte stores, and every such load then
-  // waits for the store before it (one memory round trip per kept row).
-  __shared__ int32_t s_tab[PASS == 1 ? M : 1];
-  if constexpr (PASS == 1) {
-    if (tid < M) s_tab[tid] = a.tab[tid * 64 + k];
-    __syncthreads();
-  } else if (a.row_part && blockIdx.x == 0 && blockIdx.y == 0) {
-    const float m = wave_max(part_max(a.row_part, (int)a.row_nparts, 1, tid));
-    if (lane == 0) s_max[wave] = m;
-    __syncthreads();
-    if (tid == 0) a.row_absmax[0] = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-    __syncthreads();
-  }
-  float v[M];
-  if (active) {
-    const float* t = a.T + ((blk * M) * a.nk + kc) * a.C + c;
-#pragma unroll
-    for (int j = 0; j < M; ++j) v[j] = t[(int64_t)j * a.nk * a.C];
-  } else {
-#pragma unroll
-    for (int j = 0; j < M; ++j) v[j] = 0.f;
-  }
-  fwht<M>(v);
-  // every coefficient is complete here: without this the compiler sinks the last butterfly stage into
-  // the conditional code below and holds both stages' registers (a third more than the block itself)
-  if constexpr (PASS == 1 || SAWB) {
-#pragma unroll
-    for (int j = 0; j < M; ++j) asm volatile("" : "+v"(v[j]));
-  }
-
   if constexpr (PASS == 0) {
+    if (a.row_part && blockIdx.x == 0 && blockIdx.y == 0) {
+      const float m = wave_max(part_max(a.row_part, (int)a.row_nparts, 1, tid));
+      if (lane == 0) s_max[wave] = m;
+      __syncthreads();
+      if (tid == 0) a.row_absmax[0] = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
+      __syncthreads();
+    }
+    constexpr int ITEMS = items_most<M>();
+    const uint32_t item0 = blockIdx.y * per, items = (uint32_t)(a.NB * a.nk);
+    const uint32_t mine = items - item0 < (uint32_t)per ? items - item0 : (uint32_t)per;
+    const float* const tc = a.T + (active ? c : 0);          // (what a lane without a channel reads is never used)
+    float v[ITEMS][M];
+#pragma unroll
+    for (int u = 0; u < ITEMS; ++u) {
+      if ((uint32_t)u >= mine) break;
+      const uint32_t blk = (item0 + u) / (uint32_t)a.nk, kc = item0 + u - blk * (uint32_t)a.nk;
+      const float* t = tc + ((int64_t)blk * M * a.nk + kc) * a.C;
+#pragma unroll
+      for (int j = 0; j < M; ++j) v[u][j] = t[(int64_t)j * a.nk * a.C];
+    }
     float cmax = 0.f;
     double ssq = 0.0, sab = 0.0;
 #pragma unroll
-    for (int j = 0; j < M; ++j) {
-      if ((a.keep[kc][j >> 5] >> (j & 31)) & 1u) {
-        cmax = fmaxf(cmax, fabsf(v[j]));
-        if constexpr (SAWB) { ssq += (double)v[j] * (double)v[j]; sab += (double)fabsf(v[j]); }
+    for (int u = 0; u < ITEMS; ++u) {
+      if ((uint32_t)u >= mine) break;
+      const uint32_t kc = (item0 + u) % (uint32_t)a.nk;
+      fwht<M>(v[u]);
+      // every coefficient is complete here: without this the compiler sinks the last butterfly stage into
+      // the conditional code below and holds both stages' registers (a third more than the block itself)
+      if constexpr (SAWB) {
+#pragma unroll
+        for (int j = 0; j < M; ++j) asm volatile("" : "+v"(v[u][j]));
+      }
+#pragma unroll
+      for (int j = 0; j < M; ++j) {
+        if ((a.keep[kc][j >> 5] >> (j & 31)) & 1u) {
+          cmax = fmaxf(cmax, fabsf(v[u][j]));
+          if constexpr (SAWB) { ssq += (double)v[u][j] * (double)v[u][j]; sab += (double)fabsf(v[u][j]); }
+        }
       }
     }
     if (a.mode == HOT_SCALE_ROW) {
@@ -248,7 +255,24 @@ __global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
       a.partial[2 * wg + 1] = b;
     }
   } else {
+    const int64_t blk = blockIdx.y / a.nk;
+    const int kc = (int)(blockIdx.y - blk * a.nk);
+    const int k = a.klist[kc];
+    // The table entries of this coefficient index (one per run) go through LDS: read from global memory
+    // inside the quantise loop they would sit between the loop's byte stores, and every such load then
+    // waits for the store before it (one memory round trip per kept row).
+    __shared__ int32_t s_tab[M];
+    if (tid < M) s_tab[tid] = a.tab[tid * 64 + k];
+    __syncthreads();
     if (!active) return;
+    float v[M];
+    const float* t = a.T + ((blk * M) * a.nk + kc) * a.C + c;
+#pragma unroll
+    for (int j = 0; j < M; ++j) v[j] = t[(int64_t)j * a.nk * a.C];
+    fwht<M>(v);
+    // (complete here, as above)
+#pragma unroll
+    for (int j = 0; j < M; ++j) asm volatile("" : "+v"(v[j]));
     float d, clip = 0.f;
     if (a.mode == HOT_SCALE_ROW) d = a.colmax[c] / (float)qmax + 1e-11f;
     else if (a.mode == HOT_SCALE_TENSOR) d = a.stat[0] / (float)qmax + 1e-11f;
@@ -282,22 +306,24 @@ __global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
 // in LDS as [channel][run] and leave K-major, straight into the GEMM operand.  No [K, C]
 // intermediate with its 64-byte stores, no transpose kernel.  The workgroup of a block's last
 // index group also clears the row padding behind the last block.
+// A wave takes `per` indices, as many as make 32 loads of a thread where that leaves two workgroups per CU (launch_runs): in blocks of
+// 256 tokens one index is four rows, and workgroups of four indices wrote 16 bytes of a line each (21760 x 912 bf16: 28 us).
 constexpr int KG = 4;
 template <int M, int ROUND, bool SAWB>
-__global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigArgs a, int8_t* __restrict__ out, int64_t ld_out, int groups) {
-  __shared__ __align__(16) uint8_t img[64][KG * M + 16];
+__global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigArgs a, int8_t* __restrict__ out, int64_t ld_out, int groups, int per) {
+  constexpr int MOST = items_most<M>();
+  __shared__ __align__(16) uint8_t img[64][KG * MOST * M + 16];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t c0 = (int64_t)blockIdx.x * 64, c = c0 + lane;
   const bool active = c < a.C;
   const int64_t blk = blockIdx.y / groups;
   const int grp = (int)(blockIdx.y - blk * groups);
-  const int kc = grp * KG + wave;                      // this wave's needed coefficient index
-  const bool has_k = kc < a.nk;
+  const int kc0 = grp * KG * per;                      // the workgroup's first needed coefficient index; wave w takes kc0 + KG u + w
   const int qmax = (1 << (a.bits - 1)) - 1;
   // the workgroup's K run within the block: the outputs of its coefficient indices, in list order
-  const int k_hi = (grp + 1) * KG < a.nk ? (grp + 1) * KG : a.nk;
-  const int run0 = a.kbase[grp * KG], run_len = a.kbase[k_hi] - run0;
+  const int k_hi = kc0 + KG * per < a.nk ? kc0 + KG * per : a.nk;
+  const int run0 = a.kbase[kc0], run_len = a.kbase[k_hi] - run0;
   // absmax steps come straight from the statistic (no finalize kernel in between); the workgroups of
   // the first block and index group publish them
   float d = 1.f, clip = 0.f;
@@ -314,21 +340,25 @@ __global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigAr
     clip = a.stat[2];
   }
   const float rcp = 1.0f / d;
-  if (has_k) {
-    float v[M];
-    if (active) {
-      const float* t = a.T + ((blk * M) * a.nk + kc) * a.C + c;
+  float v[MOST][M];
 #pragma unroll
-      for (int j = 0; j < M; ++j) v[j] = t[(int64_t)j * a.nk * a.C];
-    } else {
+  for (int u = 0; u < MOST; ++u) {
+    const int kc = kc0 + KG * u + wave;
+    if (u < per && kc < k_hi) {
+      const float* t = a.T + ((blk * M) * a.nk + kc) * a.C + (active ? c : 0);      // (what a lane without a channel reads is never used)
 #pragma unroll
-      for (int j = 0; j < M; ++j) v[j] = 0.f;
+      for (int j = 0; j < M; ++j) v[u][j] = t[(int64_t)j * a.nk * a.C];
     }
-    fwht<M>(v);
+  }
+#pragma unroll
+  for (int u = 0; u < MOST; ++u) {
+    const int kc = kc0 + KG * u + wave;
+    if (u >= per || kc >= k_hi) break;
+    fwht<M>(v[u]);
     // every coefficient is complete here: without this the compiler sinks the last butterfly stage into
     // the conditional code below and holds both stages' registers (a third more than the block itself)
 #pragma unroll
-    for (int j = 0; j < M; ++j) asm volatile("" : "+v"(v[j]));
+    for (int j = 0; j < M; ++j) asm volatile("" : "+v"(v[u][j]));
     // which runs keep this coefficient index: a bit mask in the kernel arguments, the same for every
     // lane of the wave, so the walk below branches on scalar registers and a kept coefficient's place
     // in the run is a running count (the list is run-major: this index's outputs are neighbours)
@@ -340,7 +370,7 @@ __global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigAr
 #pragma unroll
     for (int j = 0; j < M; ++j) {
       if (!((kw[j >> 5] >> (j & 31)) & 1u)) continue;
-      float x = v[j];
+      float x = v[u][j];
       if constexpr (SAWB) x = fminf(fmaxf(x, -clip), clip);
       int q;
       if constexpr (ROUND == HOT_ROUND_NEAREST) {
@@ -389,15 +419,18 @@ __global__ void __launch_bounds__(64 * KG, 2) big_stage2_runs_kernel(const BigAr
 
 template <int M>
 int launch_runs(const BigArgs& a, void* out, int64_t ld_out, hipStream_t st) {
-  const int groups = (a.nk + KG - 1) / KG;
+  int per = items_most<M>();
+  while (per > 1 && (a.C + 63) / 64 * a.NB * ((a.nk + KG * per - 1) / (KG * per)) < 512) --per;
+  const int groups = (a.nk + KG * per - 1) / (KG * per);
+  per = (a.nk + KG * groups - 1) / (KG * groups);      // (even groups)
   const dim3 grid((unsigned)((a.C + 63) / 64), (unsigned)(a.NB * groups));
   const bool sawb = a.mode == HOT_SCALE_SAWB, stoch = a.rounding == HOT_ROUND_STOCH;
   if (stoch) {
-    if (sawb) hipLaunchKernelGGL((big_stage2_runs_kernel<M, 1, true>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups);
-    else hipLaunchKernelGGL((big_stage2_runs_kernel<M, 1, false>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups);
+    if (sawb) hipLaunchKernelGGL((big_stage2_runs_kernel<M, 1, true>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups, per);
+    else hipLaunchKernelGGL((big_stage2_runs_kernel<M, 1, false>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups, per);
   } else {
-    if (sawb) hipLaunchKernelGGL((big_stage2_runs_kernel<M, 0, true>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups);
-    else hipLaunchKernelGGL((big_stage2_runs_kernel<M, 0, false>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups);
+    if (sawb) hipLaunchKernelGGL((big_stage2_runs_kernel<M, 0, true>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups, per);
+    else hipLaunchKernelGGL((big_stage2_runs_kernel<M, 0, false>), grid, dim3(64 * KG), 0, st, a, (int8_t*)out, ld_out, groups, per);
   }
   return check_launch("big_stage2_runs_kernel");
 }
@@ -510,7 +543,14 @@ __global__ void __launch_bounds__(256) big_finalize_kernel(const BigArgs a, int6
     return;
   }
   double q = 0.0, b = 0.0;
-  for (int64_t i = tid; i < nwg; i += 256) { q += a.partial[2 * i]; b += a.partial[2 * i + 1]; }
+  // (one after the other, sixteen loads under way: with one at a time the sums of 12544 x 3072 took 45 of the call's 131 us)
+  for (int64_t i0 = tid; i0 < nwg; i0 += 16 * 256) {
+    double2 v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = i0 + u * 256 < nwg ? reinterpret_cast<const double2*>(a.partial)[i0 + u * 256] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) { q += v[u].x; b += v[u].y; }
+  }
   s_q[tid] = q; s_b[tid] = b;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
@@ -662,16 +702,19 @@ int build_row_table(int32_t* tab, int n, const int32_t* rows, int r, uint64_t* k
 
 template <int M>
 int launch_stage2(const BigArgs& a, dim3 grid, int pass, hipStream_t st) {
+  int per = 1;
   const bool sawb = a.mode == HOT_SCALE_SAWB, stoch = a.rounding == HOT_ROUND_STOCH;
   if (pass == 0) {
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, true>), grid, dim3(BT), 0, st, a);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, false>), grid, dim3(BT), 0, st, a);
+    per = items_per(M, a.C, a.NB * a.nk);
+    grid.y = (grid.y + per - 1) / per;
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, true>), grid, dim3(BT), 0, st, a, per);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, false>), grid, dim3(BT), 0, st, a, per);
   } else if (stoch) {
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, true>), grid, dim3(BT), 0, st, a);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, false>), grid, dim3(BT), 0, st, a);
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, true>), grid, dim3(BT), 0, st, a, per);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, false>), grid, dim3(BT), 0, st, a, per);
   } else {
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, true>), grid, dim3(BT), 0, st, a);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, false>), grid, dim3(BT), 0, st, a);
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, true>), grid, dim3(BT), 0, st, a, per);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, false>), grid, dim3(BT), 0, st, a, per);
   }
   return check_launch("big_stage2_kernel");
 }
@@ -813,7 +856,7 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
   if (int rc = dispatch_stage2(m, a, g2, 0, st)) return rc;
   // (with absmax steps the run-major quantise pass reads the statistic itself and publishes the steps)
   if (!(run_major && scale_mode != HOT_SCALE_SAWB))
-    hipLaunchKernelGGL(big_finalize_kernel, dim3(1), dim3(256), 0, st, a, (int64_t)gx * NB * a.nk, kout);
+    hipLaunchKernelGGL(big_finalize_kernel, dim3(1), dim3(256), 0, st, a, gx * ((NB * a.nk + items_per(m, C, NB * a.nk) - 1) / items_per(m, C, NB * a.nk)), kout);
   if (rowmajor) {
     // untransposed [NB r, C]: the quantise pass writes the destination itself (INT8), or its [Kout, C]
     // scratch, which a second kernel packs two channels to a byte

@@ -287,6 +287,30 @@ def test_llama_shapes_properties(gpu, shape):
     assert float((gw8 - ref_gw).norm() / ref_gw.norm()) < 0.03
 
 
+@pytest.mark.parametrize("L,C", [(256 * 13, 2568), (512 * 27, 264), (1024 * 11, 528), (256, 8)])
+@pytest.mark.parametrize("scale", [orc.SCALE_TENSOR, orc.SCALE_SAWB, orc.SCALE_ROW])
+def test_large_blocks_many_items(gpu, L, C, scale):
+    """Blocks above 128 tokens where a workgroup takes several (block, coefficient) items in both passes of stage 2, the last one fewer;
+    and the smallest problem, where it takes one.  Run-major rows; codes and steps are the oracle's."""
+    from hot_amd import ops
+    from hot_amd.hadamard_matmul import run_major
+    n, rows = orc.hla_rows(L)
+    assert n == L & -L and n > 128
+    rows = tuple(int(v) for v in run_major(rows))
+    x = torch.randn(L, C, generator=torch.Generator().manual_seed(L + C))
+    if scale == orc.SCALE_ROW:
+        q, s, lp = ops.hla_tokenwise(x.to(gpu), n, rows, bits=8, rounding="nearest", scale="row")
+        xp = orc.fwht_blocks_first(x.numpy(), n, np.asarray(rows))
+        q_ref, s_ref = orc.quant(np.ascontiguousarray(xp.T), 8, orc.SCALE_ROW)
+    else:
+        q, s = ops.abc_forward(x.to(gpu), ops.HotOptions(n_o=16, hla_n=n, hla_rows=rows, act_scale=scale))
+        q_ref, s_ref = orc.abc_forward(x.numpy(), orc.HotConfig(n_o=16, hla_n=n, hla_rows=rows, act_scale=scale))
+        q_ref = q_ref.T
+    assert np.array_equal(s.cpu().numpy().ravel(), np.asarray(s_ref).ravel())
+    q = q.cpu().numpy()
+    assert np.array_equal(q[:, :q_ref.shape[1]], q_ref) and not q[:, q_ref.shape[1]:].any()
+
+
 def test_hlq_backward_op_surface(gpu):
     """HLQ_backward.backward(Go, W, X, 0, 0, 16, per_token) -> (gx, gw, 4 floats)."""
     from hot_amd import HLQ_backward
