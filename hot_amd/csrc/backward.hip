@@ -126,6 +126,13 @@ static const int32_t* identity_rows() {
   return rows.v;
 }
 
+// The job that adds up the partial column sums of g_y: as many rows as the statistics pass writes, which the workspace has room for.
+static int colsum_args(ColsumArgs& s, const float* partial, int64_t O, int64_t strips, int64_t room, void* out, int out_dtype, const char* who) {
+  if (strips > room) return fail(HOT_ERR_WORKSPACE, "%s: %lld rows of partial column sums, room for %lld", who, (long long)strips, (long long)room);
+  s.partial = partial; s.C = O; s.out = out; s.out_dtype = out_dtype; s.strips = (int32_t)strips;
+  return HOT_OK;
+}
+
 // Whether W's job shares the launches of a phase (Hadamard blocks of up to 16; with stochastic rounding of 16).
 static bool w_joins_phase(const hot_config* c) { return c->w_round == HOT_ROUND_STOCH ? c->n_o == CW_ROWS : c->n_o <= CW_ROWS; }
 
@@ -363,8 +370,8 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   }
   ColsumArgs sj;
   if (gb) {
-    sj.partial = (const float*)(ws + b.off_colsum); sj.C = O; sj.out = gb; sj.out_dtype = out_dtype;
-    sj.strips = (int32_t)colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, dtype == HOT_F32 ? 4 : 2);
+    const int64_t strips = big ? colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, elem) : col_job_strips(gj);
+    if (int e = colsum_args(sj, (const float*)(ws + b.off_colsum), O, strips, b.colsum_strips, gb, out_dtype, who)) return e;
   }
 
   // statistics
@@ -797,6 +804,7 @@ int hot_gw_luq(const void* gy, int dtype, const void* xq, const float* sx, int64
 
 struct BatchedLayout {
   int64_t ld_g, ld_w, kg, ld_gp;
+  int64_t colsum_strips;                         // as in BwdLayout
   size_t off_colw, off_colg, off_hq, off_sg, off_sw, off_sgp, off_qg, off_qw, off_qgp, off_part, part_bytes, off_colsum, total;
 };
 
@@ -824,7 +832,8 @@ static BatchedLayout batched_layout(int64_t B, int64_t T, int64_t O, int64_t I, 
   // partial column sums of g_y (bias gradient); the query knows no input type: room for either element size
   const int64_t s2 = colsum_strips_impl(L, O, c->hla_n, c->hla_r, 0, c->gw_scale, 2, B);
   const int64_t s4 = colsum_strips_impl(L, O, c->hla_n, c->hla_r, 0, c->gw_scale, 4, B);
-  b.off_colsum = o; o += align256((size_t)(s2 > s4 ? s2 : s4) * (size_t)O * 4);
+  b.colsum_strips = s2 > s4 ? s2 : s4;
+  b.off_colsum = o; o += align256((size_t)b.colsum_strips * (size_t)O * 4);
   b.total = o;
   return b;
 }
@@ -904,7 +913,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
                         1, 0, false, w_short);
   if (!rc) rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
                              HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg,
-                             colwise_group_workspace_bytes_impl(O, (int)B), who, (int)B, b.kg, false, false);
+                             colwise_group_workspace_bytes_impl(O, (int)B), who, (int)B, b.kg, false, false, 0, gb != nullptr);
   if (rc) return rc;
   HqArgs hj;
   if (hq_job) {
@@ -916,8 +925,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
   ColsumArgs sj;
   if (gb) {
     gj.a.colsum = (float*)(ws + b.off_colsum);
-    sj.partial = gj.a.colsum; sj.C = O; sj.out = gb; sj.out_dtype = out_dtype;
-    sj.strips = (int32_t)colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, dtype == HOT_F32 ? 4 : 2, B);
+    if ((rc = colsum_args(sj, gj.a.colsum, O, col_job_strips(gj), b.colsum_strips, gb, out_dtype, who))) return rc;
   }
   col_job_clear(gj, st);
   rc = phase_launch(0, dtype, &gj, w_short ? &wj : nullptr, nullptr, nullptr, st);

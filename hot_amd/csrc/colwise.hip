@@ -291,6 +291,8 @@ void col_job_row_stat(ColJob& job, int n_o) {
   a.row_absmax = a.pmax + 3 * COL_MAX_WGS;
 }
 
+int64_t col_job_strips(const ColJob& job) { return (int64_t)job.runs[0] * job.a.groups; }
+
 uint32_t col_job_blocks(const ColJob& job, int pass) {
   if (pass == 0 && job.tall_gx) return (uint32_t)round_up((int64_t)job.tall_gx * job.tall_gy, 8);
   return (uint32_t)round_up((int64_t)job.a.gx * job.runs[pass] * job.a.groups, 8);

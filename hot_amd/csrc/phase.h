@@ -86,6 +86,8 @@ int64_t col_jobs_want(int64_t workgroups);
 int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes);
 // The statistics pass also delivers the absmax of the row-wise Hadamard of blocks of n_o (1 .. 16) of the same input.
 void col_job_row_stat(ColJob& job, int n_o);
+// Rows of partial column sums that its statistics pass writes (a.colsum): one per run of token blocks.
+int64_t col_job_strips(const ColJob& job);
 // Zeroes what the statistics pass updates by atomics (nothing for most jobs).
 void col_job_clear(const ColJob& job, hipStream_t st);
 ColArgs col_job_args(const ColJob& job, int pass);

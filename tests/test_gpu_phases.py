@@ -236,6 +236,29 @@ def test_batched_bias_gradient(gpu, dt, B, T, O, variant):
     assert torch.equal(gb.cpu(), gi.double().reshape(-1, O).sum(0).float())
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T,O", [(8191, 2064), (12608, 3072), (16384, 768)])
+def test_bias_gradient_of_one_long_sample(gpu, dt, T, O):
+    """One sample with a step per channel and so many runs of token blocks that the statistics pass would rather take longer ones: the
+    bias gradient adds up the rows that this call wrote, in both entry points.  NaN wherever the call has not written; integers, of
+    which every order gives the exact sum."""
+    from hot_amd import ops
+    n, rows = orc.hla_rows(min(T & -T, 64))
+    opt = ops.HotOptions(n_o=16, hla_n=n, hla_rows=tuple(int(v) for v in rows), gx_scale="row", gw_scale="row")
+    g = torch.Generator(device=gpu).manual_seed(T)
+    gy = torch.randint(-8, 9, (1, T, O), generator=g, device=gpu).to(dt)
+    w, x = torch.rand(O, 16, generator=g, device=gpu).to(dt), torch.randn(1, T, 16, generator=g, device=gpu).to(dt)
+    ref = gy[0].double().sum(0).float()
+    ws = torch.empty(1 << 28, dtype=torch.uint8, device=gpu)
+    for back, buf, v in ((ops.linear_backward_batched, ops.abc_forward_batched, gy), (ops.linear_backward, lambda t, o: ops.abc_forward(t[0], o), gy[0])):
+        xq, sx = buf(x, opt)
+        ws.view(torch.float32).fill_(float("nan"))
+        gx, gw, gb = back(v, w, xq, sx, opt, out_dtype=torch.float32, workspace=ws, bias_grad=True)
+        assert torch.equal(gb, ref)
+        gx0, gw0 = back(v, w, xq, sx, opt, out_dtype=torch.float32, workspace=ws)      # (this one takes the longer runs)
+        assert torch.equal(gx, gx0) and torch.equal(gw, gw0)
+
+
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("O", [96, 100])
 def test_layer_bias_gradient_per_sample(gpu, fresh_args, dt, O):
