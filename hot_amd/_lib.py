@@ -26,7 +26,7 @@ STREAM_GX, STREAM_GW, STREAM_W, STREAM_ACT = 0, 1, 2, 3
 HOT_STATIC_MAX_CHANNELS = 16384
 
 EXPORTS = (
-    "hot_last_error", "hot_abi_version", "hot_backward_streams", "hot_backward_products", "hot_backward_pair_rows", "hot_kpad", "hot_hq_rowwise", "hot_hla_tokenwise",
+    "hot_last_error", "hot_abi_version", "hot_backward_streams", "hot_backward_products", "hot_backward_pair_rows", "hot_backward_gy_runs", "hot_kpad", "hot_hq_rowwise", "hot_hla_tokenwise",
     "hot_wq_colwise", "hot_colwise_workspace_bytes", "hot_gemm_i8", "hot_abc_workspace_bytes",
     "hot_abc_forward", "hot_backward_workspace_bytes", "hot_linear_backward", "hot_linear_backward_kernels",
     "hot_gemm_splits", "hot_hla_workspace_bytes", "hot_linear_backward_bias",
@@ -74,6 +74,8 @@ def _declare(lib):
     lib.hot_backward_products.argtypes = [i64, i64, i64, cfgp]
     lib.hot_backward_pair_rows.restype = i32
     lib.hot_backward_pair_rows.argtypes = [i64, i64, i64, cfgp]
+    lib.hot_backward_gy_runs.restype = i32
+    lib.hot_backward_gy_runs.argtypes = [i64, i64, i64, i64, cfgp, i32, i32, C.POINTER(i32)]
     lib.hot_kpad.restype = i64
     lib.hot_kpad.argtypes = [i64]
     lib.hot_hq_rowwise.restype = i32

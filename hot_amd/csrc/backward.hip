@@ -299,6 +299,23 @@ struct Marks {
   int seq = 0;
 };
 
+// The fewest workgroups of a column-wise job (col_jobs_want) from those of all jobs of the quantise phase: W's, g_y's along the tokens,
+// and as many as g_y's row-wise quantiser takes by itself, which stand for it also where another kernel or another launch has it.
+static int64_t flat_want(int64_t L, int64_t O, int64_t I, const hot_config* c, int dtype) {
+  const int elem = dtype == HOT_F32 ? 4 : 2;
+  const int64_t w = col_job_workgroups(O, I, c->n_o, c->n_o, c->w_bits == 4, c->w_scale, elem);
+  const int64_t g = c->hla_n > COL_MAX_N ? 0 : col_job_workgroups(L, O, c->hla_n, c->hla_r, 0, c->gw_scale, elem);
+  return col_jobs_want(w + g + L * O / (256 * HQ_UNROLL * EPL));
+}
+
+// g_y along the tokens, in blocks of up to 128: of a call, and of one with steps per sample.
+static int flat_gy_job(ColJob& job, const void* gy, int dtype, int64_t L, int64_t O, const hot_config* c, const BwdLayout& b, uint8_t* ws,
+                       int64_t want, bool bias, const char* who) {
+  return col_job_impl(job, gy, dtype, L, O, c->hla_n, cfg_rows(c), c->hla_r, c->gw_bits, c->gw_round, c->seed, HOT_STREAM_GW, c->gw_scale,
+                      ws + b.off_qgp, b.ld_gp, 0, (float*)(ws + b.off_sgp), ws + b.off_colg, colwise_workspace_bytes_impl(O), who,
+                      1, 0, false, false, want, bias);
+}
+
 static int run_backward(const void* gy, const void* w, int dtype, const void* xq, const float* sx, int64_t L,
                         int64_t O, int64_t I, const hot_config* cfg, void* gx, void* gw, int out_dtype,
                         void* workspace, size_t workspace_bytes, Marks* marks, hipStream_t st,
@@ -340,9 +357,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   // the launches of the two phases (phase.h); larger ones have kernels of their own.
   const bool big = cfg->hla_n > COL_MAX_N, w_short = w_joins_phase(cfg);
   ColJob gj, wj;
-  const int elem = dtype == HOT_F32 ? 4 : 2;
-  const int64_t want = col_jobs_want(col_job_workgroups(O, I, cfg->n_o, cfg->n_o, cfg->w_bits == 4, cfg->w_scale, elem) +
-                                     (big ? 0 : col_job_workgroups(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, elem)) + L * O / 8192);
+  const int64_t want = flat_want(L, O, I, cfg, dtype);
   rc = col_job_impl(wj, w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed, HOT_STREAM_W,
                     cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw, colwise_workspace_bytes_impl(I), who,
                     1, 0, false, w_short, want);
@@ -354,9 +369,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   const bool row_fused = hq_job && row_tensor;
   float* const slots = (float*)(ws + b.off_hq);
   if (!big) {
-    rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
-                      HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg, colwise_workspace_bytes_impl(O), who,
-                      1, 0, false, false, want, gb != nullptr);
+    rc = flat_gy_job(gj, gy, dtype, L, O, cfg, b, ws, want, gb != nullptr, who);
     if (rc) return rc;
     if (row_fused) col_job_row_stat(gj, cfg->n_o);
     if (gb) gj.a.colsum = (float*)(ws + b.off_colsum);
@@ -370,7 +383,7 @@ static int run_backward(const void* gy, const void* w, int dtype, const void* xq
   }
   ColsumArgs sj;
   if (gb) {
-    const int64_t strips = big ? colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, elem) : col_job_strips(gj);
+    const int64_t strips = big ? colsum_strips_impl(L, O, cfg->hla_n, cfg->hla_r, 0, cfg->gw_scale, dtype == HOT_F32 ? 4 : 2) : col_job_strips(gj);
     if (int e = colsum_args(sj, (const float*)(ws + b.off_colsum), O, strips, b.colsum_strips, gb, out_dtype, who)) return e;
   }
 
@@ -878,6 +891,31 @@ size_t hot_backward_batched_workspace_bytes(int64_t B, int64_t T, int64_t O, int
   return batched_layout(B, T, O, I, cfg).total;
 }
 
+static int batched_gy_job(ColJob& job, const void* gy, int dtype, int64_t B, int64_t T, int64_t O, const hot_config* c, const BatchedLayout& b,
+                          uint8_t* ws, bool bias, const char* who) {
+  return col_job_impl(job, gy, dtype, B * T, O, c->hla_n, cfg_rows(c), c->hla_r, c->gw_bits, c->gw_round, c->seed, HOT_STREAM_GW, c->gw_scale,
+                      ws + b.off_qgp, b.ld_gp, 0, (float*)(ws + b.off_sgp), ws + b.off_colg, colwise_group_workspace_bytes_impl(O, (int)B),
+                      who, (int)B, b.kg, false, false, 0, bias);
+}
+
+int hot_backward_gy_runs(int64_t B, int64_t T, int64_t O, int64_t I, const hot_config* cfg, int dtype, int bias, int32_t* out4) {
+  const char* who = "hot_backward_gy_runs";
+  if (!out4) return fail(HOT_ERR_INVALID, "%s: null pointer", who);
+  if (int e = B ? check_batched(cfg, B, T, who) : check_cfg(cfg, who)) return e;
+  if (T <= 0 || O <= 0 || I <= 0 || O % cfg->n_o || I % 8) return fail(HOT_ERR_INVALID, "%s: bad shape T=%lld O=%lld I=%lld", who, (long long)T, (long long)O, (long long)I);
+  // (the job is filled and nothing launched: any aligned address does for its operands)
+  uint8_t* const at = (uint8_t*)4096;
+  ColJob g;
+  const int rc = B ? batched_gy_job(g, at, dtype, B, T, O, cfg, batched_layout(B, T, O, I, cfg), at, bias != 0, who)
+                   : flat_gy_job(g, at, dtype, T, O, cfg, bwd_layout(T, O, I, cfg), at, flat_want(T, O, I, cfg, dtype), bias != 0, who);
+  if (rc) return rc;
+  out4[0] = g.runs[0];
+  out4[1] = g.runs[1];
+  out4[2] = g.a.colmax_own ? g.a.ncolmax : 0;
+  out4[3] = g.tall_gx != 0;
+  return HOT_OK;
+}
+
 // gb: [O] of out_dtype, the column sums of g_y (bias gradient), or null.  They come out of the statistics pass, which
 // holds the sum of every token block, and a job of the quantise phase adds them up: training step of
 // 64 x 197 tokens 768 -> 768 bf16 197 us with a reduction of g_y behind the call, 188 with this; 128 x 197, 768 -> 3072 727 / 669.
@@ -911,9 +949,7 @@ static int run_backward_batched(const char* who, const void* gy, const void* w, 
   int rc = col_job_impl(wj, w, dtype, O, I, cfg->n_o, identity_rows(), cfg->n_o, cfg->w_bits, cfg->w_round, cfg->seed, HOT_STREAM_W,
                         cfg->w_scale, ws + b.off_qw, b.ld_w, cfg->w_bits == 4, sw, ws + b.off_colw, colwise_workspace_bytes_impl(I), who,
                         1, 0, false, w_short);
-  if (!rc) rc = col_job_impl(gj, gy, dtype, L, O, cfg->hla_n, cfg_rows(cfg), cfg->hla_r, cfg->gw_bits, cfg->gw_round, cfg->seed,
-                             HOT_STREAM_GW, cfg->gw_scale, ws + b.off_qgp, b.ld_gp, 0, sgp, ws + b.off_colg,
-                             colwise_group_workspace_bytes_impl(O, (int)B), who, (int)B, b.kg, false, false, 0, gb != nullptr);
+  if (!rc) rc = batched_gy_job(gj, gy, dtype, B, T, O, cfg, b, ws, gb != nullptr, who);
   if (rc) return rc;
   HqArgs hj;
   if (hq_job) {

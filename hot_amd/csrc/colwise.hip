@@ -96,43 +96,54 @@ size_t colwise_group_workspace_bytes_impl(int64_t C, int groups) {
 }
 
 // Token blocks per workgroup of the quantise pass (tb) and of an absmax statistics pass (tb0).
-// The staged run of a channel (tb * r codes) must be a whole number of output dwords and cover the
-// blocks that share a 16-row step, and is at least 32 bytes long.  Beyond that, runs grow (up to 128
-// bytes) only while the grid keeps four workgroups per CU and the staging area does not cost a
-// resident workgroup: with the ring of a 16-bit input three workgroups share a CU up to 80 staged
-// bytes per channel, and the quantise pass lost a quarter of its speed each time a longer run took
-// one away (measured at 8192 x 11008 and 11008 x 4096; the L2 of an XCD merges the short runs of
-// neighbouring workgroups anyway).  (Runs below 32 bytes make a small W kernel faster on its own,
-// 8 us instead of 11 at 3072 x 768, but its four times as many workgroups then get in the way of the
-// g_y statistics pass it runs beside: the step came out 2 us slower.)  Absmax statistics stage nothing: while the grid has fewer than 2048
-// workgroups they take shorter workgroups, down to 64 rows (measured 1 us faster at 12608 x 3072).
-// The SAWB sums are order-sensitive and keep the partition of the quantise pass.
+// The staged run of a channel (tb * r codes) must be a whole number of output dwords and cover the blocks that share a 16-row step.
+// In a launch that fills the chip it is 32 bytes and more (shorter runs of W, 3072 x 768, beside g_y: W's own kernel 8 us instead of 11,
+// but four times as many workgroups in the way of g_y's, and the step 2 us longer), and grows up to 128 bytes while the grid keeps four
+// workgroups per CU and the staging area does not cost a resident workgroup: the quantise pass lost a quarter of its speed each time
+// a longer run took one of three away (measured at 8192 x 11008 and 11008 x 4096; the L2 of an XCD merges the short runs of
+// neighbouring workgroups anyway).  col_ring_bytes: a workgroup of one or two steps has a ring of as many buffers, which is what
+// lets more of them share a CU.
 // With fewer workgroups than `want` the runs go below 32 bytes, down to one step or one output word: a workgroup's time is then
 // a chain (rows on their way, transform, store), and two workgroups on two CUs take half of it each (col_jobs_want).
-// col_ring_bytes: a workgroup of one or two steps has a ring of as many buffers, which is what lets more of them share a CU.
-struct ColPartition { int tb, tb0; };
-static ColPartition col_partition(int n, int r, int store4, int mode, int64_t C, int64_t NB, int elem_bytes, int64_t want, bool keep_stat) {
-  const int BPS = n >= CW_ROWS ? 1 : CW_ROWS / n;
-  const int64_t gx = (C + CW - 1) / CW;
-  auto run_bytes = [&](int t) { return store4 ? t * r / 2 : t * r; };   // t * r is a multiple of 8 when store4
-  auto wgs = [&](int t) { return gx * ((NB + t - 1) / t); };
+// Absmax statistics stage nothing: while the grid has fewer than 2048 workgroups they take shorter workgroups, down to 64 rows
+// (measured 1 us faster at 12608 x 3072).
+// Sums depend on the partition, in their last bits: those of SAWB steps and of a bias gradient (keep_stat) take one that neither
+// `want` nor the length of a ring moves.
+struct ColShape { int n, r, store4, mode; int64_t C, NB; int elem_bytes; };
+static int col_bps(const ColShape& s) { return s.n >= CW_ROWS ? 1 : CW_ROWS / s.n; }       // blocks that share a 16-row step
+// (runs are powers of two blocks)
+static int64_t col_wgs(const ColShape& s, int t) { return (s.C + CW - 1) / CW * ((s.NB + t - 1) >> __builtin_ctz(t)); }
+static int col_least(const ColShape& s) {
+  int t = col_bps(s);
+  while ((t * s.r) % (s.store4 ? 8 : 4) != 0) t <<= 1;
+  return t;
+}
+// whole_ring: every ring counts as one of all its buffers, whatever the workgroup takes
+static int col_long_run(const ColShape& s, bool whole_ring) {
+  auto run_bytes = [&](int t) { return s.store4 ? t * s.r / 2 : t * s.r; };   // t * r is a multiple of 8 when store4
   auto resident = [&](int t) {   // workgroups of the quantise pass per CU, as far as LDS decides (three are enough)
-    const size_t per = col_ring_bytes(t * n, elem_bytes) + (size_t)CW * (t * r + 4) + 256;
-    const int k = (int)((160u * 1024u) / per);
+    const unsigned per = (unsigned)col_ring_bytes(whole_ring ? 4 * CW_ROWS : t * s.n, s.elem_bytes) + CW * (t * s.r + 4) + 256;
+    const int k = (int)(160u * 1024u / per);
     return k > 3 ? 3 : k;
   };
-  int least = BPS;
-  while ((least * r) % (store4 ? 8 : 4) != 0) least <<= 1;
-  int tb = least;
-  while (run_bytes(tb) < 32) tb <<= 1;
-  while (run_bytes(tb) < 128 && wgs(2 * tb) >= 1024 && resident(2 * tb) >= resident(tb)) tb <<= 1;
-  const int whole = tb;
-  if (mode != HOT_SCALE_SAWB)
-    while (tb > least && wgs(tb) < want) tb >>= 1;
-  int tb0 = keep_stat ? whole : tb;
-  if (mode != HOT_SCALE_SAWB)
-    while (tb0 > BPS && (tb0 & 1) == 0 && tb0 * n > 64 && wgs(tb0) < 2048) tb0 >>= 1;
-  return {tb, tb0};
+  int t = col_least(s);
+  while (run_bytes(t) < 32) t <<= 1;
+  while (run_bytes(t) < 128 && col_wgs(s, 2 * t) >= 1024 && resident(2 * t) >= resident(t)) t <<= 1;
+  return t;
+}
+// of an absmax statistics pass, from those of a quantise pass
+static int col_stat_run(const ColShape& s, int t) {
+  const int least = col_bps(s);
+  if (s.mode != HOT_SCALE_SAWB)
+    while (t > least && (t & 1) == 0 && t * s.n > 64 && col_wgs(s, t) < 2048) t >>= 1;
+  return t;
+}
+struct ColPartition { int tb, tb0; };
+static ColPartition col_partition(const ColShape& s, int64_t want, bool keep_stat) {
+  int tb = col_long_run(s, s.mode == HOT_SCALE_SAWB);
+  if (s.mode != HOT_SCALE_SAWB)
+    for (const int least = col_least(s); tb > least && col_wgs(s, tb) < want;) tb >>= 1;
+  return {tb, col_stat_run(s, keep_stat ? col_long_run(s, true) : tb)};
 }
 
 // The fewest workgroups that each column-wise job of a launch should have, given how many all jobs of the launch have while none
@@ -144,8 +155,8 @@ static ColPartition col_partition(int n, int r, int store4, int mode, int64_t C,
 int64_t col_jobs_want(int64_t workgroups) { return workgroups < 2048 ? 256 : 128; }
 
 int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes) {
-  const ColPartition cp = col_partition(n, r, store4, mode, C, R / n, elem_bytes, 0, false);
-  return (C + CW - 1) / CW * ((R / n + cp.tb - 1) / cp.tb);
+  const ColShape s = {n, r, store4, mode, C, R / n, elem_bytes};
+  return col_wgs(s, col_long_run(s, mode == HOT_SCALE_SAWB));
 }
 
 // ---- jobs -----------------------------------------------------------------------
@@ -236,7 +247,7 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
 
   // grids: strips of channels x runs of token blocks, per sample group (a run never leaves its sample)
   const int elem = dtype == HOT_F32 ? 4 : 2;
-  const ColPartition cp = col_partition(n, r, store4, scale_mode, C, a.NB, elem, groups > 1 ? 0 : want, keep_stat);
+  const ColPartition cp = col_partition({n, r, store4, scale_mode, C, a.NB, elem}, groups > 1 ? 0 : want, keep_stat);
   const int64_t gx = (C + CW - 1) / CW, runs = (a.NBs + cp.tb - 1) / cp.tb;
   int tb0 = cp.tb0;
   int64_t runs0 = (a.NBs + tb0 - 1) / tb0;
@@ -414,9 +425,9 @@ int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int m
     const int64_t rows = colsum_strip_rows_big(R, C);
     return (R + rows - 1) / rows;
   }
-  const int64_t NB = R / n;
-  const ColPartition part = col_partition(n, r, store4, mode, C, NB, elem_bytes, 0, true);
-  return (NB / groups + part.tb0 - 1) / part.tb0 * groups;
+  const ColShape s = {n, r, store4, mode, C, R / n, elem_bytes};
+  const int tb0 = col_stat_run(s, col_long_run(s, true));
+  return (s.NB / groups + tb0 - 1) / tb0 * groups;
 }
 
 int colsum_finish_impl(const ColsumArgs& a, hipStream_t st) {

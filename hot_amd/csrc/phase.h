@@ -80,7 +80,7 @@ int col_job_impl(ColJob& job, const void* in, int dtype, int64_t R, int64_t C, i
                  float* scales_out, void* workspace, size_t workspace_bytes, const char* who, int groups, int64_t kpad_group,
                  bool rowmajor, bool as_short, int64_t want = 0, bool keep_stat = false);
 // want: the fewest workgroups it should have (one group, absmax steps; 0: as many as long runs give).  keep_stat: the statistics
-// pass keeps the partition of want = 0, on which the order of the column sums depends.
+// pass keeps a partition that depends on the shape alone, and with it the order of the column sums.
 int64_t col_jobs_want(int64_t workgroups);
 // Workgroups of the quantise pass with want = 0.
 int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes);

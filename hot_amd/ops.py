@@ -383,6 +383,14 @@ def backward_pair_rows(L: int, O: int, I: int, opt: HotOptions) -> int:
     return int(_lib.lib().hot_backward_pair_rows(int(L), int(O), int(I), C.byref(opt.to_c())))
 
 
+def backward_gy_runs(B: int, T: int, O: int, I: int, opt: HotOptions, dtype: torch.dtype, bias: bool = False) -> Tuple[int, int, int, bool]:
+    """How the passes over g_y along the tokens run (hot_backward_gy_runs; B = 0: linear_backward of T tokens): runs of token blocks of the
+    statistics pass and of the quantise pass, per-channel maxima that workgroups have to themselves, 64 channels and four runs to one."""
+    out = (C.c_int32 * 4)()
+    _lib.check(_lib.lib().hot_backward_gy_runs(int(B), int(T), int(O), int(I), C.byref(opt.to_c()), _DTYPES[dtype], int(bias), out))
+    return out[0], out[1], out[2], bool(out[3])
+
+
 def kpad_group(T: int, opt: HotOptions) -> int:
     """Code bytes every sample takes in the K dimension of the batched g_W operands."""
     return _size(opt, "kpad_group", int(T))

@@ -127,6 +127,12 @@ enum hot_products_launch {
 HOT_API int hot_backward_products(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
 /* Rows of g_x in a tile of that launch, 64, 128 or 192 (0: the products do not share one, or the size is refused). */
 HOT_API int hot_backward_pair_rows(int64_t L, int64_t O, int64_t I, const hot_config* cfg);
+/* How the passes over g_y along the tokens run, in blocks of up to 128, for the same purpose: B = 0 asks for hot_linear_backward of T
+ * tokens, B > 0 for hot_linear_backward_batched of B samples, bias != 0 for their forms with a bias gradient.  out4: runs of token blocks
+ * (per sample) of the statistics pass, and of the quantise pass; arrays of per-channel maxima (per sample) that workgroups of the
+ * statistics pass have to themselves (0: they share some, or there is no step per channel); 1 where such a workgroup takes 64
+ * channels and four runs. */
+HOT_API int hot_backward_gy_runs(int64_t B, int64_t T, int64_t O, int64_t I, const hot_config* cfg, int dtype, int bias, int32_t* out4);
 HOT_API int hot_abi_version(void);
 
 /* Bytes of the leading dimension (row pitch) the library uses for a K-major

@@ -366,3 +366,27 @@ def test_tiling_of_the_paired_products():
     assert rows(12608, 3072, 768) == rows(12608, 2304, 768) == rows(12608, 3072, 768, 8) == 128
     assert rows(12608, 768, 3072, 8) == rows(8192, 11008, 4096) == 192
     assert rows(64, 64, 64, streams=2) == rows(64, 8192, 64) == rows(0, 64, 64) == rows(64, 64, 20) == 0
+
+
+@pytest.mark.parametrize("B,T,O", [(0, 15425, 2048), (0, 4597, 9568), (0, 16411, 16), (0, 1023, 32), (0, 272, 128), (0, 12608, 3072),
+                                   (1, 12608, 3072), (64, 577, 1464), (128, 197, 912), (64, 208, 768)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_runs_of_the_column_sums(B, T, O, dtype):
+    """The partial sums of a bias gradient cover runs of token blocks that depend on the shape alone, so that its last bits do: 32 to 128
+    codes of a channel while there are 1024 workgroups and no resident one is lost (rings of three fp32 or four 16-bit steps), cut to
+    64 rows below 2048 workgroups."""
+    from hot_amd import ops
+    n, rows = orc.hla_rows(min(T & -T, 128))
+    r, strips, size = len(rows), -(-O // 256), 4 if dtype == torch.float32 else 2
+    wgs = lambda t: strips * -(-((B or 1) * T // n) // t)
+    resident = lambda t: min(3, 160 * 1024 // ((3 if size == 4 else 4) * 16 * 256 * size + 256 * (t * r + 4) + 256))
+    t = max(1, 16 // n)
+    while t * r % 4 or t * r < 32:
+        t *= 2
+    while t * r < 128 and wgs(2 * t) >= 1024 and resident(2 * t) >= resident(t):
+        t *= 2
+    while t > max(1, 16 // n) and t * n > 64 and wgs(t) < 2048:
+        t //= 2
+    for scale in ("tensor", "row"):
+        opt = ops.HotOptions(n_o=8, hla_n=n, hla_rows=tuple(int(v) for v in rows), gx_scale=scale, gw_scale=scale)
+        assert ops.backward_gy_runs(B, T, O, 64, opt, dtype, bias=True)[0] == -(-(T // n) // t)
