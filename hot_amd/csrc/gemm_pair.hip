@@ -110,7 +110,11 @@ bool gemm_pair_pays(const GemmProduct& w, const GemmProduct& x) {
 // start and end of a tile, g_x and g_W; with INT8 operands a stage of g_x has half the multiplications: x_int8 of it.  Fitted to
 // 157 shapes of 49 .. 25216 tokens and 64 .. 11008 channels, INT4 and INT8, all types, each timed in all three tilings: the choice is on
 // average 0.3 % slower than the best of the three (two tilings and the line alone: 5.1 %).  On the wrong side of the line 128 x 2304 x 5248
-// 49.0 / 46.5 / 52.0 and 512 x 4352 x 7336 127 / 118 / 127.
+// 49.0 / 46.5 / 52.0 and 512 x 4352 x 7336 127 / 118 / 127.  (1700 further shapes, the narrow ones among them: 0.5 %.)
+// Up to 256 out-features a tile of g_x is little but its own store, which the model does not see: tiles of 192 rows, two to a CU, wait
+// for theirs.  Where it would take them, us of the whole backward in 128 / 192: 15199 x 128 x 7848 160 / 215, 10496 x 80 x 5520 INT8 65 / 80,
+// 11776 x 168 x 4992 52 / 61, 9728 x 256 x 9856 81.5 / 82.8 (24 such shapes: 6 % on average, the worst 7424 x 144 x 8168 78.6 / 74.3).
+constexpr int64_t PAIR_192_LEAST_K = 256;
 static int gemm_pair_tiling(const GemmProduct& w, const GemmProduct& x) {
   struct Tiling { int xm, xn, wm, wn; double chain_x, chain_w, full_x, full_w, ends_x, ends_w, x_int8; };
   static const Tiling tilings[3] = {{64, 64, 64, 64, 0.20, 0.16, 0.22, 0.18, 2.0, 1.5, 0.8},
@@ -121,7 +125,7 @@ static int gemm_pair_tiling(const GemmProduct& w, const GemmProduct& x) {
   if (tiles(w, 192, 128) >= 256) return PAIR_192;
   int best = PAIR_128;
   double least = 0.0;
-  for (int k = PAIR_64; k <= PAIR_192; ++k) {
+  for (int k = PAIR_64; k <= (x.K > PAIR_192_LEAST_K ? PAIR_192 : PAIR_128); ++k) {
     const Tiling& t = tilings[k];
     const double sx = stages(x) * (x.bits == 8 ? t.x_int8 : 1.0), sw = stages(w);
     const double full = (tiles(x, t.xm, t.xn) * (sx * t.full_x + t.ends_x) + tiles(w, t.wm, t.wn) * (sw * t.full_w + t.ends_w)) / 512.0;

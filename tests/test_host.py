@@ -365,6 +365,9 @@ def test_tiling_of_the_paired_products():
     assert rows(49, 3072, 768) == rows(64, 64, 64) == rows(3003, 1000, 520) == 64
     assert rows(12608, 3072, 768) == rows(12608, 2304, 768) == rows(12608, 3072, 768, 8) == 128
     assert rows(12608, 768, 3072, 8) == rows(8192, 11008, 4096) == 192
+    # up to 256 out-features no tiles of 192 rows, of any width (wider g_x, long runs of tokens), unless g_W fills the chip with them
+    assert rows(15199, 128, 7848) == rows(10496, 80, 5520, 8) == rows(11776, 168, 4992) == rows(9728, 256, 9856) == 128
+    assert rows(9728, 264, 9856) == rows(9728, 200, 17000) == 192
     assert rows(64, 64, 64, streams=2) == rows(64, 8192, 64) == rows(0, 64, 64) == rows(64, 64, 20) == 0
 
 
