@@ -129,6 +129,24 @@ def test_backward_small_grids(gpu, L, O, I, dtype, variant):
     assert torch.equal(gx.cpu(), torch.from_numpy(tr.g_x).to(dtype)) and torch.equal(gw.cpu(), torch.from_numpy(tr.g_w).to(dtype))
 
 
+@pytest.mark.parametrize("L,runs", [(8191, 256), (8193, 257)])
+def test_step_from_the_last_workgroup(gpu, L, runs):
+    """The largest gradient is in the last run of token blocks, whose maximum is the last of the 256 that take a load of each thread or
+    the first behind them; so too in a sample of a batch."""
+    from hot_amd import ops
+    x, w, gy = make_case(L, 16, 16, seed=L)
+    gy[-1, -1] = 8 * gy.abs().max()
+    ocfg, opt = both_configs(L)
+    assert ops.backward_gy_runs(0, L, 16, 16, opt, gy.dtype)[0] == ops.backward_gy_runs(2, L, 16, 16, opt, gy.dtype)[0] == runs
+    gx, gw, tr = run_both(x, w, gy, ocfg, opt, gpu)
+    assert np.array_equal(gx.cpu().numpy(), tr.g_x) and np.array_equal(gw.cpu().numpy(), tr.g_w)
+    x3, g3 = torch.stack([x, -x]), torch.stack([gy, gy / 64])
+    gx, gw = ops.linear_backward_batched(g3.to(gpu), w.to(gpu), *ops.abc_forward_batched(x3.to(gpu), opt), opt)
+    gx_ref, gw_ref, _ = orc.linear_backward_batched(g3.numpy(), w.numpy(), *orc.abc_forward_batched(x3.numpy(), ocfg), ocfg,
+                                                    gw_ranges=ops.backward_batched_ranges(2, L, 16, 16, opt))
+    assert np.array_equal(gx.cpu().numpy(), gx_ref) and np.array_equal(gw.cpu().numpy(), gw_ref)
+
+
 @pytest.mark.parametrize("L", [4096 + 16, 4163, 16411])
 def test_bias_gradient_of_many_runs(gpu, L):
     """A step per channel and the bias gradient from one statistics pass of more than 64 runs of token blocks: every run leaves its own
