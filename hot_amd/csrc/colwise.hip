@@ -101,14 +101,15 @@ size_t colwise_group_workspace_bytes_impl(int64_t C, int groups) {
 // but four times as many workgroups in the way of g_y's, and the step 2 us longer), and grows up to 128 bytes while the grid keeps four
 // workgroups per CU and the staging area does not cost a resident workgroup: the quantise pass lost a quarter of its speed each time
 // a longer run took one of three away (measured at 8192 x 11008 and 11008 x 4096; the L2 of an XCD merges the short runs of
-// neighbouring workgroups anyway).  col_ring_bytes: a workgroup of one or two steps has a ring of as many buffers, which is what
-// lets more of them share a CU.
+// neighbouring workgroups anyway).  Every ring counts with all its buffers there: that those of one or two steps are shorter
+// (col_ring_bytes) lets more workgroups share a CU, but with the shorter runs that would go with it the stores lose more (us of the whole
+// backward, fp32, runs of 64 / 32 tokens: 6879 x 7424 x 1232 328 / 348, 2561 x 9280 x 2432 203 / 210, 64 x 577 x 1464 x 200 271 / 280).
 // With fewer workgroups than `want` the runs go below 32 bytes, down to one step or one output word: a workgroup's time is then
 // a chain (rows on their way, transform, store), and two workgroups on two CUs take half of it each (col_jobs_want).
 // Absmax statistics stage nothing: while the grid has fewer than 2048 workgroups they take shorter workgroups, down to 64 rows
 // (measured 1 us faster at 12608 x 3072).
-// Sums depend on the partition, in their last bits: those of SAWB steps and of a bias gradient (keep_stat) take one that neither
-// `want` nor the length of a ring moves.
+// Sums depend on the partition, in their last bits: those of SAWB steps and of a bias gradient (keep_stat) take one that `want` does
+// not move.
 struct ColShape { int n, r, store4, mode; int64_t C, NB; int elem_bytes; };
 static int col_bps(const ColShape& s) { return s.n >= CW_ROWS ? 1 : CW_ROWS / s.n; }       // blocks that share a 16-row step
 // (runs are powers of two blocks)
@@ -118,11 +119,10 @@ static int col_least(const ColShape& s) {
   while ((t * s.r) % (s.store4 ? 8 : 4) != 0) t <<= 1;
   return t;
 }
-// whole_ring: every ring counts as one of all its buffers, whatever the workgroup takes
-static int col_long_run(const ColShape& s, bool whole_ring) {
+static int col_long_run(const ColShape& s) {
   auto run_bytes = [&](int t) { return s.store4 ? t * s.r / 2 : t * s.r; };   // t * r is a multiple of 8 when store4
   auto resident = [&](int t) {   // workgroups of the quantise pass per CU, as far as LDS decides (three are enough)
-    const unsigned per = (unsigned)col_ring_bytes(whole_ring ? 4 * CW_ROWS : t * s.n, s.elem_bytes) + CW * (t * s.r + 4) + 256;
+    const unsigned per = (unsigned)col_ring_bytes(4 * CW_ROWS, s.elem_bytes) + CW * (t * s.r + 4) + 256;
     const int k = (int)(160u * 1024u / per);
     return k > 3 ? 3 : k;
   };
@@ -140,10 +140,11 @@ static int col_stat_run(const ColShape& s, int t) {
 }
 struct ColPartition { int tb, tb0; };
 static ColPartition col_partition(const ColShape& s, int64_t want, bool keep_stat) {
-  int tb = col_long_run(s, s.mode == HOT_SCALE_SAWB);
+  const int whole = col_long_run(s);
+  int tb = whole;
   if (s.mode != HOT_SCALE_SAWB)
     for (const int least = col_least(s); tb > least && col_wgs(s, tb) < want;) tb >>= 1;
-  return {tb, col_stat_run(s, keep_stat ? col_long_run(s, true) : tb)};
+  return {tb, col_stat_run(s, keep_stat ? whole : tb)};
 }
 
 // The fewest workgroups that each column-wise job of a launch should have, given how many all jobs of the launch have while none
@@ -156,7 +157,7 @@ int64_t col_jobs_want(int64_t workgroups) { return workgroups < 2048 ? 256 : 128
 
 int64_t col_job_workgroups(int64_t R, int64_t C, int n, int r, int store4, int mode, int elem_bytes) {
   const ColShape s = {n, r, store4, mode, C, R / n, elem_bytes};
-  return col_wgs(s, col_long_run(s, mode == HOT_SCALE_SAWB));
+  return col_wgs(s, col_long_run(s));
 }
 
 // ---- jobs -----------------------------------------------------------------------
@@ -426,7 +427,7 @@ int64_t colsum_strips_impl(int64_t R, int64_t C, int n, int r, int store4, int m
     return (R + rows - 1) / rows;
   }
   const ColShape s = {n, r, store4, mode, C, R / n, elem_bytes};
-  const int tb0 = col_stat_run(s, col_long_run(s, true));
+  const int tb0 = col_stat_run(s, col_long_run(s));
   return (s.NB / groups + tb0 - 1) / tb0 * groups;
 }
 

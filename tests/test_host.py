@@ -393,3 +393,14 @@ def test_runs_of_the_column_sums(B, T, O, dtype):
     for scale in ("tensor", "row"):
         opt = ops.HotOptions(n_o=8, hla_n=n, hla_rows=tuple(int(v) for v in rows), gx_scale=scale, gw_scale=scale)
         assert ops.backward_gy_runs(B, T, O, 64, opt, dtype, bias=True)[0] == -(-(T // n) // t)
+
+
+@pytest.mark.parametrize("B,T,O,tokens", [(0, 6879, 7424, 64), (0, 2561, 9280, 64), (0, 6698, 3712, 64), (0, 12608, 2304, 64), (64, 577, 1464, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_runs_of_a_full_launch(B, T, O, tokens, dtype):
+    """Where the launch fills the chip the quantise pass takes the longest runs that cost no resident workgroup, as if every ring had all
+    its buffers, in 32-bit types too: a shorter ring is no reason for a shorter run."""
+    from hot_amd import ops
+    n, rows = orc.hla_rows(min(T & -T, 64))
+    opt = ops.HotOptions(n_o=8, hla_n=n, hla_rows=tuple(int(v) for v in rows))
+    assert ops.backward_gy_runs(B, T, O, 1024, opt, dtype)[1] == -(-T // tokens)
