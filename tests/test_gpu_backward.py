@@ -116,9 +116,12 @@ def test_backward_matches_oracle(gpu, dtype, shape, variant):
     (3001, 144, 16),     # blocks of one token, many of them: the last run of nine rows
     (1023, 32, 16),      # 64 runs: with a step per channel each has maxima of its own
     (1025, 32, 16),      # 65: a workgroup takes four of them, the last one a single run
-    (4163, 80, 16),      # 66 runs of 64 tokens, the last of three, a second strip of sixteen channels
-    (16411, 16, 16),     # 257 runs: eight copies that the workgroups share
-    (1023, 2064, 8),     # 64 runs of more channels than there is room for
+    (1041, 80, 16),      # 66 runs, the last of one token, a second strip of sixteen channels
+    (4163, 80, 16),      # 261 of 16 tokens: eight copies that the workgroups share
+    (8191, 16, 16),      # 256 runs: 64 arrays of maxima
+    (8193, 16, 16),      # 257
+    (1023, 2064, 8),     # 32 runs of many channels
+    (4095, 3600, 8),     # 64 runs, twice as long as the shape's own: more channels than there is room for, so four to a workgroup
 ])
 def test_backward_small_grids(gpu, L, O, I, dtype, variant):
     """Problems whose column-wise jobs are cut into short runs of token blocks (col_partition): rings of one to four
@@ -307,9 +310,11 @@ def test_llama_shapes_properties(gpu, shape):
 
 @pytest.mark.parametrize("L,C", [(256 * 13, 2568), (512 * 27, 264), (1024 * 11, 528), (256, 8)])
 @pytest.mark.parametrize("scale", [orc.SCALE_TENSOR, orc.SCALE_SAWB, orc.SCALE_ROW])
-def test_large_blocks_many_items(gpu, L, C, scale):
+@pytest.mark.parametrize("rounding", ["nearest", "stoch"])
+def test_large_blocks_many_items(gpu, L, C, scale, rounding):
     """Blocks above 128 tokens where a workgroup takes several (block, coefficient) items in both passes of stage 2, the last one fewer;
-    and the smallest problem, where it takes one.  Run-major rows; codes and steps are the oracle's."""
+    and the smallest problem, where it takes one.  Run-major rows, both
+    roundings; codes and steps are the oracle's."""
     from hot_amd import ops
     from hot_amd.hadamard_matmul import run_major
     n, rows = orc.hla_rows(L)
@@ -317,12 +322,14 @@ def test_large_blocks_many_items(gpu, L, C, scale):
     rows = tuple(int(v) for v in run_major(rows))
     x = torch.randn(L, C, generator=torch.Generator().manual_seed(L + C))
     if scale == orc.SCALE_ROW:
-        q, s, lp = ops.hla_tokenwise(x.to(gpu), n, rows, bits=8, rounding="nearest", scale="row")
+        q, s, lp = ops.hla_tokenwise(x.to(gpu), n, rows, bits=8, rounding=rounding, scale="row", seed=31)
         xp = orc.fwht_blocks_first(x.numpy(), n, np.asarray(rows))
-        q_ref, s_ref = orc.quant(np.ascontiguousarray(xp.T), 8, orc.SCALE_ROW)
+        q_ref, s_ref = orc.quant(np.ascontiguousarray(xp.T), 8, orc.SCALE_ROW, orc.ROUND_STOCH if rounding == "stoch" else orc.ROUND_NEAREST, 31,
+                              orc.STREAM_GW, index=orc.colwise_rng_index(C, L // n, rows))
     else:
-        q, s = ops.abc_forward(x.to(gpu), ops.HotOptions(n_o=16, hla_n=n, hla_rows=rows, act_scale=scale))
-        q_ref, s_ref = orc.abc_forward(x.numpy(), orc.HotConfig(n_o=16, hla_n=n, hla_rows=rows, act_scale=scale))
+        act = dict(n_o=16, hla_n=n, hla_rows=rows, act_scale=scale, act_round=orc.ROUND_STOCH if rounding == "stoch" else orc.ROUND_NEAREST, seed=31)
+        q, s = ops.abc_forward(x.to(gpu), ops.HotOptions(**act))
+        q_ref, s_ref = orc.abc_forward(x.numpy(), orc.HotConfig(**act))
         q_ref = q_ref.T
     assert np.array_equal(s.cpu().numpy().ravel(), np.asarray(s_ref).ravel())
     q = q.cpu().numpy()
@@ -445,6 +452,7 @@ def test_hq_linear_3d_input(gpu, fresh_args, mode):
     (1, 128, 48, 24, dict()),                                                     # a batch of one
     (3, 64, 16, 8, dict(gw_scale=orc.SCALE_ROW)),                                 # one block per sample, smallest widths
     (2, 576, 256, 384, dict(gx_bits=8, w_bits=8)),                                # 324 codes per sample: three stages per group
+    (16, 577, 688, 8, dict(gw_scale=orc.SCALE_ROW)),                              # 19 runs per sample, more maxima than there is room for
 ])
 def test_backward_batched_matches_oracle(gpu, dtype, B, T, O, I, variant):
     """3-D activations through the batched entry points (one call per layer, one set of steps per
@@ -1200,7 +1208,7 @@ def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_arg
     gy = torch.randn(L, O, device=gpu) * 1e-3
 
     def run(overlap):
-        qm.overlap_buffer_write = overlap
+        monkeypatch.setattr(qm, "overlap_buffer_write", overlap)
         fresh_args.sr_step = 0
         for m in lins:
             m.zero_grad(set_to_none=True)
@@ -1213,16 +1221,13 @@ def test_hq_linear_under_autocast_matches_the_inline_buffer_write(gpu, fresh_arg
         torch.cuda.synchronize()
         return [x.grad.clone()] + [m.weight.grad.clone() for m in lins] + [m.bias.grad.clone() for m in lins]
 
-    try:
-        ref = run(False)
-        assert taken == [None] * 3
-        for _ in range(3):
-            got = run(True)
-            for a, b in zip(got, ref):
-                assert torch.equal(a, b)
-        assert len(taken) == 12 and None not in taken[3:]
-    finally:
-        qm.overlap_buffer_write = True
+    ref = run(False)
+    assert taken == [None] * 3
+    for _ in range(3):
+        got = run(True)
+        for a, b in zip(got, ref):
+            assert torch.equal(a, b)
+    assert len(taken) == 12 and None not in taken[3:]
 
 
 @pytest.mark.parametrize("rows,beside", [(24 * 1024, True), (24 * 1024 - 1, False)])

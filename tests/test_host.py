@@ -404,3 +404,29 @@ def test_runs_of_a_full_launch(B, T, O, tokens, dtype):
     n, rows = orc.hla_rows(min(T & -T, 64))
     opt = ops.HotOptions(n_o=8, hla_n=n, hla_rows=tuple(int(v) for v in rows))
     assert ops.backward_gy_runs(B, T, O, 1024, opt, dtype)[1] == -(-T // tokens)
+
+
+def test_paths_of_the_channel_maxima():
+    """Which arrays of per-channel maxima a statistics pass keeps, at the sizes that the tests on the GPU take for them: one for each run
+    of token blocks up to 64, one for four of them up to 256 and where there is no more room, else copies that runs share (0)."""
+    from hot_amd import ops
+
+    def path(B, T, O, I, dtype=torch.float32, **kw):
+        n, rows = orc.hla_rows(min(T & -T, 128))
+        opt = ops.HotOptions(n_o=16, hla_n=n, hla_rows=tuple(int(v) for v in rows), gw_scale="row", **kw)
+        runs, _, own, tall = ops.backward_gy_runs(B, T, O, I, opt, dtype)
+        return runs, own, tall
+
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+        for L, O, I, expected in ((1023, 32, 16, (64, 64, False)), (1025, 32, 16, (65, 17, True)), (1041, 80, 16, (66, 17, True)),
+                                  (4163, 80, 16, (261, 0, False)), (8191, 16, 16, (256, 64, True)), (8193, 16, 16, (257, 0, False)),
+                                  (1023, 2064, 8, (32, 32, False)), (4095, 3600, 8, (64, 16, True))):
+            assert path(0, L, O, I, dtype, gx_bits=8, w_bits=8) == expected, (L, O)
+        assert path(16, 577, 688, 8, dtype) == (19, 0, False)
+        assert path(16, 577, 512, 8, dtype) == (19, 19, False)      # (as many of fewer channels have room)
+    # one long sample: the runs of a call with a bias gradient, and the longer ones without
+    for T, O, kept, longer in ((8191, 2064, 128, 64), (12608, 3072, 197, 50), (16384, 768, 256, 128)):
+        n, rows = orc.hla_rows(min(T & -T, 64))
+        opt = ops.HotOptions(n_o=16, hla_n=n, hla_rows=tuple(int(v) for v in rows), gx_scale="row", gw_scale="row")
+        for B in (0, 1):
+            assert [ops.backward_gy_runs(B, T, O, 16, opt, torch.float32, bias)[0] for bias in (True, False)] == [kept, longer]
