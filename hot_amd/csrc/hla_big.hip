@@ -48,6 +48,7 @@ struct BigArgs {
   int64_t R, C, NB;    // NB = R / n blocks
   int32_t n, r, rpad, bits, rounding, mode;
   int32_t nk;          // coefficients of a 64-run that some kept row needs
+  uint32_t per;        // items of a workgroup of the statistics pass of stage 2 (items_per)
   uint64_t kmask;      // bit k: coefficient k is one of them
   uint8_t klist[64];   // the nk set bits of kmask in increasing order
   // which runs keep needed coefficient index kc (bit j of keep[kc]: natural row 64 j + klist[kc] is kept); for run-major lists
@@ -179,7 +180,7 @@ int items_per(int m, int64_t C, int64_t items) {
   return per;
 }
 template <int M, int PASS, int ROUND, bool SAWB>
-__global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a, int per) {
+__global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a) {
   __shared__ float s_max[BT / 64];
   __shared__ double s_sum[2][BT / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -195,8 +196,8 @@ __global__ void __launch_bounds__(BT) big_stage2_kernel(const BigArgs a, int per
       __syncthreads();
     }
     constexpr int ITEMS = items_most<M>();
-    const uint32_t item0 = blockIdx.y * per, items = (uint32_t)(a.NB * a.nk);
-    const uint32_t mine = items - item0 < (uint32_t)per ? items - item0 : (uint32_t)per;
+    const uint32_t item0 = blockIdx.y * a.per, items = (uint32_t)(a.NB * a.nk);
+    const uint32_t mine = items - item0 < a.per ? items - item0 : a.per;
     const float* const tc = a.T + (active ? c : 0);          // (what a lane without a channel reads is never used)
     float v[ITEMS][M];
 #pragma unroll
@@ -451,8 +452,7 @@ int dispatch_runs(int m, const BigArgs& a, void* out, int64_t ld_out, hipStream_
 // of 13 bits each (3744 bytes of the 4 KiB a launch may carry; larger selections go in pieces of that
 // size).  Entry of natural row i: its output coefficient (the position of i in the caller's list) in
 // the low half, its visit number (the rank of i among the kept rows in natural order, which numbers
-// the elements of stochastic rounding) in the high half; -1 for dropped rows (written by the clear
-// kernel).  The rank is counted on the device: thread k compares its row with every row of the call.
+// the elements of stochastic rounding) in the high half; -1 for dropped rows.  The rank is counted on the device.
 constexpr int TAB_ROWS = 2304;
 struct TabRows { uint32_t packed[(TAB_ROWS * 13 + 31) / 32]; int32_t count; };
 __device__ __host__ inline int tab_row_get(const uint32_t* packed, int i) {
@@ -466,9 +466,10 @@ inline void tab_row_put(uint32_t* packed, int i, int row) {
   packed[w] |= (uint32_t)row << sh;
   if (sh > 19) packed[w + 1] |= (uint32_t)row >> (32 - sh);
 }
-__global__ void __launch_bounds__(256) big_table_kernel(int32_t* tab, const TabRows p) {
-  // every workgroup marks the kept rows in a bitmap of the block's n <= 8192 natural rows; the rank
-  // of a row is the number of marks below it
+// Every workgroup marks the kept rows in a bitmap of the block's n <= 8192 natural rows (the rank of a row is the number of marks
+// below it); thread i of the grid writes -1 for natural row i when it is dropped, and the entry of the i-th row of the caller's list.
+// Dropped and kept rows are disjoint, so the two writes never meet.
+__global__ void __launch_bounds__(256) big_table_kernel(int32_t* tab, int n, const TabRows p) {
   __shared__ uint32_t s_map[8192 / 32];
   __shared__ uint32_t s_below[8192 / 32];
   const int tid = threadIdx.x;
@@ -481,32 +482,6 @@ __global__ void __launch_bounds__(256) big_table_kernel(int32_t* tab, const TabR
   __syncthreads();
   {
     // marks in the words before word `tid` (256 words: a serial sum per thread is short)
-    uint32_t acc = 0;
-    for (int w = 0; w < tid; ++w) acc += (uint32_t)__popc(s_map[w]);
-    s_below[tid] = acc;
-  }
-  __syncthreads();
-  const int k = blockIdx.x * 256 + tid;
-  if (k >= p.count) return;
-  const int row = tab_row_get(p.packed, k);
-  const int rank = (int)(s_below[row >> 5] + (uint32_t)__popc(s_map[row >> 5] & ((1u << (row & 31)) - 1u)));
-  tab[row] = k | (rank << 16);
-}
-// The whole table in one launch (selections of up to TAB_ROWS rows): every workgroup marks the kept rows in its own LDS bitmap;
-// thread i of the grid writes -1 for natural row i when it is dropped, and the entry of the i-th row of the caller's list.
-// Dropped and kept rows are disjoint, so the two writes never meet.
-__global__ void __launch_bounds__(256) big_prepare_kernel(int32_t* tab, int n, const TabRows p) {
-  __shared__ uint32_t s_map[8192 / 32];
-  __shared__ uint32_t s_below[8192 / 32];
-  const int tid = threadIdx.x;
-  s_map[tid] = 0u;
-  __syncthreads();
-  for (int j = tid; j < p.count; j += 256) {
-    const int row = tab_row_get(p.packed, j);
-    atomicOr(&s_map[row >> 5], 1u << (row & 31));
-  }
-  __syncthreads();
-  {
     uint32_t acc = 0;
     for (int w = 0; w < tid; ++w) acc += (uint32_t)__popc(s_map[w]);
     s_below[tid] = acc;
@@ -661,29 +636,21 @@ __global__ void tab_clear_kernel(int32_t* tab, int n) {
   if (i < n) tab[i] = -1;
 }
 
-// Checks the row list and writes the table of a block (every entry: the clear kernel's -1 or a kept
-// row's slot | visit << 16) with launches alone.
-int build_row_table(int32_t* tab, int n, const int32_t* rows, int r, uint64_t* kmask_out, hipStream_t st, const char* who) {
-  std::unique_ptr<int32_t[]> slot_of(new int32_t[(size_t)n]);
-  for (int i = 0; i < n; ++i) slot_of[(size_t)i] = -1;
-  uint64_t kmask = 0;
-  for (int k = 0; k < r; ++k) {
-    if (rows[k] < 0 || rows[k] >= n) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d outside [0, %d)", who, k, rows[k], n);
-    if (slot_of[(size_t)rows[k]] != -1) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d listed twice", who, k, rows[k]);
-    slot_of[(size_t)rows[k]] = k;
-    kmask |= 1ull << (rows[k] & 63);
-  }
-  if (kmask_out) *kmask_out = kmask;
+// Writes the table of a block (every entry: -1 or a kept row's slot | visit << 16) with launches alone.
+int build_row_table(int32_t* tab, int n, const int32_t* rows, int r, hipStream_t st) {
+  const dim3 grid((unsigned)((n + 255) / 256));
   if (r <= TAB_ROWS) {
     TabRows tr;
     memset(&tr, 0, sizeof(tr));
     tr.count = r;
     for (int k = 0; k < r; ++k) tab_row_put(tr.packed, k, rows[k]);
-    hipLaunchKernelGGL(big_table_kernel, dim3((unsigned)((r + 255) / 256)), dim3(256), 0, st, tab, tr);
+    hipLaunchKernelGGL(big_table_kernel, grid, dim3(256), 0, st, tab, n, tr);
   } else {
+    hipLaunchKernelGGL(tab_clear_kernel, grid, dim3(256), 0, st, tab, n);
     // rows in natural order: the visit number of a piece's entry i is its position in the sorted list
-    std::unique_ptr<int32_t[]> sorted(new int32_t[(size_t)r]);
+    std::unique_ptr<int32_t[]> sorted(new int32_t[(size_t)r]), slot_of(new int32_t[(size_t)n]);
     for (int k = 0; k < r; ++k) sorted[(size_t)k] = rows[k];
+    for (int k = 0; k < r; ++k) slot_of[(size_t)rows[k]] = k;
     std::sort(sorted.get(), sorted.get() + r);
     for (int v0 = 0; v0 < r; v0 += TAB_PIECE) {
       TabPiece piece;
@@ -701,20 +668,19 @@ int build_row_table(int32_t* tab, int n, const int32_t* rows, int r, uint64_t* k
 }
 
 template <int M>
-int launch_stage2(const BigArgs& a, dim3 grid, int pass, hipStream_t st) {
-  int per = 1;
+int launch_stage2(BigArgs a, dim3 grid, int pass, hipStream_t st) {
   const bool sawb = a.mode == HOT_SCALE_SAWB, stoch = a.rounding == HOT_ROUND_STOCH;
   if (pass == 0) {
-    per = items_per(M, a.C, a.NB * a.nk);
-    grid.y = (grid.y + per - 1) / per;
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, true>), grid, dim3(BT), 0, st, a, per);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, false>), grid, dim3(BT), 0, st, a, per);
+    a.per = (uint32_t)items_per(M, a.C, a.NB * a.nk);
+    grid.y = (grid.y + a.per - 1) / a.per;
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, true>), grid, dim3(BT), 0, st, a);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 0, 0, false>), grid, dim3(BT), 0, st, a);
   } else if (stoch) {
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, true>), grid, dim3(BT), 0, st, a, per);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, false>), grid, dim3(BT), 0, st, a, per);
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, true>), grid, dim3(BT), 0, st, a);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 1, false>), grid, dim3(BT), 0, st, a);
   } else {
-    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, true>), grid, dim3(BT), 0, st, a, per);
-    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, false>), grid, dim3(BT), 0, st, a, per);
+    if (sawb) hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, true>), grid, dim3(BT), 0, st, a);
+    else hipLaunchKernelGGL((big_stage2_kernel<M, 1, 0, false>), grid, dim3(BT), 0, st, a);
   }
   return check_launch("big_stage2_kernel");
 }
@@ -817,18 +783,8 @@ int hla_big_impl(const void* in, int dtype, int64_t R, int64_t C, int n, const i
       if ((rows[i] & 63) != last_k) { last_k = rows[i] & 63; a.kbase[++kc] = (uint16_t)i; }
     for (int q = kc + 1; q <= 64; ++q) a.kbase[q] = (uint16_t)r;
   } else {
-    // the quantise pass of any other list reads a table of its rows, written piece by piece when it is long
-    if (r <= TAB_ROWS) {
-      TabRows tr;
-      memset(&tr, 0, sizeof(tr));
-      tr.count = r;
-      for (int k = 0; k < r; ++k) tab_row_put(tr.packed, k, rows[k]);
-      hipLaunchKernelGGL(big_prepare_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (int32_t*)(ws + b.off_tab), n, tr);
-      if (int rc = check_launch("big_prepare_kernel")) return rc;
-    } else {
-      hipLaunchKernelGGL(tab_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (int32_t*)(ws + b.off_tab), n);
-      if (int rc = build_row_table((int32_t*)(ws + b.off_tab), n, rows, r, nullptr, st, who)) return rc;
-    }
+    // the quantise pass of any other list reads a table of its rows
+    if (int rc = build_row_table((int32_t*)(ws + b.off_tab), n, rows, r, st)) return rc;
   }
   const dim3 g1((unsigned)gx, (unsigned)(R / 64));
   a.row_absmax = row16_absmax_out;
@@ -894,8 +850,13 @@ int hla_expand_big_impl(const float* t, int64_t nb, int64_t C, int n, const int3
   ExpandBigArgs a;
   a.t = t; a.U = (float*)((uint8_t*)workspace + round_up((int64_t)n * 4, 256)); a.out = out; a.tab = tab; a.C = C;
   a.r = r; a.m = m; a.post = post;
-  hipLaunchKernelGGL(tab_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, tab, n);
-  if (int rc = build_row_table(tab, n, rows, r, nullptr, st, who)) return rc;
+  std::unique_ptr<bool[]> listed(new bool[(size_t)n]());
+  for (int k = 0; k < r; ++k) {
+    if (rows[k] < 0 || rows[k] >= n) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d outside [0, %d)", who, k, rows[k], n);
+    if (listed[(size_t)rows[k]]) return fail(HOT_ERR_INVALID, "%s: rows[%d]=%d listed twice", who, k, rows[k]);
+    listed[(size_t)rows[k]] = true;
+  }
+  if (int rc = build_row_table(tab, n, rows, r, st)) return rc;
   const unsigned gx = (unsigned)((C + BT - 1) / BT);
   hipLaunchKernelGGL(expand_runs_kernel, dim3(gx, (unsigned)(nb * m)), dim3(BT), 0, st, a);
   if (int rc = check_launch("expand_runs_kernel")) return rc;
