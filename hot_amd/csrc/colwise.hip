@@ -14,8 +14,8 @@
 //
 // Data movement.  A workgroup owns 256 adjacent channels (columns) and a run
 // of token blocks.  Rows arrive 16 at a time through coalesced 16-byte loads
-// (each row of the tile is one contiguous segment of HBM), are parked in a
-// double-buffered LDS tile, and every thread then pulls ITS channel's 16
+// (each row of the tile is one contiguous segment of HBM) in a ring of up to
+// four LDS buffers, and every thread then pulls ITS channel's 16
 // values out of LDS: from there on a thread holds whole columns, so the
 // butterflies (stage order h = 1, 2, 4, ..., the canonical fp32 order) need
 // no cross-lane traffic.  Quantised codes are staged in LDS as [channel][k]
@@ -524,7 +524,7 @@ extern "C" int hot_hla_tokenwise_static(const void* in, int dtype, int64_t R, in
                 (long long)C, (long long)STATIC_MAX_C);
   uint8_t* ws = nullptr;
   if (int rc = static_scratch_ptr(&ws, who)) return rc;
-  // (per-channel maxima are cleared by the first kernel of the call, everything else is written before it is read)
+  // (per-channel maxima that runs share are cleared by the first kernel of the call, everything else is written before it is read)
   return colwise_quant_impl(in, dtype, R, C, n, rows, r, bits, rounding, seed, rng_stream, scale_mode, codes_out,
                             ld_out, /*store4=*/0, scales_out, ws, STATIC_SCRATCH_BYTES, (hipStream_t)hip_stream, who);
 }

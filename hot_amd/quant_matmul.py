@@ -197,11 +197,14 @@ _PLAIN_APPLY = hasattr(torch._C, "_are_functorch_transforms_active")
 # the buffer kernels there and makes the current stream wait for them.  One side stream per device,
 # default priority.  Not under stream capture (a capture must not be forked behind its back).
 #
-# It pays only for fp32 products of 2^35 multiply-adds and more.  A product in 16 bits leaves the buffer kernels one workgroup per
+# It is done only for fp32 products of 2^35 multiply-adds and more.  A product in 16 bits leaves the buffer kernels one workgroup per
 # CU (124 KB of LDS), loses what it gives them, and the fork and the join cost the host 30 us; us of a training step of one
 # layer, canonical recipe, tokens x in -> out, beside / in line: bf16 25216 x 3072 -> 768 376 / 359, 8191 x 3072 -> 1024 235 / 203,
 # 12608 x 3072 -> 768 267 / 196, 8192 x 4096 -> 11008 1475 / 1448, 16384 x 4096 -> 4096 1029 / 999, the MLP of 25216 x 768 886 / 873;
-# fp32 16000 x 1024 -> 1024 (2^34) 414 / 390, 12608 x 1024 -> 3072 (2^35.2) 859 / 871.
+# fp32 2^33 and below 8192 x 1024 -> 1024 309 / 282, 12608 x 768 -> 768 266 / 248, 16384 x 512 -> 1024 331 / 305; about 2^34 one or the other,
+# 16000 x 1024 -> 1024 414 / 390, 6304 x 3072 -> 768 368 / 354, 25216 x 768 -> 768 395 / 404; from 2^35 on the two differ by less than runs of
+# one side do, 25216 x 3072 -> 768 1186 / 1238, 12608 x 1024 -> 3072 859 / 871, 25216 x 768 -> 3072 1280 / 1286, 8192 x 2048 -> 2048 760 / 733,
+# 4096 x 4096 -> 4096 1280 / 1248, and beside is kept.
 #
 # overlap_buffer_write: None = that rule; True = beside from OVERLAP_MIN_BYTES of input on, whatever the product; False = in line.
 _FWD = threading.local()

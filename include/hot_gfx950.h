@@ -79,7 +79,7 @@ enum hot_scale_mode {
 /* Counter-based RNG stream identifiers (Philox counter word 2). */
 enum hot_rng_stream { HOT_STREAM_GX = 0, HOT_STREAM_GW = 1, HOT_STREAM_W = 2, HOT_STREAM_ACT = 3 };
 
-#define HOT_HQ_WORKSPACE_BYTES 2048 /* per-tensor absmax of hot_hq_rowwise: 16 partial maxima, one per 128-byte line */
+#define HOT_HQ_WORKSPACE_BYTES 2048 /* per-tensor absmax of hot_hq_rowwise: up to 512 partial maxima */
 #define HOT_MAX_HLA_N 64        /* largest block with its rows inline in hot_config     */
 #define HOT_MAX_HLA_BIG 8192    /* largest block at all (rows through hla_rows_big)     */
 
@@ -250,8 +250,8 @@ HOT_API int hot_abc_forward(const void* x, int dtype, int64_t L, int64_t I, cons
  *               the call synchronise the stream and run its kernels one after the
  *               other on `hip_stream`
  * Without timing the transforms take two launches (statistics, then everything that needs a
- * step), each a grid of independent jobs, behind a clear when g_W has a step per channel, and the
- * two products one.  Products that are faster apart (a g_x of few tiles and a long K, two products
+ * step), each a grid of independent jobs, behind a clear when g_W has a step per channel and the
+ * maxima of its runs of token blocks find no room of their own, and the two products one.  Products that are faster apart (a g_x of few tiles and a long K, two products
  * that fill their rounds of large tiles) follow one another.  With cfg->streams = 2, or by the rule
  * of hot_backward_streams when an operand of 4 GiB or more rules the shared launch out, and a g_W
  * product too small to fill the chip, the g_x product runs on a side stream of the library (one per
